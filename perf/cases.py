@@ -231,6 +231,87 @@ def run(s):
     return {"logits": s["logits"], **act}
 
 
+# ---- the same functions in 64 bits -----------------------------------------------------------------------------------
+def _dequantised(fmt, w, rows, k):
+    """f64 [rows x k] of the raw blocks: Q4_K and Q6_K as GGML lays them out, Q5_K with eight contiguous 12-bit (scale, min)
+    fields and value i's fifth bit in bit i % 8 of byte 144 + i // 8."""
+    b = w.view(rows * (k // 256), SUPER_BLOCK[fmt])
+    half = lambda at: b[:, at:at + 2].contiguous().view(torch.float16).double()
+    if fmt == "q6k":
+        i = torch.arange(256, device=w.device)
+        h, g, l = i // 128, i % 128 // 32, i % 32
+        low = (b[:, 64 * h + l + 32 * (g & 1)] >> (4 * (g >> 1))) & 15
+        high = (b[:, 128 + 32 * h + l] >> (2 * g)) & 3
+        scale = b[:, 192:208].contiguous().view(torch.int8).double()[:, 8 * h + l // 16 + 2 * g]
+        return (half(208) * scale * ((low + 16 * high).double() - 32.0)).view(rows, k)
+    quants = b[:, 16:144].view(-1, 4, 1, 32)
+    q = torch.cat((quants & 15, quants >> 4), 2).reshape(-1, 256).double()
+    f = b[:, 4:16].long()
+    if fmt == "q4k":
+        s = torch.cat((f[:, 0:4] & 63, (f[:, 8:12] & 15) | (f[:, 0:4] >> 6 << 4)), 1)
+        m = torch.cat((f[:, 4:8] & 63, (f[:, 8:12] >> 4) | (f[:, 4:8] >> 6 << 4)), 1)
+    else:
+        even, odd = f[:, 0::3] | (f[:, 1::3] & 15) << 8, f[:, 1::3] >> 4 | f[:, 2::3] << 4
+        fields = torch.stack((even, odd), 2).reshape(-1, 8)
+        s, m = fields & 63, fields >> 6
+        bits = torch.arange(8, device=w.device, dtype=torch.uint8)
+        q += 16.0 * ((b[:, 144:176, None] >> bits) & 1).reshape(-1, 256)
+    spread = lambda v: v.double().repeat_interleave(32, 1)
+    return (half(0) * spread(s) * q - half(2) * spread(m)).view(rows, k)
+
+
+def _exact_product(fmt, w, n, k, a):
+    """f64 a [.. x k] times the matrix, in runs of rows that keep the dequantised part small."""
+    step, size = max(1, (1 << 25) // k), (k // 256) * SUPER_BLOCK[fmt]
+    return torch.cat([a @ _dequantised(fmt, w[r * size:min(r + step, n) * size], min(step, n - r), k).T for r in range(0, n, step)], -1)
+
+
+def _exact_attention(q, k, v):
+    """softmax(q . k / sqrt(dim)) v per head; the heads of a group share a KV head."""
+    group = q.shape[0] // k.shape[0]
+    out = []
+    for h in range(q.shape[0]):
+        p = torch.softmax(k[h // group].double() @ q[h] * q.shape[1] ** -0.5, 0)
+        out.append(p @ v[h // group].double())
+    return torch.stack(out)
+
+
+def _normalised(x, eps, gamma=1.0):
+    return x / torch.sqrt((x * x).mean() + eps) * gamma
+
+
+def exact(case, seed):
+    s, op = prepare(case, seed), case["op"]
+    if op in ("gemv", "gemm"):
+        return _exact_product(case["fmt"], s["w"], case["n"], case["k"], s["x"].double())
+    if op == "gemv_f32":
+        return s["x"].double() @ s["w"].double()
+    if op == "attention":
+        return _exact_attention(s["q"].double(), s["cache_k"][0], s["cache_v"][0])
+    shape = {name: (fmt, n, k) for name, fmt, n, k in _layer_matrices(case)}
+    product = lambda l, name, x: _exact_product(shape[name][0], s["w"][l][name], *shape[name][1:], x)
+    head = lambda x: _exact_product("q6k", s["head_w"], case["vocab"], case["hidden"], x)
+    if op == "list":
+        out = {name: [] for name in shape}
+        for l in range(case["layers"]):
+            x, got = s["x"][l].double(), {}
+            for name in shape:
+                source = {"o": "q", "down": "gate"}.get(name)
+                got[name] = product(l, name, x if source is None else _normalised(got[source], 1e-6))
+                out[name].append(got[name])
+        return {"logits": head(_normalised(out["down"][-1], 1e-6)), **{name: torch.stack(v) for name, v in out.items()}}
+    h, (g1, g2), act = s["embedding"].double(), (g.double() for g in s["gammas"]), {}
+    for l in range(case["layers"]):
+        x = _normalised(h, 1e-5, g1)
+        act.update({name: product(l, name, x) for name in ("q", "k", "v")})
+        act["attention"] = _exact_attention(act["q"].view(case["heads"], case["dim"]), s["cache_k"][l], s["cache_v"][l]).view(-1)
+        act["h1"] = h + product(l, "o", act["attention"])
+        x = _normalised(act["h1"], 1e-5, g2)
+        act.update({name: product(l, name, x) for name in ("gate", "up")})
+        h = act["h"] = act["h1"] + product(l, "down", torch.nn.functional.silu(act["gate"]) * act["up"])
+    return {"logits": head(_normalised(h, 1e-5, g1)), **{name: act.get(name) for name in s["act"]}}      # "o" and "down" go into h1 and h
+
+
 # ---- what a pass cannot do without, and what it may be off by --------------------------------------------------------
 def _product(fmt, m, n, k):
     return n * (k // 256) * SUPER_BLOCK[fmt] + 4 * m * k + 4 * m * n, 2 * m * n * k
