@@ -17,7 +17,9 @@
  * keeps a host pointer after a synchronous call returns.  Device memory for the caller's data comes
  * from trn_mem_alloc only.  Beside it the library keeps scratch of its own, per (device, stream),
  * allocated on first use and freed with the stream: the partial sums and arrival counters of the
- * products that are cut along K (trn_q*k_gemm, trn_gemv_f32, trn_incremental_attention), the tables
+ * products that are cut along K (trn_q*k_gemm, trn_gemv_f32, trn_incremental_attention), the activations of
+ * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB; kept until the stream goes once a captured
+ * graph uses them; while a stream is captured what is there is used and nothing allocated), the tables
  * of a list's launches of more than sixteen entries (trn_kquant_gemv_batch), the tables of the
  * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB per GPU
  * (trn_q4k_gemm_noalloc).  The calls that never allocate: the GEMV launchers, trn_kquant_gemv_batch
@@ -164,7 +166,8 @@ TRN_API trn_status trn_q6k_gemm(trn_stream stream, trn_dptr a, trn_dptr b_quant,
  * image: a static device array of 16 MiB + 64 KiB, of which every GPU the library runs on holds one copy until the
  * process ends.  After the library's first use on the device (any launcher, or trn_ctx_set_current, loads the kernels
  * and looks the buffer's address up once) it calls nothing that allocates or frees.  The product is cut exactly as
- * trn_q4k_gemm would cut it - hence the same bits - and when that cut needs more scratch than the buffer holds the call
+ * trn_q4k_gemm would cut it - hence the same bits; a product of many tokens goes through the buffer in several runs of
+ * them, as trn_q4k_gemm itself does from 256 MiB of scratch on - and when that cut needs more scratch than the buffer holds the call
  * returns TRN_ERROR_SCRATCH_TOO_SMALL and launches nothing; no other failure is reported under that name (every cut that
  * the library chooses by itself needs at most 11.2 MB on 256 CUs; a cut forced with trn_set_tuning may need more; m = 1
  * and unaligned operands take kernels that need no scratch).  All calls on

@@ -396,3 +396,94 @@ def test_gemm_few_tokens_by_the_rule(gpu):
             _tune("gemm_few", 0)
         assert kq.rel_l2(c, _c64("q4k", buf, a, n, k)) <= TOL
         assert np.array_equal(c, other) != taken, (m, n, k)
+
+
+@pytest.mark.parametrize("parts", (0, 1, 3))
+@pytest.mark.parametrize("m,n,k", [(33, 1, 256), (64, 255, 512), (65, 257, 1280), (97, 700, 2304)])
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_many_tokens_kernel(gpu, fmt, m, n, k, parts):
+    """The kernel for many tokens, forced: rows that fill neither a strip of 64 nor a group of 256, tokens that do not fill
+    a tile of 32, one super-block, K in one part, three (of unequal length) and as many as the library takes: within
+    tolerance and the same bits on every run, a token's values large against the others' of its tile, and a run with an
+    infinity not finite - in its own token only."""
+    buf, a = kq.gen_matrix(fmt, 600 + m, n, k), kq.gen_x(610 + m, m, k)
+    a[1] *= np.float32(1e6)
+    a[m - 1] *= np.float32(1e-6)
+    c64 = _c64(fmt, buf, a, n, k)
+    # a single result may cancel: each is held to 1e-5 of the sum of its terms' sizes (about forty roundings of 2^-24 in a
+    # row at worst, the minimum's term on top), a whole token's results to the usual relative L2
+    terms = np.abs(a).astype(np.float64) @ np.abs(kq.dequant_matrix(fmt, buf, n, k)).astype(np.float64).T
+    try:
+        _tune("gemm_tall", 2)
+        _tune("gemm_k_parts", parts)
+        c = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert np.all(np.abs(c - c64) <= TOL * terms)
+        for row in (slice(0, 1), slice(1, 2), slice(2, m - 1), slice(m - 1, m)):
+            assert n < 255 or kq.rel_l2(c[row], c64[row]) <= TOL
+        again = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert np.array_equal(again.view(np.uint32), c.view(np.uint32))
+        a[3, 7] = np.inf
+        c = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert not np.any(np.isfinite(c[3])) and np.all(np.isfinite(np.delete(c, 3, axis=0)))
+        assert np.array_equal(np.delete(c, 3, axis=0), np.delete(again, 3, axis=0))
+    finally:
+        _tune("gemm_tall", 0)
+        _tune("gemm_k_parts", 0)
+
+
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_many_tokens_no_less_exact_than_sixteen_at_a_time(gpu, fmt):
+    """The rule's own choice for 200 tokens against 8192 x 2048, and the kernel that takes sixteen at a time: the error
+    against fp64 is no larger (bound 1.02: what the seeds' scatter moves the ratio by)."""
+    m, n, k = 200, 8192, 2048
+    buf, a = kq.gen_matrix(fmt, 640, n, k), kq.gen_x(641, m, k)
+    c64 = _c64(fmt, buf, a, n, k)
+    err = {}
+    try:
+        for name, value in (("rule", 0), ("tall", 2), ("sixteen", 1)):
+            _tune("gemm_tall", value)
+            err[name] = kq.rel_l2(gpu_gemm(gpu, fmt, buf, a, m, n, k), c64)
+    finally:
+        _tune("gemm_tall", 0)
+    assert err["rule"] == err["tall"] != err["sixteen"]
+    assert err["tall"] <= 1.02 * err["sixteen"]
+
+
+def test_gemm_many_tokens_under_capture_and_without_allocation(gpu):
+    """Twice the same bits through a captured graph after a larger product has grown the workspace, and from
+    trn_q4k_gemm_noalloc, whose buffer takes the tokens in several runs."""
+    import ctypes as C
+    from trueno_amd import _ffi
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = [C.c_void_p]
+    hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    ctx, stream = gpu
+    m, n, k = 700, 4096, 8192
+    buf, a = kq.gen_matrix("q4k", 650, n, k), kq.gen_x(651, m, k)
+    want = gpu_gemm(gpu, "q4k", buf, a, m, n, k)
+    dw, da = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, a)
+    dc = t.GpuBuffer.from_host(ctx, np.full(m * n, np.nan, np.float32))
+    assert _ffi.lib().trn_q4k_gemm_noalloc(stream.raw(), da.as_ptr(), dw.as_ptr(), dc.as_ptr(), m, n, k) == 0
+    stream.synchronize()
+    assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), want.view(np.uint32))
+    graph, gexec = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream.raw(), 0) == 0
+    t.QuantizeKernel.ggml(m, n, k).launch(stream, da, dw, dc)
+    assert hip.hipStreamEndCapture(stream.raw(), C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(gexec), graph, None, None, 0) == 0
+    try:
+        gpu_gemm(gpu, "q4k", buf, np.concatenate((a, a)), 2 * m, n, k)      # grows the workspace: the graph's stays
+        for _ in range(3):
+            dc.copy_from_host(np.full(m * n, np.nan, np.float32))
+            assert hip.hipGraphLaunch(gexec, stream.raw()) == 0
+            stream.synchronize()
+            assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), want.view(np.uint32))
+            again = gpu_gemm(gpu, "q4k", buf, a, m, n, k)
+            assert np.array_equal(again.view(np.uint32), want.view(np.uint32))
+    finally:
+        hip.hipGraphExecDestroy(gexec)
+        hip.hipGraphDestroy(graph)

@@ -13,6 +13,7 @@
 #endif
 #include "kquant_chain.hip.h"
 #include "kquant_gemm_f16.hip.h"
+#include "kquant_gemm_tall.hip.h"
 #include "kquant_few_i8.hip.h"
 #include "decode_glue.hip.h"
 #include "gemv_f32.hip.h"
@@ -344,6 +345,26 @@ KQ_GEMM_F16(q4k_gemm_f16_w8t2, 512, kq_body<FMT_Q4K KQ_COMMA 8 KQ_COMMA 2>)
 KQ_GEMM_F16(q5k_gemm_f16_w8t2, 512, kq_body<FMT_Q5K KQ_COMMA 8 KQ_COMMA 2>)
 KQ_GEMM_F16(q6k_gemm_f16_w8, 512, q6k_body<1>)
 KQ_GEMM_F16(q6k_gemm_f16_w4, 256, q6k_body<2>)
+
+// Many tokens (kquant_gemm_tall.hip.h): the activations as operands, the product, the sum over the parts of K.
+extern "C" __global__ void __launch_bounds__(256) kq_tall_operands(const float* a, uint8_t* ops, u32 m, u32 nsb) {
+  gemm_tall::convert_body(a, ops, m, nsb);
+}
+extern "C" __global__ void __launch_bounds__(256) kq_tall_sum(float* c, const float* parts, uint64_t mn, u32 kparts) {
+  gemm_tall::sum_parts_body(c, parts, mn, kparts);
+}
+#define KQ_GEMM_TALL(name, BODY)                                                                                        \
+  extern "C" __global__ void __launch_bounds__(256, 2)                                                                   \
+  name(const uint8_t* ops, const uint8_t* w, float* c, u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups,           \
+       u32 tiles, u32 run) {                                                                                           \
+    extern __shared__ uint8_t tall_lds[];                                                                                \
+    const u32 lds_base =                                                                                                 \
+        static_cast<u32>(reinterpret_cast<size_t>((const __attribute__((address_space(3))) uint8_t*)tall_lds));         \
+    gemm_tall::BODY(ops, w, c, m, n, nsb, ksb, kparts, groups, tiles, run, lds_base);                                  \
+  }
+KQ_GEMM_TALL(q4k_gemm_tall, body<FMT_Q4K>)
+KQ_GEMM_TALL(q5k_gemm_tall, body<FMT_Q5K>)
+KQ_GEMM_TALL(q6k_gemm_tall, q6k_body)
 
 // Q4_K product for two to four tokens on the integer matrix cores (kquant_few_i8.hip.h): workgroup b takes the rows
 // b * rows_per_wg .. of W, k <= 4096.

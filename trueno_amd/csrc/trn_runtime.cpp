@@ -86,6 +86,8 @@ struct DeviceKernels {
   hipFunction_t gemm_f16[NFMT][2] = {};   // [format][4 or 8 strips per workgroup]
   hipFunction_t gemm_f16_w12 = nullptr;   // Q4_K: 12 strips per workgroup
   hipFunction_t gemm_f16_t2[2] = {};      // Q4_K, Q5_K: 8 strips and two token tiles per workgroup
+  hipFunction_t gemm_tall[NFMT] = {};     // many tokens
+  hipFunction_t tall_operands = nullptr, tall_sum = nullptr;
   hipFunction_t gemm_few[2] = {};         // Q4_K, integer matrix cores, built for 2 and 4 tokens
   hipFunction_t gemm_simplified = nullptr, dequant_simplified = nullptr;
 };
@@ -121,6 +123,7 @@ std::atomic<int> g_tune_group_stream_min_rows{0};  // an entry of a launch of up
 std::atomic<int> g_tune_many_item_kb{0};    // what a further piece of work costs a workgroup of such a launch, in KB of weights (0: default)
 std::atomic<int> g_tune_many_slab_weight{0};  // percent such a launch adds to an entry's bytes per slab of 4096 columns beyond the first (0: default)
 std::atomic<int> g_tune_stream_waves{0};    // waves per workgroup of a single streamed GEMV (0: default)
+std::atomic<int> g_tune_gemm_tall{0};       // the kernel for many tokens: 0 by the rule, 1 never, 2 wherever it can run (from 33 tokens on)
 std::atomic<int> g_tune_gemm_few{0};        // the integer matrix-core kernel for two to four tokens: 0 by the rule, 1 wherever it can run, 2 never
 
 inline trn_status st(hipError_t e) { return static_cast<trn_status>(e); }
@@ -186,6 +189,11 @@ hipError_t device_kernels(DeviceKernels** out) {
         (e = get_fn(m, &t.gemm_f16_t2[1], "q5k_gemm_f16_w8t2")) != hipSuccess ||
         (e = get_fn(m, &t.gemm_f16[2][0], "q6k_gemm_f16_w4")) != hipSuccess ||
         (e = get_fn(m, &t.gemm_f16[2][1], "q6k_gemm_f16_w8")) != hipSuccess ||
+        (e = get_fn(m, &t.tall_operands, "kq_tall_operands")) != hipSuccess ||
+        (e = get_fn(m, &t.tall_sum, "kq_tall_sum")) != hipSuccess ||
+        (e = get_fn(m, &t.gemm_tall[0], "q4k_gemm_tall")) != hipSuccess ||
+        (e = get_fn(m, &t.gemm_tall[1], "q5k_gemm_tall")) != hipSuccess ||
+        (e = get_fn(m, &t.gemm_tall[2], "q6k_gemm_tall")) != hipSuccess ||
         (e = get_fn(m, &t.gemm_few[0], "q4k_gemm_few_t2")) != hipSuccess ||
         (e = get_fn(m, &t.gemm_few[1], "q4k_gemm_few_t4")) != hipSuccess ||
         (e = get_fn(m, &t.fill_u32, "kq_fill_u32")) != hipSuccess) {
@@ -589,16 +597,155 @@ hipError_t launch_gemm_few(DeviceKernels* d, hipStream_t stream, uint64_t a, uin
   return hipModuleLaunchKernel(d->gemm_few[idx], grid, 1, 1, 512, 1, 1, lds, stream, args, nullptr);
 }
 
+// ---- many tokens (kquant_gemm_tall.hip.h) -----------------------------------------------------------------------------
+constexpr uint32_t kTallRows = 256, kTallTile = 32, kTallOperandBytes = 32u * 1024u + 2048u;      // rows and tokens of a workgroup; of a (tile, super-block)
+constexpr size_t kTallWorkspaceMax = size_t(256) << 20;      // products that need more go through it in runs of tokens
+constexpr size_t kTallWorkspaceLeast = size_t(16) << 20;     // every cut works within this much (trn_q4k_gemm_noalloc has no more)
+struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit; };
+uint32_t tall_lds_bytes(Fmt f) { return (f == Q6K ? 2u : 4u) * 8192u + 2u * 2048u + 4u * 64u * (f == Q6K ? 224u : kSbBytes[f]); }
+size_t tall_bytes(uint32_t tokens, uint32_t n, uint32_t nsb, uint32_t kparts) {
+  const size_t tiles = (tokens + kTallTile - 1u) / kTallTile;
+  return tiles * nsb * kTallOperandBytes + (kparts > 1u ? (size_t(kparts) * tokens * n * 4u + 255u) / 256u * 256u : 0u);
+}
+// The parts of K with the least estimated time.  Times in microseconds fitted to measurements on MI355X (1024 x 4096 ..
+// 32000 x 4096 and 4096 x 11008, 33 .. 1024 tokens, within about 10 % from 64 tokens on): 9 for the launches and the first
+// super-block; the operands at 4 TB/s; a super-block takes a round of two workgroups per CU 4.3 / 5.1 / 7.5 (Q4_K / Q5_K /
+// Q6_K), one workgroup alone on its CU 2.3 / 2.7 / 4.2; with K in parts 3 for the sum's launch, 0.4 a part, and the parts'
+// bytes at 4 TB/s.
+TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k) {
+  TallCut best;
+  const uint32_t nsb = k / 256u, groups = (n + kTallRows - 1u) / kTallRows, tiles = (m + kTallTile - 1u) / kTallTile, cus = uint32_t(d.cu_count);
+  const uint64_t units = uint64_t(groups) * tiles;
+  const double pair = f == Q4K ? 4.3 : f == Q5K ? 5.1 : 7.5, alone = f == Q4K ? 2.3 : f == Q5K ? 2.7 : 4.2;
+  const uint32_t most = g_tune_gemm_ksplit > 0 ? std::min<uint32_t>(uint32_t(g_tune_gemm_ksplit), nsb)
+                                               : uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>((2u * cus + units / 2u) / units, nsb)));
+  for (uint32_t kp = most; kp >= 1u; --kp) {
+    TallCut c;
+    c.ksb = (nsb + kp - 1u) / kp;
+    c.kparts = (nsb + c.ksb - 1u) / c.ksb;
+    if (tall_bytes(kTallTile, n, nsb, c.kparts) > kTallWorkspaceLeast) continue;
+    const uint64_t wgs = units * c.kparts, rounds = wgs / (2u * cus), rest = wgs - rounds * 2u * cus;
+    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * double(rest - cus) / cus;
+    c.us = 9.0 + double(m) * k * 8.0 / 4.0e6 + c.ksb * (double(rounds) * pair + last) +
+           (c.kparts > 1u ? 3.0 + 0.4 * c.kparts + double(c.kparts + 1u) * m * n * 4.0 / 4.0e6 : 0.0);
+    if (c.us < best.us) best = c;
+    if (g_tune_gemm_ksplit > 0) break;
+  }
+  return best;
+}
+
+// One buffer per (device, stream): the operands, then the parts of K.  A product is two or three launches that share it, so
+// a lock is held from the first to the last: another thread's product on the same stream may not come between them.  A
+// buffer whose address a captured graph holds stays until the stream goes; while a stream is captured nothing is allocated.
+struct TallWorkspace {
+  void* buf = nullptr;
+  size_t cap = 0;
+  bool captured = false;
+  std::vector<void*> retired;
+};
+std::map<std::pair<int, hipStream_t>, TallWorkspace> g_tall_ws;
+std::mutex g_tall_mutex;
+
+hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
+                            uint32_t k, const TallCut& cut, uint64_t ws) {
+  uint32_t nsb = k / 256u, tiles = (m + kTallTile - 1u) / kTallTile, kparts = cut.kparts, ksb = cut.ksb;
+  uint32_t groups = (n + kTallRows - 1u) / kTallRows;
+  uint32_t run = 1u;      // super-blocks summed by themselves: about the root of a part's
+  while (run * run < ksb) ++run;
+  uint64_t ops = ws, parts = kparts > 1u ? ws + size_t(tiles) * nsb * kTallOperandBytes : c, mn = uint64_t(m) * n;
+  void* oargs[] = {&a, &ops, &m, &nsb};
+  hipError_t e = hipModuleLaunchKernel(d->tall_operands, tiles * nsb, 1, 1, 256, 1, 1, 0, stream, oargs, nullptr);
+  if (e != hipSuccess) return e;
+  void* margs[] = {&ops, &w, &parts, &m, &n, &nsb, &ksb, &kparts, &groups, &tiles, &run};
+  const uint32_t grid = (groups * tiles * kparts + 7u) / 8u * 8u;
+  if ((e = hipModuleLaunchKernel(d->gemm_tall[f], grid, 1, 1, 256, 1, 1, tall_lds_bytes(f), stream, margs, nullptr)) != hipSuccess) return e;
+  if (kparts == 1u) return hipSuccess;
+  void* sargs[] = {&c, &parts, &mn, &kparts};
+  const uint32_t sgrid = uint32_t(std::min<uint64_t>((mn + 255u) / 256u, uint64_t(d->cu_count) * 8u));
+  return hipModuleLaunchKernel(d->tall_sum, sgrid, 1, 1, 256, 1, 1, 0, stream, sargs, nullptr);
+}
+
+// The product through `cap` bytes of workspace, in runs of as many token tiles as it holds (a tile's bits do not depend on
+// its company).  g_tall_mutex held.
+hipError_t launch_tall(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n, uint32_t k,
+                       const TallCut& cut, uint64_t ws, size_t cap) {
+  const uint32_t nsb = k / 256u;
+  uint32_t step = m;
+  if (tall_bytes(m, n, nsb, cut.kparts) > cap) {
+    step = uint32_t(std::min<size_t>(cap / tall_bytes(kTallTile, n, nsb, cut.kparts), m / kTallTile)) * kTallTile;
+    if (step == 0u) return hipErrorInvalidValue;
+  }
+  for (uint32_t t = 0; t < m; t += step) {
+    const uint32_t len = std::min(step, m - t);
+    const hipError_t e = launch_tall_once(d, f, stream, a + uint64_t(t) * k * 4u, w, c + uint64_t(t) * n * 4u, len, n, k, cut, ws);
+    if (e != hipSuccess) return e;
+    if (m - t <= step) break;
+  }
+  return hipSuccess;
+}
+
+// *done = false: the stream is being captured and its workspace is too small (the caller takes another kernel)
+hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
+                                 uint32_t k, bool* done) {
+  *done = false;
+  const TallCut cut = tall_cut(*d, f, m, n, k);
+  const size_t need = std::min(tall_bytes(m, n, k / 256u, cut.kparts), kTallWorkspaceMax);
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_tall_mutex);
+  TallWorkspace& ws = g_tall_ws[std::make_pair(dev, stream)];
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if ((e = hipStreamIsCapturing(stream, &capture)) != hipSuccess) return e;
+  if (capture != hipStreamCaptureStatusNone) {
+    if (ws.cap < tall_bytes(kTallTile, n, k / 256u, cut.kparts)) return hipSuccess;
+    ws.captured = true;
+  } else if (ws.cap < need) {
+    if (ws.buf) {
+      if (ws.captured) {
+        ws.retired.push_back(ws.buf);
+      } else {
+        if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
+        (void)hipFree(ws.buf);
+      }
+      ws.buf = nullptr;
+      ws.cap = 0;
+      ws.captured = false;
+    }
+    if ((e = hipMalloc(&ws.buf, need)) != hipSuccess) return e;
+    ws.cap = need;
+  }
+  *done = true;
+  return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.buf), ws.cap);
+}
+
 constexpr double kBigAloneBytes = 64e6;      // from this size on a matrix alone takes the list kernel (launch_gemm_like, trn_kquant_gemv_batch)
 bool list_groupable(DeviceKernels* dk, const trn_gemv_desc& d);
 extern "C" {      // (defined further down inside the extern "C" part of the file: the same language linkage here)
 hipError_t launch_gemv_group(DeviceKernels* d, hipStream_t stream, const trn_gemv_desc* descs, uint32_t len);
 }
 
+// Does the kernel for many tokens take this product?  From 33 tokens on, where its estimate is
+// below the other's: that one holds for Q4_K, while Q5_K takes 1.1 and Q6_K 1.3 to 1.6 times as long from 64 tokens on (the
+// factors below stay at the lower end).  Up to 32 tokens, one tile, it gained nothing anywhere (Q5_K 11008 x 4096, 17
+// tokens: 28 against 23 us).  Both sides measured over nine shapes, 17 .. 1024 tokens (us, sixteen at a time -> this kernel):
+//   14336 x 4096, 2048 tokens, Q4_K 835 -> 525;   11008 x 4096, 512 tokens: Q4_K 180 -> 126, Q5_K 190 -> 142, Q6_K 318 -> 201
+//   4096 x 11008, 512 tokens: Q4_K 159 -> 129, Q5_K 167 -> 150, Q6_K 288 -> 195;   32000 x 4096, 64 tokens: 60 -> 55, 68 -> 63, 110 -> 84
+//   4096 x 4096, 64 tokens: 16 and 21 (Q4_K), 20 and 26 (Q6_K): stays;   1024 x 4096, 512 tokens, Q4_K: 24 and 29: stays
+bool tall_ok(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k, bool forced) {
+  if (g_tune_gemm_tall == 1 || m <= 32u || k / 256u > 0x3FFFu || uint64_t((n + kTallRows - 1u) / kTallRows) * ((m + kTallTile - 1u) / kTallTile) > 0xFFFFFu)
+    return false;
+  const double us = tall_cut(d, f, m, n, k).us;
+  if (g_tune_gemm_tall == 2) return us < kCutDoesNotFit;
+  if (forced) return false;
+  return us < gemm_cut(d, f, m, n, k).us * (f == Q4K ? 1.0 : f == Q5K ? (m < 64u ? 1.05 : 1.1) : (m < 64u ? 1.1 : 1.3));
+}
+
 // Which kernel takes a product of m >= 1 tokens: the integer matrix cores (Q4_K, two to four tokens, where their fitted
-// time is below the other ways'), the f16 matrix cores, or the GEMV engine with a pass per token (also: whatever the
+// time is below the other ways'), the f16 matrix cores - the kernel for many tokens where its fitted time is below that of
+// the one that takes sixteen at a time -, or the GEMV engine with a pass per token (also: whatever the
 // matrix-core forms cannot take).  A forced cut of the f16 form (tuning) takes that form.
-enum class GemmRoute { kFew, kCores, kOther };
+enum class GemmRoute { kFew, kCores, kTall, kOther };
 GemmRoute gemm_route(const DeviceKernels& d, Fmt f, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n, uint32_t k) {
   const bool cores_ok = q4k_gemm_f16_ok(a, w, c, m, n, k, f);
   const bool forced = g_tune_gemm_ksplit > 0 || g_tune_gemm_waves > 0 || g_tune_gemm_tiles > 0;
@@ -608,6 +755,7 @@ GemmRoute gemm_route(const DeviceKernels& d, Fmt f, uint64_t a, uint64_t w, uint
     const double cores = !cores_ok ? 1e30 : gemm_cut(d, f, m, n, k).waves == 4u ? 7.2 + mb / 4.0 : 12.0 + mb / 9.4;
     if (g_tune_gemm_few == 1 || gemm_few_us(d, m, n) < std::min(engine, cores)) return GemmRoute::kFew;
   }
+  if (cores_ok && tall_ok(d, f, m, n, k, forced)) return GemmRoute::kTall;
   if (cores_ok && (forced || !gemm_few_tokens_by_engine(d, f, m, n, k))) return GemmRoute::kCores;
   return GemmRoute::kOther;
 }
@@ -623,7 +771,12 @@ hipError_t launch_gemm_like(Fmt f, hipStream_t stream, uint64_t a, uint64_t w, u
   if (!is_gemv) {
     const GemmRoute route = gemm_route(*d, f, a, w, c, m, n, k);
     if (route == GemmRoute::kFew) return launch_gemm_few(d, stream, a, w, c, m, n, k);
-    if (route == GemmRoute::kCores) return launch_kq_gemm_f16(d, f, stream, a, w, c, m, n, k);
+    if (route == GemmRoute::kTall) {
+      bool done = false;
+      e = launch_tall_on_stream(d, f, stream, a, w, c, m, n, k, &done);
+      if (done || e != hipSuccess) return e;
+    }
+    if (route != GemmRoute::kOther) return launch_kq_gemm_f16(d, f, stream, a, w, c, m, n, k);
   }
   const uint32_t grid_y = std::min<uint32_t>(m, 65535u);
   // GEMV parameter order is (y, w, x, k, n); GEMM is (a, b_quant, c, m, n, k)
@@ -1276,6 +1429,18 @@ void release_list_plans(hipStream_t stream);      // the cached plans of trn_kqu
 // The per-(device, stream) scratch buffers of a stream that is going away (partial sums, arrival counters, the
 // resident executor's tables).  The stream must be idle.
 static void release_stream_workspaces(hipStream_t stream) {
+  {
+    std::lock_guard<std::mutex> lock(g_tall_mutex);
+    for (auto it = g_tall_ws.begin(); it != g_tall_ws.end();) {
+      if (it->first.second == stream) {
+        if (it->second.buf) (void)hipFree(it->second.buf);
+        for (void* p : it->second.retired) (void)hipFree(p);
+        it = g_tall_ws.erase(it);
+      } else {
+        ++it;
+      }
+    }
+  }
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   auto drop_simple = [&](auto& map) {
     for (auto it = map.begin(); it != map.end();) {
@@ -1914,13 +2079,18 @@ trn_status trn_q4k_gemm_noalloc(trn_stream s, trn_dptr a, trn_dptr b, trn_dptr c
   hipStream_t stream = static_cast<hipStream_t>(s);
   DeviceKernels* d = nullptr;
   TRN_TRY(device_kernels(&d));
-  // the same choice of kernel as trn_q4k_gemm, so the same bits: only the f16 matrix-core form needs scratch at all
-  if (gemm_route(*d, Q4K, a, b, c, m, n, k) != GemmRoute::kCores) return st(launch_gemm_like(Q4K, stream, a, b, c, m, n, k, false));
+  // the same choice of kernel as trn_q4k_gemm, so the same bits: only the f16 matrix-core forms need scratch at all
+  const GemmRoute route = gemm_route(*d, Q4K, a, b, c, m, n, k);
+  if (route != GemmRoute::kCores && route != GemmRoute::kTall) return st(launch_gemm_like(Q4K, stream, a, b, c, m, n, k, false));
   int dev = 0;
   TRN_TRY(hipGetDevice(&dev));
   size_t cap = 0;
   const uint64_t base = trn_noalloc_scratch(dev, &cap);
   if (!base) return TRN_ERROR_INVALID_VALUE;
+  if (route == GemmRoute::kTall) {      // behind the counters, which stay as they are; every cut fits, in runs of tokens if need be
+    std::lock_guard<std::mutex> lock(g_tall_mutex);
+    return st(launch_tall(d, Q4K, stream, a, b, c, m, n, k, tall_cut(*d, Q4K, m, n, k), base + kGemmCounterBytes, cap - kGemmCounterBytes));
+  }
   // the cut trn_q4k_gemm would take (so the bits are its bits): refused by name when its partial sums do not fit
   const GemmCut cut = gemm_cut(*d, Q4K, m, n, k);
   const size_t part_bytes = gemm_part_bytes(cut.kparts, (m + 15u) / 16u, cut.groups, cut.waves);
@@ -2047,6 +2217,7 @@ trn_status trn_set_tuning(const char* key, int value) {
   if (!std::strcmp(key, "gemv_stream_q6k")) { g_tune_stream_q6k = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_cost")) { g_tune_stream_cost = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_min_rows")) { g_tune_stream_min_rows = value; return TRN_SUCCESS; }
+  if (!std::strcmp(key, "gemm_tall")) { if (value > 2) return TRN_ERROR_INVALID_VALUE; g_tune_gemm_tall = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_few")) { g_tune_gemm_few = value; return TRN_SUCCESS; }
   return TRN_ERROR_INVALID_VALUE;
 }
