@@ -95,3 +95,37 @@ def test_gpu_attention_by_name_extremes_and_bad_arguments(gpu):
     assert L.trn_incremental_attention(stream.raw(), *args, seq, 512, heads, heads, max_seq, 0.125) != 0
     assert L.trn_incremental_attention(stream.raw(), *args, seq, dim, heads, heads + 1, max_seq, 0.125) != 0
     assert L.trn_incremental_attention(stream.raw(), 0, dk.as_ptr(), dv.as_ptr(), do.as_ptr(), seq, dim, heads, heads, max_seq, 0.125) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", (64, 128))
+@pytest.mark.parametrize("heads,kv_heads,max_seq,seq", [(1, 1, 5, 1), (4, 4, 40, 16), (8, 2, 40, 17), (24, 2, 300, 129), (16, 16, 600, 513),
+                                                        (32, 4, 5000, 4097), (6, 4, 64, 63)])
+def test_gpu_attention_heads_of_a_kv_head_together(gpu, heads, kv_heads, max_seq, seq, dim):
+    """The matrix-core form (head dimension 64 or 128): one position, one tile of 16 and one more, twelve query heads of a KV
+    head (two groups), chunks of unequal length, a last tile that is not full; and head counts that do not divide (the
+    other kernel).  An infinite value at the last position makes its dim infinite and nothing else."""
+    ctx, stream = gpu
+    q, k, v = _case(heads * 100 + seq + dim, heads, kv_heads, max_seq, dim, spread=2.0)
+    k[:, seq:], v[:, seq:] = np.nan, np.nan                         # what lies behind the positions is not read into the result
+    dq, dk, dv = (t.GpuBuffer.from_host(ctx, a.reshape(-1)) for a in (q, k, v))
+    kern = t.IncrementalAttentionKernel.with_gqa(max_seq, dim, heads, kv_heads)
+
+    def run(dv):
+        do = t.GpuBuffer.from_host(ctx, np.full(heads * dim, np.nan, np.float32))
+        kern.launch(stream, dq, dk, dv, do, seq)
+        stream.synchronize()
+        return do.copy_to_host().reshape(heads, dim)
+
+    L = t._ffi.lib()
+    assert L.trn_set_tuning(b"attention_tiled", 2) == 0             # also where a head alone would take the other kernel
+    try:
+        got, want = run(dv), glue.attention_fp64(q, k[:, :seq], v[:, :seq], seq)
+        again = run(dv)
+        v[:, seq - 1, 3] = np.inf
+        got_inf = run(t.GpuBuffer.from_host(ctx, v.reshape(-1)))
+    finally:
+        L.trn_set_tuning(b"attention_tiled", 0)
+    assert kq.rel_l2(got, want) <= 2e-6       # f32: a score's error (about 3e-7 of 2 sigma) is its weight's, the sums add less
+    assert np.array_equal(again.view(np.uint32), got.view(np.uint32))
+    assert np.all(np.delete(got_inf, 3, axis=1) == np.delete(got, 3, axis=1)) and not np.any(np.isfinite(got_inf[:, 3]))

@@ -83,6 +83,7 @@ struct DeviceKernels {
   hipFunction_t copy_u128 = nullptr, read_u128 = nullptr;
   hipFunction_t residual_add = nullptr, swiglu = nullptr, rmsnorm = nullptr, residual_rmsnorm = nullptr;
   hipFunction_t gemv_f32_fast = nullptr, gemv_f32_generic = nullptr, q5k_from_ggml = nullptr, attention = nullptr;
+  hipFunction_t attention_tiled[2] = {};  // head dimension 64, 128
   hipFunction_t gemm_f16[NFMT][2] = {};   // [format][4 or 8 strips per workgroup]
   hipFunction_t gemm_f16_w12 = nullptr;   // Q4_K: 12 strips per workgroup
   hipFunction_t gemm_f16_t2[2] = {};      // Q4_K, Q5_K: 8 strips and two token tiles per workgroup
@@ -112,6 +113,7 @@ std::atomic<int> g_tune_group_window{0};       // entries of a list a launch may
 std::atomic<int> g_tune_group_waves{0};        // least waves per workgroup of a launch of up to sixteen entries (0: 8, or what the widest entry needs)
 std::atomic<int> g_tune_group_max{0};          // most entries in one launch (0: as many as the list offers, up to kManyMax)
 std::atomic<int> g_tune_slab_weight{0};        // percent a launch adds to an entry's bytes per slab of 4096 columns beyond the first (0: 40)
+std::atomic<int> g_tune_attention_tiled{0};    // the matrix-core form of the single-query attention: 0 by the rule, 1 never, 2 wherever it can run
 std::atomic<int> g_tune_attention_per_cu{0};   // workgroups per CU the single-query attention aims at (0: default)
 std::atomic<int> g_tune_gemm_waves{0};      // strips of 32 rows per workgroup of the matrix-core GEMM: 4, 8 or (Q4_K) 12 (0: default)
 std::atomic<int> g_tune_stream_off{0};      // 1: one-slab GEMVs load their rows into registers straight from memory (no LDS ring)
@@ -170,6 +172,8 @@ hipError_t device_kernels(DeviceKernels** out) {
         (e = get_fn(m, &t.gemv_f32_fast, "gemv_f32_fast")) != hipSuccess ||
         (e = get_fn(m, &t.q5k_from_ggml, "q5k_from_ggml")) != hipSuccess ||
         (e = get_fn(m, &t.attention, "incremental_attention")) != hipSuccess ||
+        (e = get_fn(m, &t.attention_tiled[0], "kq_attention_tiled_64")) != hipSuccess ||
+        (e = get_fn(m, &t.attention_tiled[1], "kq_attention_tiled_128")) != hipSuccess ||
         (e = get_fn(m, &t.gemv_f32_generic, "gemv_coalesced")) != hipSuccess ||
         (e = get_fn(m, &t.residual_add, "residual_add")) != hipSuccess ||
         (e = get_fn(m, &t.swiglu, "fused_swiglu")) != hipSuccess ||
@@ -413,6 +417,25 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
   DeviceKernels* d = nullptr;
   hipError_t e = device_kernels(&d);
   if (e != hipSuccess) return e;
+  if ((head_dim == 64u || head_dim == 128u) && num_heads % num_kv_heads == 0u && g_tune_attention_tiled != 1 &&
+      (num_heads > num_kv_heads || head_dim == 64u || seq_len >= 4096u || g_tune_attention_tiled == 2)) {
+    // the query heads of a KV head together, in tiles of 16 positions (both sides measured: decode_attention.hip.h; a
+    // head alone with 128 dims only with many positions: 32 heads, 2048 positions 16.7 against 16.1 us, 8192 43.3 against 45.5): a
+    // workgroup per CU (two are slower at every length, 28.8 against 18.7 us with 8 KV heads and 8192 positions), at least a tile a wave
+    const uint32_t waves = head_dim == 64u ? 8u : 4u, most_heads = 8u, step = 16u * waves;
+    uint32_t per_kv = num_heads / num_kv_heads, subs = (per_kv + most_heads - 1u) / most_heads, groups = num_kv_heads * subs;
+    const uint32_t per_cu = g_tune_attention_per_cu > 0 ? uint32_t(g_tune_attention_per_cu) : 1u;
+    uint32_t chunks = std::max(1u, per_cu * uint32_t(d->cu_count) / groups);
+    uint32_t chunk = (seq_len + chunks - 1u) / chunks;
+    chunk = (chunk + step - 1u) / step * step;
+    chunks = (seq_len + chunk - 1u) / chunk;
+    const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (chunks > 1u ? size_t(groups) * chunks * most_heads * (head_dim / 4u + 1u) * 16u : 0u);
+    uint64_t cnt = 0;
+    if ((e = acquire_scratch(g_attention_ws, d, stream, need, cnt_cap, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
+    uint64_t part = cnt + cnt_cap;
+    void* args[] = {&q, &k, &v, &out, &seq_len, &per_kv, &subs, &max_seq_len, &scale, &chunk, &chunks, &groups, &part, &cnt};
+    return hipModuleLaunchKernel(d->attention_tiled[head_dim == 128u], groups * chunks, 1, 1, 64u * waves, 1, 1, 0, stream, args, nullptr);
+  }
   uint32_t lpp_log2 = 0;
   while ((4u << lpp_log2) < head_dim) ++lpp_log2;
   const uint32_t lpp = 1u << lpp_log2, step = 4u * (64u >> lpp_log2);       // positions a workgroup takes at a time
@@ -2207,6 +2230,7 @@ trn_status trn_set_tuning(const char* key, int value) {
   if (!std::strcmp(key, "group_waves")) { g_tune_group_waves = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "group_slab_weight")) { g_tune_slab_weight = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "attention_per_cu")) { g_tune_attention_per_cu = value; return TRN_SUCCESS; }
+  if (!std::strcmp(key, "attention_tiled")) { g_tune_attention_tiled = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "attention_min_steps")) { g_tune_attention_min_steps = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_off")) { g_tune_stream_off = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_waves")) { g_tune_stream_waves = value; return TRN_SUCCESS; }
