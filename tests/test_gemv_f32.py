@@ -78,3 +78,27 @@ def test_gpu_gemv_f32_by_name_and_edges(gpu):
     stream.synchronize()
     assert np.all(dy.copy_to_host() == 0.0)
     assert L.trn_gemv_f32(stream.raw(), 0, da.as_ptr(), dx.as_ptr(), k, n) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,n", [(9, 260), (63, 260), (65, 260), (71, 516), (129, 260), (1003, 43008), (520, 33028)])
+def test_gpu_gemv_f32_last_rows_and_wide_matrices(gpu, k, n):
+    """Rows that do not fill a wave's last eight, and matrices wide enough for two workgroups per CU; an infinity in the
+    last row, which stands in for the rows behind it, makes its own column infinite and no other."""
+    ctx, stream = gpu
+    rng = np.random.default_rng(k * 37 + n)
+    a, x = rng.standard_normal((k, n)).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    want = a.astype(np.float64).T @ x.astype(np.float64)
+
+    def run(a):
+        da, dx = t.GpuBuffer.from_host(ctx, a.reshape(-1)), t.GpuBuffer.from_host(ctx, x)
+        dy = t.GpuBuffer.from_host(ctx, np.full(n, np.nan, np.float32))
+        t.CoalescedGemvKernel(k, n).launch(stream, dy, da, dx)
+        stream.synchronize()
+        return dy.copy_to_host()
+
+    got = run(a)
+    assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)      # f32: about twenty roundings of 2^-24 in a row
+    a[k - 1, 5] = np.inf
+    bad = run(a)
+    assert np.isinf(bad[5]) and np.array_equal(np.delete(bad, 5), np.delete(got, 5))

@@ -388,8 +388,11 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
     return hipModuleLaunchKernel(d->gemv_f32_generic, (n + 255u) / 256u, 1, 1, 256, 1, 1, 0, stream, args, nullptr);
   }
   const uint32_t tiles = (n + 255u) / 256u;
-  // parts of K: about two workgroups of 8 waves per CU, at least 64 rows (8 per wave) each
-  uint32_t parts = std::max(1u, (2u * uint32_t(d->cu_count) + tiles / 2u) / tiles);
+  // parts of K: as many workgroups of 8 waves as there are CUs or somewhat fewer (gemv_f32.hip.h), two per CU only where one
+  // would leave a third of them idle; at least 64 rows (8 per wave) each
+  const uint32_t cus = uint32_t(d->cu_count);
+  uint32_t parts = std::max(1u, cus / tiles);
+  if (parts * tiles * 3u < cus * 2u) parts = 2u * cus / tiles;
   parts = std::max(1u, std::min(parts, (k + 63u) / 64u));
   uint32_t rows_per_part = (k + parts - 1u) / parts;
   rows_per_part = (rows_per_part + 7u) / 8u * 8u;
