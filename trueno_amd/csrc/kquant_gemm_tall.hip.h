@@ -16,10 +16,10 @@
 //     super-block's again).
 //   * Rounding.  The hi pieces' sums are kept apart from the lo pieces' (alone they are whole numbers on a coarse grid and
 //     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by after
-//     about the root of their number.  Against fp64 the error is 0.86 .. 1.02 times the 16-token kernel's (most 0.96).
+//     about the root of their number.  Against fp64 the error is 0.84 .. 1.0 times the 16-token kernel's.
 //   * Measured (us, the 16-token kernel -> this one): Q4_K 14336 x 4096, 2048 tokens 835 -> 525 (matrix cores busy 52 % of
 //     the cycles at 1.7 GHz, the power limit's clock; the vector unit issues 40 %; a library f16 product with as many
-//     matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 195.
+//     matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 190.
 #pragma once
 #include "kquant_gemm_f16.hip.h"
 #include <utility>
