@@ -18,8 +18,10 @@
  * from trn_mem_alloc only.  Beside it the library keeps scratch of its own, per (device, stream),
  * allocated on first use and freed with the stream: the partial sums and arrival counters of the
  * products that are cut along K (trn_q*k_gemm, trn_gemv_f32, trn_incremental_attention), the activations of
- * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB; kept until the stream goes once a captured
- * graph uses them; while a stream is captured what is there is used and nothing allocated), the tables
+ * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB; what one stream adds to one capture has a
+ * buffer of its own instead, allocated during the capture and kept until the process ends, so that the graph can be
+ * replayed on any stream, beside anything but another instance of itself; at most 8 GiB per GPU for all captures, beyond
+ * that a captured product takes the kernel that needs none), the tables
  * of a list's launches of more than sixteen entries (trn_kquant_gemv_batch), the tables of the
  * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB per GPU
  * (trn_q4k_gemm_noalloc).  The calls that never allocate: the GEMV launchers, trn_kquant_gemv_batch

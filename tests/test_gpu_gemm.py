@@ -1,5 +1,7 @@
 """GPU parity, batched GEMM C = A . dequant(W)^T: within 1e-5 relative L2 of fp64 for M in {1, 4, 16, 64},
 row-major C, m = 1 equal to the GEMV; typed launcher and launch-by-name."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -487,3 +489,105 @@ def test_gemm_many_tokens_under_capture_and_without_allocation(gpu):
     finally:
         hip.hipGraphExecDestroy(gexec)
         hip.hipGraphDestroy(graph)
+
+
+class _Dim3(C.Structure):
+    _fields_ = [("x", C.c_uint), ("y", C.c_uint), ("z", C.c_uint)]
+
+
+class _KernelNodeParams(C.Structure):
+    _fields_ = [("block", _Dim3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", _Dim3), ("args", C.POINTER(C.c_void_p)),
+                ("lds", C.c_uint)]
+
+
+def _hip():
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphGetRootNodes.argtypes = [C.c_void_p, C.POINTER(C.c_void_p), C.POINTER(C.c_size_t)]
+    hip.hipGraphKernelNodeGetParams.argtypes = [C.c_void_p, C.POINTER(_KernelNodeParams)]
+    hip.hipGraphExecDestroy.argtypes = [C.c_void_p]
+    hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    return hip
+
+
+class _Captured:
+    """What `issue` puts on the stream, as a graph."""
+
+    def __init__(self, stream, issue):
+        self.hip, self.graph, self.instance = _hip(), C.c_void_p(), C.c_void_p()
+        assert self.hip.hipStreamBeginCapture(stream.raw(), 0) == 0
+        try:
+            issue()
+        finally:
+            rc = self.hip.hipStreamEndCapture(stream.raw(), C.byref(self.graph))
+        assert rc == 0 and self.hip.hipGraphInstantiate(C.byref(self.instance), self.graph, None, None, 0) == 0
+
+    def replay(self, stream):
+        assert self.hip.hipGraphLaunch(self.instance, stream.raw()) == 0
+
+    def first_kernel(self):
+        """(workgroups, the second argument as an address) of the kernel that the graph starts with."""
+        node, count, p = C.c_void_p(), C.c_size_t(1), _KernelNodeParams()
+        assert self.hip.hipGraphGetRootNodes(self.graph, C.byref(node), C.byref(count)) == 0 and count.value == 1
+        assert self.hip.hipGraphKernelNodeGetParams(node, C.byref(p)) == 0
+        return p.grid.x, C.cast(p.args[1], C.POINTER(C.c_uint64))[0]
+
+    def close(self):
+        assert self.hip.hipGraphExecDestroy(self.instance) == 0 and self.hip.hipGraphDestroy(self.graph) == 0
+
+
+def test_gemm_many_tokens_captured_products_keep_to_themselves(gpu):
+    """Two graphs captured on one stream, the first of them before that stream has seen any product: each has operand
+    memory of its own, and both give the eager call's bits when they are replayed on other streams at once, beside eager
+    products on the stream they were captured on, and after that stream is gone and its memory with it."""
+    ctx, other = gpu
+    shapes, stream, kernel = ((97, 1), (200, 2)), t.CudaStream(ctx), "q4k"
+    n, k = 700, 2304
+    buf = kq.gen_matrix(kernel, 660, n, k)
+    dw, graphs, want, out, held = t.GpuBuffer.from_host(ctx, buf), [], [], [], []
+    streams = [t.CudaStream(ctx) for _ in shapes]
+    _tune("gemm_tall", 2)
+    try:
+        for m, seed in shapes:
+            a = kq.gen_x(660 + seed, m, k)
+            want.append(gpu_gemm(gpu, kernel, buf, a, m, n, k).view(np.uint32))
+            da, dc = t.GpuBuffer.from_host(ctx, a), t.GpuBuffer.from_host(ctx, np.full(m * n, np.nan, np.float32))
+            held.append(da)
+            out.append(dc)
+            graphs.append(_Captured(stream, lambda: t.QuantizeKernel.ggml(m, n, k).launch(stream, da, dw, dc)))
+        first = [g.first_kernel() for g in graphs]
+        assert [grid for grid, _ in first] == [(m + 31) // 32 * (k // 256) for m, _ in shapes]      # the kernel for many tokens
+        assert first[0][1] != first[1][1]
+
+        def replay_both():
+            for dc in out:
+                dc.copy_from_host(np.full(dc.len(), np.nan, np.float32))
+            for _ in range(3):
+                for g, s in zip(graphs, streams):
+                    g.replay(s)
+
+        def check():
+            for dc, w, s in zip(out, want, streams):
+                s.synchronize()
+                assert np.array_equal(dc.copy_to_host().reshape(w.shape).view(np.uint32), w)
+
+        big = kq.gen_x(669, 400, k)
+        big_want = gpu_gemm(gpu, kernel, buf, big, 400, n, k).view(np.uint32)
+        for _ in range(3):
+            replay_both()
+            assert np.array_equal(gpu_gemm((ctx, stream), kernel, buf, big, 400, n, k).view(np.uint32), big_want)
+            check()
+        stream.destroy()
+        poison = [t.GpuBuffer.from_host(ctx, np.full(1 << 20, np.nan, np.float32)) for _ in range(8)]      # takes what was freed
+        for _ in range(3):
+            replay_both()
+            check()
+        assert all(np.all(np.isnan(p.copy_to_host())) for p in poison)
+    finally:
+        _tune("gemm_tall", 0)
+        other.synchronize()
+        for g in graphs:
+            g.close()

@@ -661,16 +661,29 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
 }
 
 // One buffer per (device, stream): the operands, then the parts of K.  A product is two or three launches that share it, so
-// a lock is held from the first to the last: another thread's product on the same stream may not come between them.  A
-// buffer whose address a captured graph holds stays until the stream goes; while a stream is captured nothing is allocated.
+// a lock is held from the first to the last: another thread's product on the same stream may not come between them.
+// A captured product has no part in it: a graph can be replayed for as long as the process lives, on any stream, beside
+// eager products and beside other graphs.  The products that one stream adds to one capture run one after the other and
+// share a buffer that nothing else uses and that is never freed.
 struct TallWorkspace {
   void* buf = nullptr;
   size_t cap = 0;
-  bool captured = false;
-  std::vector<void*> retired;
+  unsigned long long capture = 0;      // the stream's last capture, and its buffer
+  void* graph_buf = nullptr;
+  size_t graph_cap = 0;
 };
 std::map<std::pair<int, hipStream_t>, TallWorkspace> g_tall_ws;
+std::map<int, size_t> g_tall_graph_bytes;      // by device: what is left to graphs
 std::mutex g_tall_mutex;
+constexpr size_t kTallGraphBytesMax = size_t(8) << 30;      // of it in all; further captured products take the other kernel
+
+// While this exists, what its thread allocates does not count as part of a capture in progress (hipMalloc would be refused).
+struct AllocationBesideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  AllocationBesideCapture(const AllocationBesideCapture&) = delete;
+};
 
 hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
                             uint32_t k, const TallCut& cut, uint64_t ws) {
@@ -710,10 +723,11 @@ hipError_t launch_tall(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, 
   return hipSuccess;
 }
 
-// *done = false: the stream is being captured and its workspace is too small (the caller takes another kernel)
+// *done = false: no workspace for this product (the caller takes another kernel)
 hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
                                  uint32_t k, bool* done) {
   *done = false;
+  if (stream == hipStreamPerThread) return hipSuccess;      // one handle for as many streams as there are threads
   const TallCut cut = tall_cut(*d, f, m, n, k);
   const size_t need = std::min(tall_bytes(m, n, k / 256u, cut.kparts), kTallWorkspaceMax);
   int dev = 0;
@@ -722,21 +736,32 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
   std::lock_guard<std::mutex> lock(g_tall_mutex);
   TallWorkspace& ws = g_tall_ws[std::make_pair(dev, stream)];
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if ((e = hipStreamIsCapturing(stream, &capture)) != hipSuccess) return e;
+  unsigned long long id = 0;
+  if ((e = hipStreamGetCaptureInfo(stream, &capture, &id)) != hipSuccess) return e;
   if (capture != hipStreamCaptureStatusNone) {
-    if (ws.cap < tall_bytes(kTallTile, n, k / 256u, cut.kparts)) return hipSuccess;
-    ws.captured = true;
-  } else if (ws.cap < need) {
-    if (ws.buf) {
-      if (ws.captured) {
-        ws.retired.push_back(ws.buf);
-      } else {
-        if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
-        (void)hipFree(ws.buf);
+    if (!ws.graph_buf || ws.capture != id || ws.graph_cap < need) {
+      size_t& left = g_tall_graph_bytes[dev];
+      if (left + need > kTallGraphBytesMax) return hipSuccess;
+      void* buf = nullptr;
+      const AllocationBesideCapture beside;
+      if (hipMalloc(&buf, need) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipSuccess;
       }
+      left += need;
+      ws.capture = id;
+      ws.graph_buf = buf;
+      ws.graph_cap = need;
+    }
+    *done = true;
+    return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), ws.graph_cap);
+  }
+  if (ws.cap < need) {
+    if (ws.buf) {
+      if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
+      (void)hipFree(ws.buf);
       ws.buf = nullptr;
       ws.cap = 0;
-      ws.captured = false;
     }
     if ((e = hipMalloc(&ws.buf, need)) != hipSuccess) return e;
     ws.cap = need;
@@ -1459,8 +1484,7 @@ static void release_stream_workspaces(hipStream_t stream) {
     std::lock_guard<std::mutex> lock(g_tall_mutex);
     for (auto it = g_tall_ws.begin(); it != g_tall_ws.end();) {
       if (it->first.second == stream) {
-        if (it->second.buf) (void)hipFree(it->second.buf);
-        for (void* p : it->second.retired) (void)hipFree(p);
+        if (it->second.buf) (void)hipFree(it->second.buf);      // (a graph's buffer stays)
         it = g_tall_ws.erase(it);
       } else {
         ++it;
