@@ -18,10 +18,11 @@
  * from trn_mem_alloc only.  Beside it the library keeps scratch of its own, per (device, stream),
  * allocated on first use and freed with the stream: the partial sums and arrival counters of the
  * products that are cut along K (trn_q*k_gemm, trn_gemv_f32, trn_incremental_attention), the activations of
- * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB; what one stream adds to one capture has a
+ * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB, or none where that cannot be had: the product then
+ * takes the kernel that needs none; what one stream adds to one capture has a
  * buffer of its own instead, allocated during the capture and kept until the process ends, so that the graph can be
  * replayed on any stream, beside anything but another instance of itself; at most 8 GiB per GPU for all captures, beyond
- * that a captured product takes the kernel that needs none), the tables
+ * that again the other kernel), the tables
  * of a list's launches of more than sixteen entries (trn_kquant_gemv_batch), the tables of the
  * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB per GPU
  * (trn_q4k_gemm_noalloc).  The calls that never allocate: the GEMV launchers, trn_kquant_gemv_batch
@@ -337,6 +338,9 @@ TRN_API trn_status trn_device_cu_count(int* count);
  * that form cuts K; "gemm_waves": 4, 8 or (Q4_K) 12 strips of 32 rows per workgroup; "gemm_tiles": 1 or 2 tiles of 16 tokens per
  * workgroup (0 for each of the three = chosen from the shape by an estimated time; any of them set also keeps a
  * product of a few tokens on the matrix cores);
+ * "gemm_tall": the kernel for many tokens - 0 = from 33 tokens on where its estimated time is the lower, 1 = never, 2 =
+ * wherever it can run; "gemm_workspace_none": 1 = as if no memory were left for a further workspace of that kernel (it then
+ * leaves the product to the other one);
  * "attention_per_cu": workgroups per CU the single-query attention aims at (0 = 2); "attention_min_steps": least
  * number of steps (of 8 positions at head_dim 128) in a chunk of positions (0 = 8). */
 TRN_API trn_status trn_set_tuning(const char* key, int value);

@@ -591,3 +591,44 @@ def test_gemm_many_tokens_captured_products_keep_to_themselves(gpu):
         other.synchronize()
         for g in graphs:
             g.close()
+
+
+def test_gemm_many_tokens_without_memory_for_a_workspace(gpu):
+    """Where no workspace can be had the product goes to the kernel that takes sixteen tokens at a time: on a fresh stream, on
+    one whose workspace is too small (which it keeps for smaller products), and under capture on a stream that has seen
+    only products of many tokens."""
+    ctx, _ = gpu
+    n, k, (small, large) = 700, 2304, (64, 300)
+    buf = kq.gen_matrix("q5k", 680, n, k)
+    a = {m: kq.gen_x(681 + m, m, k) for m in (small, large)}
+    bits, refused, used = {}, t.CudaStream(ctx), t.CudaStream(ctx)
+
+    def run(stream, m):
+        return gpu_gemm((ctx, stream), "q5k", buf, a[m], m, n, k).view(np.uint32)
+
+    dw, da = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, a[large])
+    dc = t.GpuBuffer.from_host(ctx, np.full(large * n, np.nan, np.float32))
+    try:
+        for tall in (1, 2):
+            _tune("gemm_tall", tall)
+            bits[tall] = {m: run(gpu[1], m) for m in a}
+        assert not any(np.array_equal(bits[1][m], bits[2][m]) for m in a)
+        assert np.array_equal(run(used, small), bits[2][small])
+        _tune("gemm_workspace_none", 1)
+        for m in a:
+            assert np.array_equal(run(refused, m), bits[1][m])
+        assert np.array_equal(run(used, large), bits[1][large]) and np.array_equal(run(used, small), bits[2][small])
+        _tune("gemm_workspace_none", 0)
+        warm = t.CudaStream(ctx)
+        assert np.array_equal(run(warm, large), bits[2][large])
+        _tune("gemm_workspace_none", 1)
+        graph = _Captured(warm, lambda: t.Q5KKernel(large, n, k).launch(warm, da, dw, dc))
+        for _ in range(3):
+            dc.copy_from_host(np.full(large * n, np.nan, np.float32))
+            graph.replay(warm)
+            warm.synchronize()
+            assert np.array_equal(dc.copy_to_host().reshape(large, n).view(np.uint32), bits[1][large])
+        graph.close()
+    finally:
+        _tune("gemm_tall", 0)
+        _tune("gemm_workspace_none", 0)

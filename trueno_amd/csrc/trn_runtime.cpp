@@ -126,6 +126,7 @@ std::atomic<int> g_tune_many_item_kb{0};    // what a further piece of work cost
 std::atomic<int> g_tune_many_slab_weight{0};  // percent such a launch adds to an entry's bytes per slab of 4096 columns beyond the first (0: default)
 std::atomic<int> g_tune_stream_waves{0};    // waves per workgroup of a single streamed GEMV (0: default)
 std::atomic<int> g_tune_gemm_tall{0};       // the kernel for many tokens: 0 by the rule, 1 never, 2 wherever it can run (from 33 tokens on)
+std::atomic<int> g_tune_gemm_workspace_none{0};  // 1: the many-token kernel finds no memory for a further workspace
 std::atomic<int> g_tune_gemm_few{0};        // the integer matrix-core kernel for two to four tokens: 0 by the rule, 1 wherever it can run, 2 never
 
 inline trn_status st(hipError_t e) { return static_cast<trn_status>(e); }
@@ -684,6 +685,14 @@ struct AllocationBesideCapture {
   ~AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
   AllocationBesideCapture(const AllocationBesideCapture&) = delete;
 };
+void* tall_alloc(size_t bytes) {      // nullptr: none to be had, and no error is left behind
+  if (g_tune_gemm_workspace_none) return nullptr;
+  const AllocationBesideCapture beside;
+  void* buf = nullptr;
+  if (hipMalloc(&buf, bytes) == hipSuccess) return buf;
+  (void)hipGetLastError();
+  return nullptr;
+}
 
 hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
                             uint32_t k, const TallCut& cut, uint64_t ws) {
@@ -733,41 +742,62 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(g_tall_mutex);
-  TallWorkspace& ws = g_tall_ws[std::make_pair(dev, stream)];
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  unsigned long long id = 0;
-  if ((e = hipStreamGetCaptureInfo(stream, &capture, &id)) != hipSuccess) return e;
-  if (capture != hipStreamCaptureStatusNone) {
-    if (!ws.graph_buf || ws.capture != id || ws.graph_cap < need) {
-      size_t& left = g_tall_graph_bytes[dev];
-      if (left + need > kTallGraphBytesMax) return hipSuccess;
-      void* buf = nullptr;
-      const AllocationBesideCapture beside;
-      if (hipMalloc(&buf, need) != hipSuccess) {
-        (void)hipGetLastError();
-        return hipSuccess;
+  void* old = nullptr;
+  bool first = false;
+  {
+    std::lock_guard<std::mutex> lock(g_tall_mutex);
+    TallWorkspace& ws = g_tall_ws[std::make_pair(dev, stream)];
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(stream, &capture, &id) != hipSuccess) {
+      (void)hipGetLastError();
+      return hipSuccess;
+    }
+    if (capture != hipStreamCaptureStatusNone) {
+      if (!ws.graph_buf || ws.capture != id || ws.graph_cap < need) {
+        size_t& left = g_tall_graph_bytes[dev];
+        void* buf = left + need > kTallGraphBytesMax ? nullptr : tall_alloc(need);
+        if (!buf) return hipSuccess;
+        left += need;
+        ws.capture = id;
+        ws.graph_buf = buf;
+        ws.graph_cap = need;
       }
-      left += need;
-      ws.capture = id;
-      ws.graph_buf = buf;
-      ws.graph_cap = need;
+      *done = true;
+      return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), ws.graph_cap);
+    }
+    first = ws.buf == nullptr;
+    if (ws.cap < need) {
+      void* buf = tall_alloc(need);
+      if (!buf) return hipSuccess;      // (what the stream has stays: a smaller product finds it)
+      old = ws.buf;
+      ws.buf = buf;
+      ws.cap = need;
     }
     *done = true;
-    return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), ws.graph_cap);
+    e = launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.buf), ws.cap);
   }
-  if (ws.cap < need) {
-    if (ws.buf) {
-      if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
-      (void)hipFree(ws.buf);
-      ws.buf = nullptr;
-      ws.cap = 0;
+  // what waits for the stream waits without the lock: the work ahead may depend on another thread's product
+  if (old) {
+    const hipError_t idle = hipStreamSynchronize(stream);   // work in flight may still use the old buffer
+    if (e == hipSuccess) e = idle;
+    const AllocationBesideCapture beside;
+    if (idle == hipSuccess) (void)hipFree(old);
+  }
+  if (first && e == hipSuccess) {
+    // a program that warms a stream up with a long prompt may capture products of a few tokens next: the other kernel's
+    // buffer has to be there by then (a buffer that is there stays as it is)
+    bool there = false;
+    {
+      std::lock_guard<std::mutex> lock(g_ws_mutex);
+      auto it = g_gemm_ws.find(std::make_pair(dev, stream));
+      there = it != g_gemm_ws.end() && it->second.buf != nullptr;
     }
-    if ((e = hipMalloc(&ws.buf, need)) != hipSuccess) return e;
-    ws.cap = need;
+    uint64_t base = 0;
+    if (!there && acquire_scratch(g_gemm_ws, d, stream, kGemmCounterBytes + (size_t(16) << 20), kGemmCounterBytes, &base) != hipSuccess)
+      (void)hipGetLastError();      // (this product did not need it)
   }
-  *done = true;
-  return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.buf), ws.cap);
+  return e;
 }
 
 constexpr double kBigAloneBytes = 64e6;      // from this size on a matrix alone takes the list kernel (launch_gemm_like, trn_kquant_gemv_batch)
@@ -2269,6 +2299,7 @@ trn_status trn_set_tuning(const char* key, int value) {
   if (!std::strcmp(key, "gemv_stream_cost")) { g_tune_stream_cost = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_min_rows")) { g_tune_stream_min_rows = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_tall")) { if (value > 2) return TRN_ERROR_INVALID_VALUE; g_tune_gemm_tall = value; return TRN_SUCCESS; }
+  if (!std::strcmp(key, "gemm_workspace_none")) { g_tune_gemm_workspace_none = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_few")) { g_tune_gemm_few = value; return TRN_SUCCESS; }
   return TRN_ERROR_INVALID_VALUE;
 }
