@@ -24,7 +24,7 @@
  * replayed on any stream, beside anything but another instance of itself; at most 8 GiB per GPU for all captures, beyond
  * that again the other kernel), the tables
  * of a list's launches of more than sixteen entries (trn_kquant_gemv_batch), the tables of the
- * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB per GPU
+ * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB and 256 MiB allocated on first use per GPU
  * (trn_q4k_gemm_noalloc).  The calls that never allocate: the GEMV launchers, trn_kquant_gemv_batch
  * for lists whose launches hold at most sixteen entries or while the stream is being captured,
  * trn_q4k_gemm_noalloc, the element-wise launchers.  All entry points may be called from any thread;
@@ -167,13 +167,15 @@ TRN_API trn_status trn_q6k_gemm(trn_stream stream, trn_dptr a, trn_dptr b_quant,
  * results; but where trn_q4k_gemm keeps a per-stream scratch buffer that it allocates and grows on demand (partial
  * results of the parts of K and their arrival counters), this entry point uses a buffer that is part of the library
  * image: a static device array of 16 MiB + 64 KiB, of which every GPU the library runs on holds one copy until the
- * process ends.  After the library's first use on the device (any launcher, or trn_ctx_set_current, loads the kernels
- * and looks the buffer's address up once) it calls nothing that allocates or frees.  The product is cut exactly as
- * trn_q4k_gemm would cut it - hence the same bits; a product of many tokens goes through the buffer in several runs of
- * them, as trn_q4k_gemm itself does from 256 MiB of scratch on - and when that cut needs more scratch than the buffer holds the call
+ * process ends; and, for products of many tokens, 256 MiB that the library allocates there once with it.  After the
+ * library's first use on the device (any launcher, or trn_ctx_set_current, loads the kernels, looks the buffer's address up
+ * and allocates the 256 MiB) it calls nothing that allocates or frees.  The product is cut exactly as
+ * trn_q4k_gemm would cut it - hence the same bits; a product of many tokens that needs more than 256 MiB goes through them
+ * in several runs of tokens, in both entry points - and when the cut's partial sums need more than the static array holds the call
  * returns TRN_ERROR_SCRATCH_TOO_SMALL and launches nothing; no other failure is reported under that name (every cut that
  * the library chooses by itself needs at most 11.2 MB on 256 CUs; a cut forced with trn_set_tuning may need more; m = 1
- * and unaligned operands take kernels that need no scratch).  All calls on
+ * and unaligned operands take kernels that need no scratch).  (The bits differ only where memory for a workspace ran out
+ * for one of the two, see the head of this file: that one then takes the other matrix-core kernel.)  All calls on
  * one GPU share that GPU's buffer: calls that overlap in time on different streams of one GPU race - keep them on
  * one stream, or order the streams.  The kernels leave the counters at zero for the next call. */
 TRN_API trn_status trn_q4k_gemm_noalloc(trn_stream stream, trn_dptr a, trn_dptr b_quant, trn_dptr c, uint32_t m, uint32_t n, uint32_t k);
@@ -339,7 +341,7 @@ TRN_API trn_status trn_device_cu_count(int* count);
  * workgroup (0 for each of the three = chosen from the shape by an estimated time; any of them set also keeps a
  * product of a few tokens on the matrix cores);
  * "gemm_tall": the kernel for many tokens - 0 = from 33 tokens on where its estimated time is the lower, 1 = never, 2 =
- * wherever it can run; "gemm_workspace_none": 1 = as if no memory were left for a further workspace of that kernel (it then
+ * wherever it can run; "gemm_workspace_mb": what its workspace may hold, in MiB, at most 256 (0 = 256); "gemm_workspace_none": 1 = as if no memory were left for a further workspace of that kernel (it then
  * leaves the product to the other one);
  * "attention_per_cu": workgroups per CU the single-query attention aims at (0 = 2); "attention_min_steps": least
  * number of steps (of 8 positions at head_dim 128) in a chunk of positions (0 = 8). */

@@ -7,6 +7,7 @@ import pytest
 
 import trueno_amd as t
 from oracle import kquant as kq
+from trueno_amd import _ffi
 from tests.kq_helpers import REF_SLACK, gpu_gemm, gpu_gemv, record_ratio
 
 pytestmark = pytest.mark.gpu
@@ -453,7 +454,7 @@ def test_gemm_many_tokens_no_less_exact_than_sixteen_at_a_time(gpu, fmt):
 
 def test_gemm_many_tokens_under_capture_and_without_allocation(gpu):
     """Twice the same bits through a captured graph after a larger product has grown the workspace, and from
-    trn_q4k_gemm_noalloc, whose buffer takes the tokens in several runs."""
+    trn_q4k_gemm_noalloc, whose workspace is the library's own."""
     import ctypes as C
     from trueno_amd import _ffi
     hip = C.CDLL("libamdhip64.so")
@@ -632,3 +633,47 @@ def test_gemm_many_tokens_without_memory_for_a_workspace(gpu):
     finally:
         _tune("gemm_tall", 0)
         _tune("gemm_workspace_none", 0)
+
+
+def test_gemm_many_tokens_in_runs(gpu):
+    """A workspace that holds three token tiles: the same bits in four runs as in one, from both entry points, and in as many
+    runs of one tile.  The rule prices the runs: a product that it gives to the kernel for many tokens in one run goes sixteen
+    tokens at a time in a workspace that would cut it into runs of a few tiles, from both entry points again."""
+    ctx, stream = gpu
+    L = _ffi.lib()
+
+    def both(buf, a, n, k):
+        m = a.shape[0]
+        got = gpu_gemm(gpu, "q4k", buf, a, m, n, k).view(np.uint32)
+        dw, da = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, a)
+        dc = t.GpuBuffer.from_host(ctx, np.full(m * n, np.nan, np.float32))
+        assert L.trn_q4k_gemm_noalloc(stream.raw(), da.as_ptr(), dw.as_ptr(), dc.as_ptr(), m, n, k) == 0
+        stream.synchronize()
+        assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), got)
+        return got
+
+    try:
+        n, k = 300, 2304                                  # a tile of 32 tokens: 9 x 34 KiB, in one part of K
+        buf, a = kq.gen_matrix("q4k", 690, n, k), kq.gen_x(691, 321, k)
+        _tune("gemm_tall", 2)
+        for parts in (1, 3):
+            _tune("gemm_k_parts", parts)
+            _tune("gemm_workspace_mb", 0)
+            whole = both(buf, a, n, k)
+            for mb in (1, 2):
+                _tune("gemm_workspace_mb", mb)
+                assert np.array_equal(both(buf, a, n, k), whole), (parts, mb)
+        _tune("gemm_tall", 0)
+        _tune("gemm_k_parts", 0)
+        n, k = 4096, 4096
+        buf, a = kq.gen_matrix("q4k", 692, n, k), kq.gen_x(693, 512, k)
+        bits = {}
+        for name, tall, mb in (("tall", 2, 0), ("sixteen", 1, 0), ("rule", 0, 0), ("rule, small", 0, 2)):
+            _tune("gemm_tall", tall)
+            _tune("gemm_workspace_mb", mb)
+            bits[name] = both(buf, a, n, k)
+        assert np.array_equal(bits["rule"], bits["tall"]) and np.array_equal(bits["rule, small"], bits["sixteen"])
+        assert not np.array_equal(bits["tall"], bits["sixteen"])
+    finally:
+        for key in ("gemm_tall", "gemm_k_parts", "gemm_workspace_mb"):
+            _tune(key, 0)

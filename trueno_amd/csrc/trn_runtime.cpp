@@ -41,6 +41,7 @@ extern "C" const unsigned char trn_builtin_hsaco_end[];
 // trn_noalloc.hip: the library's static device scratch buffer (one copy per GPU)
 extern "C" hipError_t trn_noalloc_scratch_setup(int dev);
 extern "C" uint64_t trn_noalloc_scratch(int dev, size_t* bytes);
+extern "C" uint64_t trn_noalloc_workspace(int dev, size_t* bytes);
 
 namespace {
 
@@ -126,6 +127,7 @@ std::atomic<int> g_tune_many_item_kb{0};    // what a further piece of work cost
 std::atomic<int> g_tune_many_slab_weight{0};  // percent such a launch adds to an entry's bytes per slab of 4096 columns beyond the first (0: default)
 std::atomic<int> g_tune_stream_waves{0};    // waves per workgroup of a single streamed GEMV (0: default)
 std::atomic<int> g_tune_gemm_tall{0};       // the kernel for many tokens: 0 by the rule, 1 never, 2 wherever it can run (from 33 tokens on)
+std::atomic<int> g_tune_gemm_workspace_mb{0};    // what the many-token kernel's workspace may hold, in MiB (0: default)
 std::atomic<int> g_tune_gemm_workspace_none{0};  // 1: the many-token kernel finds no memory for a further workspace
 std::atomic<int> g_tune_gemm_few{0};        // the integer matrix-core kernel for two to four tokens: 0 by the rule, 1 wherever it can run, 2 never
 
@@ -626,17 +628,26 @@ hipError_t launch_gemm_few(DeviceKernels* d, hipStream_t stream, uint64_t a, uin
 
 // ---- many tokens (kquant_gemm_tall.hip.h) -----------------------------------------------------------------------------
 constexpr uint32_t kTallRows = 256, kTallTile = 32, kTallOperandBytes = 32u * 1024u + 2048u;      // rows and tokens of a workgroup; of a (tile, super-block)
-constexpr size_t kTallWorkspaceMax = size_t(256) << 20;      // products that need more go through it in runs of tokens
-constexpr size_t kTallWorkspaceLeast = size_t(16) << 20;     // every cut works within this much (trn_q4k_gemm_noalloc has no more)
+// The most a product's workspace holds; a product that needs more goes through it in runs of tokens, and its price is that of
+// its runs: 4096 x 65536, 2048 tokens, take three.  trn_q4k_gemm_noalloc has as much (trn_noalloc.hip), so that its runs, and
+// with them the choice of kernel and the cut, are trn_q4k_gemm's: in 16 MiB 4096 x 14336, 2048 tokens, would take eight runs
+// of 128 workgroups, an estimated 1161 us against 549 in one and 721 for sixteen tokens at a time.
+constexpr size_t kTallWorkspaceMax = size_t(256) << 20;
+size_t tall_workspace_cap() { return g_tune_gemm_workspace_mb > 0 ? std::min(size_t(g_tune_gemm_workspace_mb) << 20, kTallWorkspaceMax) : kTallWorkspaceMax; }
 struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit; };
 uint32_t tall_lds_bytes(Fmt f) { return (f == Q6K ? 2u : 4u) * 8192u + 2u * 2048u + 4u * 64u * (f == Q6K ? 224u : kSbBytes[f]); }
 size_t tall_bytes(uint32_t tokens, uint32_t n, uint32_t nsb, uint32_t kparts) {
   const size_t tiles = (tokens + kTallTile - 1u) / kTallTile;
   return tiles * nsb * kTallOperandBytes + (kparts > 1u ? (size_t(kparts) * tokens * n * 4u + 255u) / 256u * 256u : 0u);
 }
-// The parts of K with the least estimated time.  Times in microseconds fitted to measurements on MI355X (1024 x 4096 ..
+// The tokens of a run through `cap` bytes: all of them, or as many whole tiles as it holds (0: not one).
+uint32_t tall_run(uint32_t m, uint32_t n, uint32_t nsb, uint32_t kparts, size_t cap) {
+  if (tall_bytes(m, n, nsb, kparts) <= cap) return m;
+  return uint32_t(std::min<size_t>(cap / tall_bytes(kTallTile, n, nsb, kparts), m / kTallTile)) * kTallTile;
+}
+// The parts of K with the least estimated time, the same for every run.  Times in microseconds fitted to measurements on MI355X (1024 x 4096 ..
 // 32000 x 4096 and 4096 x 11008, 33 .. 1024 tokens, within about 10 % from 64 tokens on): 9 for the launches and the first
-// super-block; the operands at 4 TB/s; a super-block takes a round of two workgroups per CU 4.3 / 5.1 / 7.5 (Q4_K / Q5_K /
+// super-block of a run; the operands at 4 TB/s; a super-block takes a round of two workgroups per CU 4.3 / 5.1 / 7.5 (Q4_K / Q5_K /
 // Q6_K), one workgroup alone on its CU 2.3 / 2.7 / 4.2; with K in parts 3 for the sum's launch, 0.4 a part, and the parts'
 // bytes at 4 TB/s.
 TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k) {
@@ -646,16 +657,21 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
   const double pair = f == Q4K ? 4.3 : f == Q5K ? 5.1 : 7.5, alone = f == Q4K ? 2.3 : f == Q5K ? 2.7 : 4.2;
   const uint32_t most = g_tune_gemm_ksplit > 0 ? std::min<uint32_t>(uint32_t(g_tune_gemm_ksplit), nsb)
                                                : uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>((2u * cus + units / 2u) / units, nsb)));
+  auto run_us = [&](const TallCut& c, uint32_t tokens) {
+    const uint64_t wgs = uint64_t(groups) * ((tokens + kTallTile - 1u) / kTallTile) * c.kparts, rounds = wgs / (2u * cus), rest = wgs - rounds * 2u * cus;
+    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * double(rest - cus) / cus;
+    return 9.0 + double(tokens) * k * 8.0 / 4.0e6 + c.ksb * (double(rounds) * pair + last) +
+           (c.kparts > 1u ? 3.0 + 0.4 * c.kparts + double(c.kparts + 1u) * tokens * n * 4.0 / 4.0e6 : 0.0);
+  };
   for (uint32_t kp = most; kp >= 1u; --kp) {
     TallCut c;
     c.ksb = (nsb + kp - 1u) / kp;
     c.kparts = (nsb + c.ksb - 1u) / c.ksb;
-    if (tall_bytes(kTallTile, n, nsb, c.kparts) > kTallWorkspaceLeast) continue;
-    const uint64_t wgs = units * c.kparts, rounds = wgs / (2u * cus), rest = wgs - rounds * 2u * cus;
-    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * double(rest - cus) / cus;
-    c.us = 9.0 + double(m) * k * 8.0 / 4.0e6 + c.ksb * (double(rounds) * pair + last) +
-           (c.kparts > 1u ? 3.0 + 0.4 * c.kparts + double(c.kparts + 1u) * m * n * 4.0 / 4.0e6 : 0.0);
-    if (c.us < best.us) best = c;
+    const uint32_t step = tall_run(m, n, nsb, c.kparts, tall_workspace_cap());
+    if (step != 0u) {
+      c.us = (m / step) * run_us(c, step) + (m % step != 0u ? run_us(c, m % step) : 0.0);
+      if (c.us < best.us) best = c;
+    }
     if (g_tune_gemm_ksplit > 0) break;
   }
   return best;
@@ -717,12 +733,8 @@ hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_
 // its company).  g_tall_mutex held.
 hipError_t launch_tall(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n, uint32_t k,
                        const TallCut& cut, uint64_t ws, size_t cap) {
-  const uint32_t nsb = k / 256u;
-  uint32_t step = m;
-  if (tall_bytes(m, n, nsb, cut.kparts) > cap) {
-    step = uint32_t(std::min<size_t>(cap / tall_bytes(kTallTile, n, nsb, cut.kparts), m / kTallTile)) * kTallTile;
-    if (step == 0u) return hipErrorInvalidValue;
-  }
+  const uint32_t step = tall_run(m, n, k / 256u, cut.kparts, cap);
+  if (step == 0u) return hipErrorInvalidValue;
   for (uint32_t t = 0; t < m; t += step) {
     const uint32_t len = std::min(step, m - t);
     const hipError_t e = launch_tall_once(d, f, stream, a + uint64_t(t) * k * 4u, w, c + uint64_t(t) * n * 4u, len, n, k, cut, ws);
@@ -738,7 +750,7 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
   *done = false;
   if (stream == hipStreamPerThread) return hipSuccess;      // one handle for as many streams as there are threads
   const TallCut cut = tall_cut(*d, f, m, n, k);
-  const size_t need = std::min(tall_bytes(m, n, k / 256u, cut.kparts), kTallWorkspaceMax);
+  const size_t need = std::min(tall_bytes(m, n, k / 256u, cut.kparts), tall_workspace_cap());
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -764,7 +776,7 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
         ws.graph_cap = need;
       }
       *done = true;
-      return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), ws.graph_cap);
+      return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), need);
     }
     first = ws.buf == nullptr;
     if (ws.cap < need) {
@@ -775,7 +787,7 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
       ws.cap = need;
     }
     *done = true;
-    e = launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.buf), ws.cap);
+    e = launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.buf), need);
   }
   // what waits for the stream waits without the lock: the work ahead may depend on another thread's product
   if (old) {
@@ -2167,9 +2179,13 @@ trn_status trn_q4k_gemm_noalloc(trn_stream s, trn_dptr a, trn_dptr b, trn_dptr c
   size_t cap = 0;
   const uint64_t base = trn_noalloc_scratch(dev, &cap);
   if (!base) return TRN_ERROR_INVALID_VALUE;
-  if (route == GemmRoute::kTall) {      // behind the counters, which stay as they are; every cut fits, in runs of tokens if need be
-    std::lock_guard<std::mutex> lock(g_tall_mutex);
-    return st(launch_tall(d, Q4K, stream, a, b, c, m, n, k, tall_cut(*d, Q4K, m, n, k), base + kGemmCounterBytes, cap - kGemmCounterBytes));
+  if (route == GemmRoute::kTall && stream != hipStreamPerThread) {
+    size_t ws_cap = 0;
+    const uint64_t ws = g_tune_gemm_workspace_none ? 0 : trn_noalloc_workspace(dev, &ws_cap);
+    if (ws) {
+      std::lock_guard<std::mutex> lock(g_tall_mutex);
+      return st(launch_tall(d, Q4K, stream, a, b, c, m, n, k, tall_cut(*d, Q4K, m, n, k), ws, std::min(ws_cap, tall_workspace_cap())));
+    }
   }
   // the cut trn_q4k_gemm would take (so the bits are its bits): refused by name when its partial sums do not fit
   const GemmCut cut = gemm_cut(*d, Q4K, m, n, k);
@@ -2299,6 +2315,7 @@ trn_status trn_set_tuning(const char* key, int value) {
   if (!std::strcmp(key, "gemv_stream_cost")) { g_tune_stream_cost = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_stream_min_rows")) { g_tune_stream_min_rows = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_tall")) { if (value > 2) return TRN_ERROR_INVALID_VALUE; g_tune_gemm_tall = value; return TRN_SUCCESS; }
+  if (!std::strcmp(key, "gemm_workspace_mb")) { g_tune_gemm_workspace_mb = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_workspace_none")) { g_tune_gemm_workspace_none = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemm_few")) { g_tune_gemm_few = value; return TRN_SUCCESS; }
   return TRN_ERROR_INVALID_VALUE;
