@@ -677,3 +677,30 @@ def test_gemm_many_tokens_in_runs(gpu):
     finally:
         for key in ("gemm_tall", "gemm_k_parts", "gemm_workspace_mb"):
             _tune(key, 0)
+
+
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_many_tokens_beside_one_value_much_larger(gpu, fmt):
+    """One activation in every run of 256 is 2^12, 2^20, 2^24 times larger than the others, and the weights of its sub-block are
+    zero: the others' pieces, scaled by the run's maximum, keep all their bits.  Two pieces of eleven bits hold a value to
+    2^-23, the sums' rounding is about that much again (1.2e-7 in all without the large values): bound 2.5e-7."""
+    m, n, k = 40, 300, 2048
+    buf = kq.gen_matrix(fmt, 670, n, k).reshape(n * k // 256, -1).copy()
+    if fmt == "q4k":
+        buf[:, [4, 8]] &= 0xC0                      # scale and minimum of sub-block 0: the low six bits
+    elif fmt == "q5k":
+        buf[:, 4] = 0                               # the first of the 12-bit fields
+        buf[:, 5] &= 0xF0
+    else:
+        buf[:, 192] = 0
+    buf = buf.reshape(-1)
+    w = kq.dequant_matrix(fmt, buf, n, k)
+    assert not np.any(w[:, ::256]) and np.any(w[:, 32::256])
+    try:
+        _tune("gemm_tall", 2)
+        for power in (12, 20, 24):
+            a = kq.gen_x(671, m, k)
+            a[:, 3::256] = np.float32(2.0 ** power)
+            assert kq.rel_l2(gpu_gemm(gpu, fmt, buf, a, m, n, k), kq.gemm_fp64(a, w)) <= 2.5e-7, power
+    finally:
+        _tune("gemm_tall", 0)

@@ -16,7 +16,8 @@
 //     super-block's again).
 //   * Rounding.  The hi pieces' sums are kept apart from the lo pieces' (alone they are whole numbers on a coarse grid and
 //     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by after
-//     about the root of their number.  Against fp64 the error is 0.84 .. 1.0 times the 16-token kernel's.
+//     about the root of their number.  Against fp64 the error is 0.82 .. 0.98 times the 16-token kernel's, over 70 shapes a
+//     format drawn from 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns that the rule gives this kernel.
 //   * Measured (us, the 16-token kernel -> this one): Q4_K 14336 x 4096, 2048 tokens 835 -> 525 (matrix cores busy 52 % of
 //     the cycles at 1.7 GHz, the power limit's clock; the vector unit issues 40 %; a library f16 product with as many
 //     matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 190.
@@ -38,6 +39,7 @@ constexpr u32 kPageStride = 1024 + 16;         // LDS of the converter: pages ap
 // ---- the token operands of one (tile of 32 tokens, super-block), by one workgroup of 256 threads ----
 //   pages 2 q (lo pieces) and 2 q + 1 (hi pieces), slot 32 g + token: eight f16, elements 32 j + 8 (u % 4) + perm of the token's run, u = q / 2,
 //   j = 2 (2g + u / 4) + q % 2, perm = 0,2,1,3,4,6,5,7 - what the ANDs on a dword of nibbles leave in its 16-bit lanes
+//   (a lo piece is 2^11 times what the hi piece leaves out: it keeps its eleven bits beside a value 2^24 times larger)
 //   aux: slot 32 g + token: f16 hi pieces of 2^-5 * (sum of the scaled sub-block 4 g + e), e = 0, 2, 1, 3, then the lo pieces;
 //        at 1024: f32 2^(E+14) per token (NaN where the run holds an infinity or a NaN)
 __device__ __forceinline__ void convert_body(const float* __restrict__ a, uint8_t* __restrict__ ops, u32 m, u32 nsb) {
@@ -79,17 +81,13 @@ __device__ __forceinline__ void convert_body(const float* __restrict__ a, uint8_
     const float down = __uint_as_float((268u - eb) << 23);        // 2^-E = 2^(141 - eb): the maximum comes to [2^14, 2^15)
     _Float16 hi[8], lo[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float xs = x[e] * down;
-      hi[e] = static_cast<_Float16>(xs);
-      lo[e] = static_cast<_Float16>(xs - static_cast<float>(hi[e]));
-    }
+    for (int e = 0; e < 8; ++e) split_f16(x[e] * down, hi[e], lo[e]);
     const u32 j = c >> 2, g = j >> 2, h = j & 1u, u = 4u * ((j & 3u) >> 1) + (c & 3u), q = 2u * u + h;
     const u32x4 ph = {pack_h2(hi[0], hi[2]), pack_h2(hi[1], hi[3]), pack_h2(hi[4], hi[6]), pack_h2(hi[5], hi[7])};
     const u32x4 pl = {pack_h2(lo[0], lo[2]), pack_h2(lo[1], lo[3]), pack_h2(lo[4], lo[6]), pack_h2(lo[5], lo[7])};
     *reinterpret_cast<u32x4*>(s_page + 2u * q * kPageStride + (32u * g + token) * 16u) = pl;
     *reinterpret_cast<u32x4*>(s_page + (2u * q + 1u) * kPageStride + (32u * g + token) * 16u) = ph;
-    // the sub-block's sum out of the pieces (eleven significant bits each: thirty-two of them add up without rounding)
+    // the sub-block's sum out of the pieces (eleven significant bits each: thirty-two of similar size add up without rounding)
     const h16x2 ones = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
     float sh = __builtin_amdgcn_fdot2(as_h16x2(ph.x), ones, 0.0f, false), sl = __builtin_amdgcn_fdot2(as_h16x2(pl.x), ones, 0.0f, false);
     sh = __builtin_amdgcn_fdot2(as_h16x2(ph.y), ones, sh, false); sl = __builtin_amdgcn_fdot2(as_h16x2(pl.y), ones, sl, false);
@@ -97,9 +95,10 @@ __device__ __forceinline__ void convert_body(const float* __restrict__ a, uint8_
     sh = __builtin_amdgcn_fdot2(as_h16x2(ph.w), ones, sh, false); sl = __builtin_amdgcn_fdot2(as_h16x2(pl.w), ones, sl, false);
     sh += dpp_f32<0xB1>(sh); sl += dpp_f32<0xB1>(sl);
     sh += dpp_f32<0x4E>(sh); sl += dpp_f32<0x4E>(sl);      // the four threads of a sub-block hold its sums
-    const float sj = (sl + sh) * 0.03125f;
+    const float sj = fmaf(sl, 0.00048828125f, sh) * 0.03125f;
     if ((c & 3u) == 0u) {
-      const _Float16 s_hi = static_cast<_Float16>(sj), s_lo = static_cast<_Float16>(sj - static_cast<float>(s_hi));
+      _Float16 s_hi, s_lo;
+      split_f16(sj, s_hi, s_lo);
       _Float16* dst = reinterpret_cast<_Float16*>(s_aux + (32u * g + token) * 16u) + ((j & 1u) * 2u + ((j >> 1) & 1u));
       dst[0] = s_hi;
       dst[4] = s_lo;
@@ -251,7 +250,7 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
     };
     read_tokens(0, slot, std::integral_constant<int, 0>{});
     asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(hdr[0]), "+v"(hdr[1]), "+v"(raw[0][0]), "+v"(raw[0][1]), "+v"(qh[0]), "+v"(qh[1]) : "n"(2) : "memory");
-    float d[2], nm[2];
+    float d[2], nm[2];      // (times 2^-11 where they meet the sums of lo pieces)
     h16x2 scale[2][2], addend[2][2], mins[2][2];      // [row tile][sub-blocks 0 and 2 (low nibbles), 1 and 3 (high nibbles) of the lane's four]
     constexpr float kCentre = FMT == FMT_Q4K ? 8.0f : 16.0f;
 #pragma unroll
@@ -359,10 +358,11 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
         const f32x16 mcl = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ml), zero, 0, 0, 0);
         acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ch), acc[r], 0, 0, 0);
         low[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, cl), low[r], 0, 0, 0);
+        const float d_lo = d[r] * 0.00048828125f, nm_lo = nm[r] * 0.00048828125f;
         // (what the lo pieces gave comes first: next to no rounding is added at the size of the whole)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(d[r], acc[r][v], fmaf(nm[r], mch[v], fmaf(nm[r], mcl[v], d[r] * low[r][v]))), tot[r][v]);
+          tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(d[r], acc[r][v], fmaf(nm[r], mch[v], fmaf(nm_lo, mcl[v], d_lo * low[r][v]))), tot[r][v]);
       }
     }
     if (--left == 0u || s + 1u == ns) {      // runs of super-blocks are summed by themselves: fewer roundings at the size of the whole
@@ -381,8 +381,11 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
 // Q6_K: w = (q - 32) sc needs 13 bits, f16 holds 11.  Centred digits q - 32 = 8 (2 q2 - 3) + (nib - 8) as in
 // kquant_gemm_f16.hip.h, but three products a step instead of four: the large digit with the hi pieces in one sum (small
 // whole numbers, so that its partial sums hardly round), and in a second one, a quarter of its size, the small digit with
-// the hi pieces and the rounded whole weight with the lo pieces (what its rounding leaves out, at most 2^-12 of w against
-// pieces 2^-11 of the value, is below the sums' rounding).  Blocks of 210 bytes lie in LDS 224 apart: thirteen pieces,
+// the hi pieces and the whole weight rounded to f16 with the lo pieces.  Rounding leaves out at most 1 of odd weights above
+// 2048, 2^-11 of w, against pieces of at most 2^-11 of the value: 2^-22 of such a term, which the sums' rounding covers
+// (error 0.82 .. 0.93 times the 16-token kernel's on activations in use; where all but one in 64 activations are zero and
+// little is added up, 1.07 times).  The two digits apart against the lo pieces, a fourth product, would be exact and
+// take 8-10 % longer (4096 x 11008, 512 tokens: 212 -> 230 us).  Blocks of 210 bytes lie in LDS 224 apart: thirteen pieces,
 // then the block's last sixteen bytes (d at 222); nothing behind a block is read.
 constexpr u32 kQ6Stride = 224u, kQ6Pieces = 14u;
 
@@ -477,7 +480,9 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
       scale[r][2] = as_h16x2((y & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
       scale[r][3] = as_h16x2(((y >> 8) & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
     }
-    h16x8 wq[2], wn[2], wa[2];      // (2 q2 - 3) sc, (nib - 8) sc, their sum 8 : 1 rounded to f16; all times 2^-14
+    // (2 q2 - 3) sc 2^-20, (nib - 8) sc 2^-12, the whole weight rounded to f16 2^-23 (2^-11 of the former's scale: lo pieces
+    // carry 2^11; what is below 2^-14 is a whole multiple of 2^-24 and exact as a subnormal)
+    h16x8 wq[2], wn[2], wa[2];
     auto build = [&](int r, int q) {      // product q = 4 c + 2 i + H
       const int cc = q >> 2, i = (q >> 1) & 1, H = q & 1, hi_nib = cc >> 1, gq = 2 * hi_nib + H;
       const u32 t0 = i ? ql[r][H].z : ql[r][H].x, t1 = i ? ql[r][H].w : ql[r][H].y, c0 = i ? qh[r].z : qh[r].x, c1 = i ? qh[r].w : qh[r].y;
@@ -485,8 +490,8 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
       auto up = [](u32 v, int by) { return by >= 0 ? v << by : v >> -by; };
       const u32 a[4] = {hi_nib ? t0 : t0 << 4, hi_nib ? t0 >> 8 : t0 >> 4, hi_nib ? t1 : t1 << 4, hi_nib ? t1 >> 8 : t1 >> 4};
       const u32 b[4] = {up(c0, 4 - 2 * gq), up(c0, -4 - 2 * gq), up(c1, 4 - 2 * gq), up(c1, -4 - 2 * gq)};
-      const h16x2 sn = scale[r][cc] * h2(64.0f), an = scale[r][cc] * h2(-0.00048828125f);        // -8 * 2^-14
-      const h16x2 sq = scale[r][cc] * h2(128.0f), aq = scale[r][cc] * h2(-0.00018310546875f);    // -3 * 2^-14
+      const h16x2 sn = scale[r][cc] * h2(256.0f), an = scale[r][cc] * h2(-0.001953125f);              // -8 * 2^-12
+      const h16x2 sq = scale[r][cc] * h2(2.0f), aq = scale[r][cc] * h2(-0.00000286102294921875f);    // -3 * 2^-20
       u32 vn[4], vq[4], va[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -494,7 +499,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
         const h16x2 q2 = pk_fma_h2(b[k] & 0x00300030u, h16x2{sq[H], sq[H]}, h16x2{aq[H], aq[H]});
         vn[k] = __builtin_bit_cast(u32, n2);
         vq[k] = __builtin_bit_cast(u32, q2);
-        va[k] = __builtin_bit_cast(u32, __builtin_elementwise_fma(q2, h2(8.0f), n2));
+        va[k] = __builtin_bit_cast(u32, __builtin_elementwise_fma(n2, h2(0.00048828125f), q2));
       }
       wn[r] = __builtin_bit_cast(h16x8, u32x4{vn[0], vn[1], vn[2], vn[3]});
       wq[r] = __builtin_bit_cast(h16x8, u32x4{vq[0], vq[1], vq[2], vq[3]});
@@ -514,7 +519,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
 #pragma unroll
       for (int r = 0; r < 2; ++r)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(8.0f * d[r], acc[r][v], d[r] * low[r][v]), tot[r][v]);
+        for (int v = 0; v < 16; ++v) tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(512.0f * d[r], acc[r][v], 0.25f * d[r] * low[r][v]), tot[r][v]);      // 2^(E+14)
     };
     auto step = [&](auto i_c) {
       constexpr int I = decltype(i_c)::value, CH = I / 4, B = I & 1, X = CH + 1;
