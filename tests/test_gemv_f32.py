@@ -81,9 +81,11 @@ def test_gpu_gemv_f32_by_name_and_edges(gpu):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("k,n", [(9, 260), (63, 260), (65, 260), (71, 516), (129, 260), (1003, 43008), (520, 33028)])
+@pytest.mark.parametrize("k,n", [(9, 260), (63, 260), (65, 260), (71, 516), (129, 260), (1003, 43008), (520, 33028), (1024, 33028),
+                                 (300, 65536), (130, 65540), (65, 90000)])
 def test_gpu_gemv_f32_last_rows_and_wide_matrices(gpu, k, n):
-    """Rows that do not fill a wave's last eight, and matrices wide enough for two workgroups per CU; an infinity in the
+    """Rows that do not fill a wave's last eight, and matrices of 130 column tiles (one part of K below 1024 rows, three from
+    there on), of as many as there are CUs and one more (two parts), and of 352 (one part); an infinity in the
     last row, which stands in for the rows behind it, makes its own column infinite and no other."""
     ctx, stream = gpu
     rng = np.random.default_rng(k * 37 + n)

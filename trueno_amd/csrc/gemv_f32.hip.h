@@ -5,7 +5,8 @@
 // A lane owns four neighbouring columns, so a wave reads 1 KB of a row of A with one 128-bit load per lane, and
 // the 8 waves of a workgroup take every eighth row of the workgroup's part of K (eight rows in flight per
 // wave).  x[k] is the same for the whole wave: it comes through the scalar cache.  The waves' sums meet in LDS
-// in wave order.  K is cut in parts over the grid so that a workgroup per CU exists and no more: one in flight per CU reads
+// in wave order.  K is cut in parts over the grid so that a workgroup per CU exists and no more (up to two for matrices of
+// more than 32768 columns, whose tiles alone do not divide well among the CUs): one in flight per CU reads
 // whole lines at 6.3 TB/s, two at 5.0 (4096 x 11008, 180 MB: 36.3 -> 28.7 us; 4096 x 4096 18.3 -> 15.3, 5000 x 3000
 // 20.0 -> 16.0, 1000 x 14336 14.0 -> 12.2, 14336 x 4000 37.9 -> 36.2).  With several parts every part
 // stores its partial y through to memory and the workgroup that arrives last at the column tile's counter adds

@@ -391,11 +391,14 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
     return hipModuleLaunchKernel(d->gemv_f32_generic, (n + 255u) / 256u, 1, 1, 256, 1, 1, 0, stream, args, nullptr);
   }
   const uint32_t tiles = (n + 255u) / 256u;
-  // parts of K: as many workgroups of 8 waves as there are CUs or somewhat fewer (gemv_f32.hip.h), two per CU only where one
-  // would leave a third of them idle; at least 64 rows (8 per wave) each
+  // parts of K, at least 64 rows (8 per wave) each: as many workgroups of 8 waves as there are CUs or somewhat fewer
+  // (gemv_f32.hip.h).  Two per CU where one would leave a third of them idle, if K is long enough to be worth three parts
+  // (33028 columns: 4096 rows 104.9 in one part, 98.3 us in three; 1003 rows 28.6 and 30.3; 256 rows 9.5 and 12.2), and from 256
+  // column tiles on, where a few workgroups more than CUs are a round of their own (65792 columns, 4096 rows: 240 us in
+  // one part, 199 in two; 65536: 170 and 162; 60000, 235 tiles: 141 and 146).
   const uint32_t cus = uint32_t(d->cu_count);
   uint32_t parts = std::max(1u, cus / tiles);
-  if (parts * tiles * 3u < cus * 2u) parts = 2u * cus / tiles;
+  if (tiles >= cus || (parts * tiles * 3u < cus * 2u && k >= 1024u)) parts = std::max(1u, (2u * cus + (tiles >= cus ? tiles / 2u : 0u)) / tiles);
   parts = std::max(1u, std::min(parts, (k + 63u) / 64u));
   uint32_t rows_per_part = (k + parts - 1u) / parts;
   rows_per_part = (rows_per_part + 7u) / 8u * 8u;
