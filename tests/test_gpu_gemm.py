@@ -704,3 +704,18 @@ def test_gemm_many_tokens_beside_one_value_much_larger(gpu, fmt):
             assert kq.rel_l2(gpu_gemm(gpu, fmt, buf, a, m, n, k), kq.gemm_fp64(a, w)) <= 2.5e-7, power
     finally:
         _tune("gemm_tall", 0)
+
+
+@pytest.mark.parametrize("fmt,m,n,k,many", [("q6k", 330, 6093, 2560, False), ("q4k", 84, 4506, 7936, False), ("q6k", 330, 11008, 2560, True)])
+def test_gemm_many_tokens_by_the_rule(gpu, fmt, m, n, k, many):
+    """A few workgroups more than there are CUs: 264 and 270, which the kernel for many tokens takes 15-20 % longer for than the one
+    that takes sixteen at a time (82 and 68 us, 38 and 33 us), so that one has them; 473 go to the former."""
+    buf, a = kq.gen_matrix(fmt, 694, n, k), kq.gen_x(695, m, k)
+    bits = {}
+    try:
+        for tall in (0, 1, 2):
+            _tune("gemm_tall", tall)
+            bits[tall] = gpu_gemm(gpu, fmt, buf, a, m, n, k).view(np.uint32)
+    finally:
+        _tune("gemm_tall", 0)
+    assert np.array_equal(bits[0], bits[2 if many else 1]) and not np.array_equal(bits[1], bits[2])

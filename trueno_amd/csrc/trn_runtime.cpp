@@ -498,20 +498,21 @@ size_t gemm_part_bytes(uint32_t kparts, uint32_t tiles, uint32_t groups, uint32_
   // per part of K, token tile and strip of 32 rows: 64 lanes x 8 sums
   return kparts > 1u ? (size_t(kparts) * tiles * groups * waves * 2048u + 255u) & ~size_t(255) : 0u;
 }
+double gemm_cut_us(Fmt f, uint32_t m, uint32_t n, uint32_t k, const GemmCut& c, uint64_t rounds) {      // rounds of a workgroup per CU
+  const double weight_us = double(n) * (k / 256u) * kSbBytes[f] / 5.0e6;      // the weights once at 5 TB/s: no cut is faster
+  const double step = c.waves == 4u ? 1.5 : c.waves == 12u ? 2.6 : c.nt == 2u ? 3.2 : 2.0;
+  const double last_kb = double(c.kparts) * c.waves * c.nt * (m > 8u ? 2.0 : 1.0);
+  return (c.waves == 4u ? 3.5 : 4.0) + std::max(double(rounds) * c.ksb * step, weight_us) + (c.kparts > 1u ? 2.5 + last_kb / 40.0 : 0.0);
+}
 GemmCut gemm_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k, size_t part_cap = ~size_t(0)) {
   const uint32_t nsb = k / 256u, tiles = (m + 15u) / 16u;
-  const double weight_us = double(n) * nsb * kSbBytes[f] / 5.0e6;      // the weights once at 5 TB/s: no cut is faster
   auto cut_with = [&](uint32_t waves, uint32_t nt, uint32_t kparts) {
     GemmCut c{waves, nt, (n + 32u * waves - 1u) / (32u * waves), (tiles + nt - 1u) / nt, 1u, nsb, 0.0};
     const uint64_t units = uint64_t(c.groups) * c.tgroups;
     c.kparts = std::min(std::max(kparts, 1u), nsb);
     c.ksb = (nsb + c.kparts - 1u) / c.kparts;
     c.kparts = (nsb + c.ksb - 1u) / c.ksb;
-    const uint64_t rounds = (units * c.kparts + uint64_t(d.cu_count) - 1u) / uint64_t(d.cu_count);
-    const double step = waves == 4u ? 1.5 : waves == 12u ? 2.6 : nt == 2u ? 3.2 : 2.0;
-    const double last_kb = double(c.kparts) * waves * nt * (m > 8u ? 2.0 : 1.0);
-    c.us = (waves == 4u ? 3.5 : 4.0) + std::max(double(rounds) * c.ksb * step, weight_us) +
-           (c.kparts > 1u ? 2.5 + last_kb / 40.0 : 0.0);
+    c.us = gemm_cut_us(f, m, n, k, c, (units * c.kparts + uint64_t(d.cu_count) - 1u) / uint64_t(d.cu_count));
     if (gemm_part_bytes(c.kparts, tiles, c.groups, waves) > part_cap) c.us = kCutDoesNotFit;
     return c;
   };
@@ -637,7 +638,7 @@ constexpr uint32_t kTallRows = 256, kTallTile = 32, kTallOperandBytes = 32u * 10
 // of 128 workgroups, an estimated 1161 us against 549 in one and 721 for sixteen tokens at a time.
 constexpr size_t kTallWorkspaceMax = size_t(256) << 20;
 size_t tall_workspace_cap() { return g_tune_gemm_workspace_mb > 0 ? std::min(size_t(g_tune_gemm_workspace_mb) << 20, kTallWorkspaceMax) : kTallWorkspaceMax; }
-struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit; };
+struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit, price = kCutDoesNotFit; };      // price: against the other kernel (tall_ok)
 uint32_t tall_lds_bytes(Fmt f) { return (f == Q6K ? 2u : 4u) * 8192u + 2u * 2048u + 4u * 64u * (f == Q6K ? 224u : kSbBytes[f]); }
 size_t tall_bytes(uint32_t tokens, uint32_t n, uint32_t nsb, uint32_t kparts) {
   const size_t tiles = (tokens + kTallTile - 1u) / kTallTile;
@@ -660,9 +661,9 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
   const double pair = f == Q4K ? 4.3 : f == Q5K ? 5.1 : 7.5, alone = f == Q4K ? 2.3 : f == Q5K ? 2.7 : 4.2;
   const uint32_t most = g_tune_gemm_ksplit > 0 ? std::min<uint32_t>(uint32_t(g_tune_gemm_ksplit), nsb)
                                                : uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>((2u * cus + units / 2u) / units, nsb)));
-  auto run_us = [&](const TallCut& c, uint32_t tokens) {
+  auto run_us = [&](const TallCut& c, uint32_t tokens, double uneven) {
     const uint64_t wgs = uint64_t(groups) * ((tokens + kTallTile - 1u) / kTallTile) * c.kparts, rounds = wgs / (2u * cus), rest = wgs - rounds * 2u * cus;
-    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * double(rest - cus) / cus;
+    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * (uneven + (1.0 - uneven) * double(rest - cus) / cus);
     return 9.0 + double(tokens) * k * 8.0 / 4.0e6 + c.ksb * (double(rounds) * pair + last) +
            (c.kparts > 1u ? 3.0 + 0.4 * c.kparts + double(c.kparts + 1u) * tokens * n * 4.0 / 4.0e6 : 0.0);
   };
@@ -672,7 +673,9 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
     c.kparts = (nsb + c.ksb - 1u) / c.ksb;
     const uint32_t step = tall_run(m, n, nsb, c.kparts, tall_workspace_cap());
     if (step != 0u) {
-      c.us = (m / step) * run_us(c, step) + (m % step != 0u ? run_us(c, m % step) : 0.0);
+      auto all_us = [&](double uneven) { return (m / step) * run_us(c, step, uneven) + (m % step != 0u ? run_us(c, m % step, uneven) : 0.0); };
+      c.us = all_us(0.0);
+      c.price = all_us(0.5);
       if (c.us < best.us) best = c;
     }
     if (g_tune_gemm_ksplit > 0) break;
@@ -821,20 +824,30 @@ extern "C" {      // (defined further down inside the extern "C" part of the fil
 hipError_t launch_gemv_group(DeviceKernels* d, hipStream_t stream, const trn_gemv_desc* descs, uint32_t len);
 }
 
-// Does the kernel for many tokens take this product?  From 33 tokens on, where its estimate is
-// below the other's: that one holds for Q4_K, while Q5_K takes 1.1 and Q6_K 1.3 to 1.6 times as long from 64 tokens on (the
-// factors below stay at the lower end).  Up to 32 tokens, one tile, it gained nothing anywhere (Q5_K 11008 x 4096, 17
-// tokens: 28 against 23 us).  Both sides measured over nine shapes, 17 .. 1024 tokens (us, sixteen at a time -> this kernel):
+// Does the kernel for many tokens take this product?  From 33 tokens on, where its estimate is below the other's: that one
+// holds for Q4_K, while Q5_K takes 1.1 and Q6_K 1.3 to 1.6 times as long from 64 tokens on (the factors below stay at the
+// lower end).  Up to 32 tokens, one tile, it gained nothing anywhere (Q5_K 11008 x 4096, 17 tokens: 28 against 23 us).
+// Both sides measured over nine shapes, 17 .. 1024 tokens (us, sixteen at a time -> this kernel):
 //   14336 x 4096, 2048 tokens, Q4_K 835 -> 525;   11008 x 4096, 512 tokens: Q4_K 180 -> 126, Q5_K 190 -> 142, Q6_K 318 -> 201
 //   4096 x 11008, 512 tokens: Q4_K 159 -> 129, Q5_K 167 -> 150, Q6_K 288 -> 195;   32000 x 4096, 64 tokens: 60 -> 55, 68 -> 63, 110 -> 84
 //   4096 x 4096, 64 tokens: 16 and 21 (Q4_K), 20 and 26 (Q6_K): stays;   1024 x 4096, 512 tokens, Q4_K: 24 and 29: stays
+// The estimates that choose each kernel's cut leave two things out, and with those counted it has to be the faster one still:
+// here, where some CUs have two workgroups and the others one, the launch ends with the former (half of the step from one
+// to two comes at once: Q6_K 6093 x 2560, 330 tokens, 264 workgroups, 82 us against 68); there, the rounds are an XCD's, whose 32
+// CUs get every eighth unit (Q4_K 32000 x 4096, 33 tokens: 88 us where 46 were estimated).  Of 1200 drawn products, 33 .. 900
+// tokens, that the first comparison gives to this kernel about 135 were 3 to 17 % slower with it; the second takes 112 of
+// them back, and with them twelve that it made 3 to 10 % faster.  (What the other kernel keeps although it is the slower one,
+// as in the example, stays: the cuts would have to be fitted anew with it.)
 bool tall_ok(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k, bool forced) {
   if (g_tune_gemm_tall == 1 || m <= 32u || k / 256u > 0x3FFFu || uint64_t((n + kTallRows - 1u) / kTallRows) * ((m + kTallTile - 1u) / kTallTile) > 0xFFFFFu)
     return false;
-  const double us = tall_cut(d, f, m, n, k).us;
-  if (g_tune_gemm_tall == 2) return us < kCutDoesNotFit;
+  const TallCut cut = tall_cut(d, f, m, n, k);
+  if (g_tune_gemm_tall == 2) return cut.us < kCutDoesNotFit;
   if (forced) return false;
-  return us < gemm_cut(d, f, m, n, k).us * (f == Q4K ? 1.0 : f == Q5K ? (m < 64u ? 1.05 : 1.1) : (m < 64u ? 1.1 : 1.3));
+  const GemmCut other = gemm_cut(d, f, m, n, k);
+  if (cut.us >= other.us * (f == Q4K ? 1.0 : f == Q5K ? (m < 64u ? 1.05 : 1.1) : (m < 64u ? 1.1 : 1.3))) return false;
+  const uint64_t xcd_cus = std::max(1u, uint32_t(d.cu_count) / 8u), xcd_wgs = (uint64_t(other.groups) * other.kparts + 7u) / 8u * other.tgroups;
+  return cut.price < gemm_cut_us(f, m, n, k, other, (xcd_wgs + xcd_cus - 1u) / xcd_cus) * (f == Q4K ? 1.09 : f == Q5K ? 1.14 : 1.4);
 }
 
 // Which kernel takes a product of m >= 1 tokens: the integer matrix cores (Q4_K, two to four tokens, where their fitted
