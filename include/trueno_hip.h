@@ -154,7 +154,8 @@ TRN_API trn_status trn_q6k_gemv(trn_stream stream, trn_dptr y, trn_dptr w, trn_d
  * GEMV-family one, so m = 1 equals the GEMV.  Replace QuantizeKernel::ggml / Q5KKernel / Q6KKernel
  * (quantize.rs:347-579, :640-866, :926-1121).  Which kernel takes a product is the library's choice by its shape (one
  * token: the GEMV engine; Q4_K, two to four tokens, k <= 4096: the integer matrix cores where that is fastest; otherwise
- * the f16 matrix cores, or for a few tokens against a small matrix the GEMV engine once per token); every one of them is
+ * the f16 matrix cores, sixteen tokens at a time or from 33 tokens on in tiles of 32 where that is faster, or for a few
+ * tokens against a small matrix the GEMV engine once per token); every one of them is
  * within the 1e-5 relative L2 of fp64 and no worse than an f32 evaluation in the reference's order, but they are not
  * bit-identical to each other.  An infinity or NaN among a token's activations makes that token's results non-finite
  * (NaN where the reference's sum would give an infinity) and leaves the other tokens alone. */
@@ -337,13 +338,15 @@ TRN_API trn_status trn_device_cu_count(int* count);
  * "gemm_few": the Q4_K product of two to four tokens on the integer matrix cores - 0 = where its estimated time is the
  * lowest, 1 = wherever it can run, 2 = never.
  * "gemm_mfma_off": 1 = the k-quant GEMMs never take the f16 matrix-core form; "gemm_k_parts": into how many parts
- * that form cuts K; "gemm_waves": 4, 8 or (Q4_K) 12 strips of 32 rows per workgroup; "gemm_tiles": 1 or 2 tiles of 16 tokens per
+ * that form, or the one for many tokens, cuts K; "gemm_waves": 4, 8 or (Q4_K) 12 strips of 32 rows per workgroup; "gemm_tiles": 1 or 2 tiles of 16 tokens per
  * workgroup (0 for each of the three = chosen from the shape by an estimated time; any of them set also keeps a
  * product of a few tokens on the matrix cores);
  * "gemm_tall": the kernel for many tokens - 0 = from 33 tokens on where its estimated time is the lower, 1 = never, 2 =
  * wherever it can run; "gemm_workspace_mb": what its workspace may hold, in MiB, at most 256 (0 = 256); "gemm_workspace_none": 1 = as if no memory were left for a further workspace of that kernel (it then
  * leaves the product to the other one);
- * "attention_per_cu": workgroups per CU the single-query attention aims at (0 = 2); "attention_min_steps": least
+ * "attention_tiled": the matrix-core form of the single-query attention (head_dim 64 and 128) - 0 = by a rule on the heads
+ * and the positions, 1 = never, 2 = wherever it can run;
+ * "attention_per_cu": workgroups per CU the single-query attention aims at (0 = 2, 1 for the matrix-core form); "attention_min_steps": least
  * number of steps (of 8 positions at head_dim 128) in a chunk of positions (0 = 8). */
 TRN_API trn_status trn_set_tuning(const char* key, int value);
 

@@ -596,7 +596,8 @@ __device__ __forceinline__ void kq_body(const float* __restrict__ a, const uint8
 //     sc[8g ..]).  Token page Q of the Q4_K layout (values 128g + 64(U/4) + 32(Q%2) + 8(U%4) + .., U = Q/2) holds the
 //     eight values that the low (U/4 = 0) or high nibbles of ql dwords 8(Q%2) + 2(U%4) + {0, 1} and field 2(U/4) + Q%2 of
 //     qh dwords 2(U%4) + {0, 1} belong to: one read of a token page feeds two products.
-//   * blocks of 210 bytes are only 2-byte aligned, which the copy into LDS by DMA does not take: the weight tile of
+//   * blocks of 210 bytes are only 2-byte aligned and not whole 16-byte pieces (copies into LDS do take such sources, at 14
+//     pieces a block: kquant_gemm_tall.hip.h; here it was built otherwise): the weight tile of
 //     the NEXT super-block travels through registers (13 sixteen-byte loads and one 2-byte load per row, issued a
 //     super-block ahead, written to LDS when the current one's products are done; rows 240 bytes apart in LDS, 15 pieces).
 // Everything else (token conversion, parts of K, the sum over the parts) is the Q4_K kernel's.

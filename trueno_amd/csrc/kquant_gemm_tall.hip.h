@@ -4,7 +4,7 @@
 // f16 pieces of a run of 256 scaled by a power of two.  There a wave multiplies 32 rows of W with 16 tokens at a time and
 // builds the weight operand anew for each 16: with many tokens the vector unit and the LDS (a page of token operands per
 // matrix instruction) are what it waits for.  Here the activations are made into operands once, by a launch of their own
-// (2048 x 4096: 11 us), and a wave holds a tile of 64 rows x 32 tokens: an operand of either side feeds two matrix
+// (2048 x 4096: 11 us, 16 with the activations out of the caches), and a wave holds a tile of 64 rows x 32 tokens: an operand of either side feeds two matrix
 // instructions, so LDS reads and operand building halve.
 //   * A workgroup is four waves with a strip of 64 rows each against one tile of 32 tokens, two workgroups a CU (80 KB of
 //     LDS, 256 registers): their phases drift apart, so that one's sums and headers run under the other's products.
@@ -18,9 +18,9 @@
 //     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by after
 //     about the root of their number.  Against fp64 the error is 0.82 .. 0.98 times the 16-token kernel's, over 70 shapes a
 //     format drawn from 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns that the rule gives this kernel.
-//   * Measured (us, the 16-token kernel -> this one): Q4_K 14336 x 4096, 2048 tokens 835 -> 525 (matrix cores busy 52 % of
-//     the cycles at 1.7 GHz, the power limit's clock; the vector unit issues 40 %; a library f16 product with as many
-//     matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 190.
+//   * Measured (us, the 16-token kernel -> this one): Q4_K 14336 x 4096, 2048 tokens 835 -> 534 (matrix cores busy 56 % of
+//     the cycles at 1.7 GHz, the power limit's clock, nine vector instructions to a matrix instruction; a library f16 product
+//     with as many matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 193 (32 %, thirteen to one).
 #pragma once
 #include "kquant_gemm_f16.hip.h"
 #include <utility>

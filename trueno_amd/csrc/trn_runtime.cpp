@@ -429,7 +429,9 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
   if ((head_dim == 64u || head_dim == 128u) && num_heads % num_kv_heads == 0u && g_tune_attention_tiled != 1 &&
       (num_heads > num_kv_heads || head_dim == 64u || seq_len >= 4096u || g_tune_attention_tiled == 2)) {
     // the query heads of a KV head together, in tiles of 16 positions (both sides measured: decode_attention.hip.h; a
-    // head alone with 128 dims only with many positions: 32 heads, 2048 positions 16.7 against 16.1 us, 8192 43.3 against 45.5): a
+    // head alone with 128 dims only with many positions: 32 heads, 2048 positions 16.7 against 16.1 us, 8192 43.3 against 45.5; under 200 positions it is
+    // as fast or faster with the cache out of L2, 8 heads over one KV head x 128, 153 positions 8.6 -> 8.1, 64 over 8, 58
+    // positions 6.7 -> 5.5, and 0.2 to 0.4 us slower with it in L2, the former 1.6): a
     // workgroup per CU (two are slower at every length, 28.8 against 18.7 us with 8 KV heads and 8192 positions), at least a tile a wave
     const uint32_t waves = head_dim == 64u ? 8u : 4u, most_heads = 8u, step = 16u * waves;
     uint32_t per_kv = num_heads / num_kv_heads, subs = (per_kv + most_heads - 1u) / most_heads, groups = num_kv_heads * subs;
