@@ -36,10 +36,14 @@ extern "C" __attribute__((visibility("hidden"))) hipError_t trn_noalloc_scratch_
   if (e != hipSuccess) return e;
   if (!ptr) return hipErrorInvalidSymbol;
   if ((e = hipMemset(ptr, 0, kCounterBytes)) != hipSuccess) return e;
+  // (a capture in progress on another thread is none of this allocation's business)
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   if (hipMalloc(&g_workspace_ptr[dev], kWorkspaceBytes) != hipSuccess) {      // without it the entry point takes the other kernel
     (void)hipGetLastError();
     g_workspace_ptr[dev] = nullptr;
   }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   g_scratch_ptr[dev] = ptr;
   return hipSuccess;
 }
