@@ -129,3 +129,33 @@ def test_gpu_attention_heads_of_a_kv_head_together(gpu, heads, kv_heads, max_seq
     assert kq.rel_l2(got, want) <= 2e-6       # f32: a score's error (about 3e-7 of 2 sigma) is its weight's, the sums add less
     assert np.array_equal(again.view(np.uint32), got.view(np.uint32))
     assert np.all(np.delete(got_inf, 3, axis=1) == np.delete(got, 3, axis=1)) and not np.any(np.isfinite(got_inf[:, 3]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads,dim,max_seq,seq", [
+    (1, 1, 256, 20, 17), (8, 1, 256, 700, 641), (6, 3, 256, 2100, 2049), (24, 2, 256, 130, 127),       # 256 dims: two pairs of (head, quad) a thread, one
+    (1, 1, 128, 5000, 4993), (2, 1, 64, 9000, 8500), (8, 2, 128, 9000, 8200), (8, 1, 128, 5000, 4999),  # 79, 133, 129 and 79 chunks: 16, 8, 4 and 2 slices
+    (4, 4, 128, 1100, 1025), (4, 4, 128, 1100, 1024),                                                  # 17 chunks and 16
+    (128, 128, 128, 905, 897), (128, 128, 128, 905, 896)])                                             # four waves a workgroup and eight
+def test_gpu_attention_tiles_through_lds(gpu, heads, kv_heads, dim, max_seq, seq):
+    """The edges of the tiled form: the last tile of a chunk, how the chunks are joined, the number of waves; what lies behind
+    the positions is NaN."""
+    ctx, stream = gpu
+    q, k, v = _case(heads * 100 + seq + dim, heads, kv_heads, max_seq, dim, spread=2.0)
+    k[:, seq:], v[:, seq:] = np.nan, np.nan
+    dq, dk, dv = (t.GpuBuffer.from_host(ctx, a.reshape(-1)) for a in (q, k, v))
+    kern = t.IncrementalAttentionKernel.with_gqa(max_seq, dim, heads, kv_heads)
+    L = t._ffi.lib()
+    assert L.trn_set_tuning(b"attention_tiled", 2) == 0
+    try:
+        got = []
+        for _ in range(2):
+            do = t.GpuBuffer.from_host(ctx, np.full(heads * dim, np.nan, np.float32))
+            kern.launch(stream, dq, dk, dv, do, seq)
+            stream.synchronize()
+            got.append(do.copy_to_host().reshape(heads, dim))
+    finally:
+        L.trn_set_tuning(b"attention_tiled", 0)
+    want = glue.attention_fp64(q, k[:, :seq], v[:, :seq], seq)
+    assert kq.rel_l2(got[0], want) <= 2e-6       # as above
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))

@@ -14,6 +14,7 @@
 // are 2^x on scores pre-multiplied by log2(e), as in the reference (ex2.approx there, v_exp_f32 here).
 #pragma once
 #include "kquant_common.hip.h"
+#include <type_traits>
 
 namespace decode_attention {
 
@@ -158,28 +159,39 @@ __device__ __forceinline__ void body(const float* __restrict__ q, const float* _
   }
 }
 
-// ---- head dimensions 64 and 128, the query heads of a KV head together (matrix cores, v_mfma_f32_16x16x4_f32) ----
+// ---- head dimensions 64, 128 and 256, the query heads of a KV head together (matrix cores, v_mfma_f32_16x16x4_f32) ----
 // The kernel above reads the cache once per query head and spends about thirty vector instructions per two positions on the
 // reduction over a position's lanes and the rescaling.  Here the query heads that share a KV head are the columns of
 // a matrix product (f32 throughout; up to eight of them), so the cache is read once:
-//   scores[16 positions][heads] = K tile . q,  lane l: K[position l%16][dims 16 j + 4 g + e], g = l/16, a 16-byte load for
-//     four products;
+//   scores[16 positions][heads] = K tile . q,  lane l: K[position l%16][dims 16 j + 4 g + e], g = l/16, one 16-byte LDS read
+//     for four products;
 //   out[dims][heads] += V tile . p,  product v takes the positions 4 g + v: the score registers are its operand as they
-//     lie, and V[position 4 g + v][dims 64 h + 4 (l%16) + e] is read in whole lines.
+//     lie, and V[position 4 g + v][dims 64 h + 4 (l%16) + e] is read in whole rows.
 // A lane's running maximum and the factor of its sums belong to one head, l%16: nothing crosses lanes but the maximum of a
-// tile (two swaps).  K of the next tile is asked for when the scores are made, V when the sums are.
+// tile (two swaps).
+// Data movement: a wave's tile of 16 positions comes by copies into LDS, a KB of whole lines each and non-temporal (every line
+// is read once; without the hint 128 query heads over 32 KV heads, 16384 positions: 97 us, with it 86).  K goes to registers
+// as soon as it is there, and its place takes the next tile's K before the first product; V the same.  So every wave has one
+// to two halves of a tile on their way while it computes, no register holds a load in flight, and two waves a SIMD fit
+// (with K and V in registers they did not: 24 us where four waves took 18.7).
 // Rounding: a score is added up in a tree over sums of four products, a tile's share of the output starts at zero (eight
-// products in a row), waves and chunks meet in trees.  Against fp64 the error is, on the average over 16 inputs, 0.94 .. 1.03 times
-// the kernel's above up to 256 positions (no more: one input scatters by 5-10 %) and 0.98 .. 0.70 times from there to 8192.
-// Bound by HBM with many positions; what is in flight is the next tile of every wave (16 KB at 128 dims).  Measured (us,
-// the kernel above -> this one; 32 query heads x 128 unless said): 8 KV heads, 8192 positions 31.5 -> 18.7; 32 KV heads,
-// 8192 positions 45.5 -> 43.3, 2048 positions 17.5 -> 17.3 (cold), 512 positions 10.0 -> 9.4 (cold); 64 heads x 64 over 16
-// KV heads, 700 positions 9.4 -> 7.1.  With 128 dims workgroups of eight waves spill (24 us where four waves take 18.7),
-// with 64 dims eight waves are faster than four (14.1 against 16.7 us, 32 KV heads, 4000 positions).  256 dims need 256
-// registers for K, V, q and the sums alone: they spill, and stay with the kernel above (as do head counts that the number
-// of KV heads does not divide).
+// products in a row), waves and chunks meet in trees.  Against fp64, averages over 16 inputs: 0.88 .. 0.99 of the kernel's
+// above with a head alone, 128 dims, 64 .. 3000 positions; 0.80 .. 0.86 with 256 dims and two heads.
+// Bound by HBM with many positions, by latency with few.  A launch of 17 us (8 KV heads, 8192 positions, 67 MB) spends 1 before
+// the first copies are out (a CU has 64 KB in flight, no more), 11 on the stream, 1 on the last tile, 4 at the end: the store
+// of a chunk's state has to be acknowledged, the counter answers, the states come back.
+// Measured (us, before -> now: before is the kernel above, or for 64 dims, several heads and from 4096 positions on one that
+// kept K and V in registers, four waves a CU; 128 dims unless said): 32 heads over 8, 8192 positions 19.0 -> 17.1; 32 heads of their
+// own, 2048 positions 16.65 -> 15.2, 1024 12.3 -> 10.7, 512 9.0 -> 8.2; four heads, 16000 positions 21.5 -> 16.9; 128 heads over 32,
+// 16384 positions 84.0 -> 81.9 (6.6 TB/s); 256 dims, 64 heads over 16, 8000 positions 99.7 -> 52.
+// Waves: eight; with 128 dims four where a wave of eight would still have more than four tiles, that is more than 512 positions a
+// workgroup (128 heads over 32, 16384 positions: 85.7 with eight, 80.5-81.9 with four: fewer streams at a time; 32 over 8, 8192
+// positions: 17.0 and 17.8).  256 dims: four, an LDS tile is 32 KB.
 constexpr u32 kTiledHeads = 8;
-template <int DIM> struct Tiled { static constexpr u32 WAVES = DIM == 64 ? 8u : 4u; };
+template <int DIM, int W> struct Tiled {
+  static constexpr u32 HALF = 64u * DIM;               // bytes of a wave's tile: 16 positions of K, then of V
+  static constexpr u32 LDS = W * 2u * HALF;
+};
 
 __device__ __forceinline__ float max_over_groups(float v) {      // over the four lanes l, l ^ 16, l ^ 32, l ^ 48
   const u32 b = __float_as_uint(v);
@@ -201,23 +213,23 @@ __device__ __forceinline__ float sum_over_groups(float v) {
 __device__ __forceinline__ float factor(float a, float b) { return a == b ? 1.0f : __builtin_amdgcn_exp2f(a - b); }
 
 // N states in registers (their o for the caller's four dims) as one; N a power of two
-template <int N>
+template <u32 N>
 __device__ __forceinline__ State merge_tree(const float (&m)[N], const float (&s)[N], const f32x4 (&o)[N]) {
   float top = m[0];
 #pragma unroll
-  for (int i = 1; i < N; ++i) top = fmaxf(top, m[i]);
+  for (u32 i = 1; i < N; ++i) top = fmaxf(top, m[i]);
   float ss[N];
   f32x4 oo[N];
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
+  for (u32 i = 0; i < N; ++i) {
     const float f = factor(m[i], top);
     ss[i] = s[i] * f;
     oo[i] = o[i] * f;
   }
 #pragma unroll
-  for (int w = N / 2; w >= 1; w /= 2)
+  for (u32 w = N / 2; w >= 1; w /= 2)
 #pragma unroll
-    for (int i = 0; i < w; ++i) {
+    for (u32 i = 0; i < w; ++i) {
       ss[i] += ss[i + w];
       oo[i] += oo[i + w];
     }
@@ -225,27 +237,66 @@ __device__ __forceinline__ State merge_tree(const float (&m)[N], const float (&s
 }
 
 // group = KV head * subs + sub: the query heads head0 .. head0 + heads - 1 of a KV head (per_kv of them, eight at a time)
-template <int DIM>
+template <int DIM, int W>     // W waves
 __device__ __forceinline__ void tiled_body(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
                                            float* __restrict__ out, u32 seq_len, u32 per_kv, u32 subs, u32 max_seq_len, float scale,
-                                           u32 chunk, u32 chunks, u32 groups, float* __restrict__ partial, u32* __restrict__ counters) {
-  constexpr u32 W = Tiled<DIM>::WAVES, H = kTiledHeads, Q = DIM / 4;      // quads of a head's output
-  constexpr int KJ = DIM / 16, VH = DIM / 64;
+                                           u32 chunk, u32 chunks, u32 groups, float* __restrict__ partial, u32* __restrict__ counters,
+                                           uint8_t* lds) {
+  using T = Tiled<DIM, W>;
+  constexpr u32 H = kTiledHeads, Q = DIM / 4, kRowBytes = 4u * DIM;      // Q: quads of a head's output
+  constexpr int KJ = DIM / 16, VH = DIM / 64, COPIES = T::HALF / 1024u;
   __shared__ float s_m[W][H], s_s[W][H];
-  __shared__ f32x4 s_o[W][H][Q];
   __shared__ u32 s_old;
-  const u32 lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, col = lane & 15u, g = lane >> 4;
+  const u32 lane = threadIdx.x & 63u, col = lane & 15u, g = lane >> 4;
+  const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
   const u32 group = blockIdx.x / chunks, ci = blockIdx.x - group * chunks;
   const u32 kv_head = group / subs, sub = group - kv_head * subs;
   const u32 head0 = kv_head * per_kv + sub * H, heads = min(H, per_kv - sub * H);
-  const f32x4* kp = reinterpret_cast<const f32x4*>(k + static_cast<size_t>(kv_head) * max_seq_len * DIM) + g;
-  const f32x4* vp = reinterpret_cast<const f32x4*>(v + static_cast<size_t>(kv_head) * max_seq_len * DIM) + col;
-  f32x4 qv[KJ];
+  const u32 p0 = ci * chunk, len = min(seq_len, p0 + chunk) - p0;      // positions of this chunk (>= 1)
+  u32x4 qv[KJ];      // in asm, like the waits: the compiler would wait for every copy behind them
 #pragma unroll
-  for (int j = 0; j < KJ; ++j)
-    qv[j] = col < heads ? reinterpret_cast<const f32x4*>(q + static_cast<size_t>(head0 + col) * DIM)[4 * j + g] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int j = 0; j < KJ; ++j) {
+    const float* src = q + static_cast<size_t>(head0 + min(col, heads - 1u)) * DIM + 16 * j + 4u * g;
+    asm volatile("global_load_dwordx4 %0, %1, off" : "=&v"(qv[j]) : "v"(src) : "memory");
+  }
+  // Copies into LDS, a KB of whole lines each.  Positions behind the chunk are outside the buffer: nothing is read for them
+  // (what lies in their place has weight 0).
+  const size_t kv_at = (static_cast<size_t>(kv_head) * max_seq_len + p0) * DIM;
+  const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(k) + kv_at, 0, static_cast<int>(len * kRowBytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(v) + kv_at, 0, static_cast<int>(len * kRowBytes), 0x00020000);
+  const u32 lds_k = static_cast<u32>(reinterpret_cast<size_t>((const __attribute__((address_space(3))) uint8_t*)lds)) + wave * (2u * T::HALF);
+  const u32 lds_v = lds_k + T::HALF;
+  // V lies in LDS as in memory.  K's unit u (16 bytes) of row r lies at u ^ r: the reads below take one unit of sixteen rows.
+  constexpr u32 kRowsPerCopy = 1024u / kRowBytes;
+  const u32 row_in = lane / Q, unit = lane - row_in * Q;
+  u32 koff[COPIES];
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) koff[i] = row_in * kRowBytes + (unit ^ (i * kRowsPerCopy + row_in)) * 16u;
+  // (the whole offset in the lane's register: a scalar part of it beyond the buffer's end would wrap the bounds check)
+  auto copy = [&](__amdgpu_buffer_rsrc_t rsrc, u32 dst, u32 off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(uintptr_t)dst, 16, static_cast<int>(off), 0, 0, 2 /* nt */);
+  };
+  auto copy_k = [&](u32 p) {
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy(k_rsrc, lds_k + 1024u * i, koff[i] + (p * kRowBytes + 1024u * i));
+  };
+  auto copy_v = [&](u32 p) {
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy(v_rsrc, lds_v + 1024u * i, lane * 16u + (p * kRowBytes + 1024u * i));
+  };
+  u32 p = wave * 16u;      // of the chunk
+  // (also by a wave that has no position: outside the buffer)
+  copy_k(p);
+  copy_v(p);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * COPIES) : "memory");
+#pragma unroll
+  for (int j = 0; j < KJ; ++j) {
+    asm volatile("" : "+v"(qv[j])::"memory");
+    if (col >= heads) qv[j] = u32x4{0u, 0u, 0u, 0u};
+  }
+  const u32 k_read = lds_k + col * kRowBytes + 16u * (g ^ (col & 3u)) + 64u * (col >> 2);      // unit 4 j + g: bits 6 and 7 ^ j, then 256 bytes on
+  const u32 v_read = lds_v + 4u * g * kRowBytes + 16u * col;
   const float sl = scale * kLog2e;
-  const u32 p0 = ci * chunk, p1 = min(seq_len, p0 + chunk);
   float m = -INFINITY, s = 0.0f;
   const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
   f32x4 o[VH][4];
@@ -253,74 +304,81 @@ __device__ __forceinline__ void tiled_body(const float* __restrict__ q, const fl
   for (int h = 0; h < VH; ++h)
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[h][e] = zero4;
-  f32x4 kk[KJ], vv[4][VH];
-  auto load_k = [&](u32 p) {      // (positions behind the chunk: its last one, which the cache holds; their weight is 0)
-    const f32x4* row = kp + static_cast<size_t>(min(p + col, p1 - 1u)) * Q;
+  for (; p < len; p += W * 16u) {
+    const bool more = p + W * 16u < len;
+    u32x4 kk[KJ];
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COPIES) : "memory");      // K is there, V behind it
 #pragma unroll
-    for (int j = 0; j < KJ; ++j) kk[j] = row[4 * j];
-  };
-  auto load_v = [&](u32 p) {
+    for (int j = 0; j < KJ; ++j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(kk[j]) : "v"(k_read ^ (64u * (j & 3))), "n"(256 * (j >> 2)) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const f32x4* row = vp + static_cast<size_t>(min(p + 4u * g + a, p1 - 1u)) * Q;
-#pragma unroll
-      for (int h = 0; h < VH; ++h) vv[a][h] = __builtin_nontemporal_load(row + 16 * h);
-    }
-  };
-  u32 p = p0 + wave * 16u;
-  if (p < p1) {
-    load_k(p);
-    load_v(p);
-  }
-  for (; p < p1; p += W * 16u) {
+    for (int j = 0; j < KJ; ++j) asm volatile("" : "+v"(kk[j])::"memory");
+    if (more) copy_k(p + W * 16u);      // K is in registers: its place takes the next tile's
     f32x4 sc[KJ];
 #pragma unroll
     for (int j = 0; j < KJ; ++j) {
       f32x4 part[4];
+      const f32x4 kj = __builtin_bit_cast(f32x4, kk[j]), qj = __builtin_bit_cast(f32x4, qv[j]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[j][e], qv[j][e], zero4, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kj[e], qj[e], zero4, 0, 0, 0);
       sc[j] = (part[0] + part[1]) + (part[2] + part[3]);
-      __builtin_amdgcn_sched_barrier(0);      // (all the products first would take four times the registers, and spill)
+      __builtin_amdgcn_sched_barrier(0);      // (all the products first would take four times the registers)
     }
 #pragma unroll
     for (int w = KJ / 2; w >= 1; w /= 2)
 #pragma unroll
       for (int j = 0; j < w; ++j) sc[j] += sc[j + w];
-    const bool more = p + W * 16u < p1;
-    if (more) load_k(p + W * 16u);
     float x[4], top = -INFINITY;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       x[a] = sc[0][a] * sl;
-      if (p + 4u * g + a < p1) top = fmaxf(top, x[a]);      // (a NaN comes in again with its own weight)
+      if (p + 4u * g + a < len) top = fmaxf(top, x[a]);      // (a NaN comes in again with its own weight)
     }
     const float nm = fmaxf(m, max_over_groups(top)), c = factor(m, nm);
     m = nm;
     float w[4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) w[a] = p + 4u * g + a < p1 ? factor(x[a], nm) : 0.0f;
-    if (p + 16u > p1) {      // a last tile that is not full: what stands in for the missing rows may be infinite, their weight is 0
+    for (int a = 0; a < 4; ++a) w[a] = p + 4u * g + a < len ? factor(x[a], nm) : 0.0f;
+    s = fmaf(s, c, (w[0] + w[1]) + (w[2] + w[3]));
+    u32x4 vv[4][VH];
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(COPIES) : "memory");      // V is there, the next K behind it
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < VH; ++h)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(vv[a][h]) : "v"(v_read), "n"(a * kRowBytes + 256 * h) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < VH; ++h)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) asm volatile("" : "+v"(vv[a][h])::"memory");
+    if (more) copy_v(p + W * 16u);
+    if (p + 16u > len) {      // a last tile that is not full: what lies behind the positions may be anything, their weight is 0
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int h = 0; h < VH; ++h) vv[a][h] = p + 4u * g + a < p1 ? vv[a][h] : zero4;
+        for (int h = 0; h < VH; ++h) vv[a][h] = p + 4u * g + a < len ? vv[a][h] : u32x4{0u, 0u, 0u, 0u};
     }
-    s = fmaf(s, c, (w[0] + w[1]) + (w[2] + w[3]));
 #pragma unroll
     for (int h = 0; h < VH; ++h) {
       f32x4 t[2][4];
 #pragma unroll
-      for (int a = 0; a < 4; ++a)
+      for (int a = 0; a < 4; ++a) {
+        const f32x4 va = __builtin_bit_cast(f32x4, vv[a][h]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[a >> 1][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[a][h][e], w[a], (a & 1) ? t[a >> 1][e] : zero4, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) t[a >> 1][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[e], w[a], (a & 1) ? t[a >> 1][e] : zero4, 0, 0, 0);
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int a = 0; a < 4; ++a) o[h][e][a] = fmaf(o[h][e][a], c, t[0][e][a] + t[1][e][a]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (more) load_v(p + W * 16u);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (a wave without positions: its copies)
+  // The waves' states meet in LDS, each in its own wave's tile: [head][quad]
+  f32x4* s_o = reinterpret_cast<f32x4*>(lds);
+  constexpr u32 kWaveUnits = 2u * T::HALF / 16u;
   s = sum_over_groups(s);
   if (col < heads) {
     if (g == 0u) {
@@ -331,42 +389,39 @@ __device__ __forceinline__ void tiled_body(const float* __restrict__ q, const fl
 #pragma unroll
     for (int h = 0; h < VH; ++h)
 #pragma unroll
-      for (int a = 0; a < 4; ++a) s_o[wave][col][16 * h + 4 * g + a] = f32x4{o[h][0][a], o[h][1][a], o[h][2][a], o[h][3][a]};
+      for (int a = 0; a < 4; ++a) s_o[wave * kWaveUnits + col * Q + 16 * h + 4 * g + a] = f32x4{o[h][0][a], o[h][1][a], o[h][2][a], o[h][3][a]};
   }
   __syncthreads();
-  // a thread per (head, quad of dims): the waves in order, then the chunks in order by the workgroup that arrives last
-  const u32 hd = threadIdx.x / Q, quad = threadIdx.x - hd * Q;
-  const bool mine = hd < heads;
-  State st = {-INFINITY, 0.0f, zero4};
-  if (mine) {      // (a wave without positions brings nothing: zeros under a maximum of -infinity)
-    float wm[W], ws[W];
-    f32x4 wo[W];
-#pragma unroll
-    for (u32 w = 0; w < W; ++w) {
-      wm[w] = s_m[w][hd];
-      ws[w] = s_s[w][hd];
-      wo[w] = s_o[w][hd][quad];
-    }
-    st = merge_tree<W>(wm, ws, wo);
-  }
-  f32x4* dst = reinterpret_cast<f32x4*>(out + static_cast<size_t>(head0 + hd) * DIM) + quad;
-  if (chunks == 1u) {
-    if (mine) {
-      const float inv = 1.0f / st.s;
-      *dst = f32x4{st.o.x * inv, st.o.y * inv, st.o.z * inv, st.o.w * inv};
-    }
-    return;
-  }
+  // a thread per (head, quad of dims), or two: the waves in a tree (one without positions brings zeros under a maximum of
+  // -infinity), then the chunks by the workgroup that arrives last
+  constexpr u32 kThreads = 64u * W;
+  const u32 pairs = heads * Q;
   // [group][chunk][head][quads, then {m, s}] through to memory: 16-byte buffer accesses at agent scope (sc1)
   constexpr u32 kHeadBytes = (Q + 1u) * 16u;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(partial, 0, static_cast<int>(groups * chunks * H * kHeadBytes), 0x00020000);
-  auto slot = [&](u32 c) { return ((group * chunks + c) * H + hd) * kHeadBytes; };
-  if (mine) {
-    __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(st.o.x), __float_as_uint(st.o.y), __float_as_uint(st.o.z), __float_as_uint(st.o.w)},
-                                           rsrc, static_cast<int>(slot(ci) + quad * 16u), 0, 16);
-    if (quad == 0u)
-      __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(st.m), __float_as_uint(st.s), 0u, 0u}, rsrc, static_cast<int>(slot(ci) + Q * 16u), 0, 16);
+  auto slot = [&](u32 c, u32 hd) { return ((group * chunks + c) * H + hd) * kHeadBytes; };
+  f32x4* dst = reinterpret_cast<f32x4*>(out + static_cast<size_t>(head0) * DIM);
+  for (u32 i = threadIdx.x; i < pairs; i += kThreads) {
+    const u32 hd = i / Q, quad = i - hd * Q;
+    float wm[W], ws[W];
+    f32x4 wo[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      wm[w] = s_m[w][hd];
+      ws[w] = s_s[w][hd];
+      wo[w] = s_o[w * kWaveUnits + i];
+    }
+    const State st = merge_tree<W>(wm, ws, wo);
+    if (chunks == 1u) {
+      const float inv = 1.0f / st.s;
+      dst[i] = st.o * inv;
+    } else {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, st.o), rsrc, static_cast<int>(slot(ci, hd) + quad * 16u), 0, 16);
+      if (quad == 0u)
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(st.m), __float_as_uint(st.s), 0u, 0u}, rsrc, static_cast<int>(slot(ci, hd) + Q * 16u), 0, 16);
+    }
   }
+  if (chunks == 1u) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the coherent stores have been acknowledged
   __syncthreads();
   if (threadIdx.x == 0u) {
@@ -375,31 +430,74 @@ __device__ __forceinline__ void tiled_body(const float* __restrict__ q, const fl
     s_old = old;
   }
   __syncthreads();
-  if (s_old != chunks - 1u || !mine) return;
-  State tot = {-INFINITY, 0.0f, zero4};
-  constexpr u32 kRound = 16;
-  for (u32 c0 = 0; c0 < chunks; c0 += kRound) {
-    u32x4 ms[kRound], ov[kRound];
+  if (s_old != chunks - 1u) return;
+  // The last workgroup: runs of chunks by as many slices of its threads as there are, then the slices in order.
+  // (Up to sixteen chunks are joined in one tree: scaled once, as the waves' states are.)
+  constexpr u32 kMostSlices = 16;
+  u32 slices = 1u;
+  while (chunks > 16u && slices < kMostSlices && 2u * slices * pairs <= kThreads && slices * 8u < chunks) slices *= 2u;
+  const u32 per_slice = (chunks + slices - 1u) / slices;
+  for (u32 i0 = 0; i0 < pairs; i0 += kThreads) {
+    const u32 i = i0 + threadIdx.x, slice = i0 == 0u && slices > 1u ? threadIdx.x / pairs : 0u, pair = i - slice * pairs;
+    const bool mine = slice < slices && pair < pairs;
+    State tot = {-INFINITY, 0.0f, zero4};
+    if (mine) {
+      const u32 hd = pair / Q, quad = pair - hd * Q, c1 = min(chunks, (slice + 1u) * per_slice);
+      auto join = [&](auto n_c) {      // chunks in flight together
+        constexpr u32 N = decltype(n_c)::value;
+        for (u32 c0 = slice * per_slice; c0 < c1; c0 += N) {
+          u32x4 ms[N], ov[N];
 #pragma unroll
-    for (u32 cc = 0; cc < kRound; ++cc) {
-      const u32 at = slot(min(c0 + cc, chunks - 1u));
-      ms[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + Q * 16u), 0, 16);
-      ov[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + quad * 16u), 0, 16);
-    }
-    float cm[kRound], cs[kRound];
-    f32x4 co[kRound];
+          for (u32 cc = 0; cc < N; ++cc) {
+            const u32 at = slot(min(c0 + cc, c1 - 1u), hd);
+            ms[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + Q * 16u), 0, 16);
+            ov[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + quad * 16u), 0, 16);
+          }
+          float cm[N], cs[N];
+          f32x4 co[N];
 #pragma unroll
-    for (u32 cc = 0; cc < kRound; ++cc) {
-      const bool there = c0 + cc < chunks;
-      cm[cc] = there ? __uint_as_float(ms[cc].x) : -INFINITY;
-      cs[cc] = there ? __uint_as_float(ms[cc].y) : 0.0f;
-      co[cc] = there ? f32x4{__uint_as_float(ov[cc].x), __uint_as_float(ov[cc].y), __uint_as_float(ov[cc].z), __uint_as_float(ov[cc].w)} : zero4;
+          for (u32 cc = 0; cc < N; ++cc) {
+            const bool there = c0 + cc < c1;
+            cm[cc] = there ? __uint_as_float(ms[cc].x) : -INFINITY;
+            cs[cc] = there ? __uint_as_float(ms[cc].y) : 0.0f;
+            co[cc] = there ? __builtin_bit_cast(f32x4, ov[cc]) : zero4;
+          }
+          const State r = merge_tree<N>(cm, cs, co);
+          merge(tot, r.m, r.s, r.o);
+        }
+      };
+      if (per_slice <= 8u) join(std::integral_constant<u32, 8>{});
+      else join(std::integral_constant<u32, 16>{});
     }
-    const State r = merge_tree<kRound>(cm, cs, co);
-    merge(tot, r.m, r.s, r.o);
+    if (slices > 1u) {      // (pairs <= kThreads / 2 then: this loop's only round, and every thread is here)
+      f32x2* s_ms = reinterpret_cast<f32x2*>(s_o + kThreads);
+      s_o[threadIdx.x] = tot.o;
+      s_ms[threadIdx.x] = f32x2{tot.m, tot.s};
+      __syncthreads();
+      if (threadIdx.x >= pairs) return;
+      auto join_slices = [&](auto n_c) {
+        constexpr u32 N = decltype(n_c)::value;
+        float jm[N], js[N];
+        f32x4 jo[N];
+#pragma unroll
+        for (u32 n = 0; n < N; ++n) {
+          const f32x2 ms = s_ms[n * pairs + threadIdx.x];
+          jm[n] = ms.x;
+          js[n] = ms.y;
+          jo[n] = s_o[n * pairs + threadIdx.x];
+        }
+        tot = merge_tree<N>(jm, js, jo);
+      };
+      if (slices == 2u) join_slices(std::integral_constant<u32, 2>{});
+      else if (slices == 4u) join_slices(std::integral_constant<u32, 4>{});
+      else if (slices == 8u) join_slices(std::integral_constant<u32, 8>{});
+      else join_slices(std::integral_constant<u32, kMostSlices>{});
+    }
+    if (mine) {
+      const float inv = 1.0f / tot.s;
+      dst[pair] = tot.o * inv;
+    }
   }
-  const float inv = 1.0f / tot.s;
-  *dst = f32x4{tot.o.x * inv, tot.o.y * inv, tot.o.z * inv, tot.o.w * inv};
 }
 
 }  // namespace decode_attention

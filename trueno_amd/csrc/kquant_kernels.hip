@@ -284,15 +284,18 @@ incremental_attention(const float* q, const float* k, const float* v, float* out
                          partial, counters);
 }
 
-#define KQ_ATTENTION_TILED(name, DIM)                                                                                    \
-  extern "C" __global__ void __launch_bounds__(64 * decode_attention::Tiled<DIM>::WAVES)                             \
+#define KQ_ATTENTION_TILED(name, DIM, W)                                                                                 \
+  extern "C" __global__ void __launch_bounds__(64 * W)                                                                 \
   name(const float* q, const float* k, const float* v, float* out, u32 seq_len, u32 per_kv, u32 subs, u32 max_seq_len,   \
        float scale, u32 chunk, u32 chunks, u32 groups, float* partial, u32* counters) {                                  \
-    decode_attention::tiled_body<DIM>(q, k, v, out, seq_len, per_kv, subs, max_seq_len, scale, chunk, chunks, groups,    \
-                                      partial, counters);                                                                \
+    __shared__ __attribute__((aligned(256))) uint8_t s_tiles[decode_attention::Tiled<DIM, W>::LDS];                      \
+    decode_attention::tiled_body<DIM, W>(q, k, v, out, seq_len, per_kv, subs, max_seq_len, scale, chunk, chunks, groups, \
+                                         partial, counters, s_tiles);                                                    \
   }
-KQ_ATTENTION_TILED(kq_attention_tiled_64, 64)
-KQ_ATTENTION_TILED(kq_attention_tiled_128, 128)
+KQ_ATTENTION_TILED(kq_attention_tiled_64, 64, 8)
+KQ_ATTENTION_TILED(kq_attention_tiled_128, 128, 8)
+KQ_ATTENTION_TILED(kq_attention_tiled_128_w4, 128, 4)
+KQ_ATTENTION_TILED(kq_attention_tiled_256, 256, 4)
 
 extern "C" __global__ void __launch_bounds__(256) kq_fill_u32(u32* p, u32 n, u32 v) {
   for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;

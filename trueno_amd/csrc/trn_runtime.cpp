@@ -84,7 +84,7 @@ struct DeviceKernels {
   hipFunction_t copy_u128 = nullptr, read_u128 = nullptr;
   hipFunction_t residual_add = nullptr, swiglu = nullptr, rmsnorm = nullptr, residual_rmsnorm = nullptr;
   hipFunction_t gemv_f32_fast = nullptr, gemv_f32_generic = nullptr, q5k_from_ggml = nullptr, attention = nullptr;
-  hipFunction_t attention_tiled[2] = {};  // head dimension 64, 128
+  hipFunction_t attention_tiled[4] = {};  // head dimension 64, 128, 256; 128 with workgroups of four waves
   hipFunction_t gemm_f16[NFMT][2] = {};   // [format][4 or 8 strips per workgroup]
   hipFunction_t gemm_f16_w12 = nullptr;   // Q4_K: 12 strips per workgroup
   hipFunction_t gemm_f16_t2[2] = {};      // Q4_K, Q5_K: 8 strips and two token tiles per workgroup
@@ -177,6 +177,8 @@ hipError_t device_kernels(DeviceKernels** out) {
         (e = get_fn(m, &t.attention, "incremental_attention")) != hipSuccess ||
         (e = get_fn(m, &t.attention_tiled[0], "kq_attention_tiled_64")) != hipSuccess ||
         (e = get_fn(m, &t.attention_tiled[1], "kq_attention_tiled_128")) != hipSuccess ||
+        (e = get_fn(m, &t.attention_tiled[2], "kq_attention_tiled_256")) != hipSuccess ||
+        (e = get_fn(m, &t.attention_tiled[3], "kq_attention_tiled_128_w4")) != hipSuccess ||
         (e = get_fn(m, &t.gemv_f32_generic, "gemv_coalesced")) != hipSuccess ||
         (e = get_fn(m, &t.residual_add, "residual_add")) != hipSuccess ||
         (e = get_fn(m, &t.swiglu, "fused_swiglu")) != hipSuccess ||
@@ -415,6 +417,14 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
 // Single-query attention over the KV cache (decode_attention.hip.h).  Per (device, stream): arrival counters per
 // head and the chunks' partial softmax states.
 ScratchMap g_attention_ws;
+constexpr uint32_t kAttentionFourWaves = 512;      // positions of a workgroup from which four waves a workgroup are faster (decode_attention.hip.h)
+
+constexpr size_t kAttentionCounterBytes = 64u * 1024u;
+// The stream's first call makes room for the most that a workgroup per CU can publish, eight heads of 256 dims, so that a longer
+// sequence, or a captured call, finds it there.
+size_t attention_scratch(const DeviceKernels& d, size_t part_bytes) {
+  return kAttentionCounterBytes + std::max(part_bytes, size_t(d.cu_count) * 8u * 65u * 16u);
+}
 
 hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t v, uint64_t out, uint32_t seq_len,
                             uint32_t head_dim, uint32_t num_heads, uint32_t num_kv_heads, uint32_t max_seq_len, float scale) {
@@ -426,26 +436,36 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
   DeviceKernels* d = nullptr;
   hipError_t e = device_kernels(&d);
   if (e != hipSuccess) return e;
-  if ((head_dim == 64u || head_dim == 128u) && num_heads % num_kv_heads == 0u && g_tune_attention_tiled != 1 &&
-      (num_heads > num_kv_heads || head_dim == 64u || seq_len >= 4096u || g_tune_attention_tiled == 2)) {
-    // the query heads of a KV head together, in tiles of 16 positions (both sides measured: decode_attention.hip.h; a
-    // head alone with 128 dims only with many positions: 32 heads, 2048 positions 16.7 against 16.1 us, 8192 43.3 against 45.5; under 200 positions it is
-    // as fast or faster with the cache out of L2, 8 heads over one KV head x 128, 153 positions 8.6 -> 8.1, 64 over 8, 58
-    // positions 6.7 -> 5.5, and 0.2 to 0.4 us slower with it in L2, the former 1.6): a
-    // workgroup per CU (two are slower at every length, 28.8 against 18.7 us with 8 KV heads and 8192 positions), at least a tile a wave
-    const uint32_t waves = head_dim == 64u ? 8u : 4u, most_heads = 8u, step = 16u * waves;
-    uint32_t per_kv = num_heads / num_kv_heads, subs = (per_kv + most_heads - 1u) / most_heads, groups = num_kv_heads * subs;
-    const uint32_t per_cu = g_tune_attention_per_cu > 0 ? uint32_t(g_tune_attention_per_cu) : 1u;
-    uint32_t chunks = std::max(1u, per_cu * uint32_t(d->cu_count) / groups);
-    uint32_t chunk = (seq_len + chunks - 1u) / chunks;
-    chunk = (chunk + step - 1u) / step * step;
-    chunks = (seq_len + chunk - 1u) / chunk;
-    const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (chunks > 1u ? size_t(groups) * chunks * most_heads * (head_dim / 4u + 1u) * 16u : 0u);
-    uint64_t cnt = 0;
-    if ((e = acquire_scratch(g_attention_ws, d, stream, need, cnt_cap, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
-    uint64_t part = cnt + cnt_cap;
-    void* args[] = {&q, &k, &v, &out, &seq_len, &per_kv, &subs, &max_seq_len, &scale, &chunk, &chunks, &groups, &part, &cnt};
-    return hipModuleLaunchKernel(d->attention_tiled[head_dim == 128u], groups * chunks, 1, 1, 64u * waves, 1, 1, 0, stream, args, nullptr);
+  // The query heads of a KV head together, in tiles of 16 positions (decode_attention.hip.h), a workgroup per CU (two are
+  // slower at every length).  With 64 and 128 dims always: faster than the other kernel, or within the scatter, at every length and
+  // head count measured (64 .. 16384 positions).  256 dims: several query heads from 32 positions a CU on (16 heads over 8: 300 positions
+  // 8.5 us with the other kernel, 10.2 with this one; 3000 positions 21.6 and 18.9; 32 over 16, 700 positions 13.1 and 12.5); a head alone only
+  // where there are few and they are long (8 heads, 8000 positions: 32.0 and 31.2; 4, 16000: 38.7 and 34.7; but 32, 8000: 82.5 and 88.2 -
+  // one wave a SIMD, fifteen columns of sixteen empty).
+  uint32_t per_kv = num_heads / num_kv_heads, subs = (per_kv + 7u) / 8u;
+  const uint64_t cus = uint64_t(d->cu_count), positions = uint64_t(num_kv_heads) * subs * seq_len;
+  bool tiled = head_dim == 64u || head_dim == 128u ||
+               (head_dim == 256u && (per_kv > 1u ? positions >= 32u * cus : num_heads <= 8u && positions >= 192u * cus));
+  if (g_tune_attention_tiled == 2) tiled = head_dim == 64u || head_dim == 128u || head_dim == 256u;
+  if (tiled && num_heads % num_kv_heads == 0u && g_tune_attention_tiled != 1) {
+    const uint32_t most_heads = 8u, per_cu = g_tune_attention_per_cu > 0 ? uint32_t(g_tune_attention_per_cu) : 1u;
+    uint32_t groups = num_kv_heads * subs, most = std::max(1u, per_cu * uint32_t(d->cu_count) / groups), chunk = 0, chunks = 0;
+    // at least four tiles a workgroup (fewer make more chunks than they save: 32 heads over 8, 700 positions 9.3 us with two, 7.9 with
+    // four, 8.6 with eight); with 64 dims eight if more than eight chunks would have to be joined (700 positions, 16 KV heads 7.4 and 6.9)
+    for (uint32_t step = 64u;; step *= 2u) {
+      chunk = ((seq_len + most - 1u) / most + step - 1u) / step * step;
+      chunks = (seq_len + chunk - 1u) / chunk;
+      if (head_dim != 64u || step > 64u || chunks <= 8u) break;
+    }
+    if (uint64_t(chunk) * head_dim * 4u < (uint64_t(1) << 31)) {      // (the kernel's offsets into a chunk)
+      const size_t need = attention_scratch(*d, chunks > 1u ? size_t(groups) * chunks * most_heads * (head_dim / 4u + 1u) * 16u : 0u);
+      uint64_t cnt = 0;
+      if ((e = acquire_scratch(g_attention_ws, d, stream, need, kAttentionCounterBytes, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
+      uint64_t part = cnt + kAttentionCounterBytes;
+      void* args[] = {&q, &k, &v, &out, &seq_len, &per_kv, &subs, &max_seq_len, &scale, &chunk, &chunks, &groups, &part, &cnt};
+      const int which = head_dim == 64u ? 0 : head_dim == 256u ? 2 : chunk >= kAttentionFourWaves ? 3 : 1;
+      return hipModuleLaunchKernel(d->attention_tiled[which], groups * chunks, 1, 1, which >= 2 ? 256u : 512u, 1, 1, 0, stream, args, nullptr);
+    }
   }
   uint32_t lpp_log2 = 0;
   while ((4u << lpp_log2) < head_dim) ++lpp_log2;
@@ -459,10 +479,10 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
   uint32_t chunk = (seq_len + chunks - 1u) / chunks;
   chunk = (chunk + step - 1u) / step * step;
   chunks = (seq_len + chunk - 1u) / chunk;
-  const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (chunks > 1u ? size_t(num_heads) * chunks * lpp * 32u : 0u);
+  const size_t need = attention_scratch(*d, chunks > 1u ? size_t(num_heads) * chunks * lpp * 32u : 0u);
   uint64_t cnt = 0;
-  if ((e = acquire_scratch(g_attention_ws, d, stream, need, cnt_cap, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
-  uint64_t part = cnt + cnt_cap;
+  if ((e = acquire_scratch(g_attention_ws, d, stream, need, kAttentionCounterBytes, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
+  uint64_t part = cnt + kAttentionCounterBytes;
   void* args[] = {&q, &k, &v, &out, &seq_len, &head_dim, &num_heads, &num_kv_heads, &max_seq_len, &scale, &lpp_log2, &chunk, &chunks,
                   &part, &cnt};
   return hipModuleLaunchKernel(d->attention, num_heads * chunks, 1, 1, 256, 1, 1, 0, stream, args, nullptr);
