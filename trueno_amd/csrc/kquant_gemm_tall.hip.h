@@ -4,23 +4,23 @@
 // f16 pieces of a run of 256 scaled by a power of two.  There a wave multiplies 32 rows of W with 16 tokens at a time and
 // builds the weight operand anew for each 16: with many tokens the vector unit and the LDS (a page of token operands per
 // matrix instruction) are what it waits for.  Here the activations are made into operands once, by a launch of their own
-// (2048 x 4096: 11 us, 16 with the activations out of the caches), and a wave holds a tile of 64 rows x 32 tokens: an operand of either side feeds two matrix
-// instructions, so LDS reads and operand building halve.
-//   * A workgroup is four waves with a strip of 64 rows each against one tile of 32 tokens, two workgroups a CU (80 KB of
-//     LDS, 256 registers): their phases drift apart, so that one's sums and headers run under the other's products.
-//     (One wave a SIMD with 64 x 64 or 64 x 128 tiles: 580 us where this takes 525, its vector instructions are not hidden;
-//     eight waves in step: 563.)
-//   * Weights and token pages come by copies into LDS, pages in a ring of chunks of four products (Q6_K two chunks, its
+// (2048 x 4096: 11 us, 16 with the activations out of the caches), and a wave holds a tile of 32 rows x 64 tokens: a weight operand, which
+// costs ten vector instructions (Q6_K thirty-two), feeds four matrix instructions (Q6_K six).
+//   * What bounds it: beside other waves' vector instructions a matrix instruction takes half its cycles of a SIMD's issue and a vector
+//     instruction four and a half (measured with one wave of each on a SIMD), so a super-block takes a wave the larger of M and M / 2 + 4.5 V cycles, M = 2304
+//     (Q6_K 3072), V = 460 (Q5_K 610, Q6_K 860).  With 64 rows x 32 tokens, the same registers, V was 650 (1250 for Q6_K): us, that form -> this
+//     one, Q6_K 4096 x 11008, 512 tokens 192 -> 163, 11008 x 4096, 1024 tokens 372 -> 309; Q5_K 11008 x 4096, 512 tokens 141 -> 135; Q4_K, which the
+//     power limit holds (1.5-1.6 GHz where both run), 14336 x 4096, 2048 tokens 538 -> 531.  The tokens' LDS reads double: 90 of 128 bytes a cycle.
+//   * A workgroup is four waves with a strip of 32 rows each against the same two operand tiles of 32 tokens, two workgroups a CU (70-80 KB of
+//     LDS, 220-240 registers): their phases drift apart, so that one's sums and headers run under the other's products.
+//   * Weights and token pages come by copies into LDS, pages in a ring of three chunks of four products (Q6_K two, its
 //     weight tile is larger), the next super-block's weight tile as soon as the last of the current one is in registers.
 //     Waits are counted by hand; every path issues the same number of copies (behind the end of a run the last
-//     super-block's again).
+//     super-block's again).  A wave in its products goes first (up to 5 % against equal priorities).
 //   * Rounding.  The hi pieces' sums are kept apart from the lo pieces' (alone they are whole numbers on a coarse grid and
-//     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by after
-//     about the root of their number.  Against fp64 the error is 0.82 .. 0.98 times the 16-token kernel's, over 70 shapes a
+//     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by every few
+//     (put_by).  Against fp64 the error is 0.82 .. 0.98 times the 16-token kernel's, over 70 shapes a
 //     format drawn from 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns that the rule gives this kernel.
-//   * Measured (us, the 16-token kernel -> this one): Q4_K 14336 x 4096, 2048 tokens 835 -> 534 (matrix cores busy 56 % of
-//     the cycles at 1.7 GHz, the power limit's clock, nine vector instructions to a matrix instruction; a library f16 product
-//     with as many matrix instructions takes 405); Q6_K 4096 x 11008, 512 tokens 290 -> 193 (32 %, thirteen to one).
 #pragma once
 #include "kquant_gemm_f16.hip.h"
 #include <utility>
@@ -30,7 +30,8 @@ namespace gemm_tall {
 using namespace gemm_f16;      // the LDS helpers, split_f16, pack_h2
 
 constexpr u32 kTile = 32;                      // tokens of an operand tile
-constexpr u32 kWaves = 4, kWaveRows = 64;      // a workgroup takes 256 rows of W against one operand tile
+constexpr int kTiles = 2;                      // operand tiles a workgroup takes
+constexpr u32 kWaves = 4, kWaveRows = 32;      // its rows of W: a strip of 32 a wave
 constexpr u32 kPagesBytes = 32 * 1024;         // 16 products x (lo page, hi page) of 64 lanes x 16 bytes
 constexpr u32 kAuxBytes = 2048;                // sums (1 KB), factors (128 bytes, padded)
 constexpr u32 kOperandBytes = kPagesBytes + kAuxBytes;      // of a (token tile, super-block)
@@ -128,9 +129,9 @@ __device__ __forceinline__ h16x2 bytes_to_h2(u32 v) {
 }
 __device__ __forceinline__ h16x2 h2(float v) { return h16x2{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
 
-template <int FMT> struct Layout;      // weight tile in LDS: STRIDE bytes a row (an odd number of 16-byte pieces), DMA instructions of 64 pieces for 64 rows
-template <> struct Layout<FMT_Q4K> { static constexpr u32 SB = 144, STRIDE = 144, PIECES = 9, STAGES = 4; };
-template <> struct Layout<FMT_Q5K> { static constexpr u32 SB = 176, STRIDE = 176, PIECES = 11, STAGES = 4; };
+template <int FMT> struct Layout;      // weight tile in LDS: STRIDE bytes a row (an odd number of 16-byte pieces), COPIES of 64 pieces for 32 rows; STAGES chunks of tokens
+template <> struct Layout<FMT_Q4K> { static constexpr u32 SB = 144, STRIDE = 144, PIECES = 9, COPIES = 5, STAGES = 3; };
+template <> struct Layout<FMT_Q5K> { static constexpr u32 SB = 176, STRIDE = 176, PIECES = 11, COPIES = 6, STAGES = 3; };
 
 template <class F, int... I>
 __device__ __forceinline__ void for_each_product(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
@@ -150,143 +151,164 @@ struct Place {
   }
 };
 
-// lane l holds W row row (of strips 32 apart) and the tokens 8 (v / 4) + 4 g + v % 4 of the tile
-__device__ __forceinline__ void store_tile(const f32x16 (&sum)[2], float* __restrict__ out, u32 m, u32 n, u32 row, u32 tile, u32 g) {
+// lane l holds W row row and the tokens 8 (v / 4) + 4 g + v % 4 of either tile
+__device__ __forceinline__ void store_tiles(const f32x16 (&sum)[kTiles], float* __restrict__ out, u32 m, u32 n, u32 row, u32 token0, u32 g) {
+  if (row >= n) return;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    if (row + 32u * r < n) {
+  for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const u32 token = tile * kTile + 8u * (v >> 2) + 4u * g + (v & 3);
-        if (token < m) out[static_cast<size_t>(token) * n + row + 32u * r] = sum[r][v];
-      }
+    for (int v = 0; v < 16; ++v) {
+      const u32 token = token0 + kTile * t + 8u * (v >> 2) + 4u * g + (v & 3);
+      if (token < m) out[static_cast<size_t>(token) * n + row] = sum[t][v];
+    }
+}
+
+// The running sums are put by; LOSSLESS: what the sum of both rounds away starts the next run, so that the length of a part costs no
+// exactness (Q6_K 4096 x 11008 in one part instead of two: 4 % above the error of two without, 5 % below with it).  Q4_K, whose vector instructions weigh
+// more beside its products, would lose 2 % of its time to it and does without.
+template <bool LOSSLESS>
+__device__ __forceinline__ void put_by(f32x16& stash, f32x16& tot) {
+  __builtin_amdgcn_sched_barrier(0);      // (nothing else is alive here)
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const float s = stash[v] + tot[v], b = s - stash[v];
+    tot[v] = LOSSLESS ? (stash[v] - (s - b)) + (tot[v] - b) : 0.0f;
+    stash[v] = s;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// the copies of both bodies: a chunk in LDS is [tile][product][lo, hi][64 lanes], 16 KB, of which wave w brings product w
+constexpr u32 kChunk = kTiles * 8192u;
+constexpr int kChunkCopies = 2 * kTiles;      // of a wave's share of a chunk
+struct TokenCopies {
+  __amdgpu_buffer_rsrc_t rsrc;
+  u32 lane16, wave, tile_bytes, ring, aux;
+  // (a second tile that is not there: the first one again, its results are not stored)
+  __device__ __forceinline__ TokenCopies(const uint8_t* ops, u32 pair, u32 m, u32 nsb, u32 sb0, u32 ns, u32 lane, u32 wave_, u32 ring_, u32 aux_)
+      : lane16(lane * 16u), wave(wave_), tile_bytes((kTiles * pair + 1u) * kTile < m ? nsb * kOperandBytes : 0u), ring(ring_), aux(aux_) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ops) + (static_cast<size_t>(pair) * kTiles * nsb + sb0) * kOperandBytes, 0,
+                                             static_cast<int>(tile_bytes + ns * kOperandBytes), 0x00020000);
+  }
+  __device__ __forceinline__ void chunk(u32 s, u32 c, u32 slot) const {
+#pragma unroll
+    for (u32 t = 0; t < kTiles; ++t) {
+      const u32 src = s * kOperandBytes + t * tile_bytes + c * 8192u + wave * 2048u, dst = ring + slot * kChunk + t * 8192u + wave * 2048u;
+      buffer_dma16(rsrc, dst, lane16, src);
+      buffer_dma16(rsrc, dst + 1024u, lane16, src + 1024u);
     }
   }
-}
+  __device__ __forceinline__ void sums(u32 s, u32 buf) const {      // the tiles' aux, a KB a wave
+    buffer_dma16(rsrc, aux + buf * (kTiles * kAuxBytes) + wave * 1024u, lane16,
+                 s * kOperandBytes + (wave >> 1) * tile_bytes + kPagesBytes + (wave & 1u) * 1024u);
+  }
+};
 
 // dynamic LDS: the ring of chunks, two aux pages, a weight tile per wave (tall_lds_bytes of the runtime)
 template <int FMT>
 __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint8_t* __restrict__ w, float* __restrict__ c,
-                                     u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 tiles, u32 run, u32 lds_base) {
+                                     u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 pairs, u32 run, u32 lds_base) {
   using L = Layout<FMT>;
-  constexpr int S = static_cast<int>(L::STAGES);
-  constexpr u32 kStage = 8192u;                        // a chunk: four products' pages
-  constexpr int TD = 2;                                // copies of a wave's share of a chunk
-  constexpr int WD = static_cast<int>(L::PIECES);      // copies of a wave's weight tile
+  constexpr int S = static_cast<int>(L::STAGES), TD = kChunkCopies, WD = static_cast<int>(L::COPIES);
   const u32 lane = threadIdx.x & 63u;
   const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
-  const Place at(blockIdx.x, groups, tiles, kparts);
+  const Place at(blockIdx.x, groups, pairs, kparts);
   if (!at.valid) return;
   const u32 sb0 = at.part * ksb, ns = min(ksb, nsb - sb0);
   const u32 col = lane & 31u, g = lane >> 5;
   const u32 row0 = at.group * (kWaves * kWaveRows) + wave * kWaveRows;
   const size_t row_bytes = static_cast<size_t>(nsb) * L::SB;
 
-  const u32 lds_ring = lds_base, lds_aux = lds_base + S * kStage;
-  const u32 lds_w = lds_aux + 2u * kAuxBytes + wave * (kWaveRows * L::STRIDE);
+  const u32 lds_ring = lds_base, lds_aux = lds_base + S * kChunk;
+  const u32 lds_w = lds_aux + 2u * kTiles * kAuxBytes + wave * (WD * 1024u);
 
   u32 woff[WD];
   const u32 row_first = min(row0, n - 1u);
 #pragma unroll
   for (int t = 0; t < WD; ++t) {
-    const u32 p = 64u * t + lane, r = p / L::PIECES, cc = p - L::PIECES * r;
+    const u32 p = min(64u * t + lane, kWaveRows * L::PIECES - 1u), r = p / L::PIECES, cc = p - L::PIECES * r;
     woff[t] = (min(row0 + r, n - 1u) - row_first) * static_cast<u32>(row_bytes) + 16u * cc;
   }
   // copies into LDS by buffer instructions: the lane's offset stays in its register, what moves is scalar
-  const u32 strip_bytes = (min(row0 + kWaveRows, n) - row_first) * static_cast<u32>(row_bytes) - sb0 * L::SB;
+  const u32 strip_bytes = (min(row0 + kWaveRows, max(n, row0 + 1u)) - row0) * static_cast<u32>(row_bytes) - sb0 * L::SB;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(w) + static_cast<size_t>(row_first) * row_bytes + static_cast<size_t>(sb0) * L::SB, 0, static_cast<int>(strip_bytes), 0x00020000);
   auto issue_w = [&](u32 s) {
 #pragma unroll
     for (int t = 0; t < WD; ++t) buffer_dma16(w_rsrc, lds_w + 1024u * t, woff[t], s * L::SB);
   };
-  // a chunk in LDS is [product][lo, hi][64 lanes]: wave w brings product w
-  const __amdgpu_buffer_rsrc_t op_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(ops) + (static_cast<size_t>(at.tile) * nsb + sb0) * kOperandBytes, 0, static_cast<int>(ns * kOperandBytes), 0x00020000);
-  const u32 lane16 = lane * 16u;
-  auto issue_tokens = [&](u32 s, u32 chunk, u32 slot) {
-    const u32 src = s * kOperandBytes + chunk * 8192u + wave * 2048u, dst = lds_ring + slot * kStage + wave * 2048u;
-    buffer_dma16(op_rsrc, dst, lane16, src);
-    buffer_dma16(op_rsrc, dst + 1024u, lane16, src + 1024u);
-  };
-  auto issue_aux = [&](u32 s, u32 buf) {      // 2 KB, by two waves (and, for one count of copies, by the other two as well)
-    buffer_dma16(op_rsrc, lds_aux + buf * kAuxBytes + (wave & 1u) * 1024u, lane16, s * kOperandBytes + kPagesBytes + (wave & 1u) * 1024u);
-  };
+  const TokenCopies tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
 
-  f32x16 tot[2], stash[2];
+  // where Q4_K keeps a lane's four scales and mins: for the last four sub-blocks the upper two bits lie apart
+  [[maybe_unused]] const u32 sc_up = g ? 2u : 0u, sc_mask = g ? 0x30303030u : 0x3F3F3F3Fu, sc_rest = g ? 0x0F0F0F0Fu : 0u;
+  f32x16 tot[kTiles], stash[kTiles];
   const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-  for (int r = 0; r < 2; ++r) tot[r] = stash[r] = zero;
+  for (int t = 0; t < kTiles; ++t) tot[t] = stash[t] = zero;
 
   // chunks 0 .. S-1 of the run, behind the first weight tile and aux pages
   issue_w(0);
-  issue_aux(0, 0);
+  tokens.sums(0, 0);
 #pragma unroll
-  for (int i = 0; i < S; ++i) issue_tokens(min(i / 4u, ns - 1u), i & 3, i);
+  for (int i = 0; i < S; ++i) tokens.chunk(min(i / 4u, ns - 1u), i & 3, i);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   asm volatile("s_barrier" ::: "memory");
   u32 slot = 0;      // of the chunk being multiplied
   u32 left = run;    // super-blocks until the running sums are put by
   for (u32 s = 0; s < ns; ++s) {
-    const u32 wt0 = lds_w + col * L::STRIDE, wt1 = wt0 + 32u * L::STRIDE;
-    const u32 aux = lds_aux + (s & 1u) * kAuxBytes;
+    const u32 wt = lds_w + col * L::STRIDE;
+    const u32 aux = lds_aux + (s & 1u) * (kTiles * kAuxBytes);
     // the weight tile has landed: behind its copies those of two chunks, the last of which may be on its way
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TD) : "memory");
-    u32x4 raw[2][2], hdr[2], tok[2][2];
-    [[maybe_unused]] u32x4 qh[2] = {};
-    lds_read128<0>(hdr[0], wt0);
-    lds_read128<0>(hdr[1], wt1);
-    lds_read128<16>(raw[0][0], wt0 + g * 64u);
-    lds_read128<16>(raw[0][1], wt1 + g * 64u);
-    if constexpr (FMT == FMT_Q5K) {
-      lds_read128<144>(qh[0], wt0 + g * 16u);
-      lds_read128<144>(qh[1], wt1 + g * 16u);
-    }
+    u32x4 raw[2], hdr, tok[2][kTiles][2];
+    [[maybe_unused]] u32x4 qh = {};
+    lds_read128<0>(hdr, wt);
+    lds_read128<16>(raw[0], wt + g * 64u);
+    if constexpr (FMT == FMT_Q5K) lds_read128<144>(qh, wt + g * 16u);
     auto read_tokens = [&](int buf, u32 sl, auto page_c) {
       constexpr int PAGE = decltype(page_c)::value;
-      const u32 at = lds_ring + sl * kStage + lane * 16u;
-      lds_read128<PAGE * 2048>(tok[buf][0], at);
-      lds_read128<PAGE * 2048 + 1024>(tok[buf][1], at);
+      const u32 at = lds_ring + sl * kChunk + lane * 16u;
+      lds_read128<PAGE * 2048>(tok[buf][0][0], at);
+      lds_read128<PAGE * 2048 + 1024>(tok[buf][0][1], at);
+      lds_read128<PAGE * 2048 + 8192>(tok[buf][1][0], at);
+      lds_read128<PAGE * 2048 + 8192 + 1024>(tok[buf][1][1], at);
     };
     read_tokens(0, slot, std::integral_constant<int, 0>{});
-    asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(hdr[0]), "+v"(hdr[1]), "+v"(raw[0][0]), "+v"(raw[0][1]), "+v"(qh[0]), "+v"(qh[1]) : "n"(2) : "memory");
-    float d[2], nm[2];      // (times 2^-11 where they meet the sums of lo pieces)
-    h16x2 scale[2][2], addend[2][2], mins[2][2];      // [row tile][sub-blocks 0 and 2 (low nibbles), 1 and 3 (high nibbles) of the lane's four]
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(hdr), "+v"(raw[0]), "+v"(qh) : "n"(2 * kTiles) : "memory");
+    h16x2 scale[2], addend[2], mins[2];      // sub-blocks 0 and 2 (low nibbles), 1 and 3 (high nibbles) of the lane's four
     constexpr float kCentre = FMT == FMT_Q4K ? 8.0f : 16.0f;
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const u32x4 hd = hdr[r];
+    const float d = half_bits_to_f32(hdr.x);
+    const float nm = half_bits_to_f32(hdr.x >> 16) * -0.001953125f;       // -dmin * 2^-9: the sums carry 2^-5, the products 2^-14
+    {
       u32 s4, m4;
-      d[r] = half_bits_to_f32(hd.x);
-      nm[r] = half_bits_to_f32(hd.x >> 16) * -0.001953125f;       // -dmin * 2^-9: the sums carry 2^-5, the products 2^-14
       if constexpr (FMT == FMT_Q4K) {      // get_scale_min_k4, quantize.rs:1306-1385
-        s4 = g ? ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)) : (hd.y & 0x3F3F3F3Fu);
-        m4 = g ? (((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u)) : (hd.z & 0x3F3F3F3Fu);
+        s4 = ((hdr.y >> sc_up) & sc_mask) | (hdr.w & sc_rest);
+        m4 = ((hdr.z >> sc_up) & sc_mask) | ((hdr.w >> 4) & sc_rest);
       } else {                             // eight contiguous 12-bit fields, scale in the low six bits (quantize.rs:1607-1635)
-        const u32 lo = g ? ((hd.z >> 16) | (hd.w << 16)) : hd.y;
-        const u32 hi = g ? (hd.w >> 16) : (hd.z & 0xFFFFu);
+        const u32 lo = g ? ((hdr.z >> 16) | (hdr.w << 16)) : hdr.y;
+        const u32 hi = g ? (hdr.w >> 16) : (hdr.z & 0xFFFFu);
         const u32 f0 = lo & 0xFFFu, f1 = (lo >> 12) & 0xFFFu, f2 = ((lo >> 24) | (hi << 8)) & 0xFFFu, f3 = (hi >> 4) & 0xFFFu;
         s4 = (f0 & 63u) | ((f1 & 63u) << 8) | ((f2 & 63u) << 16) | ((f3 & 63u) << 24);
         m4 = (f0 >> 6) | ((f1 >> 6) << 8) | ((f2 >> 6) << 16) | ((f3 >> 6) << 24);
       }
       const h16x2 s02 = bytes_to_h2(s4), s13 = bytes_to_h2(s4 >> 8);
-      scale[r][0] = s02 * h2(1024.0f);
-      scale[r][1] = s13 * h2(64.0f);
-      addend[r][0] = s02 * h2(-kCentre * 0.00006103515625f);
-      addend[r][1] = s13 * h2(-kCentre * 0.00006103515625f);
-      mins[r][0] = bytes_to_h2(m4);
-      mins[r][1] = bytes_to_h2(m4 >> 8);
+      scale[0] = s02 * h2(1024.0f);
+      scale[1] = s13 * h2(64.0f);
+      addend[0] = s02 * h2(-kCentre * 0.00006103515625f);
+      addend[1] = s13 * h2(-kCentre * 0.00006103515625f);
+      mins[0] = bytes_to_h2(m4);
+      mins[1] = bytes_to_h2(m4 >> 8);
     }
-    // weight operand of product q (0..15) of a row tile, out of the four dwords of its chunk
-    auto build = [&](int r, int q, const u32x4& rw) -> h16x8 {
+    // weight operand of product q (0..15), out of the four dwords of its chunk
+    auto build = [&](int q, const u32x4& rw) -> h16x8 {
       const int u = q >> 1, h = q & 1;
       const u32 t0 = (u & 1) ? rw.z : rw.x, t1 = (u & 1) ? rw.w : rw.y;
-      const _Float16 sv = scale[r][h][u >> 2], av = addend[r][h][u >> 2];
+      const _Float16 sv = scale[h][u >> 2], av = addend[h][u >> 2];
       const h16x2 sc = {sv, sv}, ad = {av, av};
       const u32 mask = h ? 0x00F000F0u : 0x000F000Fu;
       u32 f[4] = {0u, 0u, 0u, 0u};
       if constexpr (FMT == FMT_Q5K) {      // the fifth bits (kquant_gemm_f16.hip.h)
-        const u32 word = u < 4 ? (h ? qh[r].y : qh[r].x) : (h ? qh[r].w : qh[r].z);
+        const u32 word = u < 4 ? (h ? qh.y : qh.x) : (h ? qh.w : qh.z);
 #pragma unroll
         for (int dd = 0; dd < 2; ++dd) {
           const u32 nb = (word >> (4 * ((2 * u + dd) & 7))) & 15u;
@@ -298,84 +320,81 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
                        __builtin_bit_cast(u32, pk_fma_h2((t1 & mask) | f[2], sc, ad)), __builtin_bit_cast(u32, pk_fma_h2(((t1 >> 8) & mask) | f[3], sc, ad))};
       return __builtin_bit_cast(h16x8, o);
     };
-    h16x8 frag[2][2];
-    frag[0][0] = build(0, 0, raw[0][0]);
-    frag[0][1] = build(1, 0, raw[0][1]);
-    f32x16 acc[2], low[2];      // of the hi and of the lo pieces
+    h16x8 frag[2];
+    frag[0] = build(0, raw[0]);
+    f32x16 acc[kTiles], low[kTiles];      // of the hi and of the lo pieces
     auto step = [&](auto i_c) {
       constexpr int I = decltype(i_c)::value, CH = I / 4, B = I & 1;
-      if constexpr (I % 4 == 2 && CH < 3) {      // the next chunk's weight dwords
-        lds_read128<16 + 16 * (CH + 1)>(raw[(CH + 1) & 1][0], wt0 + g * 64u);
-        lds_read128<16 + 16 * (CH + 1)>(raw[(CH + 1) & 1][1], wt1 + g * 64u);
-      }
+      if constexpr (I % 4 == 2 && CH < 3) lds_read128<16 + 16 * (CH + 1)>(raw[(CH + 1) & 1], wt + g * 64u);      // the next chunk's weight dwords
       if constexpr (I % 4 == 3) {
         // everything of this chunk is in registers: on to the next one, as soon as every wave is there
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tok[B][0]), "+v"(tok[B][1]), "+v"(raw[(CH + 1) & 1][0]), "+v"(raw[(CH + 1) & 1][1])::"memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1]), "+v"(raw[(CH + 1) & 1])::"memory");
         constexpr int X = CH + 1;                            // chunk X has landed: S - 2 chunks behind it, and what went out with them
         constexpr bool W_BEHIND = X == 4 && S >= 3;
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * TD + (W_BEHIND ? WD + 1 : 0)) : "memory");
         asm volatile("s_barrier" ::: "memory");
         if constexpr (X == 3) {      // the last of this weight tile is in registers: its place takes the next one
           issue_w(min(s + 1u, ns - 1u));
-          issue_aux(min(s + 1u, ns - 1u), (s + 1u) & 1u);
+          tokens.sums(min(s + 1u, ns - 1u), (s + 1u) & 1u);
         }
         constexpr int NX = CH + S;                           // chunk CH + S takes this chunk's place
-        issue_tokens(min(s + NX / 4u, ns - 1u), NX & 3, slot);
+        tokens.chunk(min(s + NX / 4u, ns - 1u), NX & 3, slot);
         slot = slot + 1u == S ? 0u : slot + 1u;
       }
       if constexpr (I < 15) read_tokens(1 - B, slot, std::integral_constant<int, (I + 1) & 3>{});
       if constexpr (I % 4 != 3)
-        asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(tok[B][0]), "+v"(tok[B][1]) : "n"(2) : "memory");
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1]) : "n"(2 * kTiles) : "memory");
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][1]), frag[B][r], I == 0 ? zero : acc[r], 0, 0, 0);
-        low[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][0]), frag[B][r], I == 0 ? zero : low[r], 0, 0, 0);
-        if constexpr (I < 15) frag[1 - B][r] = build(r, I + 1, raw[((I + 1) / 4) & 1][r]);
+      for (int t = 0; t < kTiles; ++t) {
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][1]), frag[B], I == 0 ? zero : acc[t], 0, 0, 0);
+        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][0]), frag[B], I == 0 ? zero : low[t], 0, 0, 0);
       }
+      if constexpr (I < 15) frag[1 - B] = build(I + 1, raw[((I + 1) / 4) & 1]);
     };
-    // (a wave in its products goes first, 5 % against equal priorities: the other workgroup's wave on the SIMD fills the rest)
+
     __builtin_amdgcn_s_setprio(1);
     for_each_product(step, std::make_integer_sequence<int, 16>{});
     __builtin_amdgcn_s_setprio(0);
     // what the centring took out, then the min term, then the super-block's share of the running sums
     {
-      u32x4 sx, f0, f1, f2, f3;
-      lds_read128<0>(sx, aux + lane * 16u);
-      lds_read128<1024>(f0, aux + g * 16u);          // 2^(E+14) of the tokens 8 a + 4 g + {0..3}, a = 0..3
-      lds_read128<1056>(f1, aux + g * 16u);
-      lds_read128<1088>(f2, aux + g * 16u);
-      lds_read128<1120>(f3, aux + g * 16u);
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sx), "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)::"memory");
-      const u32 fb[16] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, f3.x, f3.y, f3.z, f3.w};
+      // C s_j 2^-9 and m_j against the sums' hi pieces (slots 0..3 of a lane), then against their lo pieces (4..7)
+      const u32 c0 = __builtin_bit_cast(u32, addend[0] * h2(-32.0f)), c1 = __builtin_bit_cast(u32, addend[1] * h2(-32.0f));
+      const u32 m0 = __builtin_bit_cast(u32, mins[0]), m1 = __builtin_bit_cast(u32, mins[1]);
+      const u32x4 ch = {c0, c1, 0u, 0u}, cl = {0u, 0u, c0, c1}, mh = {m0, m1, 0u, 0u}, ml = {0u, 0u, m0, m1};
+      const float d_lo = d * 0.00048828125f, nm_lo = nm * 0.00048828125f;
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        // C s_j 2^-9 and m_j against the sums' hi pieces (slots 0..3 of a lane), then against their lo pieces (4..7)
-        const u32 c0 = __builtin_bit_cast(u32, addend[r][0] * h2(-32.0f)), c1 = __builtin_bit_cast(u32, addend[r][1] * h2(-32.0f));
-        const u32 m0 = __builtin_bit_cast(u32, mins[r][0]), m1 = __builtin_bit_cast(u32, mins[r][1]);
-        const u32x4 ch = {c0, c1, 0u, 0u}, cl = {0u, 0u, c0, c1}, mh = {m0, m1, 0u, 0u}, ml = {0u, 0u, m0, m1};
+      for (int t = 0; t < kTiles; ++t) {
+        u32x4 sx, f0, f1, f2, f3;
+        const u32 at_t = aux + t * kAuxBytes;
+        lds_read128<0>(sx, at_t + lane * 16u);
+        lds_read128<1024>(f0, at_t + g * 16u);          // 2^(E+14) of the tokens 8 a + 4 g + {0..3}, a = 0..3
+        lds_read128<1056>(f1, at_t + g * 16u);
+        lds_read128<1088>(f2, at_t + g * 16u);
+        lds_read128<1120>(f3, at_t + g * 16u);
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sx), "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)::"memory");
+        const u32 fb[16] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, f3.x, f3.y, f3.z, f3.w};
         const h16x8 sv = __builtin_bit_cast(h16x8, sx);
         const f32x16 mch = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, mh), zero, 0, 0, 0);
         const f32x16 mcl = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ml), zero, 0, 0, 0);
-        acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ch), acc[r], 0, 0, 0);
-        low[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, cl), low[r], 0, 0, 0);
-        const float d_lo = d[r] * 0.00048828125f, nm_lo = nm[r] * 0.00048828125f;
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ch), acc[t], 0, 0, 0);
+        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, cl), low[t], 0, 0, 0);
         // (what the lo pieces gave comes first: next to no rounding is added at the size of the whole)
 #pragma unroll
         for (int v = 0; v < 16; ++v)
-          tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(d[r], acc[r][v], fmaf(nm[r], mch[v], fmaf(nm_lo, mcl[v], d_lo * low[r][v]))), tot[r][v]);
+          tot[t][v] = fmaf(__uint_as_float(fb[v]), fmaf(d, acc[t][v], fmaf(nm, mch[v], fmaf(nm_lo, mcl[v], d_lo * low[t][v]))), tot[t][v]);
+        __builtin_amdgcn_sched_barrier(0);      // (both tiles' at once would spill)
       }
     }
-    if (--left == 0u || s + 1u == ns) {      // runs of super-blocks are summed by themselves: fewer roundings at the size of the whole
+    if (--left == 0u) {      // runs of super-blocks are summed by themselves: fewer roundings at the size of the whole
       left = run;
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        stash[r] += tot[r];
-        tot[r] = zero;
-      }
+      for (int t = 0; t < kTiles; ++t) put_by<FMT == FMT_Q5K>(stash[t], tot[t]);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the copies asked for ahead of the end land before the workgroup's LDS is another's
-  store_tile(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile, g);
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) stash[t] += tot[t];
+  store_tiles(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (kTiles * kTile), g);
 }
 
 // Q6_K: w = (q - 32) sc needs 13 bits, f16 holds 11.  Centred digits q - 32 = 8 (2 q2 - 3) + (nib - 8) as in
@@ -390,19 +409,18 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
 constexpr u32 kQ6Stride = 224u, kQ6Pieces = 14u;
 
 __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const uint8_t* __restrict__ w, float* __restrict__ c,
-                                         u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 tiles, u32 run, u32 lds_base) {
-  constexpr u32 kStage = 8192u;                        // a chunk: four products' pages
-  constexpr int TD = 2, WD = static_cast<int>(kQ6Pieces);
+                                         u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 pairs, u32 run, u32 lds_base) {
+  constexpr int TD = kChunkCopies, WD = 7;             // 32 rows x 14 pieces
   const u32 lane = threadIdx.x & 63u;
   const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
-  const Place at(blockIdx.x, groups, tiles, kparts);
+  const Place at(blockIdx.x, groups, pairs, kparts);
   if (!at.valid) return;
   const u32 sb0 = at.part * ksb, ns = min(ksb, nsb - sb0);
   const u32 col = lane & 31u, g = lane >> 5;
   const u32 row0 = at.group * (kWaves * kWaveRows) + wave * kWaveRows;
   const size_t row_bytes = static_cast<size_t>(nsb) * 210u;
-  const u32 lds_ring = lds_base, lds_aux = lds_base + 2u * kStage;
-  const u32 lds_w = lds_aux + 2u * kAuxBytes + wave * (kWaveRows * kQ6Stride);
+  const u32 lds_ring = lds_base, lds_aux = lds_base + 2u * kChunk;
+  const u32 lds_w = lds_aux + 2u * kTiles * kAuxBytes + wave * (kWaveRows * kQ6Stride);
 
   u32 woff[WD];
   const u32 row_first = min(row0, n - 1u);
@@ -417,81 +435,69 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
 #pragma unroll
     for (int t = 0; t < WD; ++t) dma16(src + woff[t], lds_w + 1024u * t);
   };
-  const __amdgpu_buffer_rsrc_t op_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<uint8_t*>(ops) + (static_cast<size_t>(at.tile) * nsb + sb0) * kOperandBytes, 0, static_cast<int>(ns * kOperandBytes), 0x00020000);
+  const TokenCopies tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
   const u32 lane16 = lane * 16u;
-  auto issue_tokens = [&](u32 s, u32 chunk, u32 slot) {
-    const u32 src = s * kOperandBytes + chunk * 8192u + wave * 2048u, dst = lds_ring + slot * kStage + wave * 2048u;
-    buffer_dma16(op_rsrc, dst, lane16, src);
-    buffer_dma16(op_rsrc, dst + 1024u, lane16, src + 1024u);
-  };
-  auto issue_aux = [&](u32 s, u32 buf) {
-    buffer_dma16(op_rsrc, lds_aux + buf * kAuxBytes + (wave & 1u) * 1024u, lane16, s * kOperandBytes + kPagesBytes + (wave & 1u) * 1024u);
-  };
 
-  f32x16 tot[2], stash[2];
+  f32x16 tot[kTiles], stash[kTiles];
   const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-  for (int r = 0; r < 2; ++r) tot[r] = stash[r] = zero;
+  for (int t = 0; t < kTiles; ++t) tot[t] = stash[t] = zero;
   issue_w(0);
-  issue_aux(0, 0);
-  issue_tokens(0, 0, 0);
-  issue_tokens(0, 1, 1);
+  tokens.sums(0, 0);
+  tokens.chunk(0, 0, 0);
+  tokens.chunk(0, 1, 1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   asm volatile("s_barrier" ::: "memory");
   u32 left = run;
   for (u32 s = 0; s < ns; ++s) {
-    const u32 wt0 = lds_w + col * kQ6Stride, wt1 = wt0 + 32u * kQ6Stride;
-    const u32 aux = lds_aux + (s & 1u) * kAuxBytes;
+    const u32 wt = lds_w + col * kQ6Stride;
+    const u32 aux = lds_aux + (s & 1u) * (kTiles * kAuxBytes);
     // the weight tile has landed: only the copies of a chunk are behind its own
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TD) : "memory");
-    u32x4 ql[2][2], qh[2], tok[2][2];
-    u32x2 scv[2];
-    u32 dv[2];
-    auto read_raw = [&](auto c_c) {
-      constexpr int SET = decltype(c_c)::value & 1;
-      lds_read128<16 * SET>(ql[0][0], wt0 + g * 64u);
-      lds_read128<32 + 16 * SET>(ql[0][1], wt0 + g * 64u);
-      lds_read128<128 + 16 * SET>(qh[0], wt0 + g * 32u);
-      lds_read128<16 * SET>(ql[1][0], wt1 + g * 64u);
-      lds_read128<32 + 16 * SET>(ql[1][1], wt1 + g * 64u);
-      lds_read128<128 + 16 * SET>(qh[1], wt1 + g * 32u);
+    u32x4 ql[2][2], qh[2], tok[2][kTiles][2];      // [set of this or the next chunk]
+    u32x2 scv;
+    u32 dv;
+    auto read_raw = [&](auto c_c) {      // of chunk c
+      constexpr int C = decltype(c_c)::value, SET = C & 1;
+      lds_read128<16 * SET>(ql[SET][0], wt + g * 64u);
+      lds_read128<32 + 16 * SET>(ql[SET][1], wt + g * 64u);
+      lds_read128<128 + 16 * SET>(qh[SET], wt + g * 32u);
     };
     auto read_tokens = [&](int buf, u32 sl, auto page_c) {
       constexpr int PAGE = decltype(page_c)::value;
-      lds_read128<PAGE * 2048>(tok[buf][0], lds_ring + sl * kStage + lane16);
-      lds_read128<PAGE * 2048 + 1024>(tok[buf][1], lds_ring + sl * kStage + lane16);
+      const u32 at = lds_ring + sl * kChunk + lane16;
+      lds_read128<PAGE * 2048>(tok[buf][0][0], at);
+      lds_read128<PAGE * 2048 + 1024>(tok[buf][0][1], at);
+      lds_read128<PAGE * 2048 + 8192>(tok[buf][1][0], at);
+      lds_read128<PAGE * 2048 + 8192 + 1024>(tok[buf][1][1], at);
     };
-    lds_read64<192>(scv[0], wt0 + g * 8u);
-    lds_read64<192>(scv[1], wt1 + g * 8u);
-    asm volatile("ds_read_u16 %0, %1 offset:222" : "=&v"(dv[0]) : "v"(wt0) : "memory");
-    asm volatile("ds_read_u16 %0, %1 offset:222" : "=&v"(dv[1]) : "v"(wt1) : "memory");
+    lds_read64<192>(scv, wt + g * 8u);
+    asm volatile("ds_read_u16 %0, %1 offset:222" : "=&v"(dv) : "v"(wt) : "memory");
     read_raw(std::integral_constant<int, 0>{});
+    read_raw(std::integral_constant<int, 1>{});      // (chunks 2 and 3 are the high nibbles of the same words)
     read_tokens(0, 0u, std::integral_constant<int, 0>{});
-    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(scv[0]), "+v"(scv[1]), "+v"(dv[0]), "+v"(dv[1])::"memory");
-    float d[2];
-    h16x2 scale[2][4];      // chunk c: sc of its products with H = 0 and 1
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      d[r] = half_bits_to_f32(dv[r]);
-      const u32 x = scv[r].x ^ 0x80808080u, y = scv[r].y ^ 0x80808080u;
-      scale[r][0] = as_h16x2((x & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
-      scale[r][1] = as_h16x2(((x >> 8) & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
-      scale[r][2] = as_h16x2((y & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
-      scale[r][3] = as_h16x2(((y >> 8) & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
+    asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(scv), "+v"(dv), "+v"(ql[0][0]), "+v"(ql[0][1]), "+v"(qh[0]), "+v"(ql[1][0]), "+v"(ql[1][1]), "+v"(qh[1]) : "n"(2 * kTiles) : "memory");
+    const float d = half_bits_to_f32(dv);
+    h16x2 scale[4];      // chunk c: sc of its products with H = 0 and 1
+    {
+      const u32 x = scv.x ^ 0x80808080u, y = scv.y ^ 0x80808080u;
+      scale[0] = as_h16x2((x & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
+      scale[1] = as_h16x2(((x >> 8) & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
+      scale[2] = as_h16x2((y & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
+      scale[3] = as_h16x2(((y >> 8) & 0x00FF00FFu) | 0x64006400u) - h2(1152.0f);
     }
     // (2 q2 - 3) sc 2^-20, (nib - 8) sc 2^-12, the whole weight rounded to f16 2^-23 (2^-11 of the former's scale: lo pieces
     // carry 2^11; what is below 2^-14 is a whole multiple of 2^-24 and exact as a subnormal)
-    h16x8 wq[2], wn[2], wa[2];
-    auto build = [&](int r, int q) {      // product q = 4 c + 2 i + H
-      const int cc = q >> 2, i = (q >> 1) & 1, H = q & 1, hi_nib = cc >> 1, gq = 2 * hi_nib + H;
-      const u32 t0 = i ? ql[r][H].z : ql[r][H].x, t1 = i ? ql[r][H].w : ql[r][H].y, c0 = i ? qh[r].z : qh[r].x, c1 = i ? qh[r].w : qh[r].y;
+    h16x8 wq, wn, wa;
+    auto build = [&](int q) {      // product q = 4 c + 2 i + H
+      const int cc = q >> 2, i = (q >> 1) & 1, H = q & 1, hi_nib = cc >> 1, gq = 2 * hi_nib + H, set = cc & 1;
+      const u32 t0 = i ? ql[set][H].z : ql[set][H].x, t1 = i ? ql[set][H].w : ql[set][H].y, c0 = i ? qh[set].z : qh[set].x, c1 = i ? qh[set].w : qh[set].y;
       // nibbles to bits 4..7 of their 16-bit lanes, fields to bits 4..5: bytes 0 and 2 first, then 1 and 3
       auto up = [](u32 v, int by) { return by >= 0 ? v << by : v >> -by; };
       const u32 a[4] = {hi_nib ? t0 : t0 << 4, hi_nib ? t0 >> 8 : t0 >> 4, hi_nib ? t1 : t1 << 4, hi_nib ? t1 >> 8 : t1 >> 4};
       const u32 b[4] = {up(c0, 4 - 2 * gq), up(c0, -4 - 2 * gq), up(c1, 4 - 2 * gq), up(c1, -4 - 2 * gq)};
-      const h16x2 sn = scale[r][cc] * h2(256.0f), an = scale[r][cc] * h2(-0.001953125f);              // -8 * 2^-12
-      const h16x2 sq = scale[r][cc] * h2(2.0f), aq = scale[r][cc] * h2(-0.00000286102294921875f);    // -3 * 2^-20
+      const h16x2 sn = scale[cc] * h2(256.0f), an = scale[cc] * h2(-0.001953125f);              // -8 * 2^-12
+      const h16x2 sq = scale[cc] * h2(2.0f), aq = scale[cc] * h2(-0.00000286102294921875f);    // -3 * 2^-20
       u32 vn[4], vq[4], va[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
@@ -501,80 +507,71 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
         vq[k] = __builtin_bit_cast(u32, q2);
         va[k] = __builtin_bit_cast(u32, __builtin_elementwise_fma(n2, h2(0.00048828125f), q2));
       }
-      wn[r] = __builtin_bit_cast(h16x8, u32x4{vn[0], vn[1], vn[2], vn[3]});
-      wq[r] = __builtin_bit_cast(h16x8, u32x4{vq[0], vq[1], vq[2], vq[3]});
-      wa[r] = __builtin_bit_cast(h16x8, u32x4{va[0], va[1], va[2], va[3]});
+      wn = __builtin_bit_cast(h16x8, u32x4{vn[0], vn[1], vn[2], vn[3]});
+      wq = __builtin_bit_cast(h16x8, u32x4{vq[0], vq[1], vq[2], vq[3]});
+      wa = __builtin_bit_cast(h16x8, u32x4{va[0], va[1], va[2], va[3]});
     };
-    f32x16 acc[2], low[2];
+    f32x16 acc[kTiles], low[kTiles];
     // half a super-block's share of the running sums: the shorter the matrix cores' own sums, the less they round (over
     // whole super-blocks the error was 2 % above the 16-token kernel's for K <= 4096)
     auto add_up = [&]() {
-      u32x4 f0, f1, f2, f3;
-      lds_read128<1024>(f0, aux + g * 16u);          // 2^(E+14) of the tokens 8 a + 4 g + {0..3}, a = 0..3
-      lds_read128<1056>(f1, aux + g * 16u);
-      lds_read128<1088>(f2, aux + g * 16u);
-      lds_read128<1120>(f3, aux + g * 16u);
-      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)::"memory");
-      const u32 fb[16] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, f3.x, f3.y, f3.z, f3.w};
 #pragma unroll
-      for (int r = 0; r < 2; ++r)
+      for (int t = 0; t < kTiles; ++t) {
+        u32x4 f0, f1, f2, f3;
+        const u32 at_t = aux + t * kAuxBytes + g * 16u;
+        lds_read128<1024>(f0, at_t);          // 2^(E+14) of the tokens 8 a + 4 g + {0..3}, a = 0..3
+        lds_read128<1056>(f1, at_t);
+        lds_read128<1088>(f2, at_t);
+        lds_read128<1120>(f3, at_t);
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)::"memory");
+        const u32 fb[16] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, f3.x, f3.y, f3.z, f3.w};
 #pragma unroll
-        for (int v = 0; v < 16; ++v) tot[r][v] = fmaf(__uint_as_float(fb[v]), fmaf(512.0f * d[r], acc[r][v], 0.25f * d[r] * low[r][v]), tot[r][v]);      // 2^(E+14)
+        for (int v = 0; v < 16; ++v) tot[t][v] = fmaf(__uint_as_float(fb[v]), fmaf(512.0f * d, acc[t][v], 0.25f * d * low[t][v]), tot[t][v]);      // 2^(E+14)
+      }
     };
     auto step = [&](auto i_c) {
       constexpr int I = decltype(i_c)::value, CH = I / 4, B = I & 1, X = CH + 1;
-      auto products = [&](int r) {
-        const h16x8 lo = __builtin_bit_cast(h16x8, tok[B][0]), hi = __builtin_bit_cast(h16x8, tok[B][1]);
-        acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, wq[r], I % 8 == 0 ? zero : acc[r], 0, 0, 0);
-        low[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, wa[r], I % 8 == 0 ? zero : low[r], 0, 0, 0);
-        low[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, wn[r], low[r], 0, 0, 0);
+      auto products = [&](int t) {
+        const h16x8 lo = __builtin_bit_cast(h16x8, tok[B][t][0]), hi = __builtin_bit_cast(h16x8, tok[B][t][1]);
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, wq, I % 8 == 0 ? zero : acc[t], 0, 0, 0);
+        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, wa, I % 8 == 0 ? zero : low[t], 0, 0, 0);
+        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, wn, low[t], 0, 0, 0);
       };
       if constexpr (I % 4 == 3) {
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tok[B][0]), "+v"(tok[B][1])::"memory");
-        build(0, I);
-        build(1, I);
-        if constexpr (CH < 3) {
-          // (the operands are made before the registers of the weights are asked for again)
-          asm volatile("" : "+v"(wq[0]), "+v"(wq[1]), "+v"(wn[0]), "+v"(wn[1]), "+v"(wa[0]), "+v"(wa[1])::"memory");
-          read_raw(std::integral_constant<int, X>{});
-          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ql[0][0]), "+v"(ql[0][1]), "+v"(qh[0]), "+v"(ql[1][0]), "+v"(ql[1][1]), "+v"(qh[1])::"memory");
-        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1])::"memory");
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(X == 4 ? WD + 1 : 0) : "memory");      // chunk X is there
         asm volatile("s_barrier" ::: "memory");
-        issue_tokens(min(s + (CH + 2) / 4u, ns - 1u), (CH + 2) & 3, CH & 1);      // chunk CH + 2 takes this one's place
-        if constexpr (X == 3) {      // the last of this weight tile is in registers: its place takes the next one
+        tokens.chunk(min(s + (CH + 2) / 4u, ns - 1u), (CH + 2) & 3, CH & 1);      // chunk CH + 2 takes this one's place
+        if constexpr (X == 3) {      // all of this weight tile is in registers: its place takes the next one
           issue_w(min(s + 1u, ns - 1u));
-          issue_aux(min(s + 1u, ns - 1u), (s + 1u) & 1u);
+          tokens.sums(min(s + 1u, ns - 1u), (s + 1u) & 1u);
         }
         if constexpr (I < 15) read_tokens(1 - B, X & 1, std::integral_constant<int, 0>{});
+        build(I);
         products(0);
         products(1);
         if constexpr (I == 7 || I == 15) add_up();
       } else {
         read_tokens(1 - B, CH & 1, std::integral_constant<int, (I + 1) & 3>{});
-        asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(tok[B][0]), "+v"(tok[B][1])::"memory");
-        if constexpr (I == 0)
-          asm volatile("" : "+v"(ql[0][0]), "+v"(ql[0][1]), "+v"(qh[0]), "+v"(ql[1][0]), "+v"(ql[1][1]), "+v"(qh[1])::"memory");
-        build(0, I);
+        build(I);
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1]) : "n"(2 * kTiles) : "memory");
         products(0);
-        build(1, I);
         products(1);
       }
     };
     __builtin_amdgcn_s_setprio(1);
     for_each_product(step, std::make_integer_sequence<int, 16>{});
     __builtin_amdgcn_s_setprio(0);
-    if (--left == 0u || s + 1u == ns) {
+    if (--left == 0u) {
       left = run;
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        stash[r] += tot[r];
-        tot[r] = zero;
-      }
+      for (int t = 0; t < kTiles; ++t) put_by<true>(stash[t], tot[t]);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  store_tile(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile, g);
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) stash[t] += tot[t];
+  store_tiles(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (kTiles * kTile), g);
 }
 
 // c = the parts of K in part order

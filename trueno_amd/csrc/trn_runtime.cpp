@@ -653,15 +653,16 @@ hipError_t launch_gemm_few(DeviceKernels* d, hipStream_t stream, uint64_t a, uin
 }
 
 // ---- many tokens (kquant_gemm_tall.hip.h) -----------------------------------------------------------------------------
-constexpr uint32_t kTallRows = 256, kTallTile = 32, kTallOperandBytes = 32u * 1024u + 2048u;      // rows and tokens of a workgroup; of a (tile, super-block)
+constexpr uint32_t kTallRows = 128, kTallTokens = 64, kTallTile = 32;      // rows and tokens of a workgroup; tokens of an operand tile
+constexpr uint32_t kTallOperandBytes = 32u * 1024u + 2048u;      // of a (tile, super-block)
 // The most a product's workspace holds; a product that needs more goes through it in runs of tokens, and its price is that of
 // its runs: 4096 x 65536, 2048 tokens, take three.  trn_q4k_gemm_noalloc has as much (trn_noalloc.hip), so that its runs, and
 // with them the choice of kernel and the cut, are trn_q4k_gemm's: in 16 MiB 4096 x 14336, 2048 tokens, would take eight runs
 // of 128 workgroups, an estimated 1161 us against 549 in one and 721 for sixteen tokens at a time.
 constexpr size_t kTallWorkspaceMax = size_t(256) << 20;
 size_t tall_workspace_cap() { return g_tune_gemm_workspace_mb > 0 ? std::min(size_t(g_tune_gemm_workspace_mb) << 20, kTallWorkspaceMax) : kTallWorkspaceMax; }
-struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit, price = kCutDoesNotFit; };      // price: against the other kernel (tall_ok)
-uint32_t tall_lds_bytes(Fmt f) { return (f == Q6K ? 2u : 4u) * 8192u + 2u * 2048u + 4u * 64u * (f == Q6K ? 224u : kSbBytes[f]); }
+struct TallCut { uint32_t kparts = 1, ksb = 0; double us = kCutDoesNotFit; };
+uint32_t tall_lds_bytes(Fmt f) { return (f == Q6K ? 2u : 3u) * 16384u + 4u * 2048u + 4u * 1024u * (f == Q4K ? 5u : f == Q5K ? 6u : 7u); }
 size_t tall_bytes(uint32_t tokens, uint32_t n, uint32_t nsb, uint32_t kparts) {
   const size_t tiles = (tokens + kTallTile - 1u) / kTallTile;
   return tiles * nsb * kTallOperandBytes + (kparts > 1u ? (size_t(kparts) * tokens * n * 4u + 255u) / 256u * 256u : 0u);
@@ -669,25 +670,27 @@ size_t tall_bytes(uint32_t tokens, uint32_t n, uint32_t nsb, uint32_t kparts) {
 // The tokens of a run through `cap` bytes: all of them, or as many whole tiles as it holds (0: not one).
 uint32_t tall_run(uint32_t m, uint32_t n, uint32_t nsb, uint32_t kparts, size_t cap) {
   if (tall_bytes(m, n, nsb, kparts) <= cap) return m;
-  return uint32_t(std::min<size_t>(cap / tall_bytes(kTallTile, n, nsb, kparts), m / kTallTile)) * kTallTile;
+  const uint32_t fit = uint32_t(std::min<size_t>(cap / tall_bytes(kTallTile, n, nsb, kparts), m / kTallTile)) * kTallTile;
+  return fit > kTallTokens ? fit / kTallTokens * kTallTokens : fit;      // (whole workgroups)
 }
-// The parts of K with the least estimated time, the same for every run.  Times in microseconds fitted to measurements on MI355X (1024 x 4096 ..
-// 32000 x 4096 and 4096 x 11008, 33 .. 1024 tokens, within about 10 % from 64 tokens on): 9 for the launches and the first
-// super-block of a run; the operands at 4 TB/s; a super-block takes a round of two workgroups per CU 4.3 / 5.1 / 7.5 (Q4_K / Q5_K /
-// Q6_K), one workgroup alone on its CU 2.3 / 2.7 / 4.2; with K in parts 3 for the sum's launch, 0.4 a part, and the parts'
-// bytes at 4 TB/s.
+// The parts of K with the least estimated time, the same for every run.  Times in microseconds fitted to 1350 measurements on
+// MI355X (367 drawn products, 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns, up to six cuts each; 4-5 % root mean square,
+// 6-8 % at the 90th percentile): 8 for the launches and the first super-block of a run; the operands at 7.5 TB/s; a super-block takes
+// a round of two workgroups per CU 4.3 / 4.5 / 6.0 (Q4_K / Q5_K / Q6_K), one workgroup alone on its CU 2.3 / 2.6 / 3.2, and some CUs with two and
+// others with one, 0.6-0.7 of the step between at once.  The rounds are an XCD's, which gets an eighth of the workgroups.  With K in
+// parts 0.5 for the sum's launch, 0.3 a part, and the parts' bytes at 2.3 TB/s.
 TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k) {
   TallCut best;
-  const uint32_t nsb = k / 256u, groups = (n + kTallRows - 1u) / kTallRows, tiles = (m + kTallTile - 1u) / kTallTile, cus = uint32_t(d.cu_count);
-  const uint64_t units = uint64_t(groups) * tiles;
-  const double pair = f == Q4K ? 4.3 : f == Q5K ? 5.1 : 7.5, alone = f == Q4K ? 2.3 : f == Q5K ? 2.7 : 4.2;
+  const uint32_t nsb = k / 256u, groups = (n + kTallRows - 1u) / kTallRows, units_m = (m + kTallTokens - 1u) / kTallTokens, cus = uint32_t(d.cu_count);
+  const uint64_t units = uint64_t(groups) * units_m, xcd_cus = std::max(1u, cus / 8u);
+  const double pair = f == Q4K ? 4.3 : f == Q5K ? 4.5 : 6.0, alone = f == Q4K ? 2.3 : f == Q5K ? 2.6 : 3.2, uneven = f == Q4K ? 0.6 : 0.7;
   const uint32_t most = g_tune_gemm_ksplit > 0 ? std::min<uint32_t>(uint32_t(g_tune_gemm_ksplit), nsb)
                                                : uint32_t(std::max<uint64_t>(1u, std::min<uint64_t>((2u * cus + units / 2u) / units, nsb)));
-  auto run_us = [&](const TallCut& c, uint32_t tokens, double uneven) {
-    const uint64_t wgs = uint64_t(groups) * ((tokens + kTallTile - 1u) / kTallTile) * c.kparts, rounds = wgs / (2u * cus), rest = wgs - rounds * 2u * cus;
-    const double last = rest == 0u ? 0.0 : rest <= cus ? alone : alone + (pair - alone) * (uneven + (1.0 - uneven) * double(rest - cus) / cus);
-    return 9.0 + double(tokens) * k * 8.0 / 4.0e6 + c.ksb * (double(rounds) * pair + last) +
-           (c.kparts > 1u ? 3.0 + 0.4 * c.kparts + double(c.kparts + 1u) * tokens * n * 4.0 / 4.0e6 : 0.0);
+  auto run_us = [&](const TallCut& c, uint32_t tokens) {
+    const uint64_t wgs = (uint64_t(groups) * ((tokens + kTallTokens - 1u) / kTallTokens) * c.kparts + 7u) / 8u, rounds = wgs / (2u * xcd_cus), rest = wgs - rounds * 2u * xcd_cus;
+    const double last = rest == 0u ? 0.0 : rest <= xcd_cus ? alone : alone + (pair - alone) * (uneven + (1.0 - uneven) * double(rest - xcd_cus) / double(xcd_cus));
+    return 8.0 + double(tokens) * k * 8.0 / 7.5e6 + c.ksb * (double(rounds) * pair + last) +
+           (c.kparts > 1u ? 0.5 + 0.3 * c.kparts + double(c.kparts + 1u) * tokens * n * 4.0 / 2.3e6 : 0.0);
   };
   for (uint32_t kp = most; kp >= 1u; --kp) {
     TallCut c;
@@ -695,9 +698,7 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
     c.kparts = (nsb + c.ksb - 1u) / c.ksb;
     const uint32_t step = tall_run(m, n, nsb, c.kparts, tall_workspace_cap());
     if (step != 0u) {
-      auto all_us = [&](double uneven) { return (m / step) * run_us(c, step, uneven) + (m % step != 0u ? run_us(c, m % step, uneven) : 0.0); };
-      c.us = all_us(0.0);
-      c.price = all_us(0.5);
+      c.us = (m / step) * run_us(c, step) + (m % step != 0u ? run_us(c, m % step) : 0.0);
       if (c.us < best.us) best = c;
     }
     if (g_tune_gemm_ksplit > 0) break;
@@ -741,15 +742,16 @@ void* tall_alloc(size_t bytes) {      // nullptr: none to be had, and no error i
 hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
                             uint32_t k, const TallCut& cut, uint64_t ws) {
   uint32_t nsb = k / 256u, tiles = (m + kTallTile - 1u) / kTallTile, kparts = cut.kparts, ksb = cut.ksb;
-  uint32_t groups = (n + kTallRows - 1u) / kTallRows;
-  uint32_t run = 1u;      // super-blocks summed by themselves: about the root of a part's
-  while (run * run < ksb) ++run;
+  uint32_t groups = (n + kTallRows - 1u) / kTallRows, pairs = (m + kTallTokens - 1u) / kTallTokens;
+  // super-blocks summed by themselves: about the root of a part's; where that is put by without loss (put_by of the kernel), six of a long part's
+  uint32_t run = 1u;
+  while (run * run < ksb && (f == Q4K || ksb <= 8u || run < 6u)) ++run;
   uint64_t ops = ws, parts = kparts > 1u ? ws + size_t(tiles) * nsb * kTallOperandBytes : c, mn = uint64_t(m) * n;
   void* oargs[] = {&a, &ops, &m, &nsb};
   hipError_t e = hipModuleLaunchKernel(d->tall_operands, tiles * nsb, 1, 1, 256, 1, 1, 0, stream, oargs, nullptr);
   if (e != hipSuccess) return e;
-  void* margs[] = {&ops, &w, &parts, &m, &n, &nsb, &ksb, &kparts, &groups, &tiles, &run};
-  const uint32_t grid = (groups * tiles * kparts + 7u) / 8u * 8u;
+  void* margs[] = {&ops, &w, &parts, &m, &n, &nsb, &ksb, &kparts, &groups, &pairs, &run};
+  const uint32_t grid = (groups * pairs * kparts + 7u) / 8u * 8u;
   if ((e = hipModuleLaunchKernel(d->gemm_tall[f], grid, 1, 1, 256, 1, 1, tall_lds_bytes(f), stream, margs, nullptr)) != hipSuccess) return e;
   if (kparts == 1u) return hipSuccess;
   void* sargs[] = {&c, &parts, &mn, &kparts};
@@ -846,30 +848,25 @@ extern "C" {      // (defined further down inside the extern "C" part of the fil
 hipError_t launch_gemv_group(DeviceKernels* d, hipStream_t stream, const trn_gemv_desc* descs, uint32_t len);
 }
 
-// Does the kernel for many tokens take this product?  From 33 tokens on, where its estimate is below the other's: that one
-// holds for Q4_K, while Q5_K takes 1.1 and Q6_K 1.3 to 1.6 times as long from 64 tokens on (the factors below stay at the
-// lower end).  Up to 32 tokens, one tile, it gained nothing anywhere (Q5_K 11008 x 4096, 17 tokens: 28 against 23 us).
-// Both sides measured over nine shapes, 17 .. 1024 tokens (us, sixteen at a time -> this kernel):
-//   14336 x 4096, 2048 tokens, Q4_K 835 -> 525;   11008 x 4096, 512 tokens: Q4_K 180 -> 126, Q5_K 190 -> 142, Q6_K 318 -> 201
-//   4096 x 11008, 512 tokens: Q4_K 159 -> 129, Q5_K 167 -> 150, Q6_K 288 -> 195;   32000 x 4096, 64 tokens: 60 -> 55, 68 -> 63, 110 -> 84
-//   4096 x 4096, 64 tokens: 16 and 21 (Q4_K), 20 and 26 (Q6_K): stays;   1024 x 4096, 512 tokens, Q4_K: 24 and 29: stays
-// The estimates that choose each kernel's cut leave two things out, and with those counted it has to be the faster one still:
-// here, where some CUs have two workgroups and the others one, the launch ends with the former (half of the step from one
-// to two comes at once: Q6_K 6093 x 2560, 330 tokens, 264 workgroups, 82 us against 68); there, the rounds are an XCD's, whose 32
-// CUs get every eighth unit (Q4_K 32000 x 4096, 33 tokens: 88 us where 46 were estimated).  Of 1200 drawn products, 33 .. 900
-// tokens, that the first comparison gives to this kernel about 135 were 3 to 17 % slower with it; the second takes 112 of
-// them back, and with them twelve that it made 3 to 10 % faster.  (What the other kernel keeps although it is the slower one,
-// as in the example, stays: the cuts would have to be fitted anew with it.)
+// Does the kernel for many tokens take this product?  From 33 tokens on, where its estimate is below the other's with that one's
+// rounds counted by XCD too: an XCD's 32 CUs get every eighth unit (Q4_K 32000 x 4096, 33 tokens: 88 us where 46 were estimated).  The
+// other's estimate was fitted to Q4_K; measured times over it, medians: with 8 or 12 strips 1.00-1.10 / 1.10-1.32 / 1.45-1.58 (Q4_K / Q5_K / Q6_K), with
+// 4 strips 0.86 / 0.98 / 1.02 up to 128 tokens; the factors below gave the least sum over the 367 products.  Up to 32 tokens, half a workgroup's,
+// it gained nothing anywhere (Q5_K 11008 x 4096, 17 tokens: 28 against 23 us).
+// Of those products the better of the two kernels with its best cut is missed by 0.7 % on the average (9 % with the estimates fitted to
+// tiles of 256 rows x 32 tokens).  Both sides (us, sixteen tokens at a time -> this kernel): 14336 x 4096, 2048 tokens, Q4_K 835 -> 522; 512 tokens: 11008 x 4096 Q4_K 180 -> 117,
+// Q5_K 190 -> 127, 4096 x 11008 Q6_K 288 -> 160; 4096 x 4096, 128 tokens, Q4_K 23.0 and 26.1: stays; Q6_K 6093 x 2560, 330 tokens: 74 -> 65, but 62 estimated
+// against 61: stays.
 bool tall_ok(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k, bool forced) {
-  if (g_tune_gemm_tall == 1 || m <= 32u || k / 256u > 0x3FFFu || uint64_t((n + kTallRows - 1u) / kTallRows) * ((m + kTallTile - 1u) / kTallTile) > 0xFFFFFu)
+  if (g_tune_gemm_tall == 1 || m <= 32u || k / 256u > 0x3FFFu || uint64_t((n + kTallRows - 1u) / kTallRows) * ((m + kTallTokens - 1u) / kTallTokens) > 0xFFFFFu)
     return false;
   const TallCut cut = tall_cut(d, f, m, n, k);
   if (g_tune_gemm_tall == 2) return cut.us < kCutDoesNotFit;
   if (forced) return false;
   const GemmCut other = gemm_cut(d, f, m, n, k);
-  if (cut.us >= other.us * (f == Q4K ? 1.0 : f == Q5K ? (m < 64u ? 1.05 : 1.1) : (m < 64u ? 1.1 : 1.3))) return false;
   const uint64_t xcd_cus = std::max(1u, uint32_t(d.cu_count) / 8u), xcd_wgs = (uint64_t(other.groups) * other.kparts + 7u) / 8u * other.tgroups;
-  return cut.price < gemm_cut_us(f, m, n, k, other, (xcd_wgs + xcd_cus - 1u) / xcd_cus) * (f == Q4K ? 1.09 : f == Q5K ? 1.14 : 1.4);
+  const double factor = other.waves == 4u ? 1.0 : f == Q4K ? 1.05 : f == Q5K ? 1.15 : 1.38;
+  return cut.us < factor * gemm_cut_us(f, m, n, k, other, (xcd_wgs + xcd_cus - 1u) / xcd_cus);
 }
 
 // Which kernel takes a product of m >= 1 tokens: the integer matrix cores (Q4_K, two to four tokens, where their fitted
