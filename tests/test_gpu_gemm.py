@@ -719,3 +719,94 @@ def test_gemm_many_tokens_by_the_rule(gpu, fmt, m, n, k, many):
     finally:
         _tune("gemm_tall", 0)
     assert np.array_equal(bits[0], bits[2 if many else 1]) and not np.array_equal(bits[1], bits[2])
+
+
+@pytest.mark.parametrize("m,n,k,parts", [(2, 1, 256, 1), (16, 67, 2048, 1), (17, 95, 2304, 1), (33, 193, 4352, 3), (48, 64, 8192, 32), (5, 130, 1280, 5)])
+@pytest.mark.parametrize("rows", (1, 2, 3, 4))
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_slices_kernel(gpu, fmt, rows, m, n, k, parts):
+    """The kernel that deals the super-blocks of its rows to its waves, forced, with every height of a workgroup: one row, one super-block
+    (seven waves idle), eight, nine (a second round for one wave) and seventeen in three parts, thirty-two parts, rows that fill no tile and
+    are no multiple of four, tokens that fill no tile: within tolerance, the same bits on every run, a token's values large or small
+    against the others', an infinity in its own token only."""
+    if rows == 4 and fmt != "q4k":
+        pytest.skip("64 rows are Q4_K's")
+    buf, a = kq.gen_matrix(fmt, 700 + m, n, k), kq.gen_x(710 + m, m, k)
+    a[0] *= np.float32(1e6)
+    a[m - 1] *= np.float32(1e-6)
+    w = kq.dequant_matrix(fmt, buf, n, k)
+    c64, terms = _c64(fmt, buf, a, n, k), np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    try:
+        _tune("gemm_slices", 2)
+        _tune("gemm_slices_rows", rows)
+        _tune("gemm_k_parts", parts)
+        c = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert np.all(np.abs(c - c64) <= TOL * terms)      # as above: 1e-5 of the sum of the terms' sizes
+        again = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert np.array_equal(again.view(np.uint32), c.view(np.uint32))
+        a[1, 7] = np.inf
+        c = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+        assert not np.any(np.isfinite(c[1])) and np.array_equal(np.delete(c, 1, axis=0), np.delete(again, 1, axis=0))
+    finally:
+        for key in ("gemm_slices", "gemm_slices_rows", "gemm_k_parts"):
+            _tune(key, 0)
+
+
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_slices_no_less_exact_than_sixteen_at_a_time(gpu, fmt):
+    """By the rule, 16 tokens: against fp64 at most 1.03 times the error of the kernel that takes sixteen tokens at a time (0.95-0.98 over
+    drawn products; the ratio of two error norms over 65536 results is stable to about 2 %)."""
+    n, k, m = 4096, 4096, 16
+    buf, a = kq.gen_matrix(fmt, 720, n, k), kq.gen_x(721, m, k)
+    c64, err = _c64(fmt, buf, a, n, k), {}
+    try:
+        for slices in (0, 1):
+            _tune("gemm_slices", slices)
+            err[slices] = kq.rel_l2(gpu_gemm(gpu, fmt, buf, a, m, n, k), c64)
+    finally:
+        _tune("gemm_slices", 0)
+    assert err[0] != err[1] and err[0] <= 1.03 * err[1], err
+
+
+def test_gemm_slices_captured_on_a_new_stream_and_without_allocation(gpu):
+    """Four tokens against 6000 x 4096, which the integer cores took without scratch memory: captured on a stream that has seen no product.
+    16 tokens against 512 x 4096, parts of K: the same bits from trn_q4k_gemm_noalloc."""
+    ctx, stream = gpu
+    for m, n, k, whole in ((4, 6000, 4096, True), (16, 512, 4096, False)):
+        buf, a = kq.gen_matrix("q4k", 730 + m, n, k), kq.gen_x(731, m, k)
+        want = gpu_gemm(gpu, "q4k", buf, a, m, n, k).view(np.uint32)
+        dw, da = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, a)
+        dc = t.GpuBuffer.from_host(ctx, np.full(m * n, np.nan, np.float32))
+        if whole:
+            new = t.CudaStream(ctx)
+            graph = _Captured(new, lambda: t.QuantizeKernel.ggml(m, n, k).launch(new, da, dw, dc))
+            for _ in range(3):
+                dc.copy_from_host(np.full(m * n, np.nan, np.float32))
+                graph.replay(new)
+                new.synchronize()
+                assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), want)
+            graph.close()
+        else:
+            for _ in range(2):
+                assert _ffi.lib().trn_q4k_gemm_noalloc(stream.raw(), da.as_ptr(), dw.as_ptr(), dc.as_ptr(), m, n, k) == 0
+                stream.synchronize()
+                assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), want)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 1, 256), (64, 255, 512), (65, 257, 1280), (97, 700, 2304)])
+@pytest.mark.parametrize("fmt", ("q4k", "q5k"))
+def test_gemm_many_tokens_either_shape_of_a_workgroup(gpu, fmt, m, n, k):
+    """256 rows x 32 tokens and 128 x 64: the same sums in the same order, so the same bits for the same parts of K."""
+    buf, a = kq.gen_matrix(fmt, 740 + m, n, k), kq.gen_x(741, m, k)
+    try:
+        _tune("gemm_tall", 2)
+        for parts in (1, 2):
+            _tune("gemm_k_parts", parts)
+            bits = []
+            for strips in (1, 2):
+                _tune("gemm_tall_strips", strips)
+                bits.append(gpu_gemm(gpu, fmt, buf, a, m, n, k).view(np.uint32))
+            assert np.array_equal(*bits)
+    finally:
+        for key in ("gemm_tall", "gemm_k_parts", "gemm_tall_strips"):
+            _tune(key, 0)

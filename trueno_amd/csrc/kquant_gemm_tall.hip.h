@@ -30,8 +30,7 @@ namespace gemm_tall {
 using namespace gemm_f16;      // the LDS helpers, split_f16, pack_h2
 
 constexpr u32 kTile = 32;                      // tokens of an operand tile
-constexpr int kTiles = 2;                      // operand tiles a workgroup takes
-constexpr u32 kWaves = 4, kWaveRows = 32;      // its rows of W: a strip of 32 a wave
+constexpr u32 kWaves = 4;                      // of a workgroup; a wave holds RT strips of 32 rows against TT operand tiles, RT TT = 2
 constexpr u32 kPagesBytes = 32 * 1024;         // 16 products x (lo page, hi page) of 64 lanes x 16 bytes
 constexpr u32 kAuxBytes = 2048;                // sums (1 KB), factors (128 bytes, padded)
 constexpr u32 kOperandBytes = kPagesBytes + kAuxBytes;      // of a (token tile, super-block)
@@ -129,9 +128,10 @@ __device__ __forceinline__ h16x2 bytes_to_h2(u32 v) {
 }
 __device__ __forceinline__ h16x2 h2(float v) { return h16x2{static_cast<_Float16>(v), static_cast<_Float16>(v)}; }
 
-template <int FMT> struct Layout;      // weight tile in LDS: STRIDE bytes a row (an odd number of 16-byte pieces), COPIES of 64 pieces for 32 rows; STAGES chunks of tokens
-template <> struct Layout<FMT_Q4K> { static constexpr u32 SB = 144, STRIDE = 144, PIECES = 9, COPIES = 5, STAGES = 3; };
-template <> struct Layout<FMT_Q5K> { static constexpr u32 SB = 176, STRIDE = 176, PIECES = 11, COPIES = 6, STAGES = 3; };
+// weight tile in LDS: STRIDE bytes a row (an odd number of 16-byte pieces), COPIES of 64 pieces for a wave's rows; STAGES chunks of tokens
+template <int FMT, int RT> struct Layout {
+  static constexpr u32 SB = FMT == FMT_Q4K ? 144u : 176u, STRIDE = SB, PIECES = SB / 16u, COPIES = (32u * RT * PIECES + 63u) / 64u, STAGES = RT == 1 ? 3u : 4u;
+};
 
 template <class F, int... I>
 __device__ __forceinline__ void for_each_product(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
@@ -151,16 +151,19 @@ struct Place {
   }
 };
 
-// lane l holds W row row and the tokens 8 (v / 4) + 4 g + v % 4 of either tile
-__device__ __forceinline__ void store_tiles(const f32x16 (&sum)[kTiles], float* __restrict__ out, u32 m, u32 n, u32 row, u32 token0, u32 g) {
-  if (row >= n) return;
+// lane l holds W row row (of strips 32 apart) and the tokens 8 (v / 4) + 4 g + v % 4 of a tile; sum i is strip i / TT, tile i % TT
+template <int RT, int TT>
+__device__ __forceinline__ void store_tiles(const f32x16 (&sum)[2], float* __restrict__ out, u32 m, u32 n, u32 row, u32 token0, u32 g) {
 #pragma unroll
-  for (int t = 0; t < kTiles; ++t)
+  for (int i = 0; i < 2; ++i) {
+    if (row + 32u * (i / TT) < n) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const u32 token = token0 + kTile * t + 8u * (v >> 2) + 4u * g + (v & 3);
-      if (token < m) out[static_cast<size_t>(token) * n + row] = sum[t][v];
+      for (int v = 0; v < 16; ++v) {
+        const u32 token = token0 + kTile * (i % TT) + 8u * (v >> 2) + 4u * g + (v & 3);
+        if (token < m) out[static_cast<size_t>(token) * n + row + 32u * (i / TT)] = sum[i][v];
+      }
     }
+  }
 }
 
 // The running sums are put by; LOSSLESS: what the sum of both rounds away starts the next run, so that the length of a part costs no
@@ -178,38 +181,44 @@ __device__ __forceinline__ void put_by(f32x16& stash, f32x16& tot) {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// the copies of both bodies: a chunk in LDS is [tile][product][lo, hi][64 lanes], 16 KB, of which wave w brings product w
-constexpr u32 kChunk = kTiles * 8192u;
-constexpr int kChunkCopies = 2 * kTiles;      // of a wave's share of a chunk
+// the copies of both bodies: a chunk in LDS is [tile][product][lo, hi][64 lanes], 8 KB a tile, of which wave w brings product w
+template <int TT>
 struct TokenCopies {
+  static constexpr u32 kChunk = TT * 8192u;
+  static constexpr int kCopies = 2 * TT;      // of a wave's share of a chunk
   __amdgpu_buffer_rsrc_t rsrc;
   u32 lane16, wave, tile_bytes, ring, aux;
   // (a second tile that is not there: the first one again, its results are not stored)
-  __device__ __forceinline__ TokenCopies(const uint8_t* ops, u32 pair, u32 m, u32 nsb, u32 sb0, u32 ns, u32 lane, u32 wave_, u32 ring_, u32 aux_)
-      : lane16(lane * 16u), wave(wave_), tile_bytes((kTiles * pair + 1u) * kTile < m ? nsb * kOperandBytes : 0u), ring(ring_), aux(aux_) {
-    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ops) + (static_cast<size_t>(pair) * kTiles * nsb + sb0) * kOperandBytes, 0,
+  __device__ __forceinline__ TokenCopies(const uint8_t* ops, u32 tiles, u32 m, u32 nsb, u32 sb0, u32 ns, u32 lane, u32 wave_, u32 ring_, u32 aux_)
+      : lane16(lane * 16u), wave(wave_), tile_bytes(TT == 2 && (TT * tiles + 1u) * kTile < m ? nsb * kOperandBytes : 0u), ring(ring_), aux(aux_) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ops) + (static_cast<size_t>(tiles) * TT * nsb + sb0) * kOperandBytes, 0,
                                              static_cast<int>(tile_bytes + ns * kOperandBytes), 0x00020000);
   }
   __device__ __forceinline__ void chunk(u32 s, u32 c, u32 slot) const {
 #pragma unroll
-    for (u32 t = 0; t < kTiles; ++t) {
+    for (u32 t = 0; t < TT; ++t) {
       const u32 src = s * kOperandBytes + t * tile_bytes + c * 8192u + wave * 2048u, dst = ring + slot * kChunk + t * 8192u + wave * 2048u;
       buffer_dma16(rsrc, dst, lane16, src);
       buffer_dma16(rsrc, dst + 1024u, lane16, src + 1024u);
     }
   }
-  __device__ __forceinline__ void sums(u32 s, u32 buf) const {      // the tiles' aux, a KB a wave
-    buffer_dma16(rsrc, aux + buf * (kTiles * kAuxBytes) + wave * 1024u, lane16,
-                 s * kOperandBytes + (wave >> 1) * tile_bytes + kPagesBytes + (wave & 1u) * 1024u);
+  __device__ __forceinline__ void sums(u32 s, u32 buf) const {      // the tiles' aux, a KB a wave (one tile: by two waves and, for one count of copies, by the others as well)
+    const u32 t = TT == 2 ? wave >> 1 : 0u;
+    buffer_dma16(rsrc, aux + buf * (TT * kAuxBytes) + t * kAuxBytes + (wave & 1u) * 1024u, lane16, s * kOperandBytes + t * tile_bytes + kPagesBytes + (wave & 1u) * 1024u);
   }
 };
+// keeps an asm's outputs behind the wait in front of this
+template <class T> __device__ __forceinline__ void landed(T& v) { asm volatile("" : "+v"(v)::"memory"); }
 
 // dynamic LDS: the ring of chunks, two aux pages, a weight tile per wave (tall_lds_bytes of the runtime)
-template <int FMT>
+template <int FMT, int RT, int TT>
 __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint8_t* __restrict__ w, float* __restrict__ c,
                                      u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 pairs, u32 run, u32 lds_base) {
-  using L = Layout<FMT>;
-  constexpr int S = static_cast<int>(L::STAGES), TD = kChunkCopies, WD = static_cast<int>(L::COPIES);
+  static_assert(RT * TT == 2, "");
+  using L = Layout<FMT, RT>;
+  using Tokens = TokenCopies<TT>;
+  constexpr u32 kWaveRows = 32u * RT;
+  constexpr int S = static_cast<int>(L::STAGES), TD = Tokens::kCopies, WD = static_cast<int>(L::COPIES);
   const u32 lane = threadIdx.x & 63u;
   const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
   const Place at(blockIdx.x, groups, pairs, kparts);
@@ -219,8 +228,8 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
   const u32 row0 = at.group * (kWaves * kWaveRows) + wave * kWaveRows;
   const size_t row_bytes = static_cast<size_t>(nsb) * L::SB;
 
-  const u32 lds_ring = lds_base, lds_aux = lds_base + S * kChunk;
-  const u32 lds_w = lds_aux + 2u * kTiles * kAuxBytes + wave * (WD * 1024u);
+  const u32 lds_ring = lds_base, lds_aux = lds_base + S * Tokens::kChunk;
+  const u32 lds_w = lds_aux + 2u * TT * kAuxBytes + wave * (WD * 1024u);
 
   u32 woff[WD];
   const u32 row_first = min(row0, n - 1u);
@@ -237,14 +246,14 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
 #pragma unroll
     for (int t = 0; t < WD; ++t) buffer_dma16(w_rsrc, lds_w + 1024u * t, woff[t], s * L::SB);
   };
-  const TokenCopies tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
+  const Tokens tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
 
   // where Q4_K keeps a lane's four scales and mins: for the last four sub-blocks the upper two bits lie apart
   [[maybe_unused]] const u32 sc_up = g ? 2u : 0u, sc_mask = g ? 0x30303030u : 0x3F3F3F3Fu, sc_rest = g ? 0x0F0F0F0Fu : 0u;
-  f32x16 tot[kTiles], stash[kTiles];
+  f32x16 tot[2], stash[2];
   const f32x16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-  for (int t = 0; t < kTiles; ++t) tot[t] = stash[t] = zero;
+  for (int i = 0; i < 2; ++i) tot[i] = stash[i] = zero;
 
   // chunks 0 .. S-1 of the run, behind the first weight tile and aux pages
   issue_w(0);
@@ -257,58 +266,71 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
   u32 left = run;    // super-blocks until the running sums are put by
   for (u32 s = 0; s < ns; ++s) {
     const u32 wt = lds_w + col * L::STRIDE;
-    const u32 aux = lds_aux + (s & 1u) * (kTiles * kAuxBytes);
+    const u32 aux = lds_aux + (s & 1u) * (TT * kAuxBytes);
     // the weight tile has landed: behind its copies those of two chunks, the last of which may be on its way
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(TD) : "memory");
-    u32x4 raw[2], hdr, tok[2][kTiles][2];
-    [[maybe_unused]] u32x4 qh = {};
-    lds_read128<0>(hdr, wt);
-    lds_read128<16>(raw[0], wt + g * 64u);
-    if constexpr (FMT == FMT_Q5K) lds_read128<144>(qh, wt + g * 16u);
+    u32x4 raw[2][RT], hdr[RT], tok[2][TT][2];
+    [[maybe_unused]] u32x4 qh[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      lds_read128<0>(hdr[r], wt + 32u * r * L::STRIDE);
+      lds_read128<16>(raw[0][r], wt + 32u * r * L::STRIDE + g * 64u);
+      if constexpr (FMT == FMT_Q5K) lds_read128<144>(qh[r], wt + 32u * r * L::STRIDE + g * 16u);
+    }
     auto read_tokens = [&](int buf, u32 sl, auto page_c) {
       constexpr int PAGE = decltype(page_c)::value;
-      const u32 at = lds_ring + sl * kChunk + lane * 16u;
-      lds_read128<PAGE * 2048>(tok[buf][0][0], at);
-      lds_read128<PAGE * 2048 + 1024>(tok[buf][0][1], at);
-      lds_read128<PAGE * 2048 + 8192>(tok[buf][1][0], at);
-      lds_read128<PAGE * 2048 + 8192 + 1024>(tok[buf][1][1], at);
+      const u32 at = lds_ring + sl * Tokens::kChunk + lane * 16u;
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        lds_read128<PAGE * 2048>(tok[buf][t][0], at + 8192u * t);
+        lds_read128<PAGE * 2048 + 1024>(tok[buf][t][1], at + 8192u * t);
+      }
     };
     read_tokens(0, slot, std::integral_constant<int, 0>{});
-    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(hdr), "+v"(raw[0]), "+v"(qh) : "n"(2 * kTiles) : "memory");
-    h16x2 scale[2], addend[2], mins[2];      // sub-blocks 0 and 2 (low nibbles), 1 and 3 (high nibbles) of the lane's four
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * TT) : "memory");
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      landed(hdr[r]);
+      landed(raw[0][r]);
+      if constexpr (FMT == FMT_Q5K) landed(qh[r]);
+    }
+    h16x2 scale[RT][2], addend[RT][2], mins[RT][2];      // sub-blocks 0 and 2 (low nibbles), 1 and 3 (high nibbles) of the lane's four
+    float d[RT], nm[RT];
     constexpr float kCentre = FMT == FMT_Q4K ? 8.0f : 16.0f;
-    const float d = half_bits_to_f32(hdr.x);
-    const float nm = half_bits_to_f32(hdr.x >> 16) * -0.001953125f;       // -dmin * 2^-9: the sums carry 2^-5, the products 2^-14
-    {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const u32x4 hd = hdr[r];
       u32 s4, m4;
+      d[r] = half_bits_to_f32(hd.x);
+      nm[r] = half_bits_to_f32(hd.x >> 16) * -0.001953125f;       // -dmin * 2^-9: the sums carry 2^-5, the products 2^-14
       if constexpr (FMT == FMT_Q4K) {      // get_scale_min_k4, quantize.rs:1306-1385
-        s4 = ((hdr.y >> sc_up) & sc_mask) | (hdr.w & sc_rest);
-        m4 = ((hdr.z >> sc_up) & sc_mask) | ((hdr.w >> 4) & sc_rest);
+        s4 = ((hd.y >> sc_up) & sc_mask) | (hd.w & sc_rest);
+        m4 = ((hd.z >> sc_up) & sc_mask) | ((hd.w >> 4) & sc_rest);
       } else {                             // eight contiguous 12-bit fields, scale in the low six bits (quantize.rs:1607-1635)
-        const u32 lo = g ? ((hdr.z >> 16) | (hdr.w << 16)) : hdr.y;
-        const u32 hi = g ? (hdr.w >> 16) : (hdr.z & 0xFFFFu);
+        const u32 lo = g ? ((hd.z >> 16) | (hd.w << 16)) : hd.y;
+        const u32 hi = g ? (hd.w >> 16) : (hd.z & 0xFFFFu);
         const u32 f0 = lo & 0xFFFu, f1 = (lo >> 12) & 0xFFFu, f2 = ((lo >> 24) | (hi << 8)) & 0xFFFu, f3 = (hi >> 4) & 0xFFFu;
         s4 = (f0 & 63u) | ((f1 & 63u) << 8) | ((f2 & 63u) << 16) | ((f3 & 63u) << 24);
         m4 = (f0 >> 6) | ((f1 >> 6) << 8) | ((f2 >> 6) << 16) | ((f3 >> 6) << 24);
       }
       const h16x2 s02 = bytes_to_h2(s4), s13 = bytes_to_h2(s4 >> 8);
-      scale[0] = s02 * h2(1024.0f);
-      scale[1] = s13 * h2(64.0f);
-      addend[0] = s02 * h2(-kCentre * 0.00006103515625f);
-      addend[1] = s13 * h2(-kCentre * 0.00006103515625f);
-      mins[0] = bytes_to_h2(m4);
-      mins[1] = bytes_to_h2(m4 >> 8);
+      scale[r][0] = s02 * h2(1024.0f);
+      scale[r][1] = s13 * h2(64.0f);
+      addend[r][0] = s02 * h2(-kCentre * 0.00006103515625f);
+      addend[r][1] = s13 * h2(-kCentre * 0.00006103515625f);
+      mins[r][0] = bytes_to_h2(m4);
+      mins[r][1] = bytes_to_h2(m4 >> 8);
     }
     // weight operand of product q (0..15), out of the four dwords of its chunk
-    auto build = [&](int q, const u32x4& rw) -> h16x8 {
+    auto build = [&](int r, int q, const u32x4& rw) -> h16x8 {
       const int u = q >> 1, h = q & 1;
       const u32 t0 = (u & 1) ? rw.z : rw.x, t1 = (u & 1) ? rw.w : rw.y;
-      const _Float16 sv = scale[h][u >> 2], av = addend[h][u >> 2];
+      const _Float16 sv = scale[r][h][u >> 2], av = addend[r][h][u >> 2];
       const h16x2 sc = {sv, sv}, ad = {av, av};
       const u32 mask = h ? 0x00F000F0u : 0x000F000Fu;
       u32 f[4] = {0u, 0u, 0u, 0u};
       if constexpr (FMT == FMT_Q5K) {      // the fifth bits (kquant_gemm_f16.hip.h)
-        const u32 word = u < 4 ? (h ? qh.y : qh.x) : (h ? qh.w : qh.z);
+        const u32 word = u < 4 ? (h ? qh[r].y : qh[r].x) : (h ? qh[r].w : qh[r].z);
 #pragma unroll
         for (int dd = 0; dd < 2; ++dd) {
           const u32 nb = (word >> (4 * ((2 * u + dd) & 7))) & 15u;
@@ -320,15 +342,29 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
                        __builtin_bit_cast(u32, pk_fma_h2((t1 & mask) | f[2], sc, ad)), __builtin_bit_cast(u32, pk_fma_h2(((t1 >> 8) & mask) | f[3], sc, ad))};
       return __builtin_bit_cast(h16x8, o);
     };
-    h16x8 frag[2];
-    frag[0] = build(0, raw[0]);
-    f32x16 acc[kTiles], low[kTiles];      // of the hi and of the lo pieces
+    h16x8 frag[2][RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) frag[0][r] = build(r, 0, raw[0][r]);
+    f32x16 acc[2], low[2];      // of the hi and of the lo pieces
     auto step = [&](auto i_c) {
       constexpr int I = decltype(i_c)::value, CH = I / 4, B = I & 1;
-      if constexpr (I % 4 == 2 && CH < 3) lds_read128<16 + 16 * (CH + 1)>(raw[(CH + 1) & 1], wt + g * 64u);      // the next chunk's weight dwords
+      if constexpr (I % 4 == 2 && CH < 3)      // the next chunk's weight dwords
+#pragma unroll
+        for (int r = 0; r < RT; ++r) lds_read128<16 + 16 * (CH + 1)>(raw[(CH + 1) & 1][r], wt + 32u * r * L::STRIDE + g * 64u);
+      auto tokens_landed = [&]() {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          landed(tok[B][t][0]);
+          landed(tok[B][t][1]);
+        }
+      };
       if constexpr (I % 4 == 3) {
         // everything of this chunk is in registers: on to the next one, as soon as every wave is there
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1]), "+v"(raw[(CH + 1) & 1])::"memory");
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        tokens_landed();
+        if constexpr (CH < 3)
+#pragma unroll
+          for (int r = 0; r < RT; ++r) landed(raw[(CH + 1) & 1][r]);
         constexpr int X = CH + 1;                            // chunk X has landed: S - 2 chunks behind it, and what went out with them
         constexpr bool W_BEHIND = X == 4 && S >= 3;
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * TD + (W_BEHIND ? WD + 1 : 0)) : "memory");
@@ -342,14 +378,18 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
         slot = slot + 1u == S ? 0u : slot + 1u;
       }
       if constexpr (I < 15) read_tokens(1 - B, slot, std::integral_constant<int, (I + 1) & 3>{});
-      if constexpr (I % 4 != 3)
-        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(tok[B][0][0]), "+v"(tok[B][0][1]), "+v"(tok[B][1][0]), "+v"(tok[B][1][1]) : "n"(2 * kTiles) : "memory");
-#pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][1]), frag[B], I == 0 ? zero : acc[t], 0, 0, 0);
-        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][0]), frag[B], I == 0 ? zero : low[t], 0, 0, 0);
+      if constexpr (I % 4 != 3) {
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(2 * TT) : "memory");
+        tokens_landed();
       }
-      if constexpr (I < 15) frag[1 - B] = build(I + 1, raw[((I + 1) / 4) & 1]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = i / TT, t = i % TT;
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][1]), frag[B][r], I == 0 ? zero : acc[i], 0, 0, 0);
+        low[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h16x8, tok[B][t][0]), frag[B][r], I == 0 ? zero : low[i], 0, 0, 0);
+        if constexpr (I < 15)
+          if (t == TT - 1) frag[1 - B][r] = build(r, I + 1, raw[((I + 1) / 4) & 1][r]);
+      }
     };
 
     __builtin_amdgcn_s_setprio(1);
@@ -357,13 +397,8 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
     __builtin_amdgcn_s_setprio(0);
     // what the centring took out, then the min term, then the super-block's share of the running sums
     {
-      // C s_j 2^-9 and m_j against the sums' hi pieces (slots 0..3 of a lane), then against their lo pieces (4..7)
-      const u32 c0 = __builtin_bit_cast(u32, addend[0] * h2(-32.0f)), c1 = __builtin_bit_cast(u32, addend[1] * h2(-32.0f));
-      const u32 m0 = __builtin_bit_cast(u32, mins[0]), m1 = __builtin_bit_cast(u32, mins[1]);
-      const u32x4 ch = {c0, c1, 0u, 0u}, cl = {0u, 0u, c0, c1}, mh = {m0, m1, 0u, 0u}, ml = {0u, 0u, m0, m1};
-      const float d_lo = d * 0.00048828125f, nm_lo = nm * 0.00048828125f;
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
+      for (int t = 0; t < TT; ++t) {
         u32x4 sx, f0, f1, f2, f3;
         const u32 at_t = aux + t * kAuxBytes;
         lds_read128<0>(sx, at_t + lane * 16u);
@@ -374,27 +409,36 @@ __device__ __forceinline__ void body(const uint8_t* __restrict__ ops, const uint
         asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sx), "+v"(f0), "+v"(f1), "+v"(f2), "+v"(f3)::"memory");
         const u32 fb[16] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w, f2.x, f2.y, f2.z, f2.w, f3.x, f3.y, f3.z, f3.w};
         const h16x8 sv = __builtin_bit_cast(h16x8, sx);
-        const f32x16 mch = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, mh), zero, 0, 0, 0);
-        const f32x16 mcl = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ml), zero, 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ch), acc[t], 0, 0, 0);
-        low[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, cl), low[t], 0, 0, 0);
-        // (what the lo pieces gave comes first: next to no rounding is added at the size of the whole)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          tot[t][v] = fmaf(__uint_as_float(fb[v]), fmaf(d, acc[t][v], fmaf(nm, mch[v], fmaf(nm_lo, mcl[v], d_lo * low[t][v]))), tot[t][v]);
-        __builtin_amdgcn_sched_barrier(0);      // (both tiles' at once would spill)
+        for (int r = 0; r < RT; ++r) {
+          const int i = r * TT + t;
+          // C s_j 2^-9 and m_j against the sums' hi pieces (slots 0..3 of a lane), then against their lo pieces (4..7)
+          const u32 c0 = __builtin_bit_cast(u32, addend[r][0] * h2(-32.0f)), c1 = __builtin_bit_cast(u32, addend[r][1] * h2(-32.0f));
+          const u32 m0 = __builtin_bit_cast(u32, mins[r][0]), m1 = __builtin_bit_cast(u32, mins[r][1]);
+          const u32x4 ch = {c0, c1, 0u, 0u}, cl = {0u, 0u, c0, c1}, mh = {m0, m1, 0u, 0u}, ml = {0u, 0u, m0, m1};
+          const float d_lo = d[r] * 0.00048828125f, nm_lo = nm[r] * 0.00048828125f;
+          const f32x16 mch = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, mh), zero, 0, 0, 0);
+          const f32x16 mcl = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ml), zero, 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, ch), acc[i], 0, 0, 0);
+          low[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sv, __builtin_bit_cast(h16x8, cl), low[i], 0, 0, 0);
+          // (what the lo pieces gave comes first: next to no rounding is added at the size of the whole)
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            tot[i][v] = fmaf(__uint_as_float(fb[v]), fmaf(d[r], acc[i][v], fmaf(nm[r], mch[v], fmaf(nm_lo, mcl[v], d_lo * low[i][v]))), tot[i][v]);
+          __builtin_amdgcn_sched_barrier(0);      // (both at once would spill)
+        }
       }
     }
     if (--left == 0u) {      // runs of super-blocks are summed by themselves: fewer roundings at the size of the whole
       left = run;
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) put_by<FMT == FMT_Q5K>(stash[t], tot[t]);
+      for (int i = 0; i < 2; ++i) put_by<FMT == FMT_Q5K>(stash[i], tot[i]);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the copies asked for ahead of the end land before the workgroup's LDS is another's
 #pragma unroll
-  for (int t = 0; t < kTiles; ++t) stash[t] += tot[t];
-  store_tiles(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (kTiles * kTile), g);
+  for (int i = 0; i < 2; ++i) stash[i] += tot[i];
+  store_tiles<RT, TT>(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (TT * kTile), g);
 }
 
 // Q6_K: w = (q - 32) sc needs 13 bits, f16 holds 11.  Centred digits q - 32 = 8 (2 q2 - 3) + (nib - 8) as in
@@ -410,7 +454,9 @@ constexpr u32 kQ6Stride = 224u, kQ6Pieces = 14u;
 
 __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const uint8_t* __restrict__ w, float* __restrict__ c,
                                          u32 m, u32 n, u32 nsb, u32 ksb, u32 kparts, u32 groups, u32 pairs, u32 run, u32 lds_base) {
-  constexpr int TD = kChunkCopies, WD = 7;             // 32 rows x 14 pieces
+  using Tokens = TokenCopies<2>;
+  constexpr int kTiles = 2, TD = Tokens::kCopies, WD = 7;             // 32 rows x 14 pieces
+  constexpr u32 kWaveRows = 32u;
   const u32 lane = threadIdx.x & 63u;
   const u32 wave = static_cast<u32>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
   const Place at(blockIdx.x, groups, pairs, kparts);
@@ -419,7 +465,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
   const u32 col = lane & 31u, g = lane >> 5;
   const u32 row0 = at.group * (kWaves * kWaveRows) + wave * kWaveRows;
   const size_t row_bytes = static_cast<size_t>(nsb) * 210u;
-  const u32 lds_ring = lds_base, lds_aux = lds_base + 2u * kChunk;
+  const u32 lds_ring = lds_base, lds_aux = lds_base + 2u * Tokens::kChunk;
   const u32 lds_w = lds_aux + 2u * kTiles * kAuxBytes + wave * (kWaveRows * kQ6Stride);
 
   u32 woff[WD];
@@ -435,7 +481,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
 #pragma unroll
     for (int t = 0; t < WD; ++t) dma16(src + woff[t], lds_w + 1024u * t);
   };
-  const TokenCopies tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
+  const Tokens tokens(ops, at.tile, m, nsb, sb0, ns, lane, wave, lds_ring, lds_aux);
   const u32 lane16 = lane * 16u;
 
   f32x16 tot[kTiles], stash[kTiles];
@@ -465,7 +511,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
     };
     auto read_tokens = [&](int buf, u32 sl, auto page_c) {
       constexpr int PAGE = decltype(page_c)::value;
-      const u32 at = lds_ring + sl * kChunk + lane16;
+      const u32 at = lds_ring + sl * Tokens::kChunk + lane16;
       lds_read128<PAGE * 2048>(tok[buf][0][0], at);
       lds_read128<PAGE * 2048 + 1024>(tok[buf][0][1], at);
       lds_read128<PAGE * 2048 + 8192>(tok[buf][1][0], at);
@@ -571,7 +617,7 @@ __device__ __forceinline__ void q6k_body(const uint8_t* __restrict__ ops, const 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) stash[t] += tot[t];
-  store_tiles(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (kTiles * kTile), g);
+  store_tiles<1, 2>(stash, c + static_cast<size_t>(at.part) * m * n, m, n, row0 + col, at.tile * (kTiles * kTile), g);
 }
 
 // c = the parts of K in part order

@@ -14,6 +14,7 @@
 #include "kquant_chain.hip.h"
 #include "kquant_gemm_f16.hip.h"
 #include "kquant_gemm_tall.hip.h"
+#include "kquant_gemm_slices.hip.h"
 #include "kquant_few_i8.hip.h"
 #include "decode_glue.hip.h"
 #include "gemv_f32.hip.h"
@@ -359,6 +360,26 @@ KQ_GEMM_F16(q5k_gemm_f16_w8t2, 512, kq_body<FMT_Q5K KQ_COMMA 8 KQ_COMMA 2>)
 KQ_GEMM_F16(q6k_gemm_f16_w8, 512, q6k_body<1>)
 KQ_GEMM_F16(q6k_gemm_f16_w4, 256, q6k_body<2>)
 
+// A few sequences together (kquant_gemm_slices.hip.h): 16 RT rows of W a workgroup, the super-blocks dealt to its waves.
+#define KQ_GEMM_SLICES(name, FMT, RT)                                                                                  \
+  extern "C" __global__ void __launch_bounds__(64 * gemm_slices::kWaves)                                                 \
+  name(const float* a, const uint8_t* w, float* c, uint8_t* ws, u32 m, u32 n, u32 nsb, uint64_t geom) {                  \
+    extern __shared__ uint8_t slices_lds[];                                                                              \
+    const u32 lds_base =                                                                                                 \
+        static_cast<u32>(reinterpret_cast<size_t>((const __attribute__((address_space(3))) uint8_t*)slices_lds));       \
+    gemm_slices::body<FMT, RT>(a, w, c, ws, m, n, nsb, geom, lds_base);                                                  \
+  }
+KQ_GEMM_SLICES(q4k_gemm_slices_r1, FMT_Q4K, 1)
+KQ_GEMM_SLICES(q4k_gemm_slices_r2, FMT_Q4K, 2)
+KQ_GEMM_SLICES(q4k_gemm_slices_r3, FMT_Q4K, 3)
+KQ_GEMM_SLICES(q4k_gemm_slices_r4, FMT_Q4K, 4)
+KQ_GEMM_SLICES(q5k_gemm_slices_r1, FMT_Q5K, 1)
+KQ_GEMM_SLICES(q5k_gemm_slices_r2, FMT_Q5K, 2)
+KQ_GEMM_SLICES(q5k_gemm_slices_r3, FMT_Q5K, 3)
+KQ_GEMM_SLICES(q6k_gemm_slices_r1, FMT_Q6K, 1)
+KQ_GEMM_SLICES(q6k_gemm_slices_r2, FMT_Q6K, 2)
+KQ_GEMM_SLICES(q6k_gemm_slices_r3, FMT_Q6K, 3)
+
 // Many tokens (kquant_gemm_tall.hip.h): the activations as operands, the product, the sum over the parts of K.
 extern "C" __global__ void __launch_bounds__(256) kq_tall_operands(const float* a, uint8_t* ops, u32 m, u32 nsb) {
   gemm_tall::convert_body(a, ops, m, nsb);
@@ -375,9 +396,12 @@ extern "C" __global__ void __launch_bounds__(256) kq_tall_sum(float* c, const fl
         static_cast<u32>(reinterpret_cast<size_t>((const __attribute__((address_space(3))) uint8_t*)tall_lds));         \
     gemm_tall::BODY(ops, w, c, m, n, nsb, ksb, kparts, groups, tiles, run, lds_base);                                  \
   }
-KQ_GEMM_TALL(q4k_gemm_tall, body<FMT_Q4K>)
-KQ_GEMM_TALL(q5k_gemm_tall, body<FMT_Q5K>)
+KQ_GEMM_TALL(q4k_gemm_tall, body<FMT_Q4K KQ_COMMA 1 KQ_COMMA 2>)
+KQ_GEMM_TALL(q5k_gemm_tall, body<FMT_Q5K KQ_COMMA 1 KQ_COMMA 2>)
 KQ_GEMM_TALL(q6k_gemm_tall, q6k_body)
+// 256 rows x 32 tokens a workgroup instead of 128 x 64
+KQ_GEMM_TALL(q4k_gemm_tall_r2, body<FMT_Q4K KQ_COMMA 2 KQ_COMMA 1>)
+KQ_GEMM_TALL(q5k_gemm_tall_r2, body<FMT_Q5K KQ_COMMA 2 KQ_COMMA 1>)
 
 // Q4_K product for two to four tokens on the integer matrix cores (kquant_few_i8.hip.h): workgroup b takes the rows
 // b * rows_per_wg .. of W, k <= 4096.
