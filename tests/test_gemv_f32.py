@@ -104,3 +104,30 @@ def test_gpu_gemv_f32_last_rows_and_wide_matrices(gpu, k, n):
     a[k - 1, 5] = np.inf
     bad = run(a)
     assert np.isinf(bad[5]) and np.array_equal(np.delete(bad, 5), np.delete(got, 5))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shift_a,shift_y", [(0, 0), (1, 0), (0, 3)])
+@pytest.mark.parametrize("k,n", [(700, 1), (12576, 2), (65, 3), (700, 5), (130, 255), (3000, 257), (1003, 8191), (5000, 514), (9, 43009), (260, 66003),
+                                 (1200, 512), (300, 516)])
+def test_gpu_gemv_f32_rows_at_any_multiple_of_four_bytes(gpu, k, n, shift_a, shift_y):
+    """Columns that are no multiple of four (fewer than four, one over a tile, one under) and buffers that do not begin at 16
+    bytes: nothing before or behind y is written, a NaN around A and x is not read into a result, every replay of the call
+    gives the same bits."""
+    ctx, stream = gpu
+    rng = np.random.default_rng(k * 41 + n)
+    a, x = rng.standard_normal((k, n)).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    want = a.astype(np.float64).T @ x.astype(np.float64)
+    pad = np.full(8, np.nan, np.float32)
+    da = t.GpuBuffer.from_host(ctx, np.concatenate([pad[:shift_a], a.reshape(-1), pad]))
+    dx = t.GpuBuffer.from_host(ctx, np.concatenate([x, pad]))
+    dy = t.GpuBuffer.from_host(ctx, np.full(shift_y + n + 8, 7.0, np.float32))
+    got = []
+    for _ in range(3):
+        assert t._ffi.lib().trn_gemv_f32(stream.raw(), dy.as_ptr() + 4 * shift_y, da.as_ptr() + 4 * shift_a, dx.as_ptr(), k, n) == 0
+        stream.synchronize()
+        got.append(dy.copy_to_host())
+    assert all(np.array_equal(g.view(np.uint32), got[0].view(np.uint32)) for g in got[1:])
+    assert np.all(got[0][:shift_y] == 7.0) and np.all(got[0][shift_y + n:] == 7.0)
+    # fewer than 67 roundings of 2^-24 in a row (eight rows, k / parts / 64 of those, the waves, the parts), each of a sum of size sqrt(k)
+    assert np.linalg.norm(got[0][shift_y:shift_y + n] - want) <= 4e-6 * np.sqrt(k) * np.sqrt(n)

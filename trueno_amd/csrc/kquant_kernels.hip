@@ -216,13 +216,17 @@ fused_residual_rmsnorm(const float* residual, const float* input, float* output,
 }
 
 // f32 GEMV under the reference's two kernel names and parameter list (gemv.rs:53-57, 222-226): one engine
-// (gemv_f32.hip.h), the two names differ only in the reference's summation order.  gemv_f32_fast takes the
-// launcher's extra arguments; the named kernels are the any-shape form.
-extern "C" __global__ void __launch_bounds__(512)
-gemv_f32_fast(float* y, const float* a, const float* x, float* partial, u32* counters, u32 k_dim, u32 n_dim, u32 rows_per_part,
-              u32 parts) {
-  gemv_f32::fast_body(y, a, x, partial, counters, k_dim, n_dim, rows_per_part, parts);
-}
+// (gemv_f32.hip.h), the two names differ only in the reference's summation order.  gemv_f32_fast, _ragged and _narrow
+// take the launcher's extra arguments; the named kernels are the plain form.
+#define GEMV_F32(name, form)                                                                                              \
+  extern "C" __global__ void __launch_bounds__(512)                                                                       \
+  name(float* y, const float* a, const float* x, float* partial, u32* counters, u32 k_dim, u32 n_dim, u32 rows_per_part,  \
+       u32 parts) {                                                                                                       \
+    gemv_f32::body<gemv_f32::form>(y, a, x, partial, counters, k_dim, n_dim, rows_per_part, parts);                       \
+  }
+GEMV_F32(gemv_f32_fast, kAligned)
+GEMV_F32(gemv_f32_ragged, kRagged)
+GEMV_F32(gemv_f32_narrow, kNarrow)
 extern "C" __global__ void __launch_bounds__(256) gemv_warp_reduce(float* y, const float* a, const float* x, u32 k_dim, u32 n_dim) {
   gemv_f32::generic_body(y, a, x, k_dim, n_dim);
 }

@@ -83,7 +83,7 @@ struct DeviceKernels {
   hipFunction_t dequant_fast[NFMT] = {}, dequant_generic[NFMT] = {};
   hipFunction_t copy_u128 = nullptr, read_u128 = nullptr;
   hipFunction_t residual_add = nullptr, swiglu = nullptr, rmsnorm = nullptr, residual_rmsnorm = nullptr;
-  hipFunction_t gemv_f32_fast = nullptr, gemv_f32_generic = nullptr, q5k_from_ggml = nullptr, attention = nullptr;
+  hipFunction_t gemv_f32_fast = nullptr, gemv_f32_ragged = nullptr, gemv_f32_narrow = nullptr, gemv_f32_generic = nullptr, q5k_from_ggml = nullptr, attention = nullptr;
   hipFunction_t attention_tiled[4] = {};  // head dimension 64, 128, 256; 128 with workgroups of four waves
   hipFunction_t gemm_f16[NFMT][2] = {};   // [format][4 or 8 strips per workgroup]
   hipFunction_t gemm_f16_w12 = nullptr;   // Q4_K: 12 strips per workgroup
@@ -180,6 +180,8 @@ hipError_t device_kernels(DeviceKernels** out) {
     if ((e = get_fn(m, &t.copy_u128, "kq_copy_u128")) != hipSuccess ||
         (e = get_fn(m, &t.read_u128, "kq_read_u128")) != hipSuccess ||
         (e = get_fn(m, &t.gemv_f32_fast, "gemv_f32_fast")) != hipSuccess ||
+        (e = get_fn(m, &t.gemv_f32_ragged, "gemv_f32_ragged")) != hipSuccess ||
+        (e = get_fn(m, &t.gemv_f32_narrow, "gemv_f32_narrow")) != hipSuccess ||
         (e = get_fn(m, &t.q5k_from_ggml, "q5k_from_ggml")) != hipSuccess ||
         (e = get_fn(m, &t.attention, "incremental_attention")) != hipSuccess ||
         (e = get_fn(m, &t.attention_tiled[0], "kq_attention_tiled_64")) != hipSuccess ||
@@ -403,6 +405,20 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
 // f32 GEMV y = A^T-style product with A K x N row-major (gemv_f32.hip.h).  Partial results of the parts of K and
 // the arrival counters live in a per-(device, stream) buffer like the GEMM's.
 ScratchMap g_gemv_f32_ws;
+constexpr size_t kGemvF32Bytes = 1024u * 1024u;      // counters and the parts of matrices of up to some 70000 columns: made at once, so it does not grow
+
+// Whether acquire_scratch can serve `need` without an allocation that a capture in progress forbids.
+bool scratch_at_hand(ScratchMap& map, hipStream_t stream, size_t need) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    const auto it = map.find(std::make_pair(dev, stream));
+    if (it != map.end() && it->second.cap >= need) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
 
 hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t x, uint32_t k, uint32_t n) {
   if (n == 0) return hipSuccess;
@@ -410,11 +426,13 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
   DeviceKernels* d = nullptr;
   hipError_t e = device_kernels(&d);
   if (e != hipSuccess) return e;
-  if (k == 0 || n % 4u != 0 || !aligned(a, 16) || !aligned(y, 16)) {
+  // Rows that do not all begin at 16 bytes: the same kernel with loads at multiples of four bytes (see there for both sides).
+  const bool ragged = n % 4u != 0 || !aligned(a, 16) || !aligned(y, 16);
+  if (k == 0 || (ragged && n > 0x7FFFFFFFu)) {      // (a grid of 512 threads for 256 columns ends at 2^31 columns)
     void* args[] = {&y, &a, &x, &k, &n};
     return hipModuleLaunchKernel(d->gemv_f32_generic, (n + 255u) / 256u, 1, 1, 256, 1, 1, 0, stream, args, nullptr);
   }
-  const uint32_t tiles = (n + 255u) / 256u;
+  const uint32_t tiles = n / 256u + (n % 256u != 0);
   // parts of K, at least 64 rows (8 per wave) each: as many workgroups of 8 waves as there are CUs or somewhat fewer
   // (gemv_f32.hip.h).  Two per CU where one would leave a third of them idle, if K is long enough to be worth three parts
   // (33028 columns: 4096 rows 104.9 in one part, 98.3 us in three; 1003 rows 28.6 and 30.3; 256 rows 9.5 and 12.2), and from 256
@@ -427,13 +445,24 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
   uint32_t rows_per_part = (k + parts - 1u) / parts;
   rows_per_part = (rows_per_part + 7u) / 8u * 8u;
   parts = (k + rows_per_part - 1u) / rows_per_part;
-  const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (parts > 1u ? size_t(parts) * n * 4u : 0u);
-  if (size_t(tiles) * 4u > cnt_cap) return hipErrorInvalidValue;
+  const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (parts > 1u ? size_t(parts) * (size_t(n) + 3u) * 4u : 0u);
   uint64_t cnt = 0;
-  if ((e = acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt)) != hipSuccess) return e;   // the kernel leaves the counters at zero
+  if (ragged) {
+    // A single part writes no partial results and counts nothing.  It also takes the call whose scratch cannot be had.
+    const bool room = size_t(tiles) * 4u <= cnt_cap && scratch_at_hand(g_gemv_f32_ws, stream, need);
+    if (parts > 1u && (!room || acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes) != hipSuccess)) {
+      (void)hipGetLastError();
+      parts = 1u;
+      rows_per_part = k;
+    }
+  } else {
+    if (size_t(tiles) * 4u > cnt_cap) return hipErrorInvalidValue;
+    if ((e = acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes)) != hipSuccess) return e;   // the kernel leaves the counters at zero
+  }
   uint64_t part = cnt + cnt_cap;
   void* args[] = {&y, &a, &x, &part, &cnt, &k, &n, &rows_per_part, &parts};
-  return hipModuleLaunchKernel(d->gemv_f32_fast, tiles * parts, 1, 1, 512, 1, 1, 0, stream, args, nullptr);
+  const hipFunction_t f = !ragged ? d->gemv_f32_fast : n < 4u ? d->gemv_f32_narrow : d->gemv_f32_ragged;
+  return hipModuleLaunchKernel(f, tiles * parts, 1, 1, 512, 1, 1, 0, stream, args, nullptr);
 }
 
 // Single-query attention over the KV cache (decode_attention.hip.h).  Per (device, stream): arrival counters per
