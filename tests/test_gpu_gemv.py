@@ -156,3 +156,24 @@ def test_q6k_streamed_through_lds_gives_the_bits_of_the_register_form(gpu, n, k)
             tune("gemv_stream_q6k", 0)
             tune("gemv_stream_min_rows", 0)
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, k, w_off)
+
+
+@pytest.mark.parametrize("fmt", ("q4k", "q5k", "q6k"))
+@pytest.mark.parametrize("n,k", [(1, 1024), (2, 2048), (3, 256), (4, 768), (5, 1024), (1023, 2048), (1538, 1280), (3001, 1792), (6145, 1024), (33003, 512),
+                                 (40001, 1536)])
+def test_gemv_rows_of_up_to_eight_super_blocks(gpu, coracle, fmt, n, k):
+    """Two or four rows to a wave, at row counts that end a workgroup or the matrix within such a batch, against fp64 and, bit for
+    bit, against the same rows in a list of two products (a row to a wave)."""
+    _check(gpu, coracle, fmt, n, k, seed=77, ref_rows=0)
+    ctx, stream = gpu
+    buf, x = kq.gen_matrix(fmt, 77, n, k), kq.gen_x(78, k)
+    w, dx = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, x)
+    ys = [t.GpuBuffer.from_host(ctx, np.full(n, np.nan, np.float32)) for _ in range(2)]
+    batch = t.GemvBatch()
+    for y in ys:
+        batch.add(fmt, k, n, y, w, dx, 0)
+    batch.launch(stream)
+    stream.synchronize()
+    one = gpu_gemv(gpu, fmt, buf, x, k, n)
+    for y in ys:
+        assert np.array_equal(y.copy_to_host().view(np.uint32), one.view(np.uint32))

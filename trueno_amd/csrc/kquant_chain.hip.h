@@ -374,7 +374,7 @@ __device__ __forceinline__ bool chain_step_stream(const ChainEntry& e, f32x4* ld
 // block_threads: blockDim.x, handed in by the kernel (an implicit kernel argument, i.e. a load: the kernel decides when).
 // chain_step_rows: the workgroup's rows are row0 .. row0 + rows_per_block - 1 (rows_per_block a multiple of U; rows
 // beyond the matrix are skipped).  chain_step: block block_id of num_blocks equal blocks of rows.
-template <int FMT, int U, bool COHERENT = false>
+template <int FMT, int U, bool COHERENT = false, bool SHORT = false>
 __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_counter, u32 spin_limit, u32* status,
                                                 f32x4* lds4, u32* s_flag, u32 row0, u32 rows_per_block, u32 block_threads) {
   using Q = Quarter<FMT>;
@@ -395,21 +395,29 @@ __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_c
   // with three waves to a SIMD the others do not fill that time.  Two sets of two rows do not fit the registers, and a
   // spilled register that is read back inside the loop waits for every load issued before it, the next rows' included.)
   constexpr int UR = 1;
-  const u32 batches = has_rows ? rows_per_block / UR : 0u;
+  // SHORT: rows of up to eight super-blocks go through the wave two at a time, of up to four four at a time: a lane group of 32 or 16
+  // lanes has a row.  (With a row a wave most lanes have nothing to do and every row costs the wave a round trip to memory: Q4_K
+  // 31598 x 1024 13.4 us and 6.0 so, Q6_K 27495 x 2048 18.1 and 11.3, Q6_K 7199 x 1024 6.8 and 4.1.)  The row sums of wave_sum_lane63
+  // stop at the group, so the bits are those of a row by itself.  An instance of its own: longer rows lose 0.1 to 0.3 us to
+  // the choice at run time (Q4_K 4096 x 4096 4.4 -> 4.6 us).
+  const u32 pack = !SHORT ? 1u : nsb <= 4u && n_dim >= 4u ? 4u : nsb <= 8u && n_dim >= 2u ? 2u : 1u;
+  const u32 batches = has_rows ? (rows_per_block + pack - 1u) / pack : 0u;
   const u32 sw = wave % sw_count, grp = wave / sw_count;
   const bool wave_active = grp < groups && grp < batches;
-  const u32 sbl = lane >> 2, c = lane & 3u;
+  const u32 group_mask = 64u / pack - 1u;
+  const u32 sbl = (lane & group_mask) >> 2, c = lane & 3u, sub = lane / (64u / pack);
   const size_t row_bytes = static_cast<size_t>(nsb) * Q::SB;
   typename Q::Regs regs[UR], regs_b[UR];
+  // the rows of batch b begin here; those at the end of the matrix move back and give some rows twice, with the same bits
+  auto first_row = [&](u32 b) -> u32 {
+    const u32 row = row0 + b * pack;
+    return row < n_dim - pack ? row : n_dim - pack;
+  };
   auto issue = [&](typename Q::Regs (&into)[UR], u32 slab, u32 b) {
     const u32 sb = slab * 16u + sbl;
     const u32 sbc = sb < nsb ? sb : nsb - 1;
-#pragma unroll
-    for (int u = 0; u < UR; ++u) {
-      u32 row = row0 + b * UR + u;
-      row = row < n_dim ? row : n_dim - 1;
-      Q::load(into[u], e.w + row * row_bytes, sbc * Q::SB, c);     // (a row is tens of KB at most: its vector must fit in LDS)
-    }
+    const u32 row = first_row(b);
+    Q::load(into[0], e.w + row * row_bytes, sbc * Q::SB + sub * static_cast<u32>(row_bytes), c);     // (a row is tens of KB at most: its vector must fit in LDS)
   };
   // Activations.  Alone on the stream (no barrier to wait for) they are requested BEFORE the weights: loads
   // return in order, so the vector (an L2 hit) is staged and summed while the weights are still on their way.
@@ -532,13 +540,13 @@ __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_c
         const u32 nb = next_of(b);
         issue(nxt, slab, nb < batches ? nb : batches - 1u);
         __builtin_amdgcn_sched_barrier(0);      // (the loads stay in front of the arithmetic whatever the register pressure)
-#pragma unroll
-        for (int u = 0; u < UR; ++u) {
-          const float p = wave_sum_lane63(Q::dot(cur[u], c, xr, sx));
-          if (lane == 63u) {
-            const u32 idx = sw * rows_per_block + b * UR + u;
-            part[idx] = (slab == sw) ? p : part[idx] + p;
-          }
+        const float p = wave_sum_groups(Q::dot(cur[0], c, xr, sx), pack);
+        // (Rows before the block, which have wrapped, and behind it are others'.  A row by itself keeps its place also behind the matrix:
+        // with several slabs the place is added to.)
+        const u32 at = pack == 1u ? b : first_row(b) - row0 + sub;
+        if ((lane & group_mask) == group_mask && at < rows_per_block) {
+          const u32 idx = sw * rows_per_block + at;
+          part[idx] = (slab == sw) ? p : part[idx] + p;
         }
         return nb;
       };
@@ -573,12 +581,12 @@ __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_c
   return true;
 }
 
-template <int FMT, int U, bool COHERENT = false>
+template <int FMT, int U, bool COHERENT = false, bool SHORT = false>
 __device__ __forceinline__ bool chain_step(const ChainEntry& e, u32* wait_counter, u32 spin_limit, u32* status,
                                            f32x4* lds4, u32* s_flag, u32 block_id, u32 num_blocks, u32 block_threads) {
   u32 rows_per_block = (e.n + num_blocks - 1) / num_blocks;
   rows_per_block = ((rows_per_block + U - 1) / U) * U;
-  return chain_step_rows<FMT, U, COHERENT>(e, wait_counter, spin_limit, status, lds4, s_flag, block_id * rows_per_block, rows_per_block,
+  return chain_step_rows<FMT, U, COHERENT, SHORT>(e, wait_counter, spin_limit, status, lds4, s_flag, block_id * rows_per_block, rows_per_block,
                                            block_threads);
 }
 

@@ -100,6 +100,20 @@ __device__ __forceinline__ float wave_sum_lane63(float v) {
   return v;
 }
 
+// The sums of 1, 2 or 4 equal groups of lanes, each in its group's last lane, with the bits that wave_sum_lane63 gives for the
+// group's values among zeros.  groups is the same in every lane.
+__device__ __forceinline__ float wave_sum_groups(float v, u32 groups) {
+  v += dpp_f32<0xB1>(v);
+  v += dpp_f32<0x4E>(v);
+  v += dpp_f32<0x141>(v);
+  v += dpp_f32<0x140>(v);
+  const float rows = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));
+  v += groups < 4u ? rows : 0.0f;
+  const float halves = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
+  v += groups < 2u ? halves : 0.0f;
+  return v;
+}
+
 // ---- byte-wise decoders: one value of one super-block -----------------------------------
 // Used by the generic (any alignment, any K) kernels and by the GEMM-family decode policy.
 // __fmul_rn/__fsub_rn keep every PTX instruction of the reference a separate rounding.

@@ -75,6 +75,13 @@ __device__ __forceinline__ void gemv_generic_body(float* __restrict__ y, const u
     chain_step<FMT, KQ_U>(e, nullptr, 0u, nullptr, lds4, &s_flag, blockIdx.x, gridDim.x, blockDim.x);                                          \
   }                                                                                                      \
   extern "C" __global__ void __launch_bounds__(768)                                                      \
+      fmtname##_gemv_short(float* y, const uint8_t* w, const float* x, u32 k_dim, u32 n_dim) {           \
+    extern __shared__ f32x4 lds4[];                                                                      \
+    __shared__ u32 s_flag;                                                                               \
+    const ChainEntry e = {FMT, k_dim, n_dim, 0u, w, x, y};                                               \
+    chain_step<FMT, KQ_U, false, true>(e, nullptr, 0u, nullptr, lds4, &s_flag, blockIdx.x, gridDim.x, blockDim.x);                             \
+  }                                                                                                      \
+  extern "C" __global__ void __launch_bounds__(768)                                                      \
       fmtname##_gemv_flags(float* y, const uint8_t* w, const float* x, u32 k_dim, u32 n_dim, u32 flags) {\
     extern __shared__ f32x4 lds4[];                                                                      \
     __shared__ u32 s_flag;                                                                               \

@@ -75,7 +75,7 @@ struct DeviceKernels {
   bool loaded = false;
   hipModule_t module = nullptr;
   int cu_count = 0;
-  hipFunction_t gemv_fast[NFMT] = {}, gemv_flags[NFMT] = {}, gemv_generic[NFMT] = {};
+  hipFunction_t gemv_fast[NFMT] = {}, gemv_short[NFMT] = {}, gemv_flags[NFMT] = {}, gemv_generic[NFMT] = {};
   hipFunction_t fill_u32 = nullptr, gemv_group = nullptr, gemv_many = nullptr, phases = nullptr;
   int cooperative = 0;
   uint32_t resident_small = 3;   // resident 256-thread GEMV workgroups per CU (occupancy of the one-slab geometry)
@@ -163,6 +163,7 @@ hipError_t device_kernels(DeviceKernels** out) {
     for (int f = 0; f < NFMT; ++f) {
       const std::string p = kFmtName[f];
       if ((e = get_fn(m, &t.gemv_fast[f], p + "_gemv_warp_reduce")) != hipSuccess ||
+          (e = get_fn(m, &t.gemv_short[f], p + "_gemv_short")) != hipSuccess ||
           (e = get_fn(m, &t.gemv_flags[f], p + "_gemv_flags")) != hipSuccess ||
           (e = get_fn(m, &t.gemv_generic[f], p + "_gemv_generic")) != hipSuccess ||
           (e = get_fn(m, &t.gemm_fast[f], p + "_gemm_ggml")) != hipSuccess ||
@@ -1090,13 +1091,16 @@ hipError_t launch_gemm_like(Fmt f, hipStream_t stream, uint64_t a, uint64_t w, u
   void** args = is_gemv ? gemv_args : gemm_args;
   // A large matrix alone is 2-5 us faster as a launch of the list kernel with one entry (workgroups of 8 waves that hand
   // their rows out among themselves) than through the single kernel: Q6_K 32000 x 4096, 108 MB, 22.7 against 27.2 us.
-  if (is_gemv && flags == 0 && !g_tune_group_off && double(n) * (k / 256u) * kSbBytes[f] >= kBigAloneBytes) {
+  // Rows of up to eight super-blocks go through the kernel that has two or four of them in a wave, at any size and with the same
+  // bits: the list kernel and the streamed one have a row a wave (Q4_K 65536 x 1024 24.9 and 8.2 us, Q5_K 40000 x 2048 23.7 and 13.1).
+  const bool short_rows = is_gemv && flags == 0 && k <= 2048u;
+  if (is_gemv && flags == 0 && !short_rows && !g_tune_group_off && double(n) * (k / 256u) * kSbBytes[f] >= kBigAloneBytes) {
     trn_gemv_desc one{};
     one.fmt = uint32_t(f) + 4u; one.k = k; one.n = n; one.y = c; one.w = w; one.x = a;
     if (list_groupable(d, one)) return launch_gemv_group(d, stream, &one, 1);
   }
   GemvGeometry g;
-  if (is_gemv && gemv_fast_ok(f, c, w, a) && stream_ok(uint32_t(f) + 4u, k, n)) {
+  if (is_gemv && !short_rows && gemv_fast_ok(f, c, w, a) && stream_ok(uint32_t(f) + 4u, k, n)) {
     g = stream_geometry(*d, f, k, n);
     if (g.fits) {
       flags |= kChainStreamFlag;
@@ -1106,7 +1110,7 @@ hipError_t launch_gemm_like(Fmt f, hipStream_t stream, uint64_t a, uint64_t w, u
   if (k != 0 && gemv_fast_ok(f, c, w, a) && (is_gemv || (aligned(uint64_t(k) * 4u, 16) && aligned(uint64_t(n) * 4u, 4))))
     g = gemv_geometry(*d, k, n, is_gemv ? kGemvMaxWaves : 8u);   // the GEMM kernels are built for 8 waves
   if (g.fits) {
-    hipFunction_t fn = is_gemv ? (flags ? d->gemv_flags[f] : d->gemv_fast[f]) : d->gemm_fast[f];
+    hipFunction_t fn = is_gemv ? (flags ? d->gemv_flags[f] : short_rows ? d->gemv_short[f] : d->gemv_fast[f]) : d->gemm_fast[f];
     return hipModuleLaunchKernel(fn, g.grid, is_gemv ? 1u : grid_y, 1, g.block, 1, 1, g.lds, stream, args, nullptr);
   }
   hipFunction_t fn = is_gemv ? d->gemv_generic[f] : d->gemm_generic[f];
