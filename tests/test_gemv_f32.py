@@ -131,3 +131,26 @@ def test_gpu_gemv_f32_rows_at_any_multiple_of_four_bytes(gpu, k, n, shift_a, shi
     assert np.all(got[0][:shift_y] == 7.0) and np.all(got[0][shift_y + n:] == 7.0)
     # fewer than 67 roundings of 2^-24 in a row (eight rows, k / parts / 64 of those, the waves, the parts), each of a sum of size sqrt(k)
     assert np.linalg.norm(got[0][shift_y:shift_y + n] - want) <= 4e-6 * np.sqrt(k) * np.sqrt(n)
+
+
+@pytest.mark.gpu
+def test_gpu_gemv_f32_rows_of_odd_length_captured_on_a_new_stream(gpu):
+    """The capture allocates nothing and its graph holds no scratch memory: replayed beside eager calls, some with more columns."""
+    from tests.test_gpu_gemm import _Captured
+    ctx, stream = gpu
+    k, n, wide = 2000, 515, 5003
+    rng = np.random.default_rng(3)
+    a, x = rng.standard_normal((k, wide)).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    da, dx = t.GpuBuffer.from_host(ctx, a.reshape(-1)), t.GpuBuffer.from_host(ctx, x)
+    dy, dz = (t.GpuBuffer.from_host(ctx, np.full(m, np.nan, np.float32)) for m in (n, wide))
+    want = a.reshape(-1)[:k * n].reshape(k, n).astype(np.float64).T @ x.astype(np.float64)
+    new = t.CudaStream(ctx)
+    graph = _Captured(new, lambda: t.CoalescedGemvKernel(k, n).launch(new, dy, da, dx))
+    for _ in range(3):
+        dy.copy_from_host(np.full(n, np.nan, np.float32))
+        graph.replay(stream)
+        t.CoalescedGemvKernel(k, wide).launch(new, dz, da, dx)
+        stream.synchronize()
+        new.synchronize()
+        assert kq.rel_l2(dy.copy_to_host(), want) <= 1e-6
+    graph.close()

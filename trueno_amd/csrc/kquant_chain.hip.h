@@ -404,20 +404,21 @@ __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_c
   const u32 batches = has_rows ? (rows_per_block + pack - 1u) / pack : 0u;
   const u32 sw = wave % sw_count, grp = wave / sw_count;
   const bool wave_active = grp < groups && grp < batches;
-  const u32 group_mask = 64u / pack - 1u;
-  const u32 sbl = (lane & group_mask) >> 2, c = lane & 3u, sub = lane / (64u / pack);
+  const u32 group_mask = SHORT ? 64u / pack - 1u : 63u;
+  const u32 sbl = SHORT ? (lane & group_mask) >> 2 : lane >> 2, c = lane & 3u, sub = SHORT ? lane / (64u / pack) : 0u;
   const size_t row_bytes = static_cast<size_t>(nsb) * Q::SB;
   typename Q::Regs regs[UR], regs_b[UR];
   // the rows of batch b begin here; those at the end of the matrix move back and give some rows twice, with the same bits
   auto first_row = [&](u32 b) -> u32 {
     const u32 row = row0 + b * pack;
+    if constexpr (!SHORT) return row < n_dim ? row : n_dim - 1;
     return row < n_dim - pack ? row : n_dim - pack;
   };
   auto issue = [&](typename Q::Regs (&into)[UR], u32 slab, u32 b) {
     const u32 sb = slab * 16u + sbl;
     const u32 sbc = sb < nsb ? sb : nsb - 1;
     const u32 row = first_row(b);
-    Q::load(into[0], e.w + row * row_bytes, sbc * Q::SB + sub * static_cast<u32>(row_bytes), c);     // (a row is tens of KB at most: its vector must fit in LDS)
+    Q::load(into[0], e.w + row * row_bytes, SHORT ? sbc * Q::SB + sub * static_cast<u32>(row_bytes) : sbc * Q::SB, c);     // (a row is tens of KB at most: its vector must fit in LDS)
   };
   // Activations.  Alone on the stream (no barrier to wait for) they are requested BEFORE the weights: loads
   // return in order, so the vector (an L2 hit) is staged and summed while the weights are still on their way.
@@ -540,11 +541,12 @@ __device__ __forceinline__ bool chain_step_rows(const ChainEntry& e, u32* wait_c
         const u32 nb = next_of(b);
         issue(nxt, slab, nb < batches ? nb : batches - 1u);
         __builtin_amdgcn_sched_barrier(0);      // (the loads stay in front of the arithmetic whatever the register pressure)
-        const float p = wave_sum_groups(Q::dot(cur[0], c, xr, sx), pack);
+        const float dot = Q::dot(cur[0], c, xr, sx);
+        const float p = SHORT ? wave_sum_groups(dot, pack) : wave_sum_lane63(dot);
         // (Rows before the block, which have wrapped, and behind it are others'.  A row by itself keeps its place also behind the matrix:
         // with several slabs the place is added to.)
         const u32 at = pack == 1u ? b : first_row(b) - row0 + sub;
-        if ((lane & group_mask) == group_mask && at < rows_per_block) {
+        if (SHORT ? (lane & group_mask) == group_mask && at < rows_per_block : lane == 63u) {
           const u32 idx = sw * rows_per_block + at;
           part[idx] = (slab == sw) ? p : part[idx] + p;
         }

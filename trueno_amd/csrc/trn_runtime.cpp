@@ -408,19 +408,6 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
 ScratchMap g_gemv_f32_ws;
 constexpr size_t kGemvF32Bytes = 1024u * 1024u;      // counters and the parts of matrices of up to some 70000 columns: made at once, so it does not grow
 
-// Whether acquire_scratch can serve `need` without an allocation that a capture in progress forbids.
-bool scratch_at_hand(ScratchMap& map, hipStream_t stream, size_t need) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return false;
-  {
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    const auto it = map.find(std::make_pair(dev, stream));
-    if (it != map.end() && it->second.cap >= need) return true;
-  }
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
-}
-
 hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t x, uint32_t k, uint32_t n) {
   if (n == 0) return hipSuccess;
   if (!y || (k != 0 && (!a || !x)) || !aligned(y, 4) || !aligned(a, 4) || !aligned(x, 4)) return hipErrorInvalidValue;
@@ -449,8 +436,10 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
   const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (parts > 1u ? size_t(parts) * (size_t(n) + 3u) * 4u : 0u);
   uint64_t cnt = 0;
   if (ragged) {
-    // A single part writes no partial results and counts nothing.  It also takes the call whose scratch cannot be had.
-    const bool room = size_t(tiles) * 4u <= cnt_cap && scratch_at_hand(g_gemv_f32_ws, stream, need);
+    // A single part writes no partial results and counts nothing: it takes the call whose scratch cannot be had, and the one that is
+    // captured, which a graph may replay on any stream and after the buffer has been replaced by a larger one.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool room = size_t(tiles) * 4u <= cnt_cap && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
     if (parts > 1u && (!room || acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes) != hipSuccess)) {
       (void)hipGetLastError();
       parts = 1u;
