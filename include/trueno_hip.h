@@ -15,8 +15,8 @@
  * device is hipErrorNoDevice = 100, which maps to GpuError::CudaNotAvailable).  Device pointers
  * are plain 64-bit integers (CUdeviceptr, sys.rs:60).  The library never owns host memory and never
  * keeps a host pointer after a synchronous call returns.  Device memory for the caller's data comes
- * from trn_mem_alloc only.  Beside it the library keeps scratch of its own, per (device, stream),
- * allocated on first use and freed with the stream: the partial sums and arrival counters of the
+ * from trn_mem_alloc only.  Beside it the library keeps scratch of its own, per (device, stream) - of
+ * hipStreamPerThread per thread -, allocated on first use and freed with the stream: the partial sums and arrival counters of the
  * products that are cut along K (trn_q*k_gemm, trn_gemv_f32, trn_incremental_attention), the activations of
  * a trn_q*k_gemm of many tokens as matrix-core operands (at most 256 MiB, or none where that cannot be had: the product then
  * takes the kernel that needs none; what one stream adds to one capture has a

@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <tuple>
@@ -360,12 +361,35 @@ hipError_t launch_rmsnorm(hipStream_t stream, uint64_t residual, uint64_t in, ui
 // threads on two streams never see a half-grown buffer; a buffer only ever belongs to one stream, and work on one
 // stream is ordered, so the kernels themselves need no lock.  New counters are zeroed by a small fill kernel, not by
 // hipMemsetAsync: the call may be recorded into a HIP graph by a capturing caller.
+// hipStreamPerThread is one handle for as many streams as there are threads, so its buffers belong to a thread as well; those of
+// threads that have ended are freed when a buffer is made next.
 struct ScratchWorkspace {
   void* buf = nullptr;
   size_t cap = 0;
+  std::weak_ptr<char> thread;      // hipStreamPerThread's only
 };
-using ScratchMap = std::map<std::pair<int, hipStream_t>, ScratchWorkspace>;
+using ScratchKey = std::tuple<int, hipStream_t, const void*>;      // device, stream, thread (see there)
+using ScratchMap = std::map<ScratchKey, ScratchWorkspace>;
 std::mutex g_ws_mutex;
+
+// The calling thread behind that handle, nothing for a stream of its own.  (An entry of a map keeps the object's address from being
+// another thread's for as long as it is there.)
+std::shared_ptr<char> stream_thread(hipStream_t stream) {
+  if (stream != hipStreamPerThread) return nullptr;
+  thread_local const std::shared_ptr<char> self = std::make_shared<char>();
+  return self;
+}
+ScratchKey scratch_key(int dev, hipStream_t stream, const std::shared_ptr<char>& thread) { return ScratchKey(dev, stream, thread.get()); }
+void free_scratch_of_ended_threads(ScratchMap& map) {      // under g_ws_mutex; hipFree waits for the work that uses a buffer
+  for (auto it = map.begin(); it != map.end();) {
+    if (std::get<2>(it->first) != nullptr && it->second.thread.expired()) {
+      if (it->second.buf) (void)hipFree(it->second.buf);
+      it = map.erase(it);
+    } else {
+      ++it;
+    }
+  }
+}
 
 // want > need: what a buffer that has to be made (or made larger) should hold, so that later calls, captured ones among them,
 // find room; the call itself does with `need`.
@@ -373,9 +397,12 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
+  const std::shared_ptr<char> thread = stream_thread(stream);
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  ScratchWorkspace& ws = map[std::make_pair(dev, stream)];
+  ScratchWorkspace& ws = map[scratch_key(dev, stream, thread)];
+  ws.thread = thread;
   if (ws.cap < need) {
+    free_scratch_of_ended_threads(map);
     if (ws.buf) {
       if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
       (void)hipFree(ws.buf);
@@ -942,7 +969,7 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
     bool there = false;
     {
       std::lock_guard<std::mutex> lock(g_ws_mutex);
-      auto it = g_gemm_ws.find(std::make_pair(dev, stream));
+      auto it = g_gemm_ws.find(scratch_key(dev, stream, nullptr));
       there = it != g_gemm_ws.end() && it->second.buf != nullptr;
     }
     uint64_t base = 0;
@@ -1739,9 +1766,10 @@ static void release_stream_workspaces(hipStream_t stream) {
     }
   }
   std::lock_guard<std::mutex> lock(g_ws_mutex);
+  const std::shared_ptr<char> thread = stream_thread(stream);
   auto drop_simple = [&](auto& map) {
     for (auto it = map.begin(); it != map.end();) {
-      if (it->first.second == stream) {
+      if (std::get<1>(it->first) == stream && std::get<2>(it->first) == thread.get()) {
         if (it->second.buf) (void)hipFree(it->second.buf);
         it = map.erase(it);
       } else {
