@@ -810,3 +810,40 @@ def test_gemm_many_tokens_either_shape_of_a_workgroup(gpu, fmt, m, n, k):
     finally:
         for key in ("gemm_tall", "gemm_k_parts", "gemm_tall_strips"):
             _tune(key, 0)
+
+
+@pytest.mark.parametrize("fmt,m,n,k,warm", [("q4k", 121, 4192, 4096, False), ("q4k", 121, 4192, 4096, True), ("q5k", 40, 2573, 5888, False),
+                                            ("q5k", 40, 2573, 5888, True), ("q4k", 16, 512, 4096, False)])
+def test_gemm_captured_products_in_parts_keep_to_themselves(gpu, fmt, m, n, k, warm):
+    """Products with K in parts that the kernels for up to sixteen and 48 tokens take by the rule, captured on a stream that has seen no product, or
+    (33 tokens and more) one that has: their counters and partial sums are the capture's own, so three replays at once with the same and other
+    products on the stream they were captured on, and after that stream is gone and its memory with it, give the eager call's bits."""
+    ctx, other = gpu
+    kernel = {"q4k": t.QuantizeKernel.ggml, "q5k": t.Q5KKernel}[fmt](m, n, k)
+    stream, buf, a = t.CudaStream(ctx), kq.gen_matrix(fmt, 750, n, k), kq.gen_x(751, m, k)
+    want = gpu_gemm(gpu, fmt, buf, a, m, n, k).view(np.uint32)
+    dw, da = t.GpuBuffer.from_host(ctx, buf), t.GpuBuffer.from_host(ctx, a)
+    dc, de = (t.GpuBuffer.from_host(ctx, np.full(m * n, np.nan, np.float32)) for _ in range(2))
+    if warm:
+        kernel.launch(stream, da, dw, de)
+        stream.synchronize()
+    graph = _Captured(stream, lambda: kernel.launch(stream, da, dw, dc))
+
+    def replay(beside):
+        dc.copy_from_host(np.full(m * n, np.nan, np.float32))
+        for _ in range(4):
+            graph.replay(other)
+            beside()
+        other.synchronize()
+        assert np.array_equal(dc.copy_to_host().reshape(m, n).view(np.uint32), want)
+
+    for _ in range(3):
+        replay(lambda: kernel.launch(stream, da, dw, de))
+        stream.synchronize()
+        assert np.array_equal(de.copy_to_host().reshape(m, n).view(np.uint32), want)
+    stream.destroy()
+    poison = [t.GpuBuffer.from_host(ctx, np.full(1 << 20, np.nan, np.float32)) for _ in range(8)]      # takes what was freed
+    for _ in range(3):
+        replay(lambda: None)
+    assert all(np.all(np.isnan(p.copy_to_host())) for p in poison)
+    graph.close()

@@ -356,6 +356,57 @@ hipError_t launch_rmsnorm(hipStream_t stream, uint64_t residual, uint64_t in, ui
   return hipModuleLaunchKernel(d->rmsnorm, 1, 1, 1, block, 1, 1, 0, stream, args, nullptr);
 }
 
+// While this exists, what its thread allocates does not count as part of a capture in progress (hipMalloc would be refused).
+struct AllocationBesideCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  AllocationBesideCapture(const AllocationBesideCapture&) = delete;
+};
+void* alloc_beside_capture(size_t bytes) {      // nullptr: none to be had, and no error is left behind
+  if (g_tune_gemm_workspace_none) return nullptr;
+  const AllocationBesideCapture beside;
+  void* buf = nullptr;
+  if (hipMalloc(&buf, bytes) == hipSuccess) return buf;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+// Scratch of captured work.  A graph can be replayed for as long as the process lives, on any stream, beside eager calls and
+// beside other graphs: what one stream adds to one capture, which runs one after the other, shares a buffer that nothing else
+// uses and that is never freed.
+constexpr size_t kCaptureBytesMax = size_t(8) << 30;      // of a device's in all; beyond that the caller does without
+std::mutex g_capture_mutex;
+std::map<int, size_t> g_capture_bytes;      // by device, under g_capture_mutex (taken last)
+struct CaptureBuffer {      // guarded by its owner's mutex
+  unsigned long long capture = 0;      // the stream's last capture, and its buffer
+  void* buf = nullptr;
+  size_t cap = 0;
+  bool take(int dev, unsigned long long id, size_t need, bool* fresh) {      // false: none to be had
+    *fresh = !buf || capture != id || cap < need;
+    if (!*fresh) return true;
+    std::lock_guard<std::mutex> lock(g_capture_mutex);
+    size_t& used = g_capture_bytes[dev];
+    void* made = used + need > kCaptureBytesMax ? nullptr : alloc_beside_capture(need);
+    if (!made) return false;
+    used += need;
+    capture = id;
+    buf = made;
+    cap = need;
+    return true;
+  }
+};
+// Is the stream being captured, and into what?  false: that cannot be told, and no error is left behind.
+bool capture_of(hipStream_t stream, bool* captured, unsigned long long* id) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamGetCaptureInfo(stream, &status, id) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  *captured = status != hipStreamCaptureStatusNone;
+  return true;
+}
+
 // Per-(device, stream) scratch buffers of the kernels that cut their work in parts (partial results + arrival
 // counters at the front).  g_ws_mutex is held across lookup, growth and the launch that zeroes new counters, so two
 // threads on two streams never see a half-grown buffer; a buffer only ever belongs to one stream, and work on one
@@ -367,6 +418,7 @@ struct ScratchWorkspace {
   void* buf = nullptr;
   size_t cap = 0;
   std::weak_ptr<char> thread;      // hipStreamPerThread's only
+  CaptureBuffer graph;
 };
 using ScratchKey = std::tuple<int, hipStream_t, const void*>;      // device, stream, thread (see there)
 using ScratchMap = std::map<ScratchKey, ScratchWorkspace>;
@@ -391,9 +443,19 @@ void free_scratch_of_ended_threads(ScratchMap& map) {      // under g_ws_mutex; 
   }
 }
 
+hipError_t clear_counters(DeviceKernels* d, hipStream_t stream, void* buf, size_t bytes) {
+  uint32_t words = uint32_t(bytes / 4u), zero = 0u;
+  void* args[] = {&buf, &words, &zero};
+  return hipModuleLaunchKernel(d->fill_u32, std::max(1u, std::min(64u, (words + 255u) / 256u)), 1, 1, 256, 1, 1, 0, stream, args, nullptr);
+}
+
 // want > need: what a buffer that has to be made (or made larger) should hold, so that later calls, captured ones among them,
 // find room; the call itself does with `need`.
-hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream, size_t need, size_t zero_bytes, uint64_t* base, size_t want = 0) {
+// Under capture the stream's buffer is taken as it is or not at all: it cannot grow (nothing may wait for the stream), and new counters would be
+// cleared by the graph's replays only.  A captured call that finds it too small, or that may not share it (apart), has the capture's own, cleared in front of it
+// by a node of the graph; apart: where there is none the stream's, as long as that is large enough.
+hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream, size_t need, size_t zero_bytes, uint64_t* base, size_t want = 0,
+                           bool apart = false) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -401,6 +463,15 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   ScratchWorkspace& ws = map[scratch_key(dev, stream, thread)];
   ws.thread = thread;
+  bool captured = false, fresh = false;
+  unsigned long long id = 0;
+  if ((apart || ws.cap < need) && capture_of(stream, &captured, &id) && captured) {
+    if (ws.graph.take(dev, id, need, &fresh)) {
+      *base = reinterpret_cast<uint64_t>(ws.graph.buf);
+      return fresh ? clear_counters(d, stream, ws.graph.buf, zero_bytes) : hipSuccess;
+    }
+    if (ws.cap < need) return hipErrorOutOfMemory;
+  }
   if (ws.cap < need) {
     free_scratch_of_ended_threads(map);
     if (ws.buf) {
@@ -421,10 +492,7 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
       ws.cap = 0;
       return e;
     }
-    uint32_t words = uint32_t(zero_bytes / 4u), zero = 0u;
-    void* fill_args[] = {&ws.buf, &words, &zero};
-    const uint32_t grid = std::max(1u, std::min(64u, (words + 255u) / 256u));
-    if ((e = hipModuleLaunchKernel(d->fill_u32, grid, 1, 1, 256, 1, 1, 0, stream, fill_args, nullptr)) != hipSuccess) return e;
+    if ((e = clear_counters(d, stream, ws.buf, zero_bytes)) != hipSuccess) return e;
   }
   *base = reinterpret_cast<uint64_t>(ws.buf);
   return hipSuccess;
@@ -560,6 +628,11 @@ ScratchMap g_gemm_ws;
 constexpr uint32_t kGemmXpStageBytes = 16 * 1024 + 512 + 64;
 constexpr size_t kGemmCounterBytes = size_t(1) << 16;   // arrival counters at the front of the GEMM's scratch buffer
 constexpr size_t kGemmPartsBytes = size_t(16) << 20;     // what a stream's buffer is made for behind them, as trn_q4k_gemm_noalloc's
+// Captured, a product of more than 32 tokens does not share the stream's buffer, whichever kernel takes it: the one for many tokens never does, and
+// which of them a shape takes is nothing a caller can know.
+hipError_t acquire_gemm_scratch(DeviceKernels* d, hipStream_t stream, uint32_t m, size_t need, uint64_t* base) {
+  return acquire_scratch(g_gemm_ws, d, stream, need, kGemmCounterBytes, base, kGemmCounterBytes + kGemmPartsBytes, m > 32u);
+}
 
 // How a product on the matrix cores is cut: `waves` strips of 32 rows and nt token tiles of 16 per workgroup (groups of
 // strips, tgroups of tiles), K in kparts parts of ksb super-blocks, so that the workgroups are about as many as the CUs.
@@ -661,8 +734,13 @@ hipError_t launch_kq_gemm_f16(DeviceKernels* d, Fmt f, hipStream_t stream, uint6
   if (ext_base != 0) {
     if (need > ext_cap) return hipErrorInvalidValue;
   } else {
-    hipError_t e = acquire_scratch(g_gemm_ws, d, stream, need, cnt_cap, &cnt, kGemmCounterBytes + kGemmPartsBytes);
-    if (e != hipSuccess) return e;
+    // (one part needs none, but an eager product makes the stream's buffer all the same: the next one may be captured)
+    bool captured = false;
+    unsigned long long id = 0;
+    if (kparts > 1u || !capture_of(stream, &captured, &id) || !captured) {
+      const hipError_t e = acquire_gemm_scratch(d, stream, m, need, &cnt);
+      if (e != hipSuccess) return e;
+    }
   }
   const uint64_t padded = (uint64_t(groups) * kparts + 7u) / 8u * 8u;
   if (ksb > 0xFFFFu || groups > 0xFFFFu || tiles > 0xFFFFu || padded * tgroups > 0x7FFFFFFFu) return hipErrorInvalidValue;
@@ -768,7 +846,7 @@ hipError_t launch_gemm_slices(DeviceKernels* d, Fmt f, hipStream_t stream, uint6
   const uint32_t tiles = (m + 15u) / 16u;
   if (ws == 0 && cut.kparts > 1u) {
     const size_t need = kGemmCounterBytes + size_t(cut.kparts) * tiles * cut.groups * cut.rt * 1024u;
-    const hipError_t e = acquire_scratch(g_gemm_ws, d, stream, need, kGemmCounterBytes, &ws, kGemmCounterBytes + kGemmPartsBytes);
+    const hipError_t e = acquire_gemm_scratch(d, stream, m, need, &ws);
     if (e != hipSuccess) return e;
   }
   uint64_t geom = uint64_t(cut.ksb) | uint64_t(cut.kparts) << 16 | uint64_t(cut.groups) << 32 | uint64_t(tiles) << 48;
@@ -845,36 +923,14 @@ TallCut tall_cut(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t
 
 // One buffer per (device, stream): the operands, then the parts of K.  A product is two or three launches that share it, so
 // a lock is held from the first to the last: another thread's product on the same stream may not come between them.
-// A captured product has no part in it: a graph can be replayed for as long as the process lives, on any stream, beside
-// eager products and beside other graphs.  The products that one stream adds to one capture run one after the other and
-// share a buffer that nothing else uses and that is never freed.
+// A captured product has no part in it (CaptureBuffer).
 struct TallWorkspace {
   void* buf = nullptr;
   size_t cap = 0;
-  unsigned long long capture = 0;      // the stream's last capture, and its buffer
-  void* graph_buf = nullptr;
-  size_t graph_cap = 0;
+  CaptureBuffer graph;
 };
 std::map<std::pair<int, hipStream_t>, TallWorkspace> g_tall_ws;
-std::map<int, size_t> g_tall_graph_bytes;      // by device: what is left to graphs
 std::mutex g_tall_mutex;
-constexpr size_t kTallGraphBytesMax = size_t(8) << 30;      // of it in all; further captured products take the other kernel
-
-// While this exists, what its thread allocates does not count as part of a capture in progress (hipMalloc would be refused).
-struct AllocationBesideCapture {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-  ~AllocationBesideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-  AllocationBesideCapture(const AllocationBesideCapture&) = delete;
-};
-void* tall_alloc(size_t bytes) {      // nullptr: none to be had, and no error is left behind
-  if (g_tune_gemm_workspace_none) return nullptr;
-  const AllocationBesideCapture beside;
-  void* buf = nullptr;
-  if (hipMalloc(&buf, bytes) == hipSuccess) return buf;
-  (void)hipGetLastError();
-  return nullptr;
-}
 
 hipError_t launch_tall_once(DeviceKernels* d, Fmt f, hipStream_t stream, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n,
                             uint32_t k, const TallCut& cut, uint64_t ws) {
@@ -926,28 +982,17 @@ hipError_t launch_tall_on_stream(DeviceKernels* d, Fmt f, hipStream_t stream, ui
   {
     std::lock_guard<std::mutex> lock(g_tall_mutex);
     TallWorkspace& ws = g_tall_ws[std::make_pair(dev, stream)];
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    bool captured = false, fresh = false;
     unsigned long long id = 0;
-    if (hipStreamGetCaptureInfo(stream, &capture, &id) != hipSuccess) {
-      (void)hipGetLastError();
-      return hipSuccess;
-    }
-    if (capture != hipStreamCaptureStatusNone) {
-      if (!ws.graph_buf || ws.capture != id || ws.graph_cap < need) {
-        size_t& left = g_tall_graph_bytes[dev];
-        void* buf = left + need > kTallGraphBytesMax ? nullptr : tall_alloc(need);
-        if (!buf) return hipSuccess;
-        left += need;
-        ws.capture = id;
-        ws.graph_buf = buf;
-        ws.graph_cap = need;
-      }
+    if (!capture_of(stream, &captured, &id)) return hipSuccess;
+    if (captured) {
+      if (!ws.graph.take(dev, id, need, &fresh)) return hipSuccess;
       *done = true;
-      return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph_buf), need);
+      return launch_tall(d, f, stream, a, w, c, m, n, k, cut, reinterpret_cast<uint64_t>(ws.graph.buf), need);
     }
     first = ws.buf == nullptr;
     if (ws.cap < need) {
-      void* buf = tall_alloc(need);
+      void* buf = alloc_beside_capture(need);
       if (!buf) return hipSuccess;      // (what the stream has stays: a smaller product finds it)
       old = ws.buf;
       ws.buf = buf;
