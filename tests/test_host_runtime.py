@@ -1,0 +1,117 @@
+"""The library's host code (trn_runtime.cpp) over a stand-in for the HIP runtime (fake_hip.cpp): which kernel is launched with which scratch memory,
+where that depends on threads, captures and failures that a GPU run cannot bring about or not every time."""
+import ctypes as C
+import os
+import subprocess
+import threading
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+A, W, Y = 1 << 32, 1 << 40, 1 << 42
+
+
+class Launch:
+    def __init__(self, name, v):
+        self.name, self.grid, self.block, self.stream, self.capture, self.args = name, v[0], v[1], v[2], v[3], list(v[4:9])
+
+
+class Runtime:
+    def __init__(self, path):
+        self.lib = lib = C.CDLL(path)
+        u64, u32 = C.c_uint64, C.c_uint32
+        lib.fake_launch.restype, lib.fake_memory.restype = C.c_char_p, u64
+        lib.fake_capture.argtypes = [u64, C.c_ulonglong]
+        lib.fake_tuning_race.argtypes = [C.c_char_p, u32, u32, u32, C.c_int]
+        lib.trn_gemv_f32.argtypes = [u64, u64, u64, u64, u32, u32]
+        for fmt in ("q4k", "q5k", "q6k"):
+            getattr(lib, f"trn_{fmt}_gemm").argtypes = [u64, u64, u64, u64, u32, u32, u32]
+        lib.trn_stream_create.argtypes = [C.POINTER(u64), C.c_uint]
+        lib.trn_stream_destroy.argtypes = [u64]
+
+    def stream(self):
+        s = C.c_uint64()
+        assert self.lib.trn_stream_create(C.byref(s), 1) == 0
+        return s.value
+
+    def launched(self, issue):
+        """(status, the launches) of one call."""
+        before = self.lib.fake_launches()
+        rc, v, out = issue(), (C.c_uint64 * 9)(), []
+        for i in range(before, self.lib.fake_launches()):
+            out.append(Launch(self.lib.fake_launch(i, v).decode(), v))
+        return rc, out
+
+    def f32(self, stream, k, n):
+        return self.launched(lambda: self.lib.trn_gemv_f32(stream, Y, A, W, k, n))
+
+    def gemm(self, fmt, stream, m, n, k):
+        return self.launched(lambda: getattr(self.lib, f"trn_{fmt}_gemm")(stream, A, W, Y, m, n, k))
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    path = tmp_path_factory.mktemp("host") / "runtime.so"
+    image = path.parent / "image"
+    image.write_bytes(b"\x7fELF" + bytes(252))
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wl,-Bsymbolic", "-D__HIP_PLATFORM_AMD__", "-DKQ_U=2",
+                    f"-I{os.environ.get('ROCM_PATH', '/opt/rocm')}/include", f'-DTRN_HSACO_PATH="{image}"', "-o", str(path),
+                    os.path.join(ROOT, "trueno_amd", "csrc", "trn_runtime.cpp"), os.path.join(ROOT, "tests", "fake_hip.cpp"), "-pthread"], check=True)
+    return Runtime(str(path))
+
+
+@pytest.fixture
+def rt(built):
+    built.lib.fake_reset()
+    yield built
+    built.lib.fake_reset()
+
+
+@pytest.mark.parametrize("n", [515, 516])
+def test_threads_have_scratch_of_their_own_behind_the_handle_they_share(rt, n):
+    counters, barrier = [], threading.Barrier(2)
+
+    def work():
+        barrier.wait()
+        counters.append(rt.f32(2, 3000, n)[0])      # hipStreamPerThread
+        barrier.wait()
+
+    before = rt.lib.fake_launches()
+    threads = [threading.Thread(target=work) for _ in range(2)]
+    for x in threads:
+        x.start()
+    for x in threads:
+        x.join()
+    v, seen = (C.c_uint64 * 9)(), set()
+    for i in range(before, rt.lib.fake_launches()):
+        if rt.lib.fake_launch(i, v).decode().startswith("gemv_f32"):
+            seen.add(v[8])
+    assert counters == [0, 0] and len(seen) == 2
+
+
+def test_scratch_of_threads_that_have_ended_is_freed(rt):
+    held = []
+    for _ in range(6):
+        x = threading.Thread(target=lambda: rt.gemm("q4k", 2, 16, 512, 4096))
+        x.start()
+        x.join()
+        held.append(rt.lib.fake_memory())
+    assert held[1:] == held[:1] * 5      # (the one before is freed when the next is made)
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("q4k", 121, 4192, 4096), ("q5k", 40, 2573, 5888)])
+@pytest.mark.parametrize("warm", (False, True))
+def test_captured_products_of_more_than_32_tokens_have_scratch_of_their_own(rt, fmt, m, n, k, warm):
+    stream = rt.stream()
+    if warm:
+        rt.gemm(fmt, stream, m, n, k)
+    rt.lib.fake_capture(stream, 7)
+    rc, (fill, first) = rt.gemm(fmt, stream, m, n, k)
+    rc2, (second,) = rt.gemm(fmt, stream, m, n, k)
+    assert rc == rc2 == 0 and fill.name == "kq_fill_u32" and fill.capture == first.capture == 7
+    assert fill.args[0] == first.args[3] == second.args[3]      # cleared in the graph, once
+    rt.lib.fake_capture(stream, 0)
+    rc, eager = rt.gemm(fmt, stream, m, n, k)
+    assert rc == 0 and eager[-1].name == first.name and eager[-1].args[3] != first.args[3]
+    assert [x.name for x in eager[:-1]] == ([] if warm else ["kq_fill_u32"])      # what the capture has cleared is not the stream's
+    rt.lib.trn_stream_destroy(stream)
