@@ -115,3 +115,33 @@ def test_captured_products_of_more_than_32_tokens_have_scratch_of_their_own(rt, 
     assert rc == 0 and eager[-1].name == first.name and eager[-1].args[3] != first.args[3]
     assert [x.name for x in eager[:-1]] == ([] if warm else ["kq_fill_u32"])      # what the capture has cleared is not the stream's
     rt.lib.trn_stream_destroy(stream)
+
+
+def test_a_buffer_whose_counters_could_not_be_cleared_is_not_kept(rt):
+    stream, other = rt.stream(), rt.stream()
+    rt.f32(other, 3000, 516)
+    before = rt.lib.fake_memory()
+    for n in (516, 515):
+        rt.lib.fake_fail(b"kq_fill_u32")
+        rc, launches = rt.f32(stream, 3000, n)
+        assert rc != 0 and not launches and rt.lib.fake_memory() == before
+    rt.lib.fake_capture(stream, 9)
+    rc, launches = rt.f32(stream, 3000, 516)
+    assert rc != 0 and not launches and rt.lib.fake_memory() == before
+    rt.lib.fake_capture(stream, 0)
+    rt.lib.fake_fail(b"")
+    for n in (515, 516):
+        rc, launches = rt.f32(stream, 3000, n)
+        assert rc == 0 and launches[-1].name == ("gemv_f32_ragged" if n == 515 else "gemv_f32_fast")
+        assert [x.name for x in launches[:-1]] == (["kq_fill_u32"] if n == 515 else [])
+    rt.lib.trn_stream_destroy(stream)
+    assert rt.lib.fake_memory() == before
+    rt.lib.trn_stream_destroy(other)
+
+
+def test_eager_calls_make_their_scratch_while_another_stream_is_captured(rt):
+    stream, captured = rt.stream(), rt.stream()
+    rt.lib.fake_capture(captured, 11)
+    for n in (515, 516):
+        rc, launches = rt.f32(stream, 3000, n)
+        assert rc == 0 and launches[-1].grid > (n + 255) // 256 and launches[-1].capture == 0      # parts of K

@@ -395,6 +395,13 @@ struct CaptureBuffer {      // guarded by its owner's mutex
     cap = need;
     return true;
   }
+  void drop(int dev) {      // nothing has been recorded with it
+    const AllocationBesideCapture beside;
+    (void)hipFree(buf);
+    std::lock_guard<std::mutex> lock(g_capture_mutex);
+    g_capture_bytes[dev] -= cap;
+    *this = CaptureBuffer();
+  }
 };
 // Is the stream being captured, and into what?  false: that cannot be told, and no error is left behind.
 bool capture_of(hipStream_t stream, bool* captured, unsigned long long* id) {
@@ -467,12 +474,17 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
   unsigned long long id = 0;
   if ((apart || ws.cap < need) && capture_of(stream, &captured, &id) && captured) {
     if (ws.graph.take(dev, id, need, &fresh)) {
+      if (fresh && (e = clear_counters(d, stream, ws.graph.buf, zero_bytes)) != hipSuccess) {
+        ws.graph.drop(dev);
+        return e;
+      }
       *base = reinterpret_cast<uint64_t>(ws.graph.buf);
-      return fresh ? clear_counters(d, stream, ws.graph.buf, zero_bytes) : hipSuccess;
+      return hipSuccess;
     }
     if (ws.cap < need) return hipErrorOutOfMemory;
   }
   if (ws.cap < need) {
+    const AllocationBesideCapture beside;      // (another stream may be captured meanwhile)
     free_scratch_of_ended_threads(map);
     if (ws.buf) {
       if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;   // work in flight may still use the old buffer
@@ -492,7 +504,12 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
       ws.cap = 0;
       return e;
     }
-    if ((e = clear_counters(d, stream, ws.buf, zero_bytes)) != hipSuccess) return e;
+    if ((e = clear_counters(d, stream, ws.buf, zero_bytes)) != hipSuccess) {      // a later call would count on them
+      (void)hipFree(ws.buf);
+      ws.buf = nullptr;
+      ws.cap = 0;
+      return e;
+    }
   }
   *base = reinterpret_cast<uint64_t>(ws.buf);
   return hipSuccess;
@@ -535,10 +552,14 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
     // captured, which a graph may replay on any stream and after the buffer has been replaced by a larger one.
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     const bool room = size_t(tiles) * 4u <= cnt_cap && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
-    if (parts > 1u && (!room || acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes) != hipSuccess)) {
-      (void)hipGetLastError();
-      parts = 1u;
-      rows_per_part = k;
+    if (parts > 1u) {
+      e = room ? acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes) : hipErrorOutOfMemory;
+      if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        parts = 1u;
+        rows_per_part = k;
+      }
     }
   } else {
     if (size_t(tiles) * 4u > cnt_cap) return hipErrorInvalidValue;
