@@ -23,10 +23,11 @@
  * of a list's launches of more than sixteen entries (trn_kquant_gemv_batch), the tables of the
  * resident executor (batch_mode 1); and one static array of 16 MiB + 64 KiB and 256 MiB allocated on first use per GPU
  * (trn_q4k_gemm_noalloc).  Under stream capture what one stream adds to one capture has a buffer of its own instead where the
- * product has more than 32 tokens, or where the stream's buffer is missing or too small: allocated during the capture and kept
+ * product has more than 32 tokens, or is an f32 one with columns that are no multiple of four or buffers that do not begin at 16
+ * bytes, or where the stream's buffer is missing or too small: allocated during the capture and kept
  * until the process ends, so that the graph can be replayed on any stream, beside anything but another instance of itself; at most
  * 8 GiB per GPU for all captures, beyond that the stream's buffer, if it is large enough (many tokens: the kernel that needs no operands in
- * memory).  Other captured calls use the stream's: their graph is replayed on that stream, before it is destroyed, and no
+ * memory; f32: the sums in one part).  Other captured calls use the stream's: their graph is replayed on that stream, before it is destroyed, and no
  * larger product is issued there in between.  The calls that never allocate: the GEMV launchers, trn_kquant_gemv_batch
  * for lists whose launches hold at most sixteen entries or while the stream is being captured,
  * trn_q4k_gemm_noalloc, the element-wise launchers.  All entry points may be called from any thread;

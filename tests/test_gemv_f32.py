@@ -135,7 +135,8 @@ def test_gpu_gemv_f32_rows_at_any_multiple_of_four_bytes(gpu, k, n, shift_a, shi
 
 @pytest.mark.gpu
 def test_gpu_gemv_f32_rows_of_odd_length_captured_on_a_new_stream(gpu):
-    """The capture allocates nothing and its graph holds no scratch memory: replayed beside eager calls, some with more columns."""
+    """Its partial sums are the capture's own: replayed on another stream beside eager calls on its own, some with more columns, and after its
+    own is gone, always the eager call's bits."""
     from tests.test_gpu_gemm import _Captured
     ctx, stream = gpu
     k, n, wide = 2000, 515, 5003
@@ -144,13 +145,21 @@ def test_gpu_gemv_f32_rows_of_odd_length_captured_on_a_new_stream(gpu):
     da, dx = t.GpuBuffer.from_host(ctx, a.reshape(-1)), t.GpuBuffer.from_host(ctx, x)
     dy, dz = (t.GpuBuffer.from_host(ctx, np.full(m, np.nan, np.float32)) for m in (n, wide))
     want = a.reshape(-1)[:k * n].reshape(k, n).astype(np.float64).T @ x.astype(np.float64)
+    t.CoalescedGemvKernel(k, n).launch(stream, dy, da, dx)
+    stream.synchronize()
+    eager = dy.copy_to_host()
+    assert kq.rel_l2(eager, want) <= 1e-6
     new = t.CudaStream(ctx)
     graph = _Captured(new, lambda: t.CoalescedGemvKernel(k, n).launch(new, dy, da, dx))
-    for _ in range(3):
+    for beside in (True, True, True, False, False):
         dy.copy_from_host(np.full(n, np.nan, np.float32))
         graph.replay(stream)
-        t.CoalescedGemvKernel(k, wide).launch(new, dz, da, dx)
+        if beside:
+            t.CoalescedGemvKernel(k, wide).launch(new, dz, da, dx)
+            t.CoalescedGemvKernel(k, n).launch(new, dz, da, dx)
+            new.synchronize()
+        else:
+            new.destroy()
         stream.synchronize()
-        new.synchronize()
-        assert kq.rel_l2(dy.copy_to_host(), want) <= 1e-6
+        assert np.array_equal(dy.copy_to_host().view(np.uint32), eager.view(np.uint32))
     graph.close()

@@ -125,10 +125,10 @@ def test_a_buffer_whose_counters_could_not_be_cleared_is_not_kept(rt):
         rt.lib.fake_fail(b"kq_fill_u32")
         rc, launches = rt.f32(stream, 3000, n)
         assert rc != 0 and not launches and rt.lib.fake_memory() == before
-    rt.lib.fake_capture(stream, 9)
-    rc, launches = rt.f32(stream, 3000, 516)
-    assert rc != 0 and not launches and rt.lib.fake_memory() == before
-    rt.lib.fake_capture(stream, 0)
+        rt.lib.fake_capture(stream, 9)
+        rc, launches = rt.f32(stream, 3000, n)
+        assert rc != 0 and not launches and rt.lib.fake_memory() == before
+        rt.lib.fake_capture(stream, 0)
     rt.lib.fake_fail(b"")
     for n in (515, 516):
         rc, launches = rt.f32(stream, 3000, n)
@@ -145,3 +145,21 @@ def test_eager_calls_make_their_scratch_while_another_stream_is_captured(rt):
     for n in (515, 516):
         rc, launches = rt.f32(stream, 3000, n)
         assert rc == 0 and launches[-1].grid > (n + 255) // 256 and launches[-1].capture == 0      # parts of K
+
+
+def test_captured_f32_products_of_odd_rows_are_cut_as_eager_ones(rt):
+    """In the capture's own memory, whether or not the stream has some, and in one part, which needs none, where that cannot be had."""
+    stream = rt.stream()
+    for i, warm in enumerate((False, True)):
+        rt.lib.fake_capture(stream, 20 + i)
+        rc, (fill, product) = rt.f32(stream, 3000, 515)
+        rt.lib.fake_capture(stream, 0)
+        rc2, eager = rt.f32(stream, 3000, 515)
+        assert rc == rc2 == 0 and fill.name == "kq_fill_u32" and product.capture == 20 + i
+        assert (product.name, product.grid) == (eager[-1].name, eager[-1].grid) and product.grid > 3
+        assert product.args[4] == fill.args[0] != eager[-1].args[4] and len(eager) == (1 if warm else 2)
+    assert rt.lib.trn_set_tuning(b"gemm_workspace_none", 1) == 0
+    rt.lib.fake_capture(stream, 30)
+    rc, (product,) = rt.f32(stream, 3000, 515)
+    assert rc == 0 and product.grid == 3
+    assert rt.lib.trn_set_tuning(b"gemm_workspace_none", 0) == 0

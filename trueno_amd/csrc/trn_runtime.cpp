@@ -459,10 +459,11 @@ hipError_t clear_counters(DeviceKernels* d, hipStream_t stream, void* buf, size_
 // want > need: what a buffer that has to be made (or made larger) should hold, so that later calls, captured ones among them,
 // find room; the call itself does with `need`.
 // Under capture the stream's buffer is taken as it is or not at all: it cannot grow (nothing may wait for the stream), and new counters would be
-// cleared by the graph's replays only.  A captured call that finds it too small, or that may not share it (apart), has the capture's own, cleared in front of it
-// by a node of the graph; apart: where there is none the stream's, as long as that is large enough.
+// cleared by the graph's replays only.  A captured call that finds it too small, or that is not to share it, has the capture's own, cleared in front of it
+// by a node of the graph.  Where there is none: kApart takes the stream's, as long as that is large enough, kApartOrNone is out of memory.
+enum class Captured { kShares, kApart, kApartOrNone };
 hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream, size_t need, size_t zero_bytes, uint64_t* base, size_t want = 0,
-                           bool apart = false) {
+                           Captured rule = Captured::kShares) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -472,7 +473,7 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
   ws.thread = thread;
   bool captured = false, fresh = false;
   unsigned long long id = 0;
-  if ((apart || ws.cap < need) && capture_of(stream, &captured, &id) && captured) {
+  if ((rule != Captured::kShares || ws.cap < need) && capture_of(stream, &captured, &id) && captured) {
     if (ws.graph.take(dev, id, need, &fresh)) {
       if (fresh && (e = clear_counters(d, stream, ws.graph.buf, zero_bytes)) != hipSuccess) {
         ws.graph.drop(dev);
@@ -481,7 +482,7 @@ hipError_t acquire_scratch(ScratchMap& map, DeviceKernels* d, hipStream_t stream
       *base = reinterpret_cast<uint64_t>(ws.graph.buf);
       return hipSuccess;
     }
-    if (ws.cap < need) return hipErrorOutOfMemory;
+    if (ws.cap < need || rule == Captured::kApartOrNone) return hipErrorOutOfMemory;
   }
   if (ws.cap < need) {
     const AllocationBesideCapture beside;      // (another stream may be captured meanwhile)
@@ -548,12 +549,10 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
   const size_t cnt_cap = 64u * 1024u, need = cnt_cap + (parts > 1u ? size_t(parts) * (size_t(n) + 3u) * 4u : 0u);
   uint64_t cnt = 0;
   if (ragged) {
-    // A single part writes no partial results and counts nothing: it takes the call whose scratch cannot be had, and the one that is
-    // captured, which a graph may replay on any stream and after the buffer has been replaced by a larger one.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    const bool room = size_t(tiles) * 4u <= cnt_cap && hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+    // A single part writes no partial results and counts nothing: it takes the call whose scratch cannot be had.
+    const bool room = size_t(tiles) * 4u <= cnt_cap;
     if (parts > 1u) {
-      e = room ? acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes) : hipErrorOutOfMemory;
+      e = room ? acquire_scratch(g_gemv_f32_ws, d, stream, need, cnt_cap, &cnt, kGemvF32Bytes, Captured::kApartOrNone) : hipErrorOutOfMemory;
       if (e != hipSuccess && e != hipErrorOutOfMemory) return e;
       if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -652,7 +651,8 @@ constexpr size_t kGemmPartsBytes = size_t(16) << 20;     // what a stream's buff
 // Captured, a product of more than 32 tokens does not share the stream's buffer, whichever kernel takes it: the one for many tokens never does, and
 // which of them a shape takes is nothing a caller can know.
 hipError_t acquire_gemm_scratch(DeviceKernels* d, hipStream_t stream, uint32_t m, size_t need, uint64_t* base) {
-  return acquire_scratch(g_gemm_ws, d, stream, need, kGemmCounterBytes, base, kGemmCounterBytes + kGemmPartsBytes, m > 32u);
+  return acquire_scratch(g_gemm_ws, d, stream, need, kGemmCounterBytes, base, kGemmCounterBytes + kGemmPartsBytes,
+                         m > 32u ? Captured::kApart : Captured::kShares);
 }
 
 // How a product on the matrix cores is cut: `waves` strips of 32 rows and nt token tiles of 16 per workgroup (groups of
