@@ -847,3 +847,25 @@ def test_gemm_captured_products_in_parts_keep_to_themselves(gpu, fmt, m, n, k, w
         replay(lambda: None)
     assert all(np.all(np.isnan(p.copy_to_host())) for p in poison)
     graph.close()
+
+
+@pytest.mark.parametrize("tall", (1, 2))
+@pytest.mark.parametrize("fmt", MFMA_FORMATS)
+def test_gemm_sums_beyond_the_largest_float_are_infinite(gpu, fmt, tall):
+    """Token r is finite, of one sign with row r's first 256 weights and so large that their sum is twice the largest float (every other term is
+    of ordinary size): plus or minus infinity in that place, through eight further super-blocks, and a number wherever the terms' sizes add up
+    to one."""
+    m, n, k = 40, 64, 2304
+    buf, a = kq.gen_matrix(fmt, 760, n, k), kq.gen_x(761, m, k)
+    w = kq.dequant_matrix(fmt, buf, n, k)
+    sign = np.where(np.arange(m) % 2 == 0, 1.0, -1.0)
+    a[:, :256] = sign[:, None] * np.sign(w[:m, :256]) * (6.8e38 / np.abs(w[:m, :256]).astype(np.float64).sum(1))[:, None]
+    assert np.all(np.isfinite(a))
+    try:
+        _tune("gemm_tall", tall)
+        c = gpu_gemm(gpu, fmt, buf, a, m, n, k)
+    finally:
+        _tune("gemm_tall", 0)
+    assert np.array_equal(c[np.arange(m), np.arange(m)], sign * np.inf)
+    small = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64).T < 3e38
+    assert np.all(np.isfinite(c[small]))

@@ -174,8 +174,8 @@ __device__ __forceinline__ void put_by(f32x16& stash, f32x16& tot) {
   __builtin_amdgcn_sched_barrier(0);      // (nothing else is alive here)
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    const float s = stash[v] + tot[v], b = s - stash[v];
-    tot[v] = LOSSLESS ? (stash[v] - (s - b)) + (tot[v] - b) : 0.0f;
+    const float s = stash[v] + tot[v], b = s - stash[v], rest = (stash[v] - (s - b)) + (tot[v] - b);
+    tot[v] = LOSSLESS && rest == rest ? rest : 0.0f;      // (a sum that is infinite stays so: what it rounds away is no number)
     stash[v] = s;
   }
   __builtin_amdgcn_sched_barrier(0);
