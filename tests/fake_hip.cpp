@@ -59,10 +59,10 @@ EXPORT const char* fake_launch(int i, uint64_t* out) {      // out: grid, block,
   std::copy(l.args, l.args + 5, out + 4);
   return l.name.c_str();
 }
-// One thread issues a product over and over while another sets `key` to 1 or back to 0.  Of `rounds` changes, how many does the first thread not
+// One thread issues a product over and over while another sets `key` to `value` or back to 0.  Of `rounds` changes, how many does the first thread not
 // follow with a call that begins after the change has returned?
 namespace { thread_local const void* t_last = nullptr; }
-EXPORT int fake_tuning_race(const char* key, uint32_t m, uint32_t n, uint32_t k, int rounds) {
+EXPORT int fake_tuning_race(const char* key, int value, uint32_t m, uint32_t n, uint32_t k, int rounds) {
   auto product = [&] {
     (void)trn_q4k_gemm(nullptr, 4096, 8192, 12288, m, n, k);
     return t_last;
@@ -70,7 +70,7 @@ EXPORT int fake_tuning_race(const char* key, uint32_t m, uint32_t n, uint32_t k,
   const void* want[2];
   g_record = false;
   for (int s : {1, 0}) {
-    (void)trn_set_tuning(key, s);
+    (void)trn_set_tuning(key, s * value);
     want[s] = product();
   }
   if (want[0] == want[1]) return -1;
@@ -79,7 +79,7 @@ EXPORT int fake_tuning_race(const char* key, uint32_t m, uint32_t n, uint32_t k,
     for (int r = 1; r <= rounds; ++r) {
       while (seen.load() < r - 1) {}
       for (int spin = 0; spin < (r * 37) % 400; ++spin) (void)done.load();
-      (void)trn_set_tuning(key, r & 1);
+      (void)trn_set_tuning(key, (r & 1) * value);
       done.store(r);
     }
   });

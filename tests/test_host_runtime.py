@@ -22,7 +22,7 @@ class Runtime:
         u64, u32 = C.c_uint64, C.c_uint32
         lib.fake_launch.restype, lib.fake_memory.restype = C.c_char_p, u64
         lib.fake_capture.argtypes = [u64, C.c_ulonglong]
-        lib.fake_tuning_race.argtypes = [C.c_char_p, u32, u32, u32, C.c_int]
+        lib.fake_tuning_race.argtypes = [C.c_char_p, C.c_int, u32, u32, u32, C.c_int]
         lib.trn_gemv_f32.argtypes = [u64, u64, u64, u64, u32, u32]
         for fmt in ("q4k", "q5k", "q6k"):
             getattr(lib, f"trn_{fmt}_gemm").argtypes = [u64, u64, u64, u64, u32, u32, u32]
@@ -163,3 +163,8 @@ def test_captured_f32_products_of_odd_rows_are_cut_as_eager_ones(rt):
     rc, (product,) = rt.f32(stream, 3000, 515)
     assert rc == 0 and product.grid == 3
     assert rt.lib.trn_set_tuning(b"gemm_workspace_none", 0) == 0
+
+
+def test_a_plan_is_not_older_than_the_tuning_call_before_it(rt):
+    """A thread that plans a product while another changes a setting follows the change as soon as that call has returned."""
+    assert rt.lib.fake_tuning_race(b"gemm_slices", 2, 64, 4096, 4096, 20000) == 0

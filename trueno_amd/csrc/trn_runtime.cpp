@@ -2583,10 +2583,15 @@ trn_status trn_device_cu_count(int* count) {
   return st(hipDeviceGetAttribute(count, hipDeviceAttributeMultiprocessorCount, dev));
 }
 
+static trn_status store_tuning(const char* key, int value);
 trn_status trn_set_tuning(const char* key, int value) {
   if (!key || value < 0) return TRN_ERROR_INVALID_VALUE;
   std::lock_guard<std::mutex> lock(g_mutex);
-  ++g_tune_epoch;
+  const trn_status status = store_tuning(key, value);
+  ++g_tune_epoch;      // behind the value: a plan reads the count first, so one made meanwhile is older than the setting, whichever value it saw
+  return status;
+}
+static trn_status store_tuning(const char* key, int value) {
   if (!std::strcmp(key, "gemv_blocks_per_cu")) { g_tune_blocks_per_cu = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "gemv_row_groups")) { g_tune_row_groups = value; return TRN_SUCCESS; }
   if (!std::strcmp(key, "batch_mode")) {
