@@ -168,3 +168,13 @@ def test_captured_f32_products_of_odd_rows_are_cut_as_eager_ones(rt):
 def test_a_plan_is_not_older_than_the_tuning_call_before_it(rt):
     """A thread that plans a product while another changes a setting follows the change as soon as that call has returned."""
     assert rt.lib.fake_tuning_race(b"gemm_slices", 2, 64, 4096, 4096, 20000) == 0
+
+
+@pytest.mark.parametrize("n", [0x7FFFFEFD, 0x7FFFFF00, 0x7FFFFF01, 0x7FFFFFFF, 0x80000001])
+@pytest.mark.parametrize("shift", (0, 4))
+def test_f32_products_of_two_thousand_million_columns_are_launched(rt, n, shift):
+    """A launch has fewer than 2^32 threads (the stand-in refuses others, as HIP does), and the kernel with a thread per column takes what the tiled one cannot."""
+    if n % 4 == 0 and shift == 0:
+        n -= 2      # (the aligned form ends at 16384 column tiles)
+    rc, (product,) = rt.launched(lambda: rt.lib.trn_gemv_f32(rt.stream(), Y, A + shift, W, 1, n))
+    assert rc == 0 and product.grid * product.block >= n and (product.name == "gemv_f32_ragged") == (n <= 0x7FFFFF00)

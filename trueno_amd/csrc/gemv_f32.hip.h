@@ -156,7 +156,7 @@ __device__ __forceinline__ void body(float* __restrict__ y, const float* __restr
 }
 
 // The named kernels' plain form: a thread per column, k in order (the summation order of the reference's gemv_coalesced).  The
-// launcher takes it only for k = 0 and for rows of more than 2^31 columns.
+// launcher takes it only for k = 0 and for rows of 2^31 columns and more.
 __device__ __forceinline__ void generic_body(float* __restrict__ y, const float* __restrict__ a, const float* __restrict__ x,
                                              u32 k_dim, u32 n_dim) {
   const u32 col = blockIdx.x * blockDim.x + threadIdx.x;

@@ -529,7 +529,7 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
   if (e != hipSuccess) return e;
   // Rows that do not all begin at 16 bytes: the same kernel with loads at multiples of four bytes (see there for both sides).
   const bool ragged = n % 4u != 0 || !aligned(a, 16) || !aligned(y, 16);
-  if (k == 0 || (ragged && n > 0x7FFFFFFFu)) {      // (a grid of 512 threads for 256 columns ends at 2^31 columns)
+  if (k == 0 || (ragged && n > 0x7FFFFF00u)) {      // (512 threads for 256 columns: 2^23 such workgroups would be 2^32 threads, one more than a launch has)
     void* args[] = {&y, &a, &x, &k, &n};
     return hipModuleLaunchKernel(d->gemv_f32_generic, (n + 255u) / 256u, 1, 1, 256, 1, 1, 0, stream, args, nullptr);
   }
