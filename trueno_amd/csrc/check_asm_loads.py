@@ -1,18 +1,20 @@
 #!/usr/bin/env python3
 """Build-time check of the gfx950 assembly of the kernels (run by the Makefile on `hipcc -S` output).
 
-The matrix-core GEMM issues some global loads in inline asm and waits for them with hand-counted `s_waitcnt vmcnt(N)`, also
-in inline asm.  Between the two the compiler does not know that the destination registers are not valid yet: if it decides
-to copy or otherwise touch one of them there, the kernel computes with stale data.
+The kernels issue some global loads and LDS reads in inline asm and wait for them with hand-counted `s_waitcnt vmcnt(N)` and
+`lgkmcnt(N)`, also in inline asm.  Between the two the compiler does not know that the destination registers are not valid
+yet: if it decides to copy, reuse or otherwise touch one of them there, the kernel computes with stale data, or what arrives
+late overwrites an address.
 
-The check models the counter the hardware keeps.  Vector-memory operations complete in the order they were issued, and
-`s_waitcnt vmcnt(N)` returns when at most N of them are outstanding: a load is known to have landed once a wait with
-N <= (operations issued after the load) has been passed.  For every kernel the script builds the control-flow graph
+The check models the counters the hardware keeps.  Vector-memory operations complete in the order they were issued, LDS
+operations among themselves as well, and `s_waitcnt vmcnt(N)` (`lgkmcnt(N)`) returns when at most N of the counter's operations
+are outstanding: a load is known to have landed once a wait with N <= (operations of its kind issued after the load) has been
+passed.  Scalar loads count in lgkmcnt too but return out of order: they are no evidence and are left out.  For every kernel the script builds the control-flow graph
 (labels, s_branch / s_cbranch_*, s_endpgm) and computes, for every load written in an asm block, the least number of
 operations issued after it over all paths to each point (a forward data-flow analysis: at a join the minimum, around a
 loop until nothing changes), so a load that is still in flight at the end of a loop body is still in flight at the top of
-the next iteration.  It fails when an instruction outside an asm block names a register of a load that is not known to
-have landed there.
+the next iteration.  It fails when any instruction, of the compiler or of an asm block, names a register of a load that is not
+known to have landed there (but for a later load of the same kind into it, which lands later).
 
 usage: check_asm_loads.py kernels.s
 """
@@ -23,8 +25,10 @@ LOAD = re.compile(r"^\s*(global_load_\w+|buffer_load_\w+|flat_load_\w+|scratch_l
 # what the counter counts on this target: every vector-memory load, store and atomic (cache maintenance is left out,
 # which can only make a load look outstanding for longer)
 VMOP = re.compile(r"^\s*(global_|buffer_|flat_|scratch_|tbuffer_|image_)(load|store|atomic)")
+LDS_READ = re.compile(r"^\s*(ds_read\w*)\s+(v\[\d+:\d+\]|v\d+)(?=[,\s])")
+LDS_OP = re.compile(r"^\s*ds_(?!nop)")
 REG = re.compile(r"\bv\[(\d+):(\d+)\]|\bv(\d+)\b")
-VMCNT = re.compile(r"vmcnt\((\d+)\)")
+WAIT = {"vm": re.compile(r"\bvmcnt\((\d+)\)"), "lds": re.compile(r"\blgkmcnt\((\d+)\)")}
 LABEL = re.compile(r"^([.A-Za-z_$][\w.$]*):")
 BRANCH = re.compile(r"^\s*(s_branch|s_cbranch_\w+)\s+([.A-Za-z_$][\w.$]*)")
 CAP = 63          # the counter's field is six bits wide; nothing waits for more
@@ -108,26 +112,40 @@ def blocks_of(items):
     return blocks
 
 
+def asm_load(text):
+    """(counter, destination) of a load into registers, else None"""
+    m = LOAD.match(text)
+    if m:
+        return None if "lds" in m.group(1) else ("vm", m.group(2))
+    m = LDS_READ.match(text)
+    return ("lds", m.group(2)) if m else None
+
+
 def step(state, ins, report=None):
-    """state: {load line: (ops issued after it, frozenset of its registers)}; returns the state behind `ins`"""
+    """state: {(line, counter): (ops issued after it, frozenset of its registers)} of loads in flight; returns the state behind `ins`"""
     text = ins.text
     if "s_waitcnt" in text:
-        m = VMCNT.search(text)
-        if m:
-            n = int(m.group(1))
-            state = {k: v for k, v in state.items() if v[0] < n}
+        for counter, wait in WAIT.items():
+            m = wait.search(text)
+            if m:
+                n = int(m.group(1))
+                state = {k: v for k, v in state.items() if k[1] != counter or v[0] < n}
         return state
-    if not ins.asm and state and report is not None:
+    if state and report is not None:
         named = regs(text)
-        for line, (_, rs) in sorted(state.items()):
-            hit = named & rs
+        load = asm_load(text) if ins.asm else None
+        # (a load into the registers of one in flight on the same counter lands behind it)
+        sources = regs(text[text.index(load[1]) + len(load[1]):]) if load else named
+        for (line, counter), (_, rs) in sorted(state.items()):
+            hit = (sources if load and load[0] == counter else named) & rs
             if hit:
                 report(ins, min(hit), line)
-    if VMOP.match(text):
-        state = {k: (min(v[0] + 1, CAP), v[1]) for k, v in state.items()}
-        m = LOAD.match(text)
-        if ins.asm and m and "lds" not in m.group(1):
-            state[ins.no] = (0, frozenset(regs(m.group(2))))
+    counter = "vm" if VMOP.match(text) else "lds" if LDS_OP.match(text) else None
+    if counter is not None:
+        state = {k: (min(v[0] + 1, CAP), v[1]) if k[1] == counter else v for k, v in state.items()}
+        load = asm_load(text) if ins.asm else None
+        if load:
+            state[(ins.no, load[0])] = (0, frozenset(regs(load[1])))
     return state
 
 
@@ -141,7 +159,7 @@ def join(a, b):
 
 
 def check_kernel(path, name, items):
-    if not any(isinstance(it, Ins) and it.asm and LOAD.match(it.text) for it in items):
+    if not any(isinstance(it, Ins) and it.asm and asm_load(it.text) for it in items):
         return []
     errors = []
     for it in items:
@@ -195,7 +213,7 @@ def main():
     for e in errors:
         print(e, file=sys.stderr)
     if errors:
-        print(f"check_asm_loads: {len(errors)} use(s) of registers of loads in flight by the compiler", file=sys.stderr)
+        print(f"check_asm_loads: {len(errors)} use(s) of registers of loads in flight", file=sys.stderr)
         return 1
     print("check_asm_loads: ok")
     return 0
