@@ -216,7 +216,7 @@ TRN_API trn_status trn_q4k_gemm_fused(trn_stream stream, trn_dptr a, trn_dptr b_
  * launches of at most sixteen entries.  What an entry computes does not depend on the company it is launched in: the results are, bit for
  * bit, those of one launch per entry in list order.
  * With trn_set_tuning("batch_mode", 1), and when every entry meets the fast kernels' alignment (x 16 B,
- * W 16 B / 2 B for Q6_K), the list runs as ONE cooperative launch of resident workgroups: the list is cut in
+ * W 16 B / 2 B for Q6_K) and the stream is not hipStreamPerThread (which stands for one per thread), the list runs as ONE cooperative launch of resident workgroups: the list is cut in
  * phases of mutually independent entries with a device-side barrier between phases.  This form keeps, per
  * (device, stream), small device buffers with the list, the work assignment and the barrier counters (allocated on
  * first use, kept until the stream is destroyed); a list identical to the previous one on that stream is not uploaded

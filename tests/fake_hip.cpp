@@ -19,7 +19,7 @@
 namespace {
 struct Launch {
   std::string name;
-  unsigned grid, block;
+  unsigned grid, block, lds;
   uint64_t stream, capture, args[5];
 };
 std::mutex g_lock;
@@ -53,10 +53,11 @@ EXPORT uint64_t fake_memory() {
   return sum;
 }
 EXPORT int fake_launches() { return int(g_launches.size()); }
-EXPORT const char* fake_launch(int i, uint64_t* out) {      // out: grid, block, stream, capture, five arguments
+EXPORT const char* fake_launch(int i, uint64_t* out) {      // out: grid, block, stream, capture, five arguments, LDS
   const Launch& l = g_launches[size_t(i)];
   out[0] = l.grid; out[1] = l.block; out[2] = l.stream; out[3] = l.capture;
   std::copy(l.args, l.args + 5, out + 4);
+  out[9] = l.lds;
   return l.name.c_str();
 }
 // One thread issues a product over and over while another sets `key` to `value` or back to 0.  Of `rounds` changes, how many does the first thread not
@@ -102,7 +103,7 @@ EXPORT hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 EXPORT hipError_t hipDeviceGet(hipDevice_t* d, int) { *d = 0; return hipSuccess; }
 EXPORT hipError_t hipDeviceGetName(char* s, int n, hipDevice_t) { std::strncpy(s, "fake", size_t(n)); return hipSuccess; }
 EXPORT hipError_t hipDeviceTotalMem(size_t* n, hipDevice_t) { *n = size_t(1) << 38; return hipSuccess; }
-EXPORT hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) { *v = a == hipDeviceAttributeMultiprocessorCount ? 256 : 0; return hipSuccess; }
+EXPORT hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) { *v = a == hipDeviceAttributeMultiprocessorCount ? 256 : a == hipDeviceAttributeCooperativeLaunch; return hipSuccess; }
 EXPORT hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
   *p = hipDeviceProp_t{};
   std::strcpy(p->gcnArchName, "gfx950");
@@ -145,7 +146,7 @@ EXPORT hipError_t hipModuleGetFunction(hipFunction_t* f, hipModule_t, const char
   return hipSuccess;
 }
 EXPORT hipError_t hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(int* n, hipFunction_t, int, size_t) { *n = 3; return hipSuccess; }
-EXPORT hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned, unsigned, unsigned, hipStream_t s,
+EXPORT hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned, unsigned, unsigned lds, hipStream_t s,
                                         void** args, void**) {
   const std::string& name = *reinterpret_cast<const std::string*>(f);
   t_last = f;
@@ -153,7 +154,7 @@ EXPORT hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned g
   std::lock_guard<std::mutex> lock(g_lock);
   if (name == g_fail) return hipErrorLaunchFailure;
   if (uint64_t(gx) * bx >= uint64_t(1) << 32) return hipErrorInvalidConfiguration;
-  Launch l{name, gx * gy * gz, bx, reinterpret_cast<uint64_t>(s), 0, {}};
+  Launch l{name, gx * gy * gz, bx, lds, reinterpret_cast<uint64_t>(s), 0, {}};
   auto capture = g_captures.find(l.stream);
   if (capture != g_captures.end()) l.capture = capture->second;
   if (name == "kq_fill_u32") std::memcpy(&l.args[0], args[0], 8);
@@ -161,8 +162,9 @@ EXPORT hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned gx, unsigned g
   g_launches.push_back(l);
   return hipSuccess;
 }
-EXPORT hipError_t hipModuleLaunchCooperativeKernel(hipFunction_t, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, hipStream_t, void**) {
-  return hipErrorNotSupported;
+EXPORT hipError_t hipModuleLaunchCooperativeKernel(hipFunction_t f, unsigned gx, unsigned gy, unsigned gz, unsigned bx, unsigned by, unsigned bz, unsigned lds,
+                                                   hipStream_t s, void** args) {
+  return hipModuleLaunchKernel(f, gx, gy, gz, bx, by, bz, lds, s, args, nullptr);
 }
 EXPORT hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = reinterpret_cast<hipStream_t>(g_next += 4096); return hipSuccess; }
 EXPORT hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }

@@ -7,13 +7,15 @@ import threading
 
 import pytest
 
+from trueno_amd._ffi import GemvDesc
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 A, W, Y = 1 << 32, 1 << 40, 1 << 42
 
 
 class Launch:
     def __init__(self, name, v):
-        self.name, self.grid, self.block, self.stream, self.capture, self.args = name, v[0], v[1], v[2], v[3], list(v[4:9])
+        self.name, self.grid, self.block, self.stream, self.capture, self.args, self.lds = name, v[0], v[1], v[2], v[3], list(v[4:9]), v[9]
 
 
 class Runtime:
@@ -26,6 +28,7 @@ class Runtime:
         lib.trn_gemv_f32.argtypes = [u64, u64, u64, u64, u32, u32]
         for fmt in ("q4k", "q5k", "q6k"):
             getattr(lib, f"trn_{fmt}_gemm").argtypes = [u64, u64, u64, u64, u32, u32, u32]
+        lib.trn_kquant_gemv_batch.argtypes = [u64, C.POINTER(GemvDesc), u32]
         lib.trn_stream_create.argtypes = [C.POINTER(u64), C.c_uint]
         lib.trn_stream_destroy.argtypes = [u64]
 
@@ -37,7 +40,7 @@ class Runtime:
     def launched(self, issue):
         """(status, the launches) of one call."""
         before = self.lib.fake_launches()
-        rc, v, out = issue(), (C.c_uint64 * 9)(), []
+        rc, v, out = issue(), (C.c_uint64 * 10)(), []
         for i in range(before, self.lib.fake_launches()):
             out.append(Launch(self.lib.fake_launch(i, v).decode(), v))
         return rc, out
@@ -47,6 +50,13 @@ class Runtime:
 
     def gemm(self, fmt, stream, m, n, k):
         return self.launched(lambda: getattr(self.lib, f"trn_{fmt}_gemm")(stream, A, W, Y, m, n, k))
+
+    def batch(self, stream, entries):
+        """A list of products with one vector: (format code, k, n, offset of the weights) each."""
+        descs = (GemvDesc * len(entries))()
+        for i, (fmt, k, n, off) in enumerate(entries):
+            descs[i] = GemvDesc(fmt=fmt, k=k, n=n, y=Y + (i << 32), w=W + (i << 34) + off, x=A)
+        return self.launched(lambda: self.lib.trn_kquant_gemv_batch(stream, descs, len(entries)))
 
 
 @pytest.fixture(scope="module")
@@ -82,7 +92,7 @@ def test_threads_have_scratch_of_their_own_behind_the_handle_they_share(rt, n):
         x.start()
     for x in threads:
         x.join()
-    v, seen = (C.c_uint64 * 9)(), set()
+    v, seen = (C.c_uint64 * 10)(), set()
     for i in range(before, rt.lib.fake_launches()):
         if rt.lib.fake_launch(i, v).decode().startswith("gemv_f32"):
             seen.add(v[8])
@@ -178,3 +188,16 @@ def test_f32_products_of_two_thousand_million_columns_are_launched(rt, n, shift)
         n -= 2      # (the aligned form ends at 16384 column tiles)
     rc, (product,) = rt.launched(lambda: rt.lib.trn_gemv_f32(rt.stream(), Y, A + shift, W, 1, n))
     assert rc == 0 and product.grid * product.block >= n and (product.name == "gemv_f32_ragged") == (n <= 0x7FFFFF00)
+
+
+def test_threads_behind_one_handle_do_not_share_the_resident_executor(rt):
+    """Its tables and barrier counters belong to a stream; on hipStreamPerThread the list goes out in launches as with batch_mode 0."""
+    entries, stream = [(4, 4096, 512, 0), (6, 2048, 300, 0)], rt.stream()
+    plain = [x.name for x in rt.batch(stream, entries)[1]]
+    assert rt.lib.trn_set_tuning(b"batch_mode", 1) == 0
+    rc, own = rt.batch(stream, entries)
+    rc2, shared = rt.batch(2, entries)
+    assert rt.lib.trn_set_tuning(b"batch_mode", 0) == 0
+    assert rc == rc2 == 0 and "kq_gemv_phases" in [x.name for x in own]
+    assert [x.name for x in shared] == plain and all(x.stream == 2 for x in shared)
+    rt.lib.trn_stream_destroy(stream)

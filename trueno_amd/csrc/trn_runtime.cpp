@@ -1501,6 +1501,7 @@ hipError_t launch_phases(DeviceKernels* d, ChainWorkspace* ws, hipStream_t strea
 hipError_t launch_chain(hipStream_t stream, const trn_gemv_desc* descs, uint32_t count, bool* handled) {
   *handled = false;
   if (g_tune_batch_mode == 0 || count < 2) return hipSuccess;
+  if (stream == hipStreamPerThread) return hipSuccess;      // one handle for as many streams as there are threads: they would meet at one barrier's counters
   DeviceKernels* d = nullptr;
   hipError_t e = device_kernels(&d);
   if (e != hipSuccess) return e;
