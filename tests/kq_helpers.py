@@ -22,6 +22,16 @@ REF_SLACK = 1.05
 # where the ratios go: a file named by TRN_RATIO_LOG, else one in the temporary directory
 RATIO_LOG = os.environ.get("TRN_RATIO_LOG") or os.path.join(tempfile.gettempdir(), "trueno_ref_order_ratios.jsonl")
 
+# Which kernel the rules take for these is checked without a GPU (test_host_runtime.py), what it computes with one.
+# Q6_K (n, k), opt-in form through LDS: alone, and behind SHORT_ROWS_BESIDE in a list (alone, rows of up to 2048 values have a kernel of
+# their own, and a thousand rows are too few)
+STREAMED_ALONE = [(4096, 4096), (32000, 4096), (4097, 3840)]
+STREAMED_IN_A_LIST = [(1001, 4096), (515, 2048), (129, 1024), (64, 256)]
+SHORT_ROWS_BESIDE = (4096, 4096)
+# (format, m, n, k) that the super-blocks-to-waves kernel takes from the GEMV engine with a pass per token
+FROM_THE_ENGINE = [("q4k", 3, 11014, 1792), ("q4k", 4, 4509, 2304), ("q4k", 8, 1191, 2560), ("q4k", 2, 14828, 1792), ("q5k", 5, 2595, 2048), ("q5k", 8, 868, 1024),
+                   ("q5k", 3, 7487, 1536)]
+
 
 def record_ratio(kind: str, fmt: str, m: int, n: int, k: int, rows: int, ours: float, ref: float) -> None:
     """one line per measured shape: our relative L2 error against fp64 over the reference-order f32 evaluation's"""

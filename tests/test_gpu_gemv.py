@@ -8,7 +8,7 @@ import pytest
 import trueno_amd as t
 from oracle import kquant as kq
 from trueno_amd import _ffi
-from tests.kq_helpers import REF_SLACK, gpu_gemv, record_ratio
+from tests.kq_helpers import REF_SLACK, SHORT_ROWS_BESIDE, STREAMED_ALONE, STREAMED_IN_A_LIST, gpu_gemv, record_ratio
 
 pytestmark = pytest.mark.gpu
 
@@ -139,22 +139,39 @@ def test_gemv_linearity_full_size(gpu):
     assert kq.rel_l2(y12, 2.0 * y1 - 0.5 * y2) <= 5e-6
 
 
-@pytest.mark.parametrize("n,k", [(4096, 4096), (32000, 4096), (515, 2048), (129, 1024), (64, 256), (1001, 4096), (2, 4096),
-                                 (4097, 3840)])
+@pytest.mark.parametrize("n,k", STREAMED_ALONE + STREAMED_IN_A_LIST + [(2, 4096)])
 def test_q6k_streamed_through_lds_gives_the_bits_of_the_register_form(gpu, n, k):
     """Q6_K rows streamed through LDS (opt-in: "gemv_stream_q6k") lie there with their 210-byte blocks re-spaced to 224;
     the arithmetic is the register form's, so every bit must be.  Weights at several alignments (a block may start at any
-    even address), ragged row counts (the last batch of a matrix starts early), short rows (fewer pieces than a slot)."""
+    even address), ragged row counts (the last batch of a matrix starts early), short rows in a list (fewer pieces than a slot).
+    That these shapes stream is checked in test_host_runtime.py; (2, 4096), too few rows for it, has to be right all the same."""
+    ctx, stream = gpu
     tune = lambda key, v: _ffi.lib().trn_set_tuning(key.encode(), int(v))
     buf, x = kq.gen_matrix("q6k", 100 + n, n, k), kq.gen_x(7, k)
+
+    def in_a_list(w_off):
+        rows, cols = SHORT_ROWS_BESIDE
+        dw, dx = t.GpuBuffer(ctx, buf.size + w_off, np.uint8), t.GpuBuffer.from_host(ctx, x)
+        dw.copy_from_host_at(np.ascontiguousarray(buf, np.uint8).reshape(-1), w_off)
+        other = [t.GpuBuffer.from_host(ctx, np.zeros(rows * cols // 256 * 144, np.uint8)), t.GpuBuffer.from_host(ctx, np.ones(cols, np.float32))]
+        ys = [t.GpuBuffer.from_host(ctx, np.full(r, np.nan, np.float32)) for r in (rows, n)]
+        batch = t.GemvBatch()
+        batch.add("q4k", cols, rows, ys[0], *other, 0)
+        batch.add("q6k", k, n, ys[1], dw.as_ptr() + w_off, dx, 0)
+        batch.launch(stream)
+        stream.synchronize()
+        assert not np.any(ys[0].copy_to_host())
+        return ys[1].copy_to_host()
+
+    streamed = in_a_list if (n, k) in STREAMED_IN_A_LIST else lambda w_off: gpu_gemv(gpu, "q6k", buf, x, k, n, w_offset=w_off)
     for w_off in (0, 2, 6):
         a = gpu_gemv(gpu, "q6k", buf, x, k, n, w_offset=w_off)
-        assert tune("gemv_stream_q6k", 1) == 0 and tune("gemv_stream_min_rows", 1) == 0
+        assert all(tune(key, 1) == 0 for key in ("gemv_stream_q6k", "gemv_stream_min_rows", "group_stream_min_rows"))
         try:
-            b = gpu_gemv(gpu, "q6k", buf, x, k, n, w_offset=w_off)
+            b = streamed(w_off)
         finally:
-            tune("gemv_stream_q6k", 0)
-            tune("gemv_stream_min_rows", 0)
+            for key in ("gemv_stream_q6k", "gemv_stream_min_rows", "group_stream_min_rows"):
+                tune(key, 0)
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (n, k, w_off)
 
 

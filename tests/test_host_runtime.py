@@ -7,6 +7,7 @@ import threading
 
 import pytest
 
+from tests.kq_helpers import FROM_THE_ENGINE, SHORT_ROWS_BESIDE, STREAMED_ALONE, STREAMED_IN_A_LIST
 from trueno_amd._ffi import GemvDesc
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -25,6 +26,7 @@ class Runtime:
         lib.fake_launch.restype, lib.fake_memory.restype = C.c_char_p, u64
         lib.fake_capture.argtypes = [u64, C.c_ulonglong]
         lib.fake_tuning_race.argtypes = [C.c_char_p, C.c_int, u32, u32, u32, C.c_int]
+        lib.trn_q6k_gemv.argtypes = [u64, u64, u64, u64, u32, u32]
         lib.trn_gemv_f32.argtypes = [u64, u64, u64, u64, u32, u32]
         for fmt in ("q4k", "q5k", "q6k"):
             getattr(lib, f"trn_{fmt}_gemm").argtypes = [u64, u64, u64, u64, u32, u32, u32]
@@ -201,3 +203,37 @@ def test_threads_behind_one_handle_do_not_share_the_resident_executor(rt):
     assert rc == rc2 == 0 and "kq_gemv_phases" in [x.name for x in own]
     assert [x.name for x in shared] == plain and all(x.stream == 2 for x in shared)
     rt.lib.trn_stream_destroy(stream)
+
+
+@pytest.mark.parametrize("off", (0, 2, 6))
+@pytest.mark.parametrize("n,k", STREAMED_ALONE + STREAMED_IN_A_LIST)
+def test_the_shapes_tested_as_streamed_are(rt, n, k, off):
+    """By the rings in LDS, which are larger with Q6_K's rows than with those of the Q4_K entry beside it; alone by the kernel's name as well."""
+    if (n, k) in STREAMED_ALONE:
+        issue = lambda: rt.launched(lambda: rt.lib.trn_q6k_gemv(0, Y, W + off, A, k, n))
+    else:
+        rows, cols = SHORT_ROWS_BESIDE
+        issue = lambda: rt.batch(0, [(4, cols, rows, 0), (6, k, n, off)])
+    seen = []
+    try:
+        for on in (0, 1):
+            for key, value in ((b"gemv_stream_q6k", on), (b"gemv_stream_min_rows", 1), (b"group_stream_min_rows", 1)):
+                assert rt.lib.trn_set_tuning(key, value) == 0
+            rc, launches = issue()
+            assert rc == 0 and len(launches) == 1
+            seen.append(launches[0])
+    finally:
+        for key in (b"gemv_stream_q6k", b"gemv_stream_min_rows", b"group_stream_min_rows"):
+            rt.lib.trn_set_tuning(key, 0)
+    listed = (n, k) in STREAMED_IN_A_LIST or n == 32000      # (a large matrix alone is a list of one)
+    assert [x.name for x in seen] == (["kq_gemv_group"] * 2 if listed else ["q6k_gemv_warp_reduce", "q6k_gemv_flags"])
+    assert seen[1].lds > seen[0].lds
+
+
+@pytest.mark.parametrize("fmt,m,n,k", FROM_THE_ENGINE)
+def test_products_taken_from_the_engine(rt, fmt, m, n, k):
+    rc, (product,) = rt.gemm(fmt, 0, m, n, k)
+    assert rt.lib.trn_set_tuning(b"gemm_slices", 1) == 0
+    rc2, (other,) = rt.gemm(fmt, 0, m, n, k)
+    assert rt.lib.trn_set_tuning(b"gemm_slices", 0) == 0
+    assert rc == rc2 == 0 and product.name.startswith(f"{fmt}_gemm_slices") and other.name == f"{fmt}_gemm_ggml"
