@@ -134,8 +134,12 @@ def test_gpu_attention_heads_of_a_kv_head_together(gpu, heads, kv_heads, max_seq
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,dim,max_seq,seq", [
     (1, 1, 256, 20, 17), (8, 1, 256, 700, 641), (6, 3, 256, 2100, 2049), (24, 2, 256, 130, 127),       # 256 dims: two pairs of (head, quad) a thread, one
-    (1, 1, 128, 5000, 4993), (2, 1, 64, 9000, 8500), (8, 2, 128, 9000, 8200), (8, 1, 128, 5000, 4999),  # 79, 133, 129 and 79 chunks: 16, 8, 4 and 2 slices
+    (1, 1, 128, 5000, 4993), (2, 1, 64, 9000, 8500), (2, 1, 128, 5000, 4993),                          # 79, 67 and 79 chunks: 16, 16 and 8 slices
+    (8, 2, 128, 9000, 8200), (8, 1, 128, 5000, 4999), (8, 1, 128, 4000, 3800),                         # 65, 40 and 60 chunks: 4, 2 and 2 slices
+    (8, 2, 64, 130, 128), (8, 2, 64, 130, 129), (3, 3, 128, 140, 127), (8, 2, 128, 130, 97),           # one chunk of 128 positions, three of 64
+    (64, 8, 128, 1600, 1500), (24, 8, 128, 1600, 1451), (12, 4, 128, 900, 833),                         # 12 chunks of 128 positions twice (eight heads, three), 14 of 64
     (4, 4, 128, 1100, 1025), (4, 4, 128, 1100, 1024),                                                  # 17 chunks and 16
+    (4, 4, 128, 32800, 32769),                                                                         # 57 chunks of 576 positions: eight waves
     (128, 128, 128, 905, 897), (128, 128, 128, 905, 896)])                                             # four waves a workgroup and eight
 def test_gpu_attention_tiles_through_lds(gpu, heads, kv_heads, dim, max_seq, seq):
     """The edges of the tiled form: the last tile of a chunk, how the chunks are joined, the number of waves; what lies behind

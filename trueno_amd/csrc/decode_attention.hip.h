@@ -177,9 +177,9 @@ __device__ __forceinline__ void body(const float* __restrict__ q, const float* _
 // Rounding: a score is added up in a tree over sums of four products, a tile's share of the output starts at zero (eight
 // products in a row), waves and chunks meet in trees.  Against fp64, averages over 16 inputs: 0.88 .. 0.99 of the kernel's
 // above with a head alone, 128 dims, 64 .. 3000 positions; 0.80 .. 0.86 with 256 dims and two heads.
-// Bound by HBM with many positions, by latency with few.  A launch of 17 us (8 KV heads, 8192 positions, 67 MB) spends 1 before
-// the first copies are out (a CU has 64 KB in flight, no more), 11 on the stream, 1 on the last tile, 4 at the end: the store
-// of a chunk's state has to be acknowledged, the counter answers, the states come back.
+// Bound: a launch's time is a fixed part and the bytes at the memory's own rate, 128 dims, caches out of the last level: 32 heads over 8 9.1 us + bytes / 7.05
+// TB/s (4096 .. 32768 positions), 32 heads of their own 6.2-7.4 + bytes / 6.9-7.05.  The fixed part is the start (1 us before the first copies are out), the last tile
+// and, with several chunks, their sum: the store of a chunk's state has to be acknowledged, the counter answers, the states come back.
 // Measured (us, before -> now: before is the kernel above, or for 64 dims, several heads and from 4096 positions on one that
 // kept K and V in registers, four waves a CU; 128 dims unless said): 32 heads over 8, 8192 positions 19.0 -> 17.1; 32 heads of their
 // own, 2048 positions 16.65 -> 15.2, 1024 12.3 -> 10.7, 512 9.0 -> 8.2; four heads, 16000 positions 21.5 -> 16.9; 128 heads over 32,
@@ -431,73 +431,73 @@ __device__ __forceinline__ void tiled_body(const float* __restrict__ q, const fl
   }
   __syncthreads();
   if (s_old != chunks - 1u) return;
-  // The last workgroup: runs of chunks by as many slices of its threads as there are, then the slices in order.
-  // (Up to sixteen chunks are joined in one tree: scaled once, as the waves' states are.)
+  // The last workgroup joins the chunks [c0, c1) of a pair, N of them in flight together and scaled once, as the waves' states are
+  auto join = [&](u32 pair, u32 c0, u32 c1, auto n_c) {
+    constexpr u32 N = decltype(n_c)::value;
+    const u32 hd = pair / Q, quad = pair - hd * Q;
+    State tot = {-INFINITY, 0.0f, zero4};
+    for (; c0 < c1; c0 += N) {
+      u32x4 ms[N], ov[N];
+#pragma unroll
+      for (u32 cc = 0; cc < N; ++cc) {
+        const u32 at = slot(min(c0 + cc, c1 - 1u), hd);
+        ms[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + Q * 16u), 0, 16);
+        ov[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + quad * 16u), 0, 16);
+      }
+      float cm[N], cs[N];
+      f32x4 co[N];
+#pragma unroll
+      for (u32 cc = 0; cc < N; ++cc) {
+        const bool there = c0 + cc < c1;
+        cm[cc] = there ? __uint_as_float(ms[cc].x) : -INFINITY;
+        cs[cc] = there ? __uint_as_float(ms[cc].y) : 0.0f;
+        co[cc] = there ? __builtin_bit_cast(f32x4, ov[cc]) : zero4;
+      }
+      const State r = merge_tree<N>(cm, cs, co);
+      merge(tot, r.m, r.s, r.o);
+    }
+    return tot;
+  };
+  auto finish = [&](u32 pair, const State& tot) {
+    const float inv = 1.0f / tot.s;
+    dst[pair] = tot.o * inv;
+  };
+  // Up to sixteen chunks in one tree.  More: as many slices of the workgroup's threads as there are take runs of chunks, eight in flight, and the slices
+  // meet in LDS.  (The way without slices in code of its own: through the other it took 0.3 us longer at every length - 32 heads over 8, 900
+  // positions 8.1 and 7.8 us.  Slices of sixteen in flight: 8 heads over one, 6000 positions 13.5 us, of eight 12.0.)
   constexpr u32 kMostSlices = 16;
   u32 slices = 1u;
   while (chunks > 16u && slices < kMostSlices && 2u * slices * pairs <= kThreads && slices * 8u < chunks) slices *= 2u;
-  const u32 per_slice = (chunks + slices - 1u) / slices;
-  for (u32 i0 = 0; i0 < pairs; i0 += kThreads) {
-    const u32 i = i0 + threadIdx.x, slice = i0 == 0u && slices > 1u ? threadIdx.x / pairs : 0u, pair = i - slice * pairs;
-    const bool mine = slice < slices && pair < pairs;
-    State tot = {-INFINITY, 0.0f, zero4};
-    if (mine) {
-      const u32 hd = pair / Q, quad = pair - hd * Q, c1 = min(chunks, (slice + 1u) * per_slice);
-      auto join = [&](auto n_c) {      // chunks in flight together
-        constexpr u32 N = decltype(n_c)::value;
-        for (u32 c0 = slice * per_slice; c0 < c1; c0 += N) {
-          u32x4 ms[N], ov[N];
-#pragma unroll
-          for (u32 cc = 0; cc < N; ++cc) {
-            const u32 at = slot(min(c0 + cc, c1 - 1u), hd);
-            ms[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + Q * 16u), 0, 16);
-            ov[cc] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(at + quad * 16u), 0, 16);
-          }
-          float cm[N], cs[N];
-          f32x4 co[N];
-#pragma unroll
-          for (u32 cc = 0; cc < N; ++cc) {
-            const bool there = c0 + cc < c1;
-            cm[cc] = there ? __uint_as_float(ms[cc].x) : -INFINITY;
-            cs[cc] = there ? __uint_as_float(ms[cc].y) : 0.0f;
-            co[cc] = there ? __builtin_bit_cast(f32x4, ov[cc]) : zero4;
-          }
-          const State r = merge_tree<N>(cm, cs, co);
-          merge(tot, r.m, r.s, r.o);
-        }
-      };
-      if (per_slice <= 8u) join(std::integral_constant<u32, 8>{});
-      else join(std::integral_constant<u32, 16>{});
-    }
-    if (slices > 1u) {      // (pairs <= kThreads / 2 then: this loop's only round, and every thread is here)
-      f32x2* s_ms = reinterpret_cast<f32x2*>(s_o + kThreads);
-      s_o[threadIdx.x] = tot.o;
-      s_ms[threadIdx.x] = f32x2{tot.m, tot.s};
-      __syncthreads();
-      if (threadIdx.x >= pairs) return;
-      auto join_slices = [&](auto n_c) {
-        constexpr u32 N = decltype(n_c)::value;
-        float jm[N], js[N];
-        f32x4 jo[N];
-#pragma unroll
-        for (u32 n = 0; n < N; ++n) {
-          const f32x2 ms = s_ms[n * pairs + threadIdx.x];
-          jm[n] = ms.x;
-          js[n] = ms.y;
-          jo[n] = s_o[n * pairs + threadIdx.x];
-        }
-        tot = merge_tree<N>(jm, js, jo);
-      };
-      if (slices == 2u) join_slices(std::integral_constant<u32, 2>{});
-      else if (slices == 4u) join_slices(std::integral_constant<u32, 4>{});
-      else if (slices == 8u) join_slices(std::integral_constant<u32, 8>{});
-      else join_slices(std::integral_constant<u32, kMostSlices>{});
-    }
-    if (mine) {
-      const float inv = 1.0f / tot.s;
-      dst[pair] = tot.o * inv;
-    }
+  if (slices == 1u) {
+    for (u32 i = threadIdx.x; i < pairs; i += kThreads)
+      finish(i, chunks <= 8u ? join(i, 0u, chunks, std::integral_constant<u32, 8>{}) : join(i, 0u, chunks, std::integral_constant<u32, 16>{}));
+    return;
   }
+  const u32 per_slice = (chunks + slices - 1u) / slices, slice = threadIdx.x / pairs;
+  State tot = {-INFINITY, 0.0f, zero4};
+  if (slice < slices) tot = join(threadIdx.x - slice * pairs, slice * per_slice, min(chunks, (slice + 1u) * per_slice), std::integral_constant<u32, 8>{});
+  f32x2* s_ms = reinterpret_cast<f32x2*>(s_o + kThreads);
+  s_o[threadIdx.x] = tot.o;
+  s_ms[threadIdx.x] = f32x2{tot.m, tot.s};
+  __syncthreads();
+  if (threadIdx.x >= pairs) return;
+  auto join_slices = [&](auto n_c) {
+    constexpr u32 N = decltype(n_c)::value;
+    float jm[N], js[N];
+    f32x4 jo[N];
+#pragma unroll
+    for (u32 n = 0; n < N; ++n) {
+      const f32x2 ms = s_ms[n * pairs + threadIdx.x];
+      jm[n] = ms.x;
+      js[n] = ms.y;
+      jo[n] = s_o[n * pairs + threadIdx.x];
+    }
+    finish(threadIdx.x, merge_tree<N>(jm, js, jo));
+  };
+  if (slices == 2u) join_slices(std::integral_constant<u32, 2>{});
+  else if (slices == 4u) join_slices(std::integral_constant<u32, 4>{});
+  else if (slices == 8u) join_slices(std::integral_constant<u32, 8>{});
+  else join_slices(std::integral_constant<u32, kMostSlices>{});
 }
 
 }  // namespace decode_attention
