@@ -30,6 +30,7 @@ class Runtime:
         lib.trn_gemv_f32.argtypes = [u64, u64, u64, u64, u32, u32]
         for fmt in ("q4k", "q5k", "q6k"):
             getattr(lib, f"trn_{fmt}_gemm").argtypes = [u64, u64, u64, u64, u32, u32, u32]
+        lib.trn_incremental_attention.argtypes = [u64] * 5 + [u32] * 5 + [C.c_float]
         lib.trn_kquant_gemv_batch.argtypes = [u64, C.POINTER(GemvDesc), u32]
         lib.trn_stream_create.argtypes = [C.POINTER(u64), C.c_uint]
         lib.trn_stream_destroy.argtypes = [u64]
@@ -237,3 +238,11 @@ def test_products_taken_from_the_engine(rt, fmt, m, n, k):
     rc2, (other,) = rt.gemm(fmt, 0, m, n, k)
     assert rt.lib.trn_set_tuning(b"gemm_slices", 0) == 0
     assert rc == rc2 == 0 and product.name.startswith(f"{fmt}_gemm_slices") and other.name == f"{fmt}_gemm_ggml"
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,seq,kernel,workgroups", [
+    (32, 32, 128, 4096, "kq_attention_tiled_128_w4", 256), (32, 32, 128, 3584, "kq_attention_tiled_128", 256), (32, 8, 128, 16000, "kq_attention_tiled_128", 256)])
+def test_the_attention_kernels_and_their_cut(rt, heads, kv_heads, dim, seq, kernel, workgroups):
+    """The lines of the rule, one position on either side: four waves."""
+    rc, launches = rt.launched(lambda: rt.lib.trn_incremental_attention(0, A, W, W << 1, Y, seq, dim, heads, kv_heads, seq, 0.1))
+    assert rc == 0 and launches[-1].name == kernel and (workgroups == 0 or launches[-1].grid == workgroups)

@@ -184,9 +184,8 @@ __device__ __forceinline__ void body(const float* __restrict__ q, const float* _
 // kept K and V in registers, four waves a CU; 128 dims unless said): 32 heads over 8, 8192 positions 19.0 -> 17.1; 32 heads of their
 // own, 2048 positions 16.65 -> 15.2, 1024 12.3 -> 10.7, 512 9.0 -> 8.2; four heads, 16000 positions 21.5 -> 16.9; 128 heads over 32,
 // 16384 positions 84.0 -> 81.9 (6.6 TB/s); 256 dims, 64 heads over 16, 8000 positions 99.7 -> 52.
-// Waves: eight; with 128 dims four where a wave of eight would still have more than four tiles, that is more than 512 positions a
-// workgroup (128 heads over 32, 16384 positions: 85.7 with eight, 80.5-81.9 with four: fewer streams at a time; 32 over 8, 8192
-// positions: 17.0 and 17.8).  256 dims: four, an LDS tile is 32 KB.
+// Waves: eight; with 128 dims four where a workgroup has 512 positions or more, four tiles for a wave of eight, and a KV head at most eight workgroups
+// (both sides at the runtime's kAttentionFourWaves: fewer streams at a time, but half the threads to join the chunks).  256 dims: four, an LDS tile is 32 KB.
 constexpr u32 kTiledHeads = 8;
 template <int DIM, int W> struct Tiled {
   static constexpr u32 HALF = 64u * DIM;               // bytes of a wave's tile: 16 positions of K, then of V

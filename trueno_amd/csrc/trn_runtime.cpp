@@ -573,7 +573,10 @@ hipError_t launch_gemv_f32(hipStream_t stream, uint64_t y, uint64_t a, uint64_t 
 // Single-query attention over the KV cache (decode_attention.hip.h).  Per (device, stream): arrival counters per
 // head and the chunks' partial softmax states.
 ScratchMap g_attention_ws;
-constexpr uint32_t kAttentionFourWaves = 512;      // positions of a workgroup from which four waves a workgroup are faster (decode_attention.hip.h)
+// Positions of a workgroup from which it has four waves, where a KV head has few workgroups (decode_attention.hip.h).  Both sides, four waves -> eight:
+// 32 KV heads, 8 chunks, 8192 positions 44.3 -> 46.2 us; 16, 16 chunks, 8192 and 16000 positions 26.1 -> 26.7 and 49.4 -> 46.5; 32 heads over 8, 32 chunks,
+// 16000 positions 28.2 -> 26.9; over 4, 64 chunks, 32000 35.9 -> 31.7.
+constexpr uint32_t kAttentionFourWaves = 512, kAttentionFourWavesChunks = 8;
 
 constexpr size_t kAttentionCounterBytes = 64u * 1024u;
 // What a stream's buffer is made for: the most that a workgroup per CU can publish, eight heads of 256 dims.
@@ -616,7 +619,7 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
       if ((e = acquire_scratch(g_attention_ws, d, stream, need, kAttentionCounterBytes, &cnt, attention_scratch(*d))) != hipSuccess) return e;   // the kernel leaves the counters at zero
       uint64_t part = cnt + kAttentionCounterBytes;
       void* args[] = {&q, &k, &v, &out, &seq_len, &per_kv, &subs, &max_seq_len, &scale, &chunk, &chunks, &groups, &part, &cnt};
-      const int which = head_dim == 64u ? 0 : head_dim == 256u ? 2 : chunk >= kAttentionFourWaves ? 3 : 1;
+      const int which = head_dim == 64u ? 0 : head_dim == 256u ? 2 : chunk >= kAttentionFourWaves && chunks <= kAttentionFourWavesChunks ? 3 : 1;
       return hipModuleLaunchKernel(d->attention_tiled[which], groups * chunks, 1, 1, which >= 2 ? 256u : 512u, 1, 1, 0, stream, args, nullptr);
     }
   }
