@@ -241,8 +241,15 @@ def test_products_taken_from_the_engine(rt, fmt, m, n, k):
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,seq,kernel,workgroups", [
+    (8, 8, 128, 128, "kq_attention_tiled_128", 8), (8, 8, 128, 129, "kq_attention_tiled_128", 24), (8, 8, 128, 512, "kq_attention_tiled_128", 64),
+    (8, 8, 128, 513, "incremental_attention", 0), (1, 1, 128, 767, "incremental_attention", 0), (1, 1, 128, 768, "kq_attention_tiled_128", 12),
+    (9, 9, 128, 513, "kq_attention_tiled_128", 81), (8, 4, 128, 513, "kq_attention_tiled_128", 36),
+    (16, 16, 64, 128, "kq_attention_tiled_64", 16), (16, 16, 64, 129, "kq_attention_tiled_64", 48),
+    (64, 8, 128, 1280, "kq_attention_tiled_128", 160), (64, 8, 128, 1281, "kq_attention_tiled_128", 88), (16, 16, 128, 1024, "kq_attention_tiled_128", 256),
+    (8, 1, 128, 3840, "kq_attention_tiled_128", 60), (8, 1, 128, 3841, "kq_attention_tiled_128", 31), (1, 1, 128, 3841, "kq_attention_tiled_128", 61),
     (32, 32, 128, 4096, "kq_attention_tiled_128_w4", 256), (32, 32, 128, 3584, "kq_attention_tiled_128", 256), (32, 8, 128, 16000, "kq_attention_tiled_128", 256)])
 def test_the_attention_kernels_and_their_cut(rt, heads, kv_heads, dim, seq, kernel, workgroups):
-    """The lines of the rule, one position on either side: four waves."""
+    """The lines of the rule, one position on either side: heads alone, one chunk of 128 positions, chunks of 128 instead of 64, four
+    waves."""
     rc, launches = rt.launched(lambda: rt.lib.trn_incremental_attention(0, A, W, W << 1, Y, seq, dim, heads, kv_heads, seq, 0.1))
     assert rc == 0 and launches[-1].name == kernel and (workgroups == 0 or launches[-1].grid == workgroups)

@@ -593,26 +593,32 @@ hipError_t launch_attention(hipStream_t stream, uint64_t q, uint64_t k, uint64_t
   hipError_t e = device_kernels(&d);
   if (e != hipSuccess) return e;
   // The query heads of a KV head together, in tiles of 16 positions (decode_attention.hip.h), a workgroup per CU (two are
-  // slower at every length).  With 64 and 128 dims always: faster than the other kernel, or within the scatter, at every length and
-  // head count measured (64 .. 16384 positions).  256 dims: several query heads from 32 positions a CU on (16 heads over 8: 300 positions
+  // slower at every length).  64 dims always; 128 dims too (32 heads over 8, 420 positions 6.7 us, with the other kernel 8.6, 8192 17.0 and 31.2; 32 alone, 160 6.50
+  // and 6.82; but 8 over one, 420 and 640 7.0 and 7.9, with the other 6.7 and 7.2), except for up to eight heads alone with 513 .. 767 positions, where nine to
+  // twelve chunks would be joined (8 heads, 640: 7.36, with the other kernel 7.20; 512: 6.56 and 6.93; 768: 7.53 and 7.50; 12 heads, 640: 7.78 and 7.75).  256 dims: several query heads from 32 positions a CU on (16 heads over 8: 300 positions
   // 8.5 us with the other kernel, 10.2 with this one; 3000 positions 21.6 and 18.9; 32 over 16, 700 positions 13.1 and 12.5); a head alone only
   // where there are few and they are long (8 heads, 8000 positions: 32.0 and 31.2; 4, 16000: 38.7 and 34.7; but 32, 8000: 82.5 and 88.2 -
   // one wave a SIMD, fifteen columns of sixteen empty).
   uint32_t per_kv = num_heads / num_kv_heads, subs = (per_kv + 7u) / 8u;
   const uint64_t cus = uint64_t(d->cu_count), positions = uint64_t(num_kv_heads) * subs * seq_len;
-  bool tiled = head_dim == 64u || head_dim == 128u ||
+  const bool few_alone = per_kv == 1u && num_heads <= 8u && seq_len > 512u && seq_len < 768u;
+  bool tiled = head_dim == 64u || (head_dim == 128u && !few_alone) ||
                (head_dim == 256u && (per_kv > 1u ? positions >= 32u * cus : num_heads <= 8u && positions >= 192u * cus));
   if (g_tune_attention_tiled == 2) tiled = head_dim == 64u || head_dim == 128u || head_dim == 256u;
   if (tiled && num_heads % num_kv_heads == 0u && g_tune_attention_tiled != 1) {
     const uint32_t most_heads = 8u, per_cu = g_tune_attention_per_cu > 0 ? uint32_t(g_tune_attention_per_cu) : 1u;
     uint32_t groups = num_kv_heads * subs, most = std::max(1u, per_cu * uint32_t(d->cu_count) / groups), chunk = 0, chunks = 0;
-    // at least four tiles a workgroup (fewer make more chunks than they save: 32 heads over 8, 700 positions 9.3 us with two, 7.9 with
-    // four, 8.6 with eight); with 64 dims eight if more than eight chunks would have to be joined (700 positions, 16 KV heads 7.4 and 6.9)
-    for (uint32_t step = 64u;; step *= 2u) {
+    auto cut = [&](uint32_t step) {
       chunk = ((seq_len + most - 1u) / most + step - 1u) / step * step;
       chunks = (seq_len + chunk - 1u) / chunk;
-      if (head_dim != 64u || step > 64u || chunks <= 8u) break;
-    }
+    };
+    // At least four tiles a workgroup (fewer make more chunks than they save: 32 heads over 8, 700 positions 9.3 us with two, 7.9 with
+    // four, 8.6 with eight).  Eight, one for each of its waves, where that leaves nothing to join (up to 128 positions: 32 heads, 96 positions 6.55 -> 5.80 us, 64
+    // dims, 16 heads 5.37 -> 4.74); with 64 dims where more than eight chunks would have to be joined (700 positions, 16 KV heads 7.4 and 6.9); with 128, heads that
+    // share a KV head and more than 160 workgroups (64 heads over 8, 1500 positions, 192: 11.2 -> 10.5, but 1030, 136: 9.6 and 10.0; 16 over 4, 3000, 188: 10.7
+    // -> 10.2, but 2048, 128: 8.8 and 9.2) or 60 chunks (8 over one, 4100: 11.7 -> 11.4, 6000: 13.7 -> 11.9, but 3000: 10.1 and 10.8).
+    cut(head_dim != 256u && seq_len <= 128u ? 128u : 64u);
+    if (head_dim == 64u ? chunks > 8u : head_dim == 128u && chunk == 64u && per_kv > 1u && (groups * chunks > 160u || chunks > 60u)) cut(128u);
     if (uint64_t(chunk) * head_dim * 4u < (uint64_t(1) << 31)) {      // (the kernel's offsets into a chunk)
       const size_t need = kAttentionCounterBytes + (chunks > 1u ? size_t(groups) * chunks * most_heads * (head_dim / 4u + 1u) * 16u : 0u);
       uint64_t cnt = 0;
