@@ -175,10 +175,10 @@ __device__ __forceinline__ void body(const float* __restrict__ q, const float* _
 // to two halves of a tile on their way while it computes, no register holds a load in flight, and two waves a SIMD fit
 // (with K and V in registers they did not: 24 us where four waves took 18.7).
 // Rounding: a score is added up in a tree over sums of four products, a tile's share of the output starts at zero (eight
-// products in a row), waves and chunks meet in trees.  Against fp64, averages over 16 inputs: 0.88 .. 0.99 of the kernel's
-// above with a head alone, 128 dims, 64 .. 3000 positions; 0.80 .. 0.86 with 256 dims and two heads.
-// Bound: a launch's time is a fixed part and the bytes at the memory's own rate, 128 dims, caches out of the last level: 32 heads over 8 9.1 us + bytes / 7.05
-// TB/s (4096 .. 32768 positions), 32 heads of their own 6.2-7.4 + bytes / 6.9-7.05.  The fixed part is the start (1 us before the first copies are out), the last tile
+// products in a row), waves and chunks meet in trees.  Against fp64, averages over 16 inputs, 64, 128 and 256 dims, heads alone and
+// in pairs and fours: 0.94 .. 1.02 of the kernel's above with 64 and 256 positions (single inputs scatter by 10-20 %), 0.72 .. 0.95 with 1024 and 2048, 0.71 .. 0.84 with 8192.
+// Bound: a launch's time is a fixed part and the bytes at the memory's own rate, 128 dims, caches out of the last level: 32 heads over 8 8-9 us + bytes / 6.8-7.05
+// TB/s (4096 .. 32768 positions), 32 heads of their own 6.2-7.6 + bytes / 6.9-7.2.  The fixed part is the start (1 us before the first copies are out), the last tile
 // and, with several chunks, their sum: the store of a chunk's state has to be acknowledged, the counter answers, the states come back.
 // Measured (us, before -> now: before is the kernel above, or for 64 dims, several heads and from 4096 positions on one that
 // kept K and V in registers, four waves a CU; 128 dims unless said): 32 heads over 8, 8192 positions 19.0 -> 17.1; 32 heads of their

@@ -3,8 +3,9 @@
 // with the operands of kquant_gemm_f16.hip.h.  There a workgroup's waves share one super-block's token operands and meet at a barrier for every
 // super-block, and a matrix of 4096 columns is cut in parts that meet through memory: 5 us to the first barrier, 1.5-2 a super-block, 3.5 for the sum.
 //   * Here a workgroup of eight waves takes 16 RT rows of W against 16 tokens, and each wave whole super-blocks of all those rows: wave w the super-blocks
-//     w, w + 8, ...: no wave waits for another until the end, where the eight sums meet in LDS.  With 256 CUs and 16 to 64 rows a workgroup K
-//     is mostly one part.
+//     w, w + 8, ...: no wave waits for another until the end, where the eight sums meet in LDS.  Half of the products that come here keep K in one
+//     part (1508 of 3111 drawn); in the others the parts meet through memory as there: 4096 x 14336 and 4096 x 4096 with 16 tokens take four, 14 super-blocks
+//     of the former's for eight waves, so that two have one and six have two.
 //   * A wave's activations go to registers in whole lines (with a token's row a lane, sixteen rows 4 K bytes apart, a load instruction took 70
 //     cycles: the rows share an L2 channel), are turned in 8 KB of LDS so that a lane holds 64 values of one token, and become the two f16 pieces there; the
 //     next super-block's are asked for before that.  Weights come by copies into LDS, two super-blocks ahead where it holds them (RT <= 2).
@@ -14,10 +15,12 @@
 //     SIMD's issue from them) and by latency: a launch of 14336 x 4096, 16 tokens, has its first activations at 1.3 us, the first products at 3 to 6.5,
 //     two super-blocks a wave done at 12.
 //   * Rounding: as there, hi and lo pieces' sums apart; a wave sums few super-blocks, the waves meet in a tree.  Error against fp64 0.95-0.98 of that
-//     kernel's over drawn products.
-//   * Measured (us, 16 tokens, that kernel -> this one): Q4_K 14336 x 4096 15.4 -> 14.7, 4096 x 14336 18.4 -> 16.3, 4096 x 4096 9.9 -> 8.7, 11008 x 4096 14.2 ->
+//     kernel's over drawn products, 0.57-0.92 of the GEMV engine's (f32 activations) over 150 of two to eight tokens that the engine had.
+//   * Measured (us, 16 tokens, that kernel -> this one): Q4_K 14336 x 4096 15.4 -> 14.7, 4096 x 14336 18.4 -> 16.3-17.0, 4096 x 4096 9.9 -> 8.7, 11008 x 4096 14.2 ->
 //     13.0; Q5_K 11008 x 4096 16.6 -> 14.9; 3 tokens, Q4_K 12000 x 1024 13.8 -> 5.4 (the integer cores); Q6_K 32000 x 4096 keeps the other (41 against 48).
-// (v_mfma_f32_16x16x16_f16, half as long, gave wrong rows in one build where its result lay over its first operand; not used.)
+//   * q5k_gemm_slices_r1 spills 13 registers and reads them back inside the loop; its times, and so the estimate that chooses it (one product in eight of
+//     Q5_K), include that.
+// (v_mfma_f32_16x16x16_f16, half as long, gave wrong rows in one build where its result lay over its first operand; the cause was not found, and it is not used.)
 #pragma once
 #include "kquant_gemm_f16.hip.h"
 

@@ -9,8 +9,11 @@
 //   * What bounds it: beside other waves' vector instructions a matrix instruction takes half its cycles of a SIMD's issue and a vector
 //     instruction four and a half (measured with one wave of each on a SIMD), so a super-block takes a wave the larger of M and M / 2 + 4.5 V cycles, M = 2304
 //     (Q6_K 3072), V = 460 (Q5_K 610, Q6_K 860).  With 64 rows x 32 tokens, the same registers, V was 650 (1250 for Q6_K): us, that form -> this
-//     one, Q6_K 4096 x 11008, 512 tokens 192 -> 163, 11008 x 4096, 1024 tokens 372 -> 309; Q5_K 11008 x 4096, 512 tokens 141 -> 135; Q4_K, which the
-//     power limit holds (1.5-1.6 GHz where both run), 14336 x 4096, 2048 tokens 538 -> 531.  The tokens' LDS reads double: 90 of 128 bytes a cycle.
+//     one, Q6_K 4096 x 11008, 512 tokens 192 -> 163, 11008 x 4096, 1024 tokens 372 -> 309; Q5_K 11008 x 4096, 512 tokens 141 -> 135; Q4_K
+//     14336 x 4096, 2048 tokens 538 -> 531.  The tokens' LDS reads double: 90 of 128 bytes a cycle.
+//   * That accounts for four fifths of the cycles: Q4_K 14336 x 4096, 2048 tokens 722 k of 906 k (matrix cores busy 57 %), Q6_K 4096 x 11008, 512 tokens 232 k of
+//     300 k; what the rest is has not been found.  The clock is not what it lacks: a library's f16 product of as many matrix operations runs at the same 1.7 GHz
+//     and takes 642 k (72 %).
 //   * A workgroup is four waves with a strip of 32 rows each against the same two operand tiles of 32 tokens, two workgroups a CU (70-80 KB of
 //     LDS, 220-240 registers): their phases drift apart, so that one's sums and headers run under the other's products.
 //   * Weights and token pages come by copies into LDS, pages in a ring of three chunks of four products (Q6_K two, its
@@ -19,8 +22,8 @@
 //     super-block's again).  A wave in its products goes first (up to 5 % against equal priorities).
 //   * Rounding.  The hi pieces' sums are kept apart from the lo pieces' (alone they are whole numbers on a coarse grid and
 //     hardly round), what is added to them is hi pieces as well, and the running sum over super-blocks is put by every few
-//     (put_by).  Against fp64 the error is 0.82 .. 0.98 times the 16-token kernel's, over 70 shapes a
-//     format drawn from 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns that the rule gives this kernel.
+//     (put_by).  Against fp64 the error is Q4_K 0.86 .. 1.02 (0.954 on the average), Q5_K 0.81 .. 1.02
+//     (0.946), Q6_K 0.81 .. 0.94 (0.878) times the 16-token kernel's, over 70 shapes a format drawn from 33 .. 2048 tokens, 512 .. 32000 rows, 1024 .. 14336 columns that the rule gives this kernel.
 #pragma once
 #include "kquant_gemm_f16.hip.h"
 #include <utility>

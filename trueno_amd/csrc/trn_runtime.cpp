@@ -1094,8 +1094,9 @@ bool tall_ok(const DeviceKernels& d, Fmt f, uint32_t m, uint32_t n, uint32_t k, 
 // matrix-core forms cannot take).  A forced cut of the f16 form (tuning) takes that form.
 // Up to 48 tokens the kernel that deals super-blocks to its waves takes the product where its estimate is at least 5 % below that of
 // the way it would go otherwise.  Of 256 drawn products of up to 32 tokens 124 are more than 3 % faster with it, 2 slower; all of them
-// together 1.10x.  Its error against fp64 is 0.95-0.98 of the sixteen-token kernel's, 0.93 of the integer cores', 0.8 of the GEMV engine's, except
-// with Q6_K, where the engine's is the smaller one (1.21): those products stay with the engine.  What needed no scratch memory needs none here.
+// together 1.10x.  Its error against fp64 is 0.95-0.98 of the sixteen-token kernel's, 0.93 of the integer cores', 0.82 of the GEMV engine's, except
+// with Q6_K, where the engine's is the smaller one (1.21): those products stay with the engine.  What needed no scratch memory (integer cores, engine) is in one
+// part here, which needs none either.
 enum class GemmRoute { kFew, kCores, kTall, kSlices, kOther };
 GemmRoute gemm_route(const DeviceKernels& d, Fmt f, uint64_t a, uint64_t w, uint64_t c, uint32_t m, uint32_t n, uint32_t k, SlicesCut* slices, TallCut* tall) {
   const bool cores_ok = q4k_gemm_f16_ok(a, w, c, m, n, k, f);
